@@ -544,7 +544,7 @@ pp_status create_impl(int R, const pp_params *prm, const pp_options *opts, const
 			if(!q) return bail(fail(PP_ERR_NOMEM, "a device buffer was not allocated"));
 	}
 
-	// host staging: SoA in particle-index order, slot j = particle j; the
+	// host staging: particles in index order, slot j = particle j; the
 	// free slots of grand-canonical replicas hold no particle (index -1)
 	{
 		std::vector<double> h((size_t) NCOMP * d.stride, 0.);
@@ -554,8 +554,8 @@ pp_status create_impl(int R, const pp_params *prm, const pp_options *opts, const
 			for(int i = 0; i < cap[k]; i++) hr[c->p_off[k] + i] = k;
 			for(int i = 0; i < n[k]; i++, src++) {
 				long long j = c->p_off[k] + i;
-				for(int a = 0; a < 3; a++) h[(size_t) a * d.stride + j] = r[3 * src + a];
-				for(int a = 0; a < 9; a++) h[(size_t) (3 + a) * d.stride + j] = O[9 * src + a];
+				for(int a = 0; a < 3; a++) h[(size_t) NCOMP * j + a] = r[3 * src + a];
+				for(int a = 0; a < 9; a++) h[(size_t) NCOMP * j + 3 + a] = O[9 * src + a];
 				hp[j] = i;
 			}
 		}
@@ -931,19 +931,19 @@ pp_status pp_download(pp_ctx *c, int rep, double *r, double *O, double box[3]) {
 	}
 	TRY(pull_reps(c));
 	const Rep &rp = c->reps[rep];
-	const int n = rp.np, off = rp.p_off, S = c->d.stride;
+	const int n = rp.np, off = rp.p_off;
 	std::vector<double> h((size_t) NCOMP * std::max(n, 1));
 	std::vector<int> hp, sorted;
-	for(int a = 0; a < NCOMP && n; a++)
-		HIPCHECK(hipMemcpy(h.data() + (size_t) a * n, c->d.f[rp.sel] + (size_t) a * S + off, n * sizeof(double),
+	if(n)
+		HIPCHECK(hipMemcpy(h.data(), c->d.f[rp.sel] + (size_t) NCOMP * off, sizeof(double) * NCOMP * n,
 		                   hipMemcpyDeviceToHost));
 	TRY(slot_indices(c, rep, hp, sorted));
 	for(int j = 0; j < n; j++) {
 		const int i = rp.gc ? rank_of(sorted, hp[j]) : hp[j];
 		if(r)
-			for(int a = 0; a < 3; a++) r[3 * i + a] = h[(size_t) a * n + j];
+			for(int a = 0; a < 3; a++) r[3 * i + a] = h[(size_t) NCOMP * j + a];
 		if(O)
-			for(int a = 0; a < 9; a++) O[9 * i + a] = h[(size_t) (3 + a) * n + j];
+			for(int a = 0; a < 9; a++) O[9 * i + a] = h[(size_t) NCOMP * j + 3 + a];
 	}
 	if(box)
 		for(int a = 0; a < 3; a++) box[a] = rp.g.box[a];
@@ -984,19 +984,19 @@ pp_status pp_snapshot_start(pp_ctx *c, int rep) {
 	}
 	TRY(pull_reps(c));
 	const Rep &rp = c->reps[rep];
-	const int n = rp.np, off = rp.p_off, S = c->d.stride, cap = c->snap_cap;
+	const int n = rp.np, off = rp.p_off;
 	// on the sweeps' stream: the slots into the staging area, then the copy
 	// to the host on the snapshot stream once they are there
-	for(int a = 0; a < NCOMP && n; a++)
-		HIPCHECK(hipMemcpyAsync(c->snap_dev + (size_t) a * cap, c->d.f[rp.sel] + (size_t) a * S + off,
-		                        sizeof(double) * n, hipMemcpyDeviceToDevice, c->stream));
-	if(n)
+	if(n) {
+		HIPCHECK(hipMemcpyAsync(c->snap_dev, c->d.f[rp.sel] + (size_t) NCOMP * off, sizeof(double) * NCOMP * n,
+		                        hipMemcpyDeviceToDevice, c->stream));
 		HIPCHECK(hipMemcpyAsync(c->snap_dev_pid, c->d.pid[rp.sel] + off, sizeof(int) * n, hipMemcpyDeviceToDevice,
 		                        c->stream));
+	}
 	HIPCHECK(hipEventRecord(c->snap_ready, c->stream));
 	HIPCHECK(hipStreamWaitEvent(c->copy_stream, c->snap_ready, 0));
 	if(n) {
-		HIPCHECK(hipMemcpyAsync(c->snap_host, c->snap_dev, sizeof(double) * NCOMP * cap, hipMemcpyDeviceToHost,
+		HIPCHECK(hipMemcpyAsync(c->snap_host, c->snap_dev, sizeof(double) * NCOMP * n, hipMemcpyDeviceToHost,
 		                        c->copy_stream));
 		HIPCHECK(hipMemcpyAsync(c->snap_host_pid, c->snap_dev_pid, sizeof(int) * n, hipMemcpyDeviceToHost,
 		                        c->copy_stream));
@@ -1015,7 +1015,7 @@ pp_status pp_snapshot_finish(pp_ctx *c, double *r, double *O, double box[3]) {
 	HIPCHECK(hipSetDevice(c->device));
 	c->snap_pending = false;
 	HIPCHECK(hipEventSynchronize(c->snap_done));
-	const int n = c->snap_n, cap = c->snap_cap;
+	const int n = c->snap_n;
 	std::vector<int> sorted(c->snap_host_pid, c->snap_host_pid + n);
 	std::sort(sorted.begin(), sorted.end());
 	for(int i = 0; i < n; i++)
@@ -1025,9 +1025,9 @@ pp_status pp_snapshot_finish(pp_ctx *c, double *r, double *O, double box[3]) {
 		const int id = c->snap_host_pid[j];
 		const int i = c->snap_gc ? rank_of(sorted, id) : id;
 		if(r)
-			for(int a = 0; a < 3; a++) r[3 * i + a] = c->snap_host[(size_t) a * cap + j];
+			for(int a = 0; a < 3; a++) r[3 * i + a] = c->snap_host[(size_t) NCOMP * j + a];
 		if(O)
-			for(int a = 0; a < 9; a++) O[9 * i + a] = c->snap_host[(size_t) (3 + a) * cap + j];
+			for(int a = 0; a < 9; a++) O[9 * i + a] = c->snap_host[(size_t) NCOMP * j + 3 + a];
 	}
 	if(box)
 		for(int a = 0; a < 3; a++) box[a] = c->snap_box[a];
@@ -1046,7 +1046,7 @@ pp_status upload_impl(pp_ctx *c, int rep, int n, const double *r, const double *
 	Rep &rp = c->reps[rep];
 	if(n != rp.np && !(rp.gc && n >= 0 && n <= rp.cap_np))
 		return fail(PP_ERR_ARG, "replica %d holds %d particles, not %d", rep, rp.np, n);
-	const int off = rp.p_off, S = c->d.stride;
+	const int off = rp.p_off;
 	if(n && (!r || !O)) return fail(PP_ERR_ARG, "positions/orientations are NULL");
 	if(rp.gc) {
 		// the replica's other slots are free
@@ -1072,12 +1072,12 @@ pp_status upload_impl(pp_ctx *c, int rep, int n, const double *r, const double *
 	std::vector<double> h((size_t) NCOMP * std::max(n, 1));
 	std::vector<int> hp(std::max(n, 1));
 	for(int i = 0; i < n; i++) {
-		for(int a = 0; a < 3; a++) h[(size_t) a * n + i] = r[3 * i + a];
-		for(int a = 0; a < 9; a++) h[(size_t) (3 + a) * n + i] = O[9 * i + a];
+		for(int a = 0; a < 3; a++) h[(size_t) NCOMP * i + a] = r[3 * i + a];
+		for(int a = 0; a < 9; a++) h[(size_t) NCOMP * i + 3 + a] = O[9 * i + a];
 		hp[i] = i;
 	}
-	for(int a = 0; a < NCOMP && n; a++)
-		HIPCHECK(hipMemcpy(c->d.f[rp.sel] + (size_t) a * S + off, h.data() + (size_t) a * n, n * sizeof(double),
+	if(n)
+		HIPCHECK(hipMemcpy(c->d.f[rp.sel] + (size_t) NCOMP * off, h.data(), sizeof(double) * NCOMP * n,
 		                   hipMemcpyHostToDevice));
 	if(n) HIPCHECK(hipMemcpy(c->d.pid[rp.sel] + off, hp.data(), n * sizeof(int), hipMemcpyHostToDevice));
 	TRY(push_reps(c));

@@ -196,9 +196,9 @@ __host__ __device__ inline void set_grid_box(Grid &G, const double box[3]) {
 
 // Device buffers of a context.
 struct DevState {
-	double *f[2];        // SoA particle data, component c of slot j at f[b][c*stride + j]
+	double *f[2];        // particle data, component c of slot j at f[b][NCOMP * j + c]
 	int *pid[2];         // particle index of slot j
-	int stride;
+	int stride;          // slots allocated
 	int Ntot;
 	int R;
 	Rep *reps;

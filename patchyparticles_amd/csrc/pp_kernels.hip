@@ -1,8 +1,8 @@
 // pp_kernels.hip -- gfx950 kernels of the Kern-Frenkel rototranslation hot path.
 //
 // Data layout in HBM (per context, all replicas concatenated):
-//   f[2][12][stride]  double  x, y, z, O00..O22 of slot j (SoA, two buffers)
-//   pid[2][stride]    int     particle index of slot j
+//   f[2][slots][12]   double  x, y, z, O00..O22 of slot j (two buffers)
+//   pid[2][slots]     int     particle index of slot j
 //   start[C+1]        int     first slot of each cell, over the concatenated
 //                             cell regions of all replicas (one region per
 //                             replica, sized for its largest grid)
@@ -144,8 +144,7 @@ __global__ void k_count(DevState d, int mode, uint64_t sweep, long long trace_po
 	int c = rp.cell_off + rp.cell_cap;
 	if(j - rp.p_off < rp.np_hw && pick_buf(d.pid, rp.sel)[j] >= 0) {
 		const double *F = pick_buf(d.f, rp.sel);
-		const int S = d.stride;
-		double p[3] = {F[j], F[S + j], F[2 * S + j]};
+		double p[3] = {part(F, j)[0], part(F, j)[1], part(F, j)[2]};
 		if(tr)
 			for(int k = 0; k < 3; k++) p[k] *= rp.trial_s[k];
 		int ix = cell_coord(p[0], sh[0], G.inv_box[0], G.n[0]);
@@ -492,7 +491,6 @@ __global__ void k_scatter(DevState d, int mode, uint64_t sweep) {
 	double v[NCOMP];
 	double *G = nullptr;
 	int *PG = nullptr;
-	const int S = d.stride;
 	if(j < d.Ntot) {
 		r = ONE ? 0 : d.prep[j];
 		const Rep &rp = d.reps[r];
@@ -508,7 +506,7 @@ __global__ void k_scatter(DevState d, int mode, uint64_t sweep) {
 			dst = d.start[d.cellid[j]] + d.slot[j];
 #pragma unroll
 			for(int c = 0; c < NCOMP; c++) {
-				v[c] = F[c * S + j];
+				v[c] = part(F, j)[c];
 				if(tr && c < 3) v[c] *= rp.trial_s[c];
 			}
 			pid = pick_buf(d.pid, sb)[j];
@@ -517,7 +515,7 @@ __global__ void k_scatter(DevState d, int mode, uint64_t sweep) {
 	if(mode == REB_SHIFT && j < d.C_total) build_record<ONE>(d, j);
 	if(!mv) return;
 #pragma unroll
-	for(int c = 0; c < NCOMP; c++) G[c * S + dst] = v[c];
+	for(int c = 0; c < NCOMP; c++) part(G, dst)[c] = v[c];
 	PG[dst] = pid;
 	if(hw) d.reps[r].np_hw = d.reps[r].np;
 }
@@ -757,7 +755,6 @@ __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int
 	// component c of neighbour u at (9 u + c) * T + lane
 	constexpr bool REG_ORI = (ONE || T == 64) && (CPL == 1 || REACH);
 	double *ori = blk + L::FIXED;
-	const int S = d.stride;
 	{
 		// 1. the cell's record: surrounding slot ranges, own range, replica
 		const int4 *rec = (const int4 *) (d.rec + ((size_t) pass * d.total_act + gi) * REC_W);
@@ -797,7 +794,7 @@ __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int
 		if(lane < cnt) {
 			my_pid = PID[s0 + lane];
 #pragma unroll
-			for(int c = 0; c < NCOMP; c++) mine[c] = F[c * S + s0 + lane];
+			for(int c = 0; c < NCOMP; c++) mine[c] = part(F, s0 + lane)[c];
 		}
 		// trials of the cell in this pass: one per member (a sweep is then N
 		// attempts), or a fixed number per non-empty cell
@@ -830,15 +827,15 @@ __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int
 				if(i >= 0 && i < M) {
 					const int q = nb_slot(i);
 					cqr[u] = q;
-					cxr[u] = nbld<DD>(F + q);
-					cyr[u] = nbld<DD>(F + S + q);
-					czr[u] = nbld<DD>(F + 2 * S + q);
+					cxr[u] = nbld<DD>(part(F, q));
+					cyr[u] = nbld<DD>(part(F, q) + 1);
+					czr[u] = nbld<DD>(part(F, q) + 2);
 				}
 			}
 #pragma unroll
 			for(int u = 0; u < CPL; u++)
 #pragma unroll
-				for(int c = 0; c < 9; c++) orv[u][c] = cqr[u] >= 0 ? nbld<DD>(F + (3 + c) * S + cqr[u]) : 0.;
+				for(int c = 0; c < 9; c++) orv[u][c] = cqr[u] >= 0 ? nbld<DD>(part(F, cqr[u]) + 3 + c) : 0.;
 		};
 		if constexpr(!DD) load_static();
 		Trial tr;
@@ -1018,9 +1015,9 @@ __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int
 				for(int b = T * CPL - cnt; b < M; b += T)
 					if(b + lane < M) {
 						const int q = nb_slot(b + lane);
-						f(nbld<DD>(F + q), nbld<DD>(F + S + q), nbld<DD>(F + 2 * S + q), [&](double *Oq) {
+						f(nbld<DD>(part(F, q)), nbld<DD>(part(F, q) + 1), nbld<DD>(part(F, q) + 2), [&](double *Oq) {
 #pragma unroll
-							for(int c = 0; c < 9; c++) Oq[c] = nbld<DD>(F + (3 + c) * S + q);
+							for(int c = 0; c < 9; c++) Oq[c] = nbld<DD>(part(F, q) + 3 + c);
 						});
 					}
 		};
@@ -1252,7 +1249,7 @@ __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int
 				for(int b = T * CPL - cnt; b < M; b += T)
 					if(b + lane < M) {
 						const int q = nb_slot(b + lane);
-						ov |= overlaps_new(tr, nbld<DD>(F + q), nbld<DD>(F + S + q), nbld<DD>(F + 2 * S + q));
+						ov |= overlaps_new(tr, nbld<DD>(part(F, q)), nbld<DD>(part(F, q) + 1), nbld<DD>(part(F, q) + 2));
 					}
 			if(team_any<T>(ov)) continue;
 
@@ -1400,9 +1397,9 @@ __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int
 			for(int e = lane; e < cnt * NCOMP; e += T) {
 				int m = e / NCOMP, c = e - m * NCOMP;
 				if constexpr(DD)
-					__hip_atomic_store(F + c * S + s0 + m, own[m * OWN_W + c], __ATOMIC_RELAXED,
+					__hip_atomic_store(part(F, s0 + m) + c, own[m * OWN_W + c], __ATOMIC_RELAXED,
 					                   __HIP_MEMORY_SCOPE_AGENT);
-				else F[c * S + s0 + m] = own[m * OWN_W + c];
+				else part(F, s0 + m)[c] = own[m * OWN_W + c];
 			}
 			if(lane < cnt) {
 				int rank = 0;
@@ -1744,11 +1741,10 @@ __global__ __launch_bounds__(256) void k_energy(DevState d, int trial, int per_p
 	const double s0 = fast ? rp.trial_s[0] : 1., s1 = fast ? rp.trial_s[1] : 1., s2 = fast ? rp.trial_s[2] : 1.;
 	const int b = (tr && !fast) ? (rp.sel ^ 1) : rp.sel;
 	const double *F = pick_buf(d.f, b);
-	const int S = d.stride;
-	const double ux = F[j], uy = F[S + j], uz = F[2 * S + j];
+	const double ux = part(F, j)[0], uy = part(F, j)[1], uz = part(F, j)[2];
 	double O[9];
 #pragma unroll
-	for(int c = 0; c < 9; c++) O[c] = F[(3 + c) * S + j];
+	for(int c = 0; c < 9; c++) O[c] = part(F, j)[3 + c];
 	double P[4][3];
 	kf_patches(O, P);
 	const int n0 = G.n[0], n1 = G.n[1], n2 = G.n[2];
@@ -1771,15 +1767,15 @@ __global__ __launch_bounds__(256) void k_energy(DevState d, int trial, int per_p
 		int s = d.start[cc], e = d.start[cc + 1];
 		for(int q = s + lane % NB::S; q < e; q += NB::S) {
 			if(q == j) continue;
-			double dx = kf_min_image(F[q] * s0 - px, Lx, iLx);
-			double dy = kf_min_image(F[S + q] * s1 - py, Ly, iLy);
-			double dz = kf_min_image(F[2 * S + q] * s2 - pz, Lz, iLz);
+			double dx = kf_min_image(part(F, q)[0] * s0 - px, Lx, iLx);
+			double dy = kf_min_image(part(F, q)[1] * s1 - py, Ly, iLy);
+			double dz = kf_min_image(part(F, q)[2] * s2 - pz, Lz, iLz);
 			double d2 = dx * dx + dy * dy + dz * dz;
 			if(d2 < 1.) ov = true;
 			else if(d2 < rp.rc2)
 				nbond += (int) pair_bonded(dx, dy, dz, d2, &P[0][0], c2, rp.cosmax, [&](double *Oq) {
 #pragma unroll
-					for(int c = 0; c < 9; c++) Oq[c] = F[(3 + c) * S + q];
+					for(int c = 0; c < 9; c++) Oq[c] = part(F, q)[3 + c];
 				});
 		}
 	}
@@ -1813,10 +1809,9 @@ __global__ void k_bond_list(DevState d, int max_per, int *count, int *partners) 
 	const Grid &G = rp.g;
 	const double *F = pick_buf(d.f, rp.sel);
 	const int *PID = pick_buf(d.pid, rp.sel);
-	const int S = d.stride;
-	const double px = F[j], py = F[S + j], pz = F[2 * S + j];
+	const double px = part(F, j)[0], py = part(F, j)[1], pz = part(F, j)[2];
 	double O[9];
-	for(int c = 0; c < 9; c++) O[c] = F[(3 + c) * S + j];
+	for(int c = 0; c < 9; c++) O[c] = part(F, j)[3 + c];
 	double P[4][3];
 	kf_patches(O, P);
 	const int n0 = G.n[0], n1 = G.n[1], n2 = G.n[2];
@@ -1830,15 +1825,15 @@ __global__ void k_bond_list(DevState d, int max_per, int *count, int *partners) 
 		const int cc = rp.cell_off + (cx * n1 + cy) * n2 + cz;
 		for(int q = d.start[cc]; q < d.start[cc + 1]; q++) {
 			if(q == j) continue;
-			double dx = kf_min_image(F[q] - px, G.box[0], G.inv_box[0]);
-			double dy = kf_min_image(F[S + q] - py, G.box[1], G.inv_box[1]);
-			double dz = kf_min_image(F[2 * S + q] - pz, G.box[2], G.inv_box[2]);
+			double dx = kf_min_image(part(F, q)[0] - px, G.box[0], G.inv_box[0]);
+			double dy = kf_min_image(part(F, q)[1] - py, G.box[1], G.inv_box[1]);
+			double dz = kf_min_image(part(F, q)[2] - pz, G.box[2], G.inv_box[2]);
 			const double d2 = dx * dx + dy * dy + dz * dz;
 			if(d2 < 1. || !(d2 < rp.rc2)) continue;
 			kf_unit(dx, dy, dz, d2);
 			if(!kf_any_p(dx, dy, dz, &P[0][0], rp.cosmax)) continue;
 			double Oq[9];
-			for(int e = 0; e < 9; e++) Oq[e] = F[(3 + e) * S + q];
+			for(int e = 0; e < 9; e++) Oq[e] = part(F, q)[3 + e];
 			if(!kf_any_q(dx, dy, dz, Oq, rp.cosmax)) continue;
 			if(nb < max_per) partners[me * max_per + nb] = PID[q];
 			nb++;
@@ -1909,7 +1904,6 @@ __global__ __launch_bounds__(256) void k_energy_rec(DevState d) {
 		const int s0 = rec[59], cnt = rec[60];
 		const int m0 = rec[32 + 13], m2 = rec[58] - m0;  // candidates in the 13 directions
 		const double *F = pick_buf(d.f, rec[63]);
-		const int S = d.stride;
 		const double t0 = rp.trial_s[0], t1 = rp.trial_s[1], t2 = rp.trial_s[2];
 		const double Lx = rp.tg.box[0], Ly = rp.tg.box[1], Lz = rp.tg.box[2];
 		const double iLx = rp.tg.inv_box[0], iLy = rp.tg.inv_box[1], iLz = rp.tg.inv_box[2];
@@ -1931,20 +1925,20 @@ __global__ __launch_bounds__(256) void k_energy_rec(DevState d) {
 				j = s0 + a;
 				q = s0 + b2;
 			}
-			const double px = F[j] * t0, py = F[S + j] * t1, pz = F[2 * S + j] * t2;
-			const double dx = kf_min_image(F[q] * t0 - px, Lx, iLx);
-			const double dy = kf_min_image(F[S + q] * t1 - py, Ly, iLy);
-			const double dz = kf_min_image(F[2 * S + q] * t2 - pz, Lz, iLz);
+			const double px = part(F, j)[0] * t0, py = part(F, j)[1] * t1, pz = part(F, j)[2] * t2;
+			const double dx = kf_min_image(part(F, q)[0] * t0 - px, Lx, iLx);
+			const double dy = kf_min_image(part(F, q)[1] * t1 - py, Ly, iLy);
+			const double dz = kf_min_image(part(F, q)[2] * t2 - pz, Lz, iLz);
 			const double d2 = dx * dx + dy * dy + dz * dz;
 			if(d2 < 1.) novl++;
 			else if(d2 < rp.rc2) {
 				double O[9], P[4][3];
 #pragma unroll
-				for(int c = 0; c < 9; c++) O[c] = F[(3 + c) * S + j];
+				for(int c = 0; c < 9; c++) O[c] = part(F, j)[3 + c];
 				kf_patches(O, P);
 				nbond += (int) pair_bonded(dx, dy, dz, d2, &P[0][0], c2, rp.cosmax, [&](double *Oq) {
 #pragma unroll
-					for(int c = 0; c < 9; c++) Oq[c] = F[(3 + c) * S + q];
+					for(int c = 0; c < 9; c++) Oq[c] = part(F, q)[3 + c];
 				});
 			}
 		}
@@ -2061,11 +2055,10 @@ __global__ __launch_bounds__(256) void k_pairs_build(DevState d) {
 				rl2 = rp.rc2 * (PAIR_LIST_FACTOR * PAIR_LIST_FACTOR);
 			}
 		}
-		const int S = d.stride;
 		auto close = [&](int j, int q) {
-			const double dx = kf_min_image(F[q] - F[j], L[0], iL[0]);
-			const double dy = kf_min_image(F[S + q] - F[S + j], L[1], iL[1]);
-			const double dz = kf_min_image(F[2 * S + q] - F[2 * S + j], L[2], iL[2]);
+			const double dx = kf_min_image(part(F, q)[0] - part(F, j)[0], L[0], iL[0]);
+			const double dy = kf_min_image(part(F, q)[1] - part(F, j)[1], L[1], iL[1]);
+			const double dz = kf_min_image(part(F, q)[2] - part(F, j)[2], L[2], iL[2]);
 			return dx * dx + dy * dy + dz * dz < rl2;
 		};
 		const int work = on ? cnt * m2 + cnt * cnt : 0;
@@ -2116,12 +2109,11 @@ __global__ __launch_bounds__(256) void k_energy_pairs(DevState d) {
 		// (the early exit may read a stale flag: it only saves work)
 		if(__hip_atomic_load(&d.vflag[r], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) continue;
 		const double *F = pick_buf(d.f, rp.sel);
-		const int S = d.stride;
 		const double t0 = rp.trial_s[0], t1 = rp.trial_s[1], t2 = rp.trial_s[2];
-		const double px = F[j] * t0, py = F[S + j] * t1, pz = F[2 * S + j] * t2;
-		const double dx = kf_min_image(F[q] * t0 - px, rp.tg.box[0], rp.tg.inv_box[0]);
-		const double dy = kf_min_image(F[S + q] * t1 - py, rp.tg.box[1], rp.tg.inv_box[1]);
-		const double dz = kf_min_image(F[2 * S + q] * t2 - pz, rp.tg.box[2], rp.tg.inv_box[2]);
+		const double px = part(F, j)[0] * t0, py = part(F, j)[1] * t1, pz = part(F, j)[2] * t2;
+		const double dx = kf_min_image(part(F, q)[0] * t0 - px, rp.tg.box[0], rp.tg.inv_box[0]);
+		const double dy = kf_min_image(part(F, q)[1] * t1 - py, rp.tg.box[1], rp.tg.inv_box[1]);
+		const double dz = kf_min_image(part(F, q)[2] * t2 - pz, rp.tg.box[2], rp.tg.inv_box[2]);
 		const double d2 = dx * dx + dy * dy + dz * dz;
 		const int slot = k & (NSLOT - 1);
 		if(d2 < 1.) {
@@ -2132,11 +2124,11 @@ __global__ __launch_bounds__(256) void k_energy_pairs(DevState d) {
 			const double c2 = rp.cosmax >= KF_FILTER_MIN_COS ? rp.cosmax * rp.cosmax : -1.;
 			double O[9], P[4][3];
 #pragma unroll
-			for(int c = 0; c < 9; c++) O[c] = F[(3 + c) * S + j];
+			for(int c = 0; c < 9; c++) O[c] = part(F, j)[3 + c];
 			kf_patches(O, P);
 			if(pair_bonded(dx, dy, dz, d2, &P[0][0], c2, rp.cosmax, [&](double *Oq) {
 #pragma unroll
-				   for(int c = 0; c < 9; c++) Oq[c] = F[(3 + c) * S + q];
+				   for(int c = 0; c < 9; c++) Oq[c] = part(F, q)[3 + c];
 			   }))
 				atomicAdd(ctr_at(d.ctr, r, C_EBONDS, slot), 2ull);
 		}
@@ -2173,8 +2165,7 @@ __global__ void k_colour_conflicts(DevState d, int rep, int n0, int n1, int n2, 
 	const int *PID = pick_buf(d.pid, rp.sel);
 	if(PID[j] < 0) return;
 	const double *F = pick_buf(d.f, rp.sel);
-	const int S = d.stride;
-	const double x = F[j], y = F[S + j], z = F[2 * S + j];
+	const double x = part(F, j)[0], y = part(F, j)[1], z = part(F, j)[2];
 	auto cell = [&](double a, double b, double c, int &cx, int &cy, int &cz) {
 		cx = cell_coord(a, G.shift[0], G.inv_box[0], G.n[0]);
 		cy = cell_coord(b, G.shift[1], G.inv_box[1], G.n[1]);
@@ -2187,7 +2178,7 @@ __global__ void k_colour_conflicts(DevState d, int rep, int n0, int n1, int n2, 
 	for(int k = 0; k < rp.np_hw && !hit; k++) {
 		const int q = rp.p_off + k;
 		if(q == j || PID[q] < 0) continue;
-		const double qx = F[q], qy = F[S + q], qz = F[2 * S + q];
+		const double qx = part(F, q)[0], qy = part(F, q)[1], qz = part(F, q)[2];
 		int cx, cy, cz;
 		cell(qx, qy, qz, cx, cy, cz);
 		if((((cx & 1) << 2) | ((cy & 1) << 1) | (cz & 1)) != col || (cx == ix && cy == iy && cz == iz)) continue;
@@ -2421,8 +2412,7 @@ __global__ void k_vol_apply(DevState d) {
 	const Rep &rp = d.reps[d.prep[j]];
 	if(!rp.vol_apply) return;
 	double *F = pick_buf(d.f, rp.sel);
-	const int S = d.stride;
-	for(int c = 0; c < 3; c++) F[(size_t) c * S + j] *= rp.trial_s[c];
+	for(int c = 0; c < 3; c++) part(F, j)[c] *= rp.trial_s[c];
 }
 
 void launch_vol_apply(const DevState &d, hipStream_t s) {
@@ -2503,7 +2493,7 @@ template <int T>
 __device__ inline int gc_bonds(const DevState &d, const Rep &rp, const double *F, int ix, int iy, int iz,
                                const double p[3], const double P[4][3], int skip, int lane, bool &any) {
 	const Grid &G = rp.g;
-	const int S = d.stride, n0 = G.n[0], n1 = G.n[1], n2 = G.n[2];
+	const int n0 = G.n[0], n1 = G.n[1], n2 = G.n[2];
 	int nb_ = 0;
 	bool ov = false;
 	for(int nb = lane; nb < 27; nb += T) {
@@ -2511,16 +2501,16 @@ __device__ inline int gc_bonds(const DevState &d, const Rep &rp, const double *F
 		const int cc = rp.cell_off + (cx * n1 + cy) * n2 + cz;
 		for(int q = d.start[cc]; q < d.start[cc + 1]; q++) {
 			if(q == skip) continue;
-			double dx = kf_min_image(F[q] - p[0], G.box[0], G.inv_box[0]);
-			double dy = kf_min_image(F[S + q] - p[1], G.box[1], G.inv_box[1]);
-			double dz = kf_min_image(F[2 * S + q] - p[2], G.box[2], G.inv_box[2]);
+			double dx = kf_min_image(part(F, q)[0] - p[0], G.box[0], G.inv_box[0]);
+			double dy = kf_min_image(part(F, q)[1] - p[1], G.box[1], G.inv_box[1]);
+			double dz = kf_min_image(part(F, q)[2] - p[2], G.box[2], G.inv_box[2]);
 			const double d2 = dx * dx + dy * dy + dz * dz;
 			if(d2 < 1.) ov = true;
 			else if(d2 < rp.rc2) {
 				kf_unit(dx, dy, dz, d2);
 				if(kf_any_p(dx, dy, dz, &P[0][0], rp.cosmax)) {
 					double Oq[9];
-					for(int c = 0; c < 9; c++) Oq[c] = F[(3 + c) * S + q];
+					for(int c = 0; c < 9; c++) Oq[c] = part(F, q)[3 + c];
 					nb_ += kf_any_q(dx, dy, dz, Oq, rp.cosmax);
 				}
 			}
@@ -2558,7 +2548,6 @@ __global__ __launch_bounds__(256) void k_gc_pass(DevState d, uint64_t sweep) {
 	const int s0 = d.start[c], cnt = d.start[c + 1] - s0;
 	double *F = pick_buf(d.f, rp.sel);
 	int *PID = pick_buf(d.pid, rp.sel);
-	const int S = d.stride;
 	const u32x4 u = rng(d.seed, r, sweep, (uint32_t) cloc, TAG_GC, (uint32_t) col, 1);
 	const u32x4 w = rng(d.seed, r, sweep, (uint32_t) cloc, TAG_GC, (uint32_t) col, 2);
 	const double vc = (rp.g.box[0] / n0) * (rp.g.box[1] / n1) * (rp.g.box[2] / n2);
@@ -2586,8 +2575,8 @@ __global__ __launch_bounds__(256) void k_gc_pass(DevState d, uint64_t sweep) {
 		const double acc = exp((double) b / rp.T) * rp.activity * vc / (double) (cnt + 1);
 		if(!inside || ov || !(u01(w.x) < acc)) return;
 		const int slot = rp.p_off + rp.gc_base + k;
-		for(int a = 0; a < 3; a++) F[(size_t) a * S + slot] = p[a];
-		for(int a = 0; a < 9; a++) F[(size_t) (3 + a) * S + slot] = O[a];
+		for(int a = 0; a < 3; a++) part(F, slot)[a] = p[a];
+		for(int a = 0; a < 9; a++) part(F, slot)[3 + a] = O[a];
 		PID[slot] = rp.gc_base + k;
 		atomicAdd(&d.reps[r].np, 1);
 		atomicAdd(ctr_at(d.ctr, r, C_ACC_ADD, cslot), 1ull);
@@ -2600,9 +2589,9 @@ __global__ __launch_bounds__(256) void k_gc_pass(DevState d, uint64_t sweep) {
 		}
 		// members sit in order of particle index: rank m is slot s0 + m
 		const int q = s0 + (int) __umulhi(u.y, (uint32_t) cnt);
-		const double p[3] = {F[q], F[S + q], F[2 * S + q]};
+		const double p[3] = {part(F, q)[0], part(F, q)[1], part(F, q)[2]};
 		double O[9], P[4][3];
-		for(int a = 0; a < 9; a++) O[a] = F[(size_t) (3 + a) * S + q];
+		for(int a = 0; a < 9; a++) O[a] = part(F, q)[3 + a];
 		kf_patches(O, P);
 		bool ov = false;
 		const int b = gc_bonds<T>(d, rp, F, ix, iy, iz, p, P, q, lane, ov);
@@ -2633,13 +2622,12 @@ __global__ void k_gram_schmidt(DevState d) {
 	const Rep &rp = d.reps[d.prep[j]];
 	if(j - rp.p_off >= rp.np) return;
 	double *F = pick_buf(d.f, rp.sel);
-	const int S = d.stride;
 	double O[9];
 #pragma unroll
-	for(int c = 0; c < 9; c++) O[c] = F[(3 + c) * S + j];
+	for(int c = 0; c < 9; c++) O[c] = part(F, j)[3 + c];
 	gram_schmidt_rows(O);
 #pragma unroll
-	for(int c = 0; c < 9; c++) F[(3 + c) * S + j] = O[c];
+	for(int c = 0; c < 9; c++) part(F, j)[3 + c] = O[c];
 }
 
 void launch_gram_schmidt(const DevState &d, hipStream_t s) {

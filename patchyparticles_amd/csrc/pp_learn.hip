@@ -558,7 +558,6 @@ struct CandLds {
 // the other members of the cell
 struct Cands {
 	const double *F;
-	int S;
 	CellView v;
 	int j;
 	const CandLds *L = nullptr;  // staged slots / positions (filled by stage())
@@ -577,7 +576,7 @@ struct Cands {
 			return;
 		}
 		const int s = slot_of(i);
-		for(int k = 0; k < 3; k++) q[k] = F[(size_t) k * S + s];
+		for(int k = 0; k < 3; k++) q[k] = part(F, s)[k];
 	}
 	// lane-strided: candidate i is staged by lane i % T of the team, the
 	// lane that reads it first (desc_collect, the energy loop)
@@ -586,14 +585,14 @@ struct Cands {
 		for(int i = tl; i < count() && i < CAND_MAX; i += T) {
 			const int s = slot_of(i);
 			W.slot[i] = s;
-			W.x[i] = F[s];
-			W.y[i] = F[(size_t) S + s];
-			W.z[i] = F[(size_t) 2 * S + s];
+			W.x[i] = part(F, s)[0];
+			W.y[i] = part(F, s)[1];
+			W.z[i] = part(F, s)[2];
 		}
 	}
 	__device__ void ori(int i, double O[9]) const {
 		const int s = slot(i);
-		for(int k = 0; k < 9; k++) O[k] = F[(size_t) (3 + k) * S + s];
+		for(int k = 0; k < 9; k++) O[k] = part(F, s)[3 + k];
 	}
 };
 
@@ -661,7 +660,6 @@ __global__ __launch_bounds__(64 * LP_WAVES) void k_learn_pass(DevState d, NetDev
 	bool live = gi < count;
 	CellView v{};
 	const double *F = nullptr;
-	const int SS = d.stride;
 	int j = 0, nv = 0;
 	__bf16 *row = S.x + cell * ACT_LD;
 	DescLds &D = S.desc[cell];
@@ -700,10 +698,10 @@ __global__ __launch_bounds__(64 * LP_WAVES) void k_learn_pass(DevState d, NetDev
 		}
 		const unsigned long long hm = (__ballot(hit) >> (lane & ~(T - 1))) & ((1ull << T) - 1ull);
 		j = v.s0 + (int) __builtin_ctzll(hm);
-		const Cands c{F, SS, v, j, &CL};
+		const Cands c{F, v, j, &CL};
 		c.stage<T>(CL, tl);
 		double p[3];
-		for(int k = 0; k < 3; k++) p[k] = F[(size_t) k * SS + j];
+		for(int k = 0; k < 3; k++) p[k] = part(F, j)[k];
 		nv = desc_collect<T>(p, c.count(), [&](int i, double q[3]) { c.pos(i, q); }, L, iL, D, row, tl);
 	}
 	else
@@ -713,10 +711,10 @@ __global__ __launch_bounds__(64 * LP_WAVES) void k_learn_pass(DevState d, NetDev
 		}
 	__syncthreads();
 	if(live) {
-		const Cands c{F, SS, v, j, &CL};
+		const Cands c{F, v, j, &CL};
 		double p[3], O[9];
-		for(int k = 0; k < 3; k++) p[k] = F[(size_t) k * SS + j];
-		for(int k = 0; k < 9; k++) O[k] = F[(size_t) (3 + k) * SS + j];
+		for(int k = 0; k < 3; k++) p[k] = part(F, j)[k];
+		for(int k = 0; k < 9; k++) O[k] = part(F, j)[3 + k];
 		desc_fill<T>(
 			p, O, nv, [&](int i, double q[3]) { c.pos(i, q); }, [&](int i, double Oq[9]) { c.ori(i, Oq); }, L, iL, D, row,
 			tl);
@@ -759,8 +757,8 @@ __global__ __launch_bounds__(64 * LP_WAVES) void k_learn_pass(DevState d, NetDev
 		vmf_sample(dir, kap, u01f(rb.y), u01f(rb.z), axf);
 		const double ang = u01(rb.w) * d.learn.theta_max;
 		double p[3], O[9];
-		for(int k = 0; k < 3; k++) p[k] = F[(size_t) k * SS + j];
-		for(int k = 0; k < 9; k++) O[k] = F[(size_t) (3 + k) * SS + j];
+		for(int k = 0; k < 3; k++) p[k] = part(F, j)[k];
+		for(int k = 0; k < 9; k++) O[k] = part(F, j)[3 + k];
 		// body -> lab: O^T d; O' = O R(a, angle) (utils.c:186-209)
 		double np[3];
 		for(int k = 0; k < 3; k++) np[k] = p[k] + (O[k] * dbody[0] + O[3 + k] * dbody[1] + O[6 + k] * dbody[2]);
@@ -782,13 +780,13 @@ __global__ __launch_bounds__(64 * LP_WAVES) void k_learn_pass(DevState d, NetDev
 		         cell_coord(np[1], rp.g.shift[1], rp.g.inv_box[1], n1) == iy &&
 		         cell_coord(np[2], rp.g.shift[2], rp.g.inv_box[2], n2) == iz;
 		if(inside) {
-			const Cands c{F, SS, v, j, &CL};
+			const Cands c{F, v, j, &CL};
 			nv = desc_collect<T>(np, c.count(), [&](int i, double q[3]) { c.pos(i, q); }, L, iL, D, row, tl);
 		}
 	}
 	__syncthreads();
 	if(live && inside) {
-		const Cands c{F, SS, v, j, &CL};
+		const Cands c{F, v, j, &CL};
 		const double *pp = S.prop[cell];
 		double np[3], On[9];
 		for(int k = 0; k < 3; k++) np[k] = pp[k];
@@ -812,8 +810,8 @@ __global__ __launch_bounds__(64 * LP_WAVES) void k_learn_pass(DevState d, NetDev
 	double *Fw = pick_buf(d.f, v.sel);
 	const double *pp = S.prop[cell];
 	double p[3], O[9], np[3], On[9];
-	for(int k = 0; k < 3; k++) p[k] = Fw[(size_t) k * SS + j];
-	for(int k = 0; k < 9; k++) O[k] = Fw[(size_t) (3 + k) * SS + j];
+	for(int k = 0; k < 3; k++) p[k] = part(Fw, j)[k];
+	for(int k = 0; k < 9; k++) O[k] = part(Fw, j)[3 + k];
 	for(int k = 0; k < 3; k++) np[k] = pp[k];
 	for(int k = 0; k < 9; k++) On[k] = pp[3 + k];
 	// reverse: displacement p - p' in the body frame of O', axis -a
@@ -845,7 +843,7 @@ __global__ __launch_bounds__(64 * LP_WAVES) void k_learn_pass(DevState d, NetDev
 	double Po[4][3], Pn[4][3];
 	kf_patches(O, Po);
 	kf_patches(On, Pn);
-	const Cands c{Fw, SS, v, j, &CL};
+	const Cands c{Fw, v, j, &CL};
 	const int n = c.count();
 	int bo = 0, bn = 0;
 	bool ov = false;
@@ -866,8 +864,8 @@ __global__ __launch_bounds__(64 * LP_WAVES) void k_learn_pass(DevState d, NetDev
 	const u32x4 rc = rng(d.seed, v.r, sweep, (uint32_t) v.cloc, TAG_LEARN_B, (uint32_t) pass, 1);
 	const double la = -dE / rp.T + log_ratio;
 	if(la >= 0. || u01(rc.x) < exp(la)) {
-		for(int k = 0; k < 3; k++) Fw[(size_t) k * SS + j] = np[k];
-		for(int k = 0; k < 9; k++) Fw[(size_t) (3 + k) * SS + j] = On[k];
+		for(int k = 0; k < 3; k++) part(Fw, j)[k] = np[k];
+		for(int k = 0; k < 9; k++) part(Fw, j)[3 + k] = On[k];
 		atomicAdd(ctr_at(d.ctr, v.r, C_ACC_ROTO, cslot), 1ull);
 		atomicAdd(ctr_at(d.ctr, v.r, C_ACC_LEARN, cslot), 1ull);
 		if(db) atomicAdd(ctr_at(d.ctr, v.r, C_DBONDS, cslot), (unsigned long long) (long long) db);
@@ -930,7 +928,6 @@ __global__ __launch_bounds__(64 * TS_WAVES) void k_train_samples(DevState d, uin
 	// the slot's cell neighbourhood (27 cells, the particle itself left out)
 	int st[27], cn[27], self = -1, j = 0, tot = 0;
 	const double *F = nullptr;
-	const int S = d.stride;
 	double L[3], iL[3];
 	auto slot_of = [&](int i) {
 		if(self >= 0 && i >= self) i++;
@@ -943,11 +940,11 @@ __global__ __launch_bounds__(64 * TS_WAVES) void k_train_samples(DevState d, uin
 	};
 	auto pos = [&](int i, double q[3]) {
 		const int s2 = slot_of(i);
-		for(int k = 0; k < 3; k++) q[k] = F[(size_t) k * S + s2];
+		for(int k = 0; k < 3; k++) q[k] = part(F, s2)[k];
 	};
 	auto ori = [&](int i, double Oq[9]) {
 		const int s2 = slot_of(i);
-		for(int k = 0; k < 9; k++) Oq[k] = F[(size_t) (3 + k) * S + s2];
+		for(int k = 0; k < 9; k++) Oq[k] = part(F, s2)[3 + k];
 	};
 	if(b < m_pad && !live) {
 		if(lane < NN_IN_PAD / 2) {
@@ -970,8 +967,8 @@ __global__ __launch_bounds__(64 * TS_WAVES) void k_train_samples(DevState d, uin
 			iL[k] = rp.g.inv_box[k];
 		}
 		double p[3], O[9];
-		for(int k = 0; k < 3; k++) p[k] = F[(size_t) k * S + j];
-		for(int k = 0; k < 9; k++) O[k] = F[(size_t) (3 + k) * S + j];
+		for(int k = 0; k < 3; k++) p[k] = part(F, j)[k];
+		for(int k = 0; k < 9; k++) O[k] = part(F, j)[3 + k];
 		// its cell on the current grid (particles never leave their cells
 		// between rebuilds) and the 27 cells around it
 		const int n0 = rp.g.n[0], n1 = rp.g.n[1], n2 = rp.g.n[2];

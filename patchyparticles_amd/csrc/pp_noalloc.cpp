@@ -113,9 +113,9 @@ pp_status na_scratch(int dev, unsigned char **out) {
 __global__ void k_na_stage(const double *aos, int n, double *f0, int *pid0, int *prep) {
 	const int j = blockIdx.x * blockDim.x + threadIdx.x;
 	if(j >= n) return;
-	for(int c = 0; c < 3; c++) f0[(size_t) c * n + j] = aos[3 * (size_t) j + c];
+	for(int c = 0; c < 3; c++) f0[NCOMP * (size_t) j + c] = aos[3 * (size_t) j + c];
 	const double *O = aos + 3 * (size_t) n;
-	for(int c = 0; c < 9; c++) f0[(size_t) (3 + c) * n + j] = O[9 * (size_t) j + c];
+	for(int c = 0; c < 9; c++) f0[NCOMP * (size_t) j + 3 + c] = O[9 * (size_t) j + c];
 	pid0[j] = j;
 	prep[j] = 0;
 }
