@@ -233,12 +233,83 @@ __device__ __forceinline__ unsigned kf_fast_q1(double dx, double dy, double dz, 
 	return kf_fast_class(kf_q_top(dx, dy, dz, Oq), bq);
 }
 
-// q side on the old (o) and the new (n) separation of a trial
-__device__ __forceinline__ void kf_fast_q2(double ox, double oy, double oz, const KfBand &boq, double nx, double ny,
-                                           double nz, const KfBand &bnq, const double Oq[9], unsigned &fo,
-                                           unsigned &fn) {
-	fo = kf_fast_q1(ox, oy, oz, boq, Oq);
-	fn = kf_fast_q1(nx, ny, nz, bnq, Oq);
+// ---------------------------------------------------------------------
+// Single-precision filter of the colour passes.  Positions are held relative
+// to the centre of the working team's cell, so they are below two cell
+// sides, and a pair is decided in single precision unless it lies so close to
+// a threshold that the roundings could matter; such a pair (about one trial
+// in 10^3 has one) is decided by the reference's own FP64 arithmetic, so that
+// every decision equals the reference's.  With s the largest cell side and rc
+// the bond range (s >= rc > 1), u = 2^-24:
+//   a component of a separation: |rel q| <= 1.5 s, |rel p'| <= s / 2 and
+//     |displacement| <= s round once each, their sum and the difference once
+//     more: error <= 4 s u = 2.4e-7 s
+//   d^2 (for d <= rc): <= 2 sqrt(3) rc 2.4e-7 s + 4 u rc^2 <= 1.1e-6 s rc
+//   e = O'^T d by two 3 x 3 products, g = +-e0 +-e1 +-e2 <= 5.2e-6 s, and
+//     g|g| - 3 cosmax^2 d^2 <= 2.2e-5 s rc (entries of O at most 1.01)
+// The bands hold these errors three times over.  Where an orientation entry
+// is larger or a coordinate beyond F32_MAX_POS (whose FP64 spacing would
+// matter), and below KF_FILTER_MIN_COS, the bands are infinite: every pair
+// within reach takes the exact arithmetic.
+constexpr float F32_BAND_D2 = 4e-6f;  // times s rc
+constexpr float F32_BAND_T = 8e-5f;   // times s rc
+constexpr double F32_MAX_POS = 1e7;
+
+struct F32Filter {
+	float rc2, c3;        // bond range squared, 3 cosmax^2
+	float eps_d2, eps_t;  // bands
+};
+
+__device__ __forceinline__ F32Filter f32_filter(double cosmax, double rc2, double side) {
+	const float cm = (float) cosmax, band = (float) (side * sqrt(rc2));
+	const bool off = !(cosmax >= KF_FILTER_MIN_COS);
+	return {(float) rc2, 3.f * (cm * cm), off ? 1e30f : F32_BAND_D2 * band, off ? 1e30f : F32_BAND_T * band};
+}
+
+__device__ __forceinline__ bool f32_orientation_ok(const float *o) {
+	// (as integers: a NaN is larger than any number)
+	unsigned m = 0;
+#pragma unroll
+	for(int c = 0; c < 9; c++) m = max(m, __float_as_uint(o[c]) & 0x7fffffffu);
+	return m <= __float_as_uint(1.01f);
+}
+
+__device__ __forceinline__ float norm2(float x, float y, float z) {
+	return __builtin_fmaf(x, x, __builtin_fmaf(y, y, z * z));
+}
+
+// M^T d for a row-major M.
+__device__ __forceinline__ void mul_t(const float *M, float dx, float dy, float dz, float &e0, float &e1, float &e2) {
+	e0 = __builtin_fmaf(dx, M[0], __builtin_fmaf(dy, M[3], dz * M[6]));
+	e1 = __builtin_fmaf(dx, M[1], __builtin_fmaf(dy, M[4], dz * M[7]));
+	e2 = __builtin_fmaf(dx, M[2], __builtin_fmaf(dy, M[5], dz * M[8]));
+}
+
+// The largest sigma_b . e over a particle's patches (the base vectors'
+// signs): d . patch_b = c sigma_b . e for e = O^T d.
+static_assert(KF_NEG == 0b101000110011u, "the signs written out in patch_top");
+__device__ __forceinline__ float patch_top(float e0, float e1, float e2) {
+	const float s = e0 + e1, t = e0 - e1;
+	return __builtin_fmaxf(__builtin_fmaxf(e2 - s, t - e2), __builtin_fmaxf(s + e2, -(t + e2)));
+}
+
+// d^2 within a band of the overlap or the bond range (a NaN is).
+__device__ __forceinline__ bool f32_near(float d2, const F32Filter &f) {
+	return !(__builtin_fminf(__builtin_fabsf(d2 - 1.f), __builtin_fabsf(d2 - f.rc2)) > f.eps_d2);
+}
+
+// The bond of a pair at separation d, with e the separation in p's body
+// frame: KF_YES, KF_NO or KF_UNSURE.
+__device__ __forceinline__ int f32_bond(float e0, float e1, float e2, float dx, float dy, float dz, float d2,
+                                        const float *Oq, const F32Filter &f) {
+	const float thr = f.c3 * d2;
+	const float lo = thr - f.eps_t, hi = thr + f.eps_t;
+	const float gp = patch_top(e0, e1, e2), tp = gp * __builtin_fabsf(gp);
+	float f0, f1, f2;
+	mul_t(Oq, -dx, -dy, -dz, f0, f1, f2);
+	const float gq = patch_top(f0, f1, f2), tq = gq * __builtin_fabsf(gq);
+	const float tm = __builtin_fminf(tp, tq);
+	return tm > hi ? KF_YES : (tm < lo ? KF_NO : KF_UNSURE);
 }
 
 // Cell coordinate of x on a grid of n cells over [s, s+L) (periodic).

@@ -384,7 +384,13 @@ pp_status create_impl(int R, const pp_params *prm, const pp_options *opts, const
 		rp.rc2 = rcut * rcut;  // SQR(1. + delta) (system.c:86)
 		rp.cosmax = p.kf_cosmax;
 		rp.T = p.temperature;
-		for(int e = 0; e < ACC_TAB; e++) rp.acc_tab[e] = exp(-(double) e / p.temperature);  // MC.c:332
+		// u < exp(-j/T) (MC.c:332) for a draw u = w 2^-32: w <= ceil(2^32 exp(-j/T)) - 1
+		rp.pg.n_thr = 0;
+		for(int j = 1; j < ACC_TAB; j++) {
+			const double a = exp(-(double) j / p.temperature);
+			if(!(a > 0.)) break;
+			rp.pg.thr[rp.pg.n_thr++] = (uint32_t) std::min(std::ceil(a * 4294967296.) - 1., 4294967295.);
+		}
 		rp.disp_max = p.disp_max;
 		rp.theta_max = p.theta_max;
 		rp.P = p.pressure;

@@ -71,45 +71,6 @@ __device__ __forceinline__ int team_sum(int v) {
 	return v;
 }
 
-// Sum of a double over a team of 16 lanes (DPP butterflies within a row, on
-// the two halves of the value).  Lanes may round differently: for bounds
-// only.
-__device__ __forceinline__ double dpp_add_f64_quad1032(double x) {
-	const long long b = __double_as_longlong(x);
-	const int lo = __builtin_amdgcn_update_dpp(0, (int) b, DPP_QUAD_1032, 0xf, 0xf, false);
-	const int hi = __builtin_amdgcn_update_dpp(0, (int) (b >> 32), DPP_QUAD_1032, 0xf, 0xf, false);
-	return x + __longlong_as_double(((long long) hi << 32) | (unsigned) lo);
-}
-__device__ __forceinline__ double dpp_add_f64_quad2301(double x) {
-	const long long b = __double_as_longlong(x);
-	const int lo = __builtin_amdgcn_update_dpp(0, (int) b, DPP_QUAD_2301, 0xf, 0xf, false);
-	const int hi = __builtin_amdgcn_update_dpp(0, (int) (b >> 32), DPP_QUAD_2301, 0xf, 0xf, false);
-	return x + __longlong_as_double(((long long) hi << 32) | (unsigned) lo);
-}
-__device__ __forceinline__ double dpp_add_f64_half_mirror(double x) {
-	const long long b = __double_as_longlong(x);
-	const int lo = __builtin_amdgcn_update_dpp(0, (int) b, DPP_HALF_MIRROR, 0xf, 0xf, false);
-	const int hi = __builtin_amdgcn_update_dpp(0, (int) (b >> 32), DPP_HALF_MIRROR, 0xf, 0xf, false);
-	return x + __longlong_as_double(((long long) hi << 32) | (unsigned) lo);
-}
-__device__ __forceinline__ double dpp_add_f64_row_mirror(double x) {
-	const long long b = __double_as_longlong(x);
-	const int lo = __builtin_amdgcn_update_dpp(0, (int) b, DPP_ROW_MIRROR, 0xf, 0xf, false);
-	const int hi = __builtin_amdgcn_update_dpp(0, (int) (b >> 32), DPP_ROW_MIRROR, 0xf, 0xf, false);
-	return x + __longlong_as_double(((long long) hi << 32) | (unsigned) lo);
-}
-__device__ __forceinline__ double team16_sum_f64(double x) {
-	x = dpp_add_f64_quad1032(x);
-	x = dpp_add_f64_quad2301(x);
-	x = dpp_add_f64_half_mirror(x);
-	return dpp_add_f64_row_mirror(x);
-}
-
-// Lanes below this one whose bit is set in mask m.
-__device__ __forceinline__ int lanes_below(unsigned long long m) {
-	return (int) __builtin_amdgcn_mbcnt_hi((unsigned) (m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned) m, 0u));
-}
-
 // Inclusive prefix sum over a whole wavefront (every lane active):
 // Hillis-Steele steps within each 16-lane row (row_shr 1, 2, 4, 8, the
 // lanes shifted in from outside the row reading 0), then row 0's total into
@@ -129,23 +90,30 @@ __device__ __forceinline__ int wave_incl_scan(int v) {
 	return v;
 }
 
-// Sum over a team of small non-negative integers (< 8): one ballot per bit.
-template <int T>
-__device__ __forceinline__ int team_sum_small(int v) {
-	const int off = (threadIdx.x & 63) & ~(T - 1);
-	const unsigned long long tm = (T == 64) ? ~0ull : ((1ull << T) - 1ull);
-	int s = 0;
-#pragma unroll
-	for(int b = 0; b < 3; b++) s += __popcll((__ballot((v >> b) & 1) >> off) & tm) << b;
-	return s;
+// A value the compiler knows nothing about: what is computed from it stays
+// where it is written, not in registers across a loop that rarely needs it.
+__device__ __forceinline__ int opaque(int v) {
+	asm volatile("" : "+v"(v)::"memory");
+	return v;
 }
 
+__device__ __forceinline__ int opaque_uniform(int v) {
+	asm volatile("" : "+s"(v)::"memory");
+	return v;
+}
+
+// The lanes of the wavefront where p holds (__ballot takes an int, which
+// costs a select and a compare when p is a combined condition).
+__device__ __forceinline__ unsigned long long ballot(bool p) { return __builtin_amdgcn_ballot_w64(p); }
+
+// Whether p holds in some lane of the team.
 template <int T>
 __device__ __forceinline__ bool team_any(bool p) {
-	unsigned long long m = __ballot(p);
-	int off = (threadIdx.x & 63) & ~(T - 1);
-	unsigned long long tm = (T == 64) ? ~0ull : ((1ull << T) - 1ull);
-	return ((m >> off) & tm) != 0ull;
+	const unsigned long long m = ballot(p);
+	const int off = (threadIdx.x & 63) & ~(T - 1);
+	if constexpr(T == 64) return m != 0ull;
+	else if constexpr(T == 32) return (off ? (unsigned) (m >> 32) : (unsigned) m) != 0u;
+	else return ((unsigned) (m >> off) & ((1u << T) - 1u)) != 0u;
 }
 
 // When a team is a whole wavefront (T = 64) every team-uniform value is
@@ -153,17 +121,6 @@ __device__ __forceinline__ bool team_any(bool p) {
 template <int T>
 __device__ __forceinline__ int uni(int v) {
 	if constexpr(T == 64) return __builtin_amdgcn_readfirstlane(v);
-	else return v;
-}
-
-template <int T>
-__device__ __forceinline__ double unid(double v) {
-	if constexpr(T == 64) {
-		long long b = __double_as_longlong(v);
-		int lo = __builtin_amdgcn_readfirstlane((int) (b & 0xffffffffll));
-		int hi = __builtin_amdgcn_readfirstlane((int) (b >> 32));
-		return __longlong_as_double(((long long) hi << 32) | (unsigned) lo);
-	}
 	else return v;
 }
 
@@ -188,49 +145,63 @@ __device__ __forceinline__ int wrapi(int i, int n) { return i < 0 ? i + n : (i >
 // axis law symmetric under a -> -a and so the proposal symmetric.
 constexpr uint32_t AXIS_BLOCKS = 64;
 
-__device__ __forceinline__ void sphere_axis(uint64_t seed, int r, uint64_t sweep, uint32_t cell, uint32_t col,
-                                            uint32_t t, double a[3]) {
-	for(uint32_t blk = 0; blk < AXIS_BLOCKS; blk++) {
-		u32x4 v = rng(seed, r, sweep, cell | (blk << 24), TAG_AXIS, col, t);
-		const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-		for(int h = 0; h < 2; h++) {
-			double u1 = 1. - 2. * u01(w[2 * h]), u2 = 1. - 2. * u01(w[2 * h + 1]);
-			double q = u1 * u1 + u2 * u2;
-			if(q < 1.) {
-				double f = 2. * __builtin_sqrt(1. - q);
-				a[0] = u1 * f;
-				a[1] = u2 * f;
-				a[2] = 1. - 2. * q;
-				return;
-			}
+__device__ __forceinline__ u32x4 axis_block(uint64_t seed, int r, uint64_t sweep, uint32_t cell, uint32_t col, uint32_t t,
+                                            uint32_t blk) {
+	return rng(seed, r, sweep, cell | (blk << 24), TAG_AXIS, col, t);
+}
+
+// v: block 0 of the draw (callers form it among their other draws, so that
+// the Philox rounds of all of them overlap).
+__device__ __forceinline__ void sphere_axis_from(u32x4 v, uint64_t seed, int r, uint64_t sweep, uint32_t cell,
+                                                 uint32_t col, uint32_t t, double a[3]) {
+	for(uint32_t blk = 0;;) {
+		// the block's first accepted pair
+		const double p1 = 1. - 2. * u01(v.x), p2 = 1. - 2. * u01(v.y), s1 = 1. - 2. * u01(v.z), s2 = 1. - 2. * u01(v.w);
+		const double p = p1 * p1 + p2 * p2, s = s1 * s1 + s2 * s2;
+		const bool one = p < 1.;
+		const double q = one ? p : s, u1 = one ? p1 : s1, u2 = one ? p2 : s2;
+		if(q < 1.) {
+			const double f = 2. * __builtin_sqrt(1. - q);
+			a[0] = u1 * f;
+			a[1] = u2 * f;
+			a[2] = 1. - 2. * q;
+			return;
 		}
+		if(++blk == AXIS_BLOCKS) break;
+		v = axis_block(seed, r, sweep, cell, col, t, blk);
 	}
-	u32x4 v = rng(seed, r, sweep, cell, TAG_AXIS_FALLBACK, col, t);
+	v = rng(seed, r, sweep, cell, TAG_AXIS_FALLBACK, col, t);
 	a[0] = 0.;
 	a[1] = 0.;
 	a[2] = (v.x & 1u) ? 1. : -1.;
 }
 
+__device__ __forceinline__ void sphere_axis(uint64_t seed, int r, uint64_t sweep, uint32_t cell, uint32_t col,
+                                            uint32_t t, double a[3]) {
+	sphere_axis_from(axis_block(seed, r, sweep, cell, col, t, 0), seed, r, sweep, cell, col, t, a);
+}
+
 // Trial t of cell cloc (colour col) in sweep `sweep`: member rank among
 // cnt, displacement uniform in +-disp_max/2 per axis (MC.c:317-319), rotation
 // by an angle uniform in [0, theta_max) about an axis uniform on the sphere
-// (MC.c:321-325, utils.c:186-202), and the acceptance draw (MC.c:332).
-__device__ __forceinline__ void make_trial(const DevState &d, const Rep &rp, int r, uint64_t sweep, int cloc, int col,
-                                           int t, int cnt, double *out) {
-	u32x4 ra = rng(d.seed, r, sweep, (uint32_t) cloc, TAG_TRIAL_A, (uint32_t) col, (uint32_t) t);
-	u32x4 rb = rng(d.seed, r, sweep, (uint32_t) cloc, TAG_TRIAL_B, (uint32_t) col, (uint32_t) t);
+// (MC.c:321-325, utils.c:186-202).  Returns the 32 bits of the acceptance
+// draw u = w 2^-32 (MC.c:332).
+__device__ __forceinline__ uint32_t make_trial(const DevState &d, const Rep &rp, int r, uint64_t sweep, int cloc, int col,
+                                               int t, int cnt, double out[TRIAL_W]) {
+	const u32x4 ra = rng(d.seed, r, sweep, (uint32_t) cloc, TAG_TRIAL_A, (uint32_t) col, (uint32_t) t);
+	const u32x4 rb = rng(d.seed, r, sweep, (uint32_t) cloc, TAG_TRIAL_B, (uint32_t) col, (uint32_t) t);
+	const u32x4 rc = axis_block(d.seed, r, sweep, (uint32_t) cloc, (uint32_t) col, (uint32_t) t, 0);
+	double axis[3], st, ct, R[9];
+	sincos(u01(rb.x) * rp.theta_max, &st, &ct);
+	sphere_axis_from(rc, d.seed, r, sweep, (uint32_t) cloc, (uint32_t) col, (uint32_t) t, axis);
 	out[0] = (double) __umulhi(ra.x, (uint32_t) cnt);
 	out[1] = (u01(ra.y) - 0.5) * rp.disp_max;
 	out[2] = (u01(ra.z) - 0.5) * rp.disp_max;
 	out[3] = (u01(ra.w) - 0.5) * rp.disp_max;
-	double axis[3], st, ct, R[9];
-	sphere_axis(d.seed, r, sweep, (uint32_t) cloc, (uint32_t) col, (uint32_t) t, axis);
-	sincos(u01(rb.x) * rp.theta_max, &st, &ct);
 	rotation_matrix(axis, st, ct, R);
 #pragma unroll
 	for(int c = 0; c < 9; c++) out[4 + c] = R[c];
-	out[13] = u01(rb.w);
+	return rb.w;
 }
 
 // Trial geometry shared by the helpers of one team.
@@ -291,9 +262,8 @@ __device__ __forceinline__ void bonds_old_new_exact(const Trial &t, const double
 
 // Bonds of neighbour q with the new position only: the filtered decision
 // (a pair inside the filter band sets `band`) and the reference's arithmetic
-// (MC.c:242-262).  For neighbours whose bonds with the old position are known.
-// bonds_new_sep takes the separation (wx, wy, wz) = sep_new(q) and its
-// square w2; bonds_new forms them.
+// (MC.c:242-262), for the separation (wx, wy, wz) = sep_new(q) and its square
+// w2.
 template <class LoadO>
 __device__ __forceinline__ void bonds_new_sep(const Trial &t, const double *Pn, double wx, double wy, double wz,
                                               double w2, LoadO load_o, int &bn, bool &band) {
@@ -308,14 +278,6 @@ __device__ __forceinline__ void bonds_new_sep(const Trial &t, const double *Pn, 
 		bn += (int) (qn & 1u);
 	}
 	band |= unsure != 0u;
-}
-
-template <class LoadO>
-__device__ __forceinline__ void bonds_new(const Trial &t, const double *Pn, double qx, double qy, double qz,
-                                          LoadO load_o, int &bn, bool &band) {
-	double wx, wy, wz;
-	const double w2 = sep_new(t, qx, qy, qz, wx, wy, wz);
-	bonds_new_sep(t, Pn, wx, wy, wz, w2, load_o, bn, band);
 }
 
 template <class LoadO>

@@ -12,7 +12,7 @@ namespace ppd {
 constexpr int CELL_CAP = 24;   // particles of one sweep cell staged in LDS
 constexpr int NSLOT = 64;      // spread of per-replica atomic counters
 constexpr int NCOMP = 12;      // x, y, z, O00..O22 per particle
-constexpr int TRIAL_W = 14;    // one trial: member rank, dx, dy, dz, R[9], acceptance draw
+constexpr int TRIAL_W = 13;    // one trial: member rank, dx, dy, dz, R[9]
 constexpr int MAX_TRIALS_PER_CELL = 16;
 // cells per scan workgroup of 256 lanes: small tiles shorten each lane's
 // chain where the whole grid is a few tiles; large ones keep the per-tile
@@ -106,6 +106,19 @@ struct Grid {
 	int pad;
 };
 
+// What the colour passes need of a replica's grid and parameters, formed once
+// per sweep (k_count) and not by every team of every pass: the divisions and
+// integer quotients alone were a fifth of a pass of one trial per member.
+struct PassGeo {
+	double box[3], inv_box[3];
+	double shift[3], side[3];   // of the sweep's cells
+	float inv_side[3];
+	F32Filter filter;           // of the single-precision pair tests
+	int n1, n2;
+	int n_thr;                  // entries of thr in use
+	uint32_t thr[ACC_TAB - 1];  // a 32-bit draw w accepts a rise of j bonds iff w <= thr[j - 1]
+};
+
 // One replica: its particle range, its cell region and its parameters.
 //
 // Slots [p_off, p_off + cap_np) belong to the replica; after a rebuild its np
@@ -168,7 +181,7 @@ struct Rep {
 	int vol_apply;   // an accepted fast trial: positions still to be rescaled in place
 	int lx_ref_rule;  // box-shape moves accepted with exp(+dE/T) as MC.c:562 (not Metropolis)
 	double lx_change_max, lyz_min, lyz_max;
-	double acc_tab[ACC_TAB];  // exp(-k / T): the acceptance factor of an energy rise of k bonds
+	PassGeo pg;  // set by the rebuild of each sweep (n_thr, thr: at creation)
 };
 
 // Cells per side for a box: the largest (even, if asked) count whose side is

@@ -91,6 +91,22 @@ __device__ __forceinline__ int replica_of_cell(const DevState &d, int c) {
 // box trial whose grid the current lists cannot serve).
 __device__ __forceinline__ bool trial_rebuilds(const Rep &rp) { return rp.trial_active && !rp.trial_fast; }
 
+__device__ __forceinline__ void set_pass_geo(Rep &rp, const Grid &G, const double sh[3]) {
+	PassGeo &p = rp.pg;
+	double smax = 0.;
+	for(int k = 0; k < 3; k++) {
+		p.box[k] = G.box[k];
+		p.inv_box[k] = G.inv_box[k];
+		p.shift[k] = sh[k];
+		p.side[k] = G.box[k] / (double) G.n[k];
+		p.inv_side[k] = (float) ((double) G.n[k] / G.box[k]);
+		smax = fmax(smax, p.side[k]);
+	}
+	p.filter = f32_filter(rp.cosmax, rp.rc2, smax);
+	p.n1 = G.n[1];
+	p.n2 = G.n[2];
+}
+
 // ONE: a context of one replica, whose table then loads to scalar registers.
 template <bool ONE>
 __global__ void k_count(DevState d, int mode, uint64_t sweep, long long trace_pos) {
@@ -130,6 +146,7 @@ __global__ void k_count(DevState d, int mode, uint64_t sweep, long long trace_po
 			u32x4 v = rng(d.seed, r, sweep, 0, TAG_COLOUR, 0, 0);
 			const uint32_t w4[4] = {v.x, v.y, v.z, v.w};
 			rp.col_perm = colour_perm_from(w4);
+			set_pass_geo(rp, G, sh);
 		}
 	}
 	if(!tr && j == rp.p_off) {
@@ -560,125 +577,69 @@ struct PassArgs {
 	unsigned mark;  // dependency-driven sweeps: the value a finished cell publishes in done[]
 };
 
-// Per-team LDS (doubles) for cells of up to CAP members: the stage row of a
-// trial's O' and patches, the cell's trials, its members ranked by particle
-// index (x, y, z, O and the 4 patch vectors; the kept form holds the
-// member's fractional cell coordinates in the first three patch slots),
-// their particle indices, their kept static bond counts and the cell's
-// record (surrounding slot ranges).
-constexpr int OWN_W = NCOMP + 12;   // x, y, z, O[9], P[12]
-constexpr int LDS_NB = REC_W / 2;   // the cell record, REC_W ints
-constexpr int LDS_STAGE = 22;       // a trial's O' (9) and patches (12), formed one value per lane
+// Per-team LDS for cells of up to CAP members (offsets in 8-byte words):
+//   SH  the members' single-precision records: position relative to the
+//       cell's centre, O, the count of bonds with static neighbours, the
+//       bits of the bonds with the other members
+//   FT  the trials in single precision: displacement, the largest energy
+//       rise their draw accepts, R, the moving member's rank
+//   OWN the members' exact state, ranked by particle index: x, y, z, O, and
+//       the position relative to the cell's centre
+//   TR  the trials' exact displacement and R
+//   PID particle indices, NB the cell's record (surrounding slot ranges)
+//   GEO constants of the exact arithmetic and the far neighbours, here so
+//       that the trial loop does not hold them in registers
+constexpr int OWN_W = 16;  // x, y, z, O[9], rel[3], one unused
+constexpr int TR_W = 12;   // dx, dy, dz, R[9]
+constexpr int SH_W = 16;   // floats: rel[3], O[9], static bonds, member bond bits, two unused
+constexpr int FT_W = 16;   // floats: dx, dy, dz, the rise it accepts, R[9], rank, two unused
+constexpr int GEO_W = 12;  // box[3], 1 / box[3], the cell's centre[3], rc^2, cosmax, one unused
 template <int CAP>
 struct TeamLds {
-	static constexpr int OWN = CAP * OWN_W;
-	static constexpr int PID = (CAP + 1) / 2;  // CAP ints
-	static constexpr int SB = (CAP + 1) / 2;   // CAP ints: each member's bonds with the static neighbours
-	// a trial per member, or a fixed number per cell
-	static constexpr int TRIAL = (CAP > MAX_TRIALS_PER_CELL ? CAP : MAX_TRIALS_PER_CELL) * TRIAL_W;
-	static constexpr int FIXED = OWN + PID + SB + TRIAL + LDS_NB + LDS_STAGE;
-	static_assert((LDS_STAGE + TRIAL + OWN + PID + SB) % 2 == 0 && FIXED % 2 == 0 && (LDS_STAGE + TRIAL) % 2 == 0 &&
-	                  TRIAL_W % 2 == 0 && OWN_W % 2 == 0,
-	              "16-byte aligned trials, members, record and team blocks");
+	static constexpr int TRIALS = CAP > MAX_TRIALS_PER_CELL ? CAP : MAX_TRIALS_PER_CELL;
+	static constexpr int SH = 0;
+	static constexpr int FT = SH + CAP * SH_W / 2;
+	static constexpr int OWN = FT + TRIALS * FT_W / 2;
+	static constexpr int TR = OWN + CAP * OWN_W;
+	static constexpr int PID = TR + TRIALS * TR_W;
+	static constexpr int NB = PID + (CAP + 1) / 2;
+	static constexpr int GEO = NB + REC_W / 2;
+	static constexpr int SIZE = GEO + GEO_W;
+	static_assert(FT % 2 == 0 && OWN % 2 == 0 && TR % 2 == 0 && NB % 2 == 0 && SIZE % 2 == 0, "16-byte aligned parts");
 };
 // Cells of the small-cell pass (dilute systems, 16-lane teams with one
-// register slot per lane): about half the LDS of a general team, so twice
-// the cells stay resident; fuller cells are deferred to the general pass.
+// register slot per lane): half the LDS of a general team, so twice the
+// cells stay resident; fuller cells are deferred to the general pass.
 constexpr int SMALL_CAP = 8;
-// + the orientations of the register neighbours, component-major (two
-// slots per lane for 16-lane teams, one per lane for the small-cell pass)
-template <int T, int CAP = CELL_CAP>
+template <int CAP = CELL_CAP>
 constexpr int team_lds() {
-	return TeamLds<CAP>::FIXED + 9 * (CAP < CELL_CAP ? T : (T < 32 ? 32 : T));
+	return TeamLds<CAP>::SIZE;
 }
-// 16 teams of 32 lanes (four 128-lane workgroups, the default shape) share a
-// CU's 160 KiB; 32 small-cell teams of 16 lanes do
-static_assert(2 * 8 * team_lds<32>() * sizeof(double) <= 160 * 1024, "two pass workgroups per CU");
-static_assert(4 * 8 * team_lds<16, SMALL_CAP>() * sizeof(double) <= 160 * 1024, "four small-cell workgroups per CU");
+// 16 general teams (four 128-thread workgroups of 32-lane teams, the default
+// shape) share a CU's 160 KiB; 32 small-cell teams do
+static_assert(16 * team_lds<>() * sizeof(double) <= 160 * 1024, "two pass workgroups per CU");
+static_assert(32 * team_lds<SMALL_CAP>() * sizeof(double) <= 160 * 1024, "eight small-cell workgroups per CU");
 
-// The same decisions through the filtered tests (no square root, no
-// divisions, no branch per patch).  A pair inside a filter band sets `band`;
-// the caller then redoes that lane's neighbours with bonds_old_new_exact.
-template <class LoadO>
-__device__ __forceinline__ void bonds_old_new(const Trial &t, const double *Po, const double *Pn, double qx, double qy,
-                                              double qz, LoadO load_o, int &bo, int &bn, bool &band) {
-	const double ox = kf_min_image(qx - t.px, t.Lx, t.iLx);
-	const double oy = kf_min_image(qy - t.py, t.Ly, t.iLy);
-	const double oz = kf_min_image(qz - t.pz, t.Lz, t.iLz);
-	const double o2 = ox * ox + oy * oy + oz * oz;
-	const double wx = kf_min_image(qx - t.nx, t.Lx, t.iLx);
-	const double wy = kf_min_image(qy - t.ny, t.Ly, t.iLy);
-	const double wz = kf_min_image(qz - t.nz, t.Lz, t.iLz);
-	const double w2 = wx * wx + wy * wy + wz * wz;
-	const KfBand bo_ = kf_band(t.c2, o2), bn_ = kf_band(t.c2, w2);
-	const unsigned fo = o2 < t.rc2 ? kf_fast_p(ox, oy, oz, Po, bo_) : 0u;
-	const unsigned fn = w2 < t.rc2 ? kf_fast_p(wx, wy, wz, Pn, bn_) : 0u;
-	unsigned unsure = ((fo | fn) >> 1) & 1u;
-	if((fo | fn) & 1u) {
-		double Oq[9];
-		load_o(Oq);
-		unsigned qo, qn;
-		kf_fast_q2(ox, oy, oz, kf_band_q(bo_), wx, wy, wz, kf_band_q(bn_), Oq, qo, qn);
-		qo = (fo & 1u) ? qo : 0u;
-		qn = (fn & 1u) ? qn : 0u;
-		unsure |= ((qo | qn) >> 1) & 1u;
-		bo += (int) (qo & 1u);
-		bn += (int) (qn & 1u);
-	}
-	band |= unsure != 0u;
-}
+constexpr float F32_CELL = 1e-5f;  // in-cell margin of the single-precision test, in cell sides
+constexpr float F32_FAR = 1e15f;   // the position of an empty slot
 
-// One cell of a colour pass: entry gi of the pass's list of non-empty cells
-// (all replicas), worked on by the T lanes of one team with its LDS block
-// `own`.  The cell's members
-// make sequential trials.  Each lane keeps up to CPL of the cell's static
-// neighbours (the 26 surrounding cells, fixed during the pass) in registers;
-// a denser neighbourhood is handled T at a time from HBM.
-// One of the 21 values of a trial's O' = O R (v < 9: O'[v]) and its patches
-// (v = 9 + 3a + kk: P'[a][kk]): the row of O it needs, the column, and for a
-// patch component the signs of patch a as sign-bit masks of the high word.
-struct RotShare {
-	int row, col;
-	bool patch;
-	unsigned long long s0, s1, s2;
+// One lane's share of an accepted move, values v = 0..14 of the moving
+// member's record: v < 3 the position, v < 12 O' = O R in the reference's
+// order (utils.c:172-184), else the position relative to the cell's centre.
+// own: three words of the member's record from `o`, tr: of the trial from
+// `r` with stride 3.
+struct MoveShare {
+	int o, r, word;  // word: the value's place in the single-precision record
+	bool dot;
 };
-
-__device__ __forceinline__ RotShare rot_share(int v) {
-	RotShare r;
-	const int idx = v < 9 ? 0 : v - 9;
-	r.patch = v >= 9;
-	r.row = v < 9 ? v / 3 : (v < 21 ? idx % 3 : 0);
-	r.col = v % 3;
-	const unsigned neg = (v >= 9 && v < 21) ? (KF_NEG >> (3 * (idx / 3))) & 7u : 0u;
-	r.s0 = (unsigned long long) (neg & 1u) << 63;
-	r.s1 = (unsigned long long) ((neg >> 1) & 1u) << 63;
-	r.s2 = (unsigned long long) ((neg >> 2) & 1u) << 63;
-	return r;
+__device__ __forceinline__ MoveShare move_share(int v) {
+	MoveShare m;
+	m.dot = v >= 3 && v < 12;
+	m.o = m.dot ? 3 + 3 * ((v - 3) / 3) : (v < 15 ? v : 0);
+	m.r = m.dot ? 3 + (v - 3) % 3 : (v < 3 ? v : (v >= 12 && v < 15 ? v - 12 : 0));
+	m.word = v < 3 ? 12 + v : (v < 12 ? v : v - 12);
+	return m;
 }
-
-// The value: row `row` of O' from that row of O (o0, o1, o2) and R (the
-// trial's tv[4..12]) in the reference's order (utils.c:172-184), then either
-// its column or, with b_a[j] = +-c and (+-x) c = +-(x c) exactly, the signed
-// sum of the row times c (utils.h:17-21).
-__device__ __forceinline__ double rot_value(const RotShare &r, double o0, double o1, double o2, const double *tv) {
-	const double r0 = o0 * tv[4] + o1 * tv[4 + 3] + o2 * tv[4 + 6];
-	const double r1 = o0 * tv[5] + o1 * tv[5 + 3] + o2 * tv[5 + 6];
-	const double r2 = o0 * tv[6] + o1 * tv[6 + 3] + o2 * tv[6 + 6];
-	if(!r.patch) return r.col == 0 ? r0 : (r.col == 1 ? r1 : r2);
-	const double m0 = r0 * KF_C, m1 = r1 * KF_C, m2 = r2 * KF_C;
-	const double a0 = __longlong_as_double(__double_as_longlong(m0) ^ (long long) r.s0);
-	const double a1 = __longlong_as_double(__double_as_longlong(m1) ^ (long long) r.s1);
-	const double a2 = __longlong_as_double(__double_as_longlong(m2) ^ (long long) r.s2);
-	return a0 + a1 + a2;
-}
-
-// Trials per cell from which the kept form pays: with fewer, the up-front
-// counts cost about what the trials save.
-constexpr int KEEP_MIN_TRIALS = 4;
-
-// Margin of the reach filter over rounding in positions and distances
-// (below 1e-12 for coordinates of a few hundred).
-constexpr double REACH_EPS = 1e-9;
 
 // A read of another cell's particle data during a pass.  In the
 // dependency-driven sweep (DD: the passes of a sweep in one launch, each cell
@@ -725,10 +686,29 @@ __device__ __forceinline__ void wait_neighbours(const DevState &d, const Rep &rp
 	__atomic_signal_fence(__ATOMIC_SEQ_CST);
 }
 
-// KEEP (fixed trials per cell, many per member): every member's bonds with
-// the static neighbours are counted up front and kept as it moves, so a trial
-// tests only the new position against them.  Without KEEP (about one trial
-// per member) every trial tests both positions.
+// One cell of a colour pass: entry gi of the pass's list of non-empty cells
+// (all replicas), worked on by the T lanes of one team with its LDS block
+// `blk`.  The cell's members make sequential trials.  Each lane keeps up to
+// CPL of the cell's static neighbours (the 26 surrounding cells, fixed during
+// the pass) in registers; a denser neighbourhood is handled T at a time from
+// HBM.
+//
+// The static neighbours do not move during the pass: a member's bonds with
+// them, and with the other members, are counted at the first trial that gets
+// as far as its bonds, and kept as members move; later trials test only the
+// new position.  The bond decision is symmetric to the bit.
+//
+// A trial is one dependent chain, and most wavefronts share their SIMD with
+// at most one other, so its length sets the pass's time.  Hence the
+// single-precision filter (F32Filter: about 150 VALU instructions per trial
+// instead of 280 in FP64, half the registers, no LDS exchange of the new
+// patches: the separation is rotated into each particle's body frame
+// instead), the trial read one ahead, and the exact new state formed one
+// value per lane on acceptance.  Measured, steps of 16 trials per cell: one
+// system of N=32768 at rho 0.5 285 -> 207 us, 8 x 4096 427 -> 212 us (its 28
+// candidates per cell also fit the second register slot now, where the FP64
+// form read 1 in 4 cells' last neighbours from HBM at every trial), 256
+// uneven replicas 4.15 -> 2.75 ms.
 //
 // DD: the pass is one of several in flight (k_pass_dd).  The cell's own
 // loads and its trials come first; the team then waits for its neighbours of
@@ -738,691 +718,496 @@ __device__ __forceinline__ void wait_neighbours(const DevState &d, const Rep &rp
 //
 // CAP < CELL_CAP (the small-cell pass): a cell of more than CAP members is
 // not worked on here but listed for the general pass that follows.
-template <int T, int CPL, bool KEEP, bool ONE, bool DD, bool REACH = false, int CAP = CELL_CAP>
-__device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int pass, int gi, int lane,
-                                          double *blk, unsigned mark) {
+template <int T, int CPL, bool ONE, bool DD, int CAP = CELL_CAP>
+__device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int pass, int gi, int lane, double *blk,
+                                          unsigned mark) {
 	using L = TeamLds<CAP>;
-	// the team's block, the per-trial data first (short LDS offsets)
-	double *stage = blk;                    // LDS_STAGE doubles
-	double *trials = blk + LDS_STAGE;       // L::TRIAL
-	double *own = trials + L::TRIAL;        // L::OWN
-	int *own_pid = (int *) (own + L::OWN);
-	int *sbond = (int *) (own + L::OWN + L::PID);  // member m's bonds with the static neighbours
-	int *nb_tab = (int *) (own + L::OWN + L::PID + L::SB);  // the cell's record (build_record)
-	// the orientations of this lane's register neighbours: in registers where
-	// they allow (scalar replica constants, and one slot per lane or a reach
-	// filter that leaves the second slot almost always empty), else in LDS,
-	// component c of neighbour u at (9 u + c) * T + lane
-	constexpr bool REG_ORI = (ONE || T == 64) && (CPL == 1 || REACH);
-	double *ori = blk + L::FIXED;
-	{
-		// 1. the cell's record: surrounding slot ranges, own range, replica
-		const int4 *rec = (const int4 *) (d.rec + ((size_t) pass * d.total_act + gi) * REC_W);
-		for(int e = lane; e < REC_W / 4; e += T) ((int4 *) nb_tab)[e] = rec[e];
-		team_sync();
-		const int M = uni<T>(nb_tab[58]);
-		const int s0 = uni<T>(nb_tab[59]);
-		const int cnt = uni<T>(nb_tab[60]);
-		const int cloc = uni<T>(nb_tab[61]);
-		const int r = ONE ? 0 : uni<T>(nb_tab[62]);
-		const int sel = uni<T>(nb_tab[63]);
-		if constexpr(CAP < CELL_CAP)
-			if(cnt > d.small_cap) {
-				// (entries < total_act: each cell is listed at most once a pass)
-				if(lane == 0) d.ovf[atomicAdd(d.ovf_n + pass, 1)] = gi;
-				return;
-			}
-		// (a team of T < CELL_CAP lanes holds one member per lane)
-		if(cnt > CELL_CAP || cnt > T) {
-			if(lane == 0) {
-				atomicOr(d.err, (int) ERR_CELL_CAP);
-				// (DD) the neighbours of later passes do not wait for it
-				if constexpr(DD)
-					__hip_atomic_store(d.done + d.reps[r].cell_off + cloc, mark, __ATOMIC_RELAXED,
-					                   __HIP_MEMORY_SCOPE_AGENT);
-			}
+	static_assert(T == 16 || T == 32 || T == 64, "teams of 16, 32 or 64 lanes");
+	float *shadow = (float *) (blk + L::SH);
+	float *ftrial = (float *) (blk + L::FT);
+	double *own = blk + L::OWN;
+	double *trials = blk + L::TR;
+	double *geo = blk + L::GEO;
+	int *own_pid = (int *) (blk + L::PID);
+	int *nb_tab = (int *) (blk + L::NB);
+
+	// 1. the cell's record: surrounding slot ranges, own range, replica
+	const int4 *rec = (const int4 *) (d.rec + ((size_t) pass * d.total_act + gi) * REC_W);
+	for(int e = lane; e < REC_W / 4; e += T) ((int4 *) nb_tab)[e] = rec[e];
+	team_sync();
+	const int M = uni<T>(nb_tab[58]);
+	const int s0 = uni<T>(nb_tab[59]);
+	const int cnt = uni<T>(nb_tab[60]);
+	const int cloc = uni<T>(nb_tab[61]);
+	const int r = ONE ? 0 : uni<T>(nb_tab[62]);
+	const int sel = uni<T>(nb_tab[63]);
+	if constexpr(CAP < CELL_CAP)
+		if(cnt > d.small_cap) {
+			// (entries < total_act: each cell is listed at most once a pass)
+			if(lane == 0) d.ovf[atomicAdd(d.ovf_n + pass, 1)] = gi;
 			return;
 		}
-		const Rep &rp = d.reps[r];
-		double *F = pick_buf(d.f, sel);
-		int *PID = pick_buf(d.pid, sel);
-
-		// 2. every load of the cell at once: the members, the static
-		// neighbours' positions and the replica's geometry
-		int my_pid = 0;
-		double mine[NCOMP];
-		if(lane < cnt) {
-			my_pid = PID[s0 + lane];
-#pragma unroll
-			for(int c = 0; c < NCOMP; c++) mine[c] = part(F, s0 + lane)[c];
+	// (a team of T < CELL_CAP lanes holds one member per lane)
+	if(cnt > CELL_CAP || cnt > T) {
+		if(lane == 0) {
+			atomicOr(d.err, (int) ERR_CELL_CAP);
+			// (DD) the neighbours of later passes do not wait for it
+			if constexpr(DD)
+				__hip_atomic_store(d.done + d.reps[r].cell_off + cloc, mark, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 		}
-		// trials of the cell in this pass: one per member (a sweep is then N
-		// attempts), or a fixed number per non-empty cell
-		const int ntrial = d.trials_per_cell > 0 ? d.trials_per_cell : cnt;
-		// slot of static neighbour i (0 <= i < M)
-		auto nb_slot = [&](int i) {
-			int lo2 = 0, hi2 = 26;
-			while(hi2 - lo2 > 1) {
-				int mid = (lo2 + hi2) >> 1;
-				if(nb_tab[32 + mid] <= i) lo2 = mid;
-				else hi2 = mid;
-			}
-			return nb_tab[lo2] + (i - nb_tab[32 + lo2]);
-		};
-		// Register slot lane + u T (u < CPL) of the team holds one neighbour:
-		// slots below cnt the cell's members (member = lane, kept current
-		// from the cell's LDS block at every trial), then the first static
-		// neighbours; the rest (dense neighbourhoods only) are read again at
-		// every trial.  A lane thus tests one neighbour per trial whether the
-		// cell holds one member or several.
-		double cxr[CPL], cyr[CPL], czr[CPL];
-		int cqr[CPL];  // the static neighbour's slot, -1: a member or none
-		double orv[CPL][9];
-		auto load_static = [&]() {
+		return;
+	}
+	const Rep &rp = d.reps[r];
+	double *F = pick_buf(d.f, sel);
+	int *PID = pick_buf(d.pid, sel);
+
+	// 2. every load of the cell at once: the members, the static neighbours
+	// and the replica's geometry
+	int my_pid = 0;
+	double mine[NCOMP];
+	if(lane < cnt) {
+		my_pid = PID[s0 + lane];
 #pragma unroll
-			for(int u = 0; u < CPL; u++) {
-				const int i = lane + u * T - cnt;
-				cqr[u] = -1;
-				cxr[u] = cyr[u] = czr[u] = 0.;
-				if(i >= 0 && i < M) {
-					const int q = nb_slot(i);
-					cqr[u] = q;
-					cxr[u] = nbld<DD>(part(F, q));
-					cyr[u] = nbld<DD>(part(F, q) + 1);
-					czr[u] = nbld<DD>(part(F, q) + 2);
+		for(int c = 0; c < NCOMP; c++) mine[c] = part(F, s0 + lane)[c];
+	}
+	// trials of the cell in this pass: one per member (a sweep is then N
+	// attempts), or a fixed number per non-empty cell
+	const int ntrial = d.trials_per_cell > 0 ? d.trials_per_cell : cnt;
+	// slot of static neighbour i (0 <= i < M)
+	auto nb_slot = [&](int i) {
+		int lo2 = 0, hi2 = 26;
+		while(hi2 - lo2 > 1) {
+			int mid = (lo2 + hi2) >> 1;
+			if(nb_tab[32 + mid] <= i) lo2 = mid;
+			else hi2 = mid;
+		}
+		return nb_tab[lo2] + (i - nb_tab[32 + lo2]);
+	};
+	// Register slot lane + u T (u < CPL) of the team holds one neighbour:
+	// slots below cnt the cell's members (member = lane, read from the
+	// shadow records at every trial), then the first static neighbours; the
+	// rest (dense neighbourhoods only) are read again at every trial.  A lane
+	// thus tests one neighbour per trial whether the cell holds one member or
+	// several.
+	int cq[CPL];  // the static neighbour's slot, -1: a member or none
+	double sd[CPL][NCOMP];
+	auto load_static = [&]() {
+#pragma unroll
+		for(int u = 0; u < CPL; u++) {
+			const int i = lane + u * T - cnt;
+			cq[u] = -1;
+			if(i >= 0 && i < M) {
+				const int q = nb_slot(i);
+				cq[u] = q;
+#pragma unroll
+				for(int c = 0; c < NCOMP; c++) sd[u][c] = nbld<DD>(part(F, q) + c);
+			}
+		}
+	};
+	if constexpr(!DD) load_static();
+	const PassGeo &pg = rp.pg;
+	const int n1 = uni<T>(pg.n1), n2 = uni<T>(pg.n2);
+	const int ix = cloc / (n1 * n2), iy = (cloc / n2) % n1, iz = cloc % n2;
+	const int col = ((ix & 1) << 2) | ((iy & 1) << 1) | (iz & 1);
+	// the cell's centre
+	const double ce0 = pg.shift[0] + ((double) ix + 0.5) * pg.side[0], ce1 = pg.shift[1] + ((double) iy + 0.5) * pg.side[1],
+	             ce2 = pg.shift[2] + ((double) iz + 0.5) * pg.side[2];
+
+	// 3. the cell's trials, one lane each (Philox: no memory traffic), and
+	// the particle indices into LDS.  A trial keeps the largest rise in bonds
+	// lost that its draw accepts: u < exp(-j/T) (MC.c:332) falls with j, and
+	// for the 32-bit draw w it reads w <= thr[j - 1] exactly, so a trial
+	// decides by comparing two integers.
+	if(lane < ntrial) {
+		double tv[TRIAL_W];
+		const uint32_t draw = make_trial(d, rp, r, sweep, cloc, col, lane, cnt, tv);
+		int most = 0;
+#pragma unroll
+		for(int j = 0; j < ACC_TAB - 1; j++) most += (int) ((j < pg.n_thr) & (draw <= pg.thr[j]));
+		const int k = (int) tv[0];
+		double *w = trials + lane * TR_W;
+		float *f = ftrial + lane * FT_W;
+#pragma unroll
+		for(int e = 0; e < TR_W; e++) w[e] = tv[1 + e];
+		f[0] = (float) tv[1];
+		f[1] = (float) tv[2];
+		f[2] = (float) tv[3];
+		f[3] = __int_as_float(most);
+#pragma unroll
+		for(int e = 0; e < 9; e++) f[4 + e] = (float) tv[4 + e];
+		f[13] = __int_as_float(k);
+	}
+	static_assert(MAX_TRIALS_PER_CELL <= 16 && CELL_CAP <= 32, "one lane per trial");
+	const int koff = (threadIdx.x & 63) & ~(T - 1);
+	// the team's lanes of a wavefront mask
+	auto team_bits = [&](unsigned long long m) {
+		if constexpr(T == 64) return m;
+		else if constexpr(T == 32) return koff ? (unsigned) (m >> 32) : (unsigned) m;
+		else return (unsigned) (m >> koff) & ((1u << T) - 1u);
+	};
+	auto count_bits = [](auto m) {
+		if constexpr(sizeof(m) == 8) return (int) __popcll(m);
+		else return (int) __popc(m);
+	};
+	if(lane < cnt) own_pid[lane] = my_pid;
+	if(lane == 0) {
+		const double g[GEO_W] = {pg.box[0], pg.box[1], pg.box[2], pg.inv_box[0], pg.inv_box[1], pg.inv_box[2],
+		                         ce0, ce1, ce2, rp.rc2, rp.cosmax, 0.};
+#pragma unroll
+		for(int e = 0; e < GEO_W; e++) geo[e] = g[e];
+	}
+	team_sync();
+	// 4. members into LDS ranked by particle index; a lane's slots become
+	// single precision, relative to the cell's centre
+	bool wild = false;  // beyond the filter's error bounds
+	auto rel3 = [&](const double *p, double *q) {
+		q[0] = kf_min_image(p[0] - ce0, pg.box[0], pg.inv_box[0]);
+		q[1] = kf_min_image(p[1] - ce1, pg.box[1], pg.inv_box[1]);
+		q[2] = kf_min_image(p[2] - ce2, pg.box[2], pg.inv_box[2]);
+		wild |= !(__builtin_fmax(__builtin_fabs(p[0]), __builtin_fmax(__builtin_fabs(p[1]), __builtin_fabs(p[2]))) < F32_MAX_POS);
+	};
+	auto check_o = [&](const float *o) {
+		wild |= !f32_orientation_ok(o);
+	};
+	if(lane < cnt) {
+		int rank = 0;
+		for(int m = 0; m < cnt; m++) rank += own_pid[m] < my_pid;
+		double *w = own + rank * OWN_W;
+		float *s = shadow + rank * SH_W;
+		double rel[3];
+		rel3(mine, rel);
+		float of[9];
+#pragma unroll
+		for(int c = 0; c < NCOMP; c++) w[c] = mine[c];
+#pragma unroll
+		for(int c = 0; c < 9; c++) of[c] = (float) mine[3 + c];
+		check_o(of);
+#pragma unroll
+		for(int c = 0; c < 3; c++) {
+			w[12 + c] = rel[c];
+			s[c] = (float) rel[c];
+		}
+#pragma unroll
+		for(int c = 0; c < 9; c++) s[3 + c] = of[c];
+	}
+	if constexpr(DD) {
+		// the neighbours' data once their earlier passes are done
+		wait_neighbours<T>(d, rp, nb_tab, pass, ix, iy, iz, rp.g.n[0], n1, n2, mark, lane);
+		load_static();
+	}
+	float qx[CPL], qy[CPL], qz[CPL], qo[CPL][9];
+#pragma unroll
+	for(int u = 0; u < CPL; u++) {
+		qx[u] = qy[u] = qz[u] = F32_FAR;
+#pragma unroll
+		for(int c = 0; c < 9; c++) qo[u][c] = 0.f;
+		if(cq[u] >= 0) {
+			double rel[3];
+			rel3(sd[u], rel);
+			qx[u] = (float) rel[0];
+			qy[u] = (float) rel[1];
+			qz[u] = (float) rel[2];
+#pragma unroll
+			for(int c = 0; c < 9; c++) qo[u][c] = (float) sd[u][3 + c];
+			check_o(qo[u]);
+		}
+	}
+	F32Filter fl = pg.filter;
+	if(team_any<T>(wild)) fl.eps_d2 = fl.eps_t = 1e30f;
+	const float is0 = pg.inv_side[0], is1 = pg.inv_side[1], is2 = pg.inv_side[2];
+	// whether any team of the wavefront has neighbours beyond the register
+	// slots (a scalar branch around those loops)
+	const bool wave_far = ballot(M + cnt > T * CPL) != 0ull;
+	// and likewise whether any uses the second slot of its lanes
+	const bool wave_2 = CPL > 1 && ballot(M + cnt > T) != 0ull;
+	team_sync();
+
+	auto hide = [](int v) { if constexpr(T == 64) return opaque_uniform(v); else return opaque(v); };
+	auto hide_rep = [&]() { if constexpr(ONE) return opaque_uniform(0); else return hide(r); };
+	// The exact arithmetic of one pair: member k moved by trial t (t < 0: as
+	// it stands) and static slot q, or member m >= 0.  OVERLAP, BOND or 0.
+	enum : unsigned { OVERLAP = 1, BOND = 2, UNSURE = 4 };
+	auto exact_pair = [&](int k, int t, int q, int m) -> unsigned {
+		k = opaque(k);
+		q = opaque(q);
+		m = opaque(m);
+		const double *p = own + k * OWN_W, *pm = own + max(m, 0) * OWN_W, *dt = trials + t * TR_W;
+		double w[3];
+		// (the member's value is read in either case and kept, so that no
+		// pointer is chosen between LDS and HBM)
+		auto other = [&](int c) {
+			double v = pm[c];
+			asm volatile("" : "+v"(v));
+			if(m < 0) v = nbld<DD>(part(F, q) + c);
+			return v;
+		};
+#pragma unroll
+		for(int c = 0; c < 3; c++)
+			w[c] = kf_min_image(other(c) - (t >= 0 ? p[c] + dt[c] : p[c]), geo[c], geo[3 + c]);
+		const double w2 = w[0] * w[0] + w[1] * w[1] + w[2] * w[2], cosmax = geo[10];
+		if(w2 < 1.) return OVERLAP;
+		if(!(w2 < geo[9])) return 0u;
+		kf_unit(w[0], w[1], w[2], w2);
+		double O[9], P[4][3];
+#pragma unroll
+		for(int c = 0; c < 9; c++) O[c] = p[3 + c];
+		if(t >= 0) {
+			double R[9], On[9];
+#pragma unroll
+			for(int c = 0; c < 9; c++) R[c] = dt[3 + c];
+			mat_mul3(O, R, On);
+#pragma unroll
+			for(int c = 0; c < 9; c++) O[c] = On[c];
+		}
+		kf_patches(O, P);
+		if(!kf_any_p(w[0], w[1], w[2], &P[0][0], cosmax)) return 0u;
+#pragma unroll
+		for(int c = 0; c < 9; c++) O[c] = other(3 + c);
+		return kf_any_q(w[0], w[1], w[2], O, cosmax) ? BOND : 0u;
+	};
+	// within a band of one of the distance thresholds (an empty slot is not)
+	auto near_d2 = [&](float d2) { return f32_near(d2, fl) & (d2 < 0.5f * F32_FAR * F32_FAR); };
+	auto bond_f32 = [&](float e0, float e1, float e2, float dx, float dy, float dz, float d2, const float *Oq) -> unsigned {
+		const int v = f32_bond(e0, e1, e2, dx, dy, dz, d2, Oq, fl);
+		return v == KF_YES ? (unsigned) BOND : (v == KF_NO ? 0u : (unsigned) UNSURE);
+	};
+	const bool is_mem = lane < cnt;
+	const MoveShare ms = move_share(lane);
+	int c_acc = 0, d_bonds = 0;
+	unsigned known = 0;  // members whose bonds are counted in their records
+	float ft[14];
+	auto read_trial = [&](int t) {
+		const float *f = ftrial + t * FT_W;
+#pragma unroll
+		for(int e = 0; e < 14; e++) ft[e] = f[e];
+	};
+	read_trial(0);
+
+	// 5. the trials
+	for(int t = 0; t < ntrial; t++) {
+		// the trial (read one ahead), the moving member's record, another
+		// member's for a member lane, and the lane's share of the exact move
+		float tv[14];
+#pragma unroll
+		for(int e = 0; e < 14; e++) tv[e] = ft[e];
+		const int k = __float_as_int(tv[13]);
+		const float *s = shadow + k * SH_W;
+		float sv[14];
+#pragma unroll
+		for(int c = 0; c < 14; c++) sv[c] = s[c];
+		if(is_mem) {
+			if(lane == k) qx[0] = F32_FAR;
+			else {
+				const float *so = shadow + lane * SH_W;
+				qx[0] = so[0];
+				qy[0] = so[1];
+				qz[0] = so[2];
+#pragma unroll
+				for(int c = 0; c < 9; c++) qo[0][c] = so[3 + c];
+			}
+		}
+		const double *dt = trials + t * TR_W;
+		const double *me = own + k * OWN_W + ms.o, *tm = dt + ms.r;
+		const double o0 = me[0], o1 = me[ms.dot ? 1 : 0], o2 = me[ms.dot ? 2 : 0];
+		const double r0 = tm[0], r1 = tm[ms.dot ? 3 : 0], r2 = tm[ms.dot ? 6 : 0];
+		read_trial(t + 1 < ntrial ? t + 1 : t);
+		const float nx = sv[0] + tv[0], ny = sv[1] + tv[1], nz = sv[2] + tv[2];
+
+		// a trial that leaves the cell, or overlaps a neighbour, is rejected;
+		// what single precision cannot tell stays for the exact arithmetic
+		const float x = __builtin_fmaxf(__builtin_fabsf(nx) * is0, __builtin_fmaxf(__builtin_fabsf(ny) * is1,
+		                                                                         __builtin_fabsf(nz) * is2));
+		const bool close = !(__builtin_fabsf(x - 0.5f) > F32_CELL) | !(x < 1.5f);
+		bool rej = (x > 0.5f) & !close, unsure = close;
+		// slots in use by the wavefront's teams (a scalar branch)
+		auto each_slot = [&](auto &&f) {
+			f(0);
+			if constexpr(CPL > 1)
+				if(wave_2) f(1);
+		};
+		float dx[CPL], dy[CPL], dz[CPL], d2[CPL];
+		bool near[CPL];
+		each_slot([&](int u) {
+			dx[u] = qx[u] - nx;
+			dy[u] = qy[u] - ny;
+			dz[u] = qz[u] - nz;
+			d2[u] = norm2(dx[u], dy[u], dz[u]);
+			near[u] = near_d2(d2[u]);
+			rej |= (d2[u] < 1.f) & !near[u];
+		});
+		if(team_any<T>(rej)) continue;
+
+		// bonds at the new position: O'^T d = R^T (O^T d)
+		unsigned b[CPL] = {}, bo[CPL] = {};
+		each_slot([&](int u) {
+			if(d2[u] < fl.rc2) {
+				float a0, a1, a2, e0, e1, e2;
+				mul_t(sv + 3, dx[u], dy[u], dz[u], a0, a1, a2);
+				mul_t(tv + 4, a0, a1, a2, e0, e1, e2);
+				b[u] = bond_f32(e0, e1, e2, dx[u], dy[u], dz[u], d2[u], qo[u]);
+			}
+			b[u] = near[u] ? (unsigned) UNSURE : b[u];
+			unsure |= b[u] == UNSURE;
+		});
+		// the bonds at the present position, when not yet counted
+		const bool first = !((known >> k) & 1u);
+		const bool wave_first = ballot(first) != 0ull;
+		if(wave_first)
+			each_slot([&](int u) {
+				const float ex = qx[u] - sv[0], ey = qy[u] - sv[1], ez = qz[u] - sv[2];
+				const float e2 = norm2(ex, ey, ez);
+				if(e2 < fl.rc2) {
+					float a0, a1, a2;
+					mul_t(sv + 3, ex, ey, ez, a0, a1, a2);
+					bo[u] = bond_f32(a0, a1, a2, ex, ey, ez, e2, qo[u]);
+				}
+				bo[u] = near_d2(e2) ? (unsigned) UNSURE : bo[u];
+				unsure |= bo[u] == UNSURE;
+			});
+		bool late = false;  // a rejection found by the exact arithmetic
+		if(__builtin_expect(ballot(unsure) != 0ull, 0)) {
+			if(close) {
+				const Grid &G = d.reps[hide_rep()].g;
+				const int at[3] = {ix, iy, iz};
+#pragma unroll 1
+				for(int a = 0; a < 3; a++)
+					late |= cell_coord(own[k * OWN_W + a] + dt[a], G.shift[a], G.inv_box[a], G.n[a]) != at[a];
+			}
+#pragma unroll 1
+			for(int v = 0; v < 2; v++)
+#pragma unroll
+				for(int u = 0; u < CPL; u++)
+					if((v ? b[u] : bo[u]) == UNSURE) {
+						const unsigned e = exact_pair(k, v ? t : -1, cq[u], u == 0 && is_mem ? lane : -1);
+						if(v) b[u] = e;
+						else bo[u] = e;
+						late |= v && e == OVERLAP;
+					}
+			late = team_any<T>(late);
+		}
+		// the counts: static neighbours, and the members' bits
+		const unsigned mem_mask = (1u << cnt) - 1u;
+		int s_new = 0, s_old = __float_as_int(sv[12]);
+		unsigned mb = 0, mb_old = __float_as_uint(sv[13]);
+		each_slot([&](int u) {
+			const auto bits = team_bits(ballot(b[u] == BOND));
+			s_new += count_bits(bits);
+			if(u == 0) mb = (unsigned) bits & mem_mask;
+		});
+		s_new -= (int) __popc(mb);
+		if(wave_first) {
+			int so = 0;
+			unsigned mo = 0;
+			each_slot([&](int u) {
+				const auto bits = team_bits(ballot(bo[u] == BOND));
+				so += count_bits(bits);
+				if(u == 0) mo = (unsigned) bits & mem_mask;
+			});
+			mb_old = first ? mo : mb_old;
+			s_old = first ? so - (int) __popc(mo) : s_old;
+		}
+		if(wave_far) {
+			// the static neighbours beyond the register slots, from HBM
+			int n = 0;  // bonds at the new position, and << 16 at the present one
+			bool ov = false;
+			for(int i = lane + T * CPL - cnt; i < M; i += T) {
+				const int q = opaque(nb_slot(i));
+				float rel[3], Oq[9];
+				wild = false;
+#pragma unroll
+				for(int c = 0; c < 3; c++) {
+					const double p = nbld<DD>(part(F, q) + c);
+					rel[c] = (float) kf_min_image(p - geo[6 + c], geo[c], geo[3 + c]);
+					wild |= !(__builtin_fabs(p) < F32_MAX_POS);
+				}
+				const float fx = rel[0], fy = rel[1], fz = rel[2];
+				const float reach = fl.rc2 + fl.eps_d2;
+				const float gn2 = norm2(fx - nx, fy - ny, fz - nz), go2 = norm2(fx - sv[0], fy - sv[1], fz - sv[2]);
+				if(!wild && !(gn2 < reach) && !(first && go2 < reach)) continue;
+#pragma unroll
+				for(int c = 0; c < 9; c++) Oq[c] = (float) nbld<DD>(part(F, q) + 3 + c);
+				check_o(Oq);
+#pragma unroll 1
+				for(int v = first ? 0 : 1; v < 2; v++) {
+					const float gx = fx - (v ? nx : sv[0]), gy = fy - (v ? ny : sv[1]), gz = fz - (v ? nz : sv[2]);
+					const float g2 = v ? gn2 : go2;
+					unsigned bf = g2 < 1.f ? (unsigned) OVERLAP : 0u;
+					if(wild || near_d2(g2)) bf = UNSURE;
+					else if(g2 >= 1.f && g2 < fl.rc2) {
+						float a0, a1, a2, e0, e1, e2;
+						mul_t(sv + 3, gx, gy, gz, a0, a1, a2);
+						mul_t(tv + 4, a0, a1, a2, e0, e1, e2);
+						bf = bond_f32(v ? e0 : a0, v ? e1 : a1, v ? e2 : a2, gx, gy, gz, g2, Oq);
+					}
+					if(bf == UNSURE) bf = exact_pair(k, v ? t : -1, q, -1);
+					ov |= v && bf == OVERLAP;
+					n += bf == BOND ? (v ? 1 : 1 << 16) : 0;
 				}
 			}
-#pragma unroll
-			for(int u = 0; u < CPL; u++)
-#pragma unroll
-				for(int c = 0; c < 9; c++) orv[u][c] = cqr[u] >= 0 ? nbld<DD>(part(F, cqr[u]) + 3 + c) : 0.;
-		};
-		if constexpr(!DD) load_static();
-		Trial tr;
-		tr.Lx = unid<T>(rp.g.box[0]);
-		tr.Ly = unid<T>(rp.g.box[1]);
-		tr.Lz = unid<T>(rp.g.box[2]);
-		tr.iLx = unid<T>(rp.g.inv_box[0]);
-		tr.iLy = unid<T>(rp.g.inv_box[1]);
-		tr.iLz = unid<T>(rp.g.inv_box[2]);
-		tr.rc2 = unid<T>(rp.rc2);
-		tr.cosmax = unid<T>(rp.cosmax);
-		tr.c2 = tr.cosmax >= KF_FILTER_MIN_COS ? tr.cosmax * tr.cosmax : -1.;
-		const double temp = unid<T>(rp.T);
-		const double sh0 = rp.g.shift[0], sh1 = rp.g.shift[1], sh2 = rp.g.shift[2];
-		const int n0 = uni<T>(rp.g.n[0]), n1 = uni<T>(rp.g.n[1]), n2 = uni<T>(rp.g.n[2]);
-		const int ix = cloc / (n1 * n2), iy = (cloc / n2) % n1, iz = cloc % n2;
-
-		// 3. the cell's trials, one lane each (Philox: no memory traffic),
-		// and the particle indices into LDS.  A trial's slot 0 (the member
-		// rank) is replaced by its acceptance bits: bit j is set iff the draw
-		// u < exp(-j/T), the replica's factor for a rise of j bonds
-		// (MC.c:332), so a trial decides without a table read.  Lane t keeps
-		// trial t's rank.
-		int my_k = 0;
-		double my_dl = 0.;  // (REACH) the length of this lane's trial displacement
-		if(lane < ntrial) {
-			double tv[TRIAL_W];
-			const int col = ((ix & 1) << 2) | ((iy & 1) << 1) | (iz & 1);
-			make_trial(d, rp, r, sweep, cloc, col, lane, cnt, tv);
-			if constexpr(REACH) my_dl = __builtin_sqrt(tv[1] * tv[1] + tv[2] * tv[2] + tv[3] * tv[3]);
-			unsigned am = 0;
-#pragma unroll
-			for(int j = 1; j < ACC_TAB; j++) am |= (unsigned) (tv[13] < rp.acc_tab[j]) << j;
-			my_k = (int) tv[0];
-			tv[0] = (double) am;
-#pragma unroll
-			for(int e = 0; e < TRIAL_W; e++) trials[lane * TRIAL_W + e] = tv[e];
+			late |= team_any<T>(ov);
+			n = team_sum<T>(n);
+			s_new += n & 0xffff;
+			if(first) s_old += n >> 16;
 		}
-		static_assert(MAX_TRIALS_PER_CELL <= 32 && CELL_CAP <= 32, "one lane per trial");
-		const int koff = (threadIdx.x & 63) & ~(T - 1);
-		if(lane < cnt) own_pid[lane] = my_pid;
-		if constexpr(!REG_ORI && !DD && !REACH) {
-#pragma unroll
-			for(int u = 0; u < CPL; u++)
-#pragma unroll
-				for(int c = 0; c < 9; c++) ori[(9 * u + c) * T + lane] = orv[u][c];
+		known |= 1u << k;
+		const int db = s_new + (int) __popc(mb) - s_old - (int) __popc(mb_old);
+		// MC.c:332: accept if dE <= 0 or a uniform draw u < exp(-dE/T), with
+		// dE = -db an integer: below ACC_TAB the trial holds the comparison
+		bool acc = -db <= __float_as_int(tv[3]);
+		if(ballot(-db >= ACC_TAB) != 0ull && -db >= ACC_TAB) {
+			const u32x4 rb = rng(d.seed, r, sweep, (uint32_t) hide(cloc), TAG_TRIAL_B, (uint32_t) col, (uint32_t) t);
+			acc = u01(rb.w) < exp((double) db / d.reps[hide_rep()].T);
 		}
+		if(acc && !late) {
+			c_acc++;
+			d_bonds += db;
+			// the new state, one value per lane, exact and single precision;
+			// lanes 0 and 1 write the new static count and member bits
+			const double rv = ms.dot ? o0 * r0 + o1 * r1 + o2 * r2 : o0 + r0;
+			if(lane < 15) {
+				own[k * OWN_W + lane] = rv;
+				shadow[k * SH_W + ms.word] =
+				    lane == 0 ? __int_as_float(s_new) : (lane == 1 ? __uint_as_float(mb) : (float) rv);
+			}
+			// the other members' bits for member k
+			if(is_mem && lane != k) {
+				unsigned *w = (unsigned *) (shadow + lane * SH_W + 13);
+				*w = (*w & ~(1u << k)) | ((b[0] >> 1) << k);
+			}
+		}
+		else if(first && lane < 2)
+			shadow[k * SH_W + 12 + lane] = lane == 0 ? __int_as_float(s_old) : __uint_as_float(mb_old);
 		team_sync();
-		// 4. members into LDS ranked by particle index, with their patch vectors
+	}
+	// 6. write the members back, ranked (the ranking permutes the cell's slots)
+	if(c_acc > 0 || cnt > 1) {
+		const int at = hide(s0);
+		for(int e = lane; e < cnt * NCOMP; e += T) {
+			int m = e / NCOMP, c = e - m * NCOMP;
+			if constexpr(DD)
+				__hip_atomic_store(part(F, at + m) + c, own[m * OWN_W + c], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+			else part(F, at + m)[c] = own[m * OWN_W + c];
+		}
 		if(lane < cnt) {
 			int rank = 0;
 			for(int m = 0; m < cnt; m++) rank += own_pid[m] < my_pid;
-			double *w = own + rank * OWN_W;
-#pragma unroll
-			for(int c = 0; c < NCOMP; c++) w[c] = mine[c];
-			double P[4][3];
-			kf_patches(mine + 3, P);
-#pragma unroll
-			for(int i = 0; i < 4; i++)
-#pragma unroll
-				for(int c = 0; c < 3; c++) w[NCOMP + 3 * i + c] = P[i][c];
+			PID[at + rank] = my_pid;
 		}
-		team_sync();
-		if constexpr(REACH) {
-			// Keep only the static neighbours a member can reach.  No member
-			// travels further during the pass than S, the summed lengths of
-			// the cell's trial displacements (triangle inequality on the
-			// periodic box), so a neighbour further than 1 + delta + S from
-			// every member's start can neither overlap nor bond with any
-			// trial position: dropping it changes no decision.  The kept ones
-			// are compacted into the register slots after the members (most
-			// teams then need one slot per lane) through the orientation
-			// block of LDS, 8 values then 5 values per slot.
-			const double S = team16_sum_f64(my_dl);
-			const double reach = __builtin_sqrt(tr.rc2) + S + REACH_EPS;
-			const double reach2 = reach * reach;
-			bool keep_u[CPL];
-#pragma unroll
-			for(int u = 0; u < CPL; u++) {
-				double dmin2 = reach2;
-				if(cqr[u] >= 0)
-					for(int m = 0; m < cnt; m++) {
-						const double *wm = own + m * OWN_W;
-						const double dx = kf_min_image(cxr[u] - wm[0], tr.Lx, tr.iLx);
-						const double dy = kf_min_image(cyr[u] - wm[1], tr.Ly, tr.iLy);
-						const double dz = kf_min_image(czr[u] - wm[2], tr.Lz, tr.iLz);
-						dmin2 = __builtin_fmin(dmin2, dx * dx + dy * dy + dz * dz);
-					}
-				keep_u[u] = cqr[u] >= 0 && dmin2 < reach2;
-			}
-			static_assert(!REACH || (T == 16 && CPL == 2), "reach filter: 16-lane teams, two slots per lane");
-			const unsigned long long tmask = ((1ull << T) - 1ull) << koff;
-			const unsigned long long k0 = __ballot(keep_u[0]) & tmask, k1 = __ballot(keep_u[CPL - 1]) & tmask;
-			const int n0 = __popcll(k0), nr = n0 + __popcll(k1);
-			const int dst[2] = {cnt + lanes_below(k0), cnt + n0 + lanes_below(k1)};
-			double *stg = ori;  // value v of slot j at stg[32 v + j]
-			double stale[CPL][5];
-#pragma unroll
-			for(int u = 0; u < CPL; u++) {
-#pragma unroll
-				for(int c = 0; c < 5; c++) stale[u][c] = orv[u][4 + c];
-				if(keep_u[u]) {
-					const int j = dst[u];
-					stg[j] = (double) cqr[u];
-					stg[32 + j] = cxr[u];
-					stg[64 + j] = cyr[u];
-					stg[96 + j] = czr[u];
-#pragma unroll
-					for(int c = 0; c < 4; c++) stg[32 * (4 + c) + j] = orv[u][c];
-				}
-			}
-			team_sync();
-#pragma unroll
-			for(int u = 0; u < CPL; u++) {
-				const int j = lane + u * T;
-				const bool in = j >= cnt && j < cnt + nr;
-				cqr[u] = in ? (int) stg[j] : -1;
-				cxr[u] = in ? stg[32 + j] : 0.;
-				cyr[u] = in ? stg[64 + j] : 0.;
-				czr[u] = in ? stg[96 + j] : 0.;
-#pragma unroll
-				for(int c = 0; c < 4; c++) orv[u][c] = in ? stg[32 * (4 + c) + j] : 0.;
-			}
-			team_sync();
-#pragma unroll
-			for(int u = 0; u < CPL; u++)
-				if(keep_u[u])
-#pragma unroll
-					for(int c = 0; c < 5; c++) stg[32 * c + dst[u]] = stale[u][c];
-			team_sync();
-#pragma unroll
-			for(int u = 0; u < CPL; u++) {
-				const int j = lane + u * T;
-				const bool in = j >= cnt && j < cnt + nr;
-#pragma unroll
-				for(int c = 0; c < 5; c++) orv[u][4 + c] = in ? stg[32 * c + j] : 0.;
-			}
-			team_sync();
-			if constexpr(!REG_ORI) {
-#pragma unroll
-				for(int u = 0; u < CPL; u++)
-#pragma unroll
-					for(int c = 0; c < 9; c++) ori[(9 * u + c) * T + lane] = orv[u][c];
-			}
-			team_sync();
-		}
-		if constexpr(DD) {
-			// the neighbours' data once their earlier passes are done
-			wait_neighbours<T>(d, rp, nb_tab, pass, ix, iy, iz, n0, n1, n2, mark, lane);
-			load_static();
-			if constexpr(!REG_ORI) {
-#pragma unroll
-				for(int u = 0; u < CPL; u++)
-#pragma unroll
-					for(int c = 0; c < 9; c++) ori[(9 * u + c) * T + lane] = orv[u][c];
-			}
-			team_sync();
-		}
-		// (orientations in LDS) a member slot's orientation, kept current by
-		// the trials that move it
-		if constexpr(!REG_ORI)
-			if(lane < cnt) {
-#pragma unroll
-				for(int c = 0; c < 9; c++) ori[c * T + lane] = own[lane * OWN_W + 3 + c];
-			}
-		// the orientation of the neighbour in register slot u
-		auto reg_o = [&](int u, double *Oq) {
-#pragma unroll
-			for(int c = 0; c < 9; c++) Oq[c] = REG_ORI ? orv[u][c] : ori[(9 * u + c) * T + lane];
-		};
-		// whether any team of the wavefront has neighbours beyond the
-		// register slots (a scalar branch around those loops)
-		const bool wave_far = __ballot(M + cnt > T * CPL) != 0ull;
-		// the static neighbours beyond the register slots, from HBM
-		auto each_far = [&](auto &&f) {
-			if(wave_far)
-				for(int b = T * CPL - cnt; b < M; b += T)
-					if(b + lane < M) {
-						const int q = nb_slot(b + lane);
-						f(nbld<DD>(part(F, q)), nbld<DD>(part(F, q) + 1), nbld<DD>(part(F, q) + 2), [&](double *Oq) {
-#pragma unroll
-							for(int c = 0; c < 9; c++) Oq[c] = nbld<DD>(part(F, q) + 3 + c);
-						});
-					}
-		};
-		team_sync();
-		// 5. KEEP: every member's bonds with the static neighbours, and with
-		// each other
-		unsigned mbits = 0;
-		if constexpr(KEEP) {
-			// each member lane's own member in its first register slot (the
-			// trials refresh it as members move)
-			const bool mem_lane = lane < cnt;
-			if(mem_lane) {
-				const double *wl = own + lane * OWN_W;
-				cxr[0] = wl[0];
-				cyr[0] = wl[1];
-				czr[0] = wl[2];
-				if constexpr(REG_ORI)
-#pragma unroll
-					for(int c = 0; c < 9; c++) orv[0][c] = wl[3 + c];
-			}
-			// Two members at a time (independent chains), one reduction for
-			// both.  Each lane tests its register slots against member mm: a
-			// static neighbour adds to the member's kept count; another
-			// member sets a bit of the lane's mbits (bit mm of lane j iff
-			// members j and mm are bonded: the pair decision is symmetric).
-			auto slot_for = [&](int u, int mm) { return u == 0 && mem_lane ? lane != mm : cqr[u] >= 0; };
-			auto add = [&](int u, int b, int &bs, int &bm) {
-				if(u == 0 && mem_lane) bm = b;
-				else bs += b;
-			};
-			for(int m = 0; m < cnt; m += 2) {
-				const bool two = m + 1 < cnt;
-				const double *w0 = own + m * OWN_W, *w1 = own + (two ? m + 1 : m) * OWN_W;
-				Trial t0 = tr, t1 = tr;
-				t0.nx = unid<T>(w0[0]);
-				t0.ny = unid<T>(w0[1]);
-				t0.nz = unid<T>(w0[2]);
-				t1.nx = unid<T>(w1[0]);
-				t1.ny = unid<T>(w1[1]);
-				t1.nz = unid<T>(w1[2]);
-				double P0[12], P1[12];
-#pragma unroll
-				for(int c = 0; c < 12; c++) {
-					P0[c] = w0[NCOMP + c];
-					P1[c] = w1[NCOMP + c];
-				}
-				int b0 = 0, b1 = 0, mb0 = 0, mb1 = 0;
-				bool band0 = tr.c2 < 0., band1 = band0;
-				if(!band0) {
-#pragma unroll
-					for(int u = 0; u < CPL; u++) {
-						auto lo = [&](double *Oq) { reg_o(u, Oq); };
-						if(slot_for(u, m)) {
-							int b = 0;
-							bonds_new(t0, P0, cxr[u], cyr[u], czr[u], lo, b, band0);
-							add(u, b, b0, mb0);
-						}
-						if(two && slot_for(u, m + 1)) {
-							int b = 0;
-							bonds_new(t1, P1, cxr[u], cyr[u], czr[u], lo, b, band1);
-							add(u, b, b1, mb1);
-						}
-					}
-					each_far([&](double qx, double qy, double qz, auto load_o) {
-						bonds_new(t0, P0, qx, qy, qz, load_o, b0, band0);
-						if(two) bonds_new(t1, P1, qx, qy, qz, load_o, b1, band1);
-					});
-				}
-				if(__ballot(band0) != 0ull && team_any<T>(band0) && band0) {
-					b0 = 0;
-					mb0 = 0;
-#pragma unroll
-					for(int u = 0; u < CPL; u++)
-						if(slot_for(u, m)) {
-							int b = 0;
-							bonds_new_exact(t0, P0, cxr[u], cyr[u], czr[u], [&](double *Oq) { reg_o(u, Oq); }, b);
-							add(u, b, b0, mb0);
-						}
-					each_far([&](double qx, double qy, double qz, auto load_o) {
-						bonds_new_exact(t0, P0, qx, qy, qz, load_o, b0);
-					});
-				}
-				if(__ballot(band1) != 0ull && team_any<T>(band1) && band1) {
-					b1 = 0;
-					mb1 = 0;
-#pragma unroll
-					for(int u = 0; u < CPL; u++)
-						if(slot_for(u, m + 1)) {
-							int b = 0;
-							bonds_new_exact(t1, P1, cxr[u], cyr[u], czr[u], [&](double *Oq) { reg_o(u, Oq); }, b);
-							add(u, b, b1, mb1);
-						}
-					each_far([&](double qx, double qy, double qz, auto load_o) {
-						bonds_new_exact(t1, P1, qx, qy, qz, load_o, b1);
-					});
-				}
-				// (each count is below the team's neighbour count, M < 65536)
-				const int b = team_sum<T>(b0 | (b1 << 16));
-				if(lane == 0) {
-					sbond[m] = b & 0xffff;
-					if(two) sbond[m + 1] = b >> 16;
-				}
-				if(mem_lane) mbits |= ((unsigned) mb0 << m) | (two ? (unsigned) mb1 << (m + 1) : 0u);
-			}
-			team_sync();
-			// The members' fractional coordinates inside the cell, u = (cell
-			// coordinate as cell_coord forms it) - (ix, iy, iz), kept in the
-			// record's patch slots (the kept form reads no old patches): a
-			// trial whose u + displacement stays 1e-9 cells clear of the
-			// faces cannot leave the cell (cell_coord's roundings are below
-			// 1e-13 cells), so it skips the exact test.
-			if(lane < cnt) {
-				double *wm = own + lane * OWN_W;
-				const double p3[3] = {wm[0], wm[1], wm[2]};
-				const double sh[3] = {sh0, sh1, sh2}, il[3] = {tr.iLx, tr.iLy, tr.iLz};
-				const int nn[3] = {n0, n1, n2}, ii[3] = {ix, iy, iz};
-#pragma unroll
-				for(int a = 0; a < 3; a++) {
-					double t = (p3[a] - sh[a]) * il[a];
-					t = t - __builtin_floor(t);
-					wm[NCOMP + a] = t * (double) nn[a] - (double) ii[a];
-				}
-			}
-			team_sync();
-		}
-		// cells per unit length along each axis (the u step of a displacement)
-		const double gnx = (double) n0 * tr.iLx, gny = (double) n1 * tr.iLy, gnz = (double) n2 * tr.iLz;
-		int c_acc = 0, d_bonds = 0;
-		// this lane's share of a trial's O' and patches (see the trial loop):
-		// value lane, and with T < 21 also value lane + T
-		static_assert(T >= 16 && CELL_CAP <= 32, "a team of 16 lanes or more");
-		const RotShare rsh = rot_share(lane), rsh2 = rot_share(lane + T);
-
-		for(int t = 0; t < ntrial; t++) {
-			// the moving member's rank, read from lane t of the team; then one
-			// LDS read round: the trial, the member's state and this lane's
-			// member
-			int k;
-			static_assert(T == 16 || T == 32 || T == 64, "teams of 16, 32 or 64 lanes");
-			if constexpr(T == 64) k = __builtin_amdgcn_readlane(my_k, t);
-			else if constexpr(T == 32) {
-				const int k0 = __builtin_amdgcn_readlane(my_k, t), k1 = __builtin_amdgcn_readlane(my_k, t + 32);
-				k = koff ? k1 : k0;
-			}
-			else {
-				const int k0 = __builtin_amdgcn_readlane(my_k, t), k1 = __builtin_amdgcn_readlane(my_k, t + 16);
-				const int k2 = __builtin_amdgcn_readlane(my_k, t + 32), k3 = __builtin_amdgcn_readlane(my_k, t + 48);
-				k = koff < 32 ? (koff ? k1 : k0) : (koff == 32 ? k2 : k3);
-			}
-			const double *tp = trials + t * TRIAL_W;
-			double tv[TRIAL_W];
-#pragma unroll
-			for(int e = 0; e < TRIAL_W; e++) tv[e] = tp[e];
-			// a member slot: the member's current state (every member but the
-			// moving one is a neighbour of the trial; a cell of one member
-			// reads nothing here)
-			const bool is_mem = lane < cnt;
-			const bool has_m = is_mem && lane != k;
-			if(has_m) {
-				const double *wl = own + lane * OWN_W;
-				cxr[0] = wl[0];
-				cyr[0] = wl[1];
-				czr[0] = wl[2];
-				if constexpr(REG_ORI)
-#pragma unroll
-					for(int c = 0; c < 9; c++) orv[0][c] = wl[3 + c];
-			}
-			// register slot u holds a neighbour of this trial
-			auto has_slot = [&](int u) { return u == 0 && is_mem ? has_m : cqr[u] >= 0; };
-			const double *me = own + k * OWN_W;
-			double ux = 0., uy = 0., uz = 0.;  // (kept form) the member's u
-			if constexpr(KEEP) {
-				ux = me[NCOMP];
-				uy = me[NCOMP + 1];
-				uz = me[NCOMP + 2];
-			}
-			// the rows of the member's O that the lane's share of O' needs
-			const double *orow = me + 3 + 3 * rsh.row;
-			const double o0 = orow[0], o1 = orow[1], o2 = orow[2];
-			double o3 = 0., o4 = 0., o5 = 0.;
-			if constexpr(T < 21) {
-				const double *orow2 = me + 3 + 3 * rsh2.row;
-				o3 = orow2[0];
-				o4 = orow2[1];
-				o5 = orow2[2];
-			}
-			double Po[12];  // the old patches (two-sided tests only)
-			if constexpr(!KEEP)
-#pragma unroll
-				for(int c = 0; c < 12; c++) Po[c] = me[NCOMP + c];
-			tr.px = unid<T>(me[0]);
-			tr.py = unid<T>(me[1]);
-			tr.pz = unid<T>(me[2]);
-			tr.nx = unid<T>(tr.px + tv[1]);
-			tr.ny = unid<T>(tr.py + tv[2]);
-			tr.nz = unid<T>(tr.pz + tv[3]);
-			// a trial that leaves the cell is rejected
-			// (kept form: skipped when u + displacement is clear of the faces)
-			double cu0 = 0., cu1 = 0., cu2 = 0.;
-			bool deep = false;
-			if constexpr(KEEP) {
-				cu0 = __builtin_fma(tv[1], gnx, ux);  // u is an estimate: fused is fine
-				cu1 = __builtin_fma(tv[2], gny, uy);
-				cu2 = __builtin_fma(tv[3], gnz, uz);
-				constexpr double CELL_EPS = 1e-9;
-				deep = __builtin_fmax(__builtin_fabs(cu0 - 0.5), __builtin_fmax(__builtin_fabs(cu1 - 0.5),
-				                                                               __builtin_fabs(cu2 - 0.5))) <
-				       0.5 - CELL_EPS;
-			}
-			if(!deep) {
-				// all three axes evaluated (no short circuit)
-				const int out = (int) (uni<T>(cell_coord(tr.nx, sh0, tr.iLx, n0)) != ix) |
-				                (int) (uni<T>(cell_coord(tr.ny, sh1, tr.iLy, n1)) != iy) |
-				                (int) (uni<T>(cell_coord(tr.nz, sh2, tr.iLz, n2)) != iz);
-				if(out) continue;
-			}
-
-			// phase 1: hard cores at the new position, wavefront-ballot early exit
-			// (the register neighbours' separations are kept for phase 2)
-			bool ov = false;
-			double sx[CPL], sy[CPL], sz[CPL], s2[CPL];
-#pragma unroll
-			for(int u = 0; u < CPL; u++)
-				if(has_slot(u)) {
-					s2[u] = sep_new(tr, cxr[u], cyr[u], czr[u], sx[u], sy[u], sz[u]);
-					ov |= s2[u] < 1.;
-				}
-			if(wave_far)
-				for(int b = T * CPL - cnt; b < M; b += T)
-					if(b + lane < M) {
-						const int q = nb_slot(b + lane);
-						ov |= overlaps_new(tr, nbld<DD>(part(F, q)), nbld<DD>(part(F, q) + 1), nbld<DD>(part(F, q) + 2));
-					}
-			if(team_any<T>(ov)) continue;
-
-			// O' = O R in the body frame (utils.c:172-184, 204-209) and its
-			// patches (utils.h:17-21), one value per lane (two on some lanes of
-			// a 16-lane team) in the reference's order: value v < 9 is O'[v],
-			// v = 9 + 3a + kk the patch component P'[a][kk] (rot_value).  The
-			// values meet in the stage row.
-			double rv = 0., rv2 = 0.;
-			if(lane < 21) {
-				rv = rot_value(rsh, o0, o1, o2, tv);
-				stage[lane] = rv;
-			}
-			if constexpr(T < 21)
-				if(lane + T < 21) {
-					rv2 = rot_value(rsh2, o3, o4, o5, tv);
-					stage[lane + T] = rv2;
-				}
-			team_sync();
-			double Pn[12];
-#pragma unroll
-			for(int c = 0; c < 12; c++) Pn[c] = stage[9 + c];
-
-			// phase 2: bonds at the old and the new position, over this lane's
-			// neighbours: its register slots (a member or static neighbours;
-			// KEEP: new position only, the old count is the member's kept one)
-			// and the static neighbours beyond them
-			int bo, bn, s_new = 0, bnm = 0;
-			if constexpr(KEEP) {
-				int bns = 0;
-				const int bom = has_m ? (int) ((mbits >> k) & 1u) : 0;
-				// a register slot's bond: with a member (slot 0 of a member
-				// lane) or with a static neighbour
-				auto add_slot = [&](int u, int b) {
-					if(u == 0) {
-						bnm += is_mem ? b : 0;
-						bns += is_mem ? 0 : b;
-					}
-					else bns += b;
-				};
-				bool band = tr.c2 < 0.;  // no filter: every lane takes the exact form
-				if(!band) {
-#pragma unroll
-					for(int u = 0; u < CPL; u++)
-						if(has_slot(u)) {
-							int b = 0;
-							bonds_new_sep(tr, Pn, sx[u], sy[u], sz[u], s2[u], [&](double *Oq) { reg_o(u, Oq); }, b,
-							              band);
-							add_slot(u, b);
-						}
-					each_far([&](double qx, double qy, double qz, auto load_o) {
-						bonds_new(tr, Pn, qx, qy, qz, load_o, bns, band);
-					});
-				}
-				if(__ballot(band) != 0ull && team_any<T>(band) && band) {
-					bns = 0;
-					bnm = 0;
-#pragma unroll
-					for(int u = 0; u < CPL; u++)
-						if(has_slot(u)) {
-							int b = 0;
-							bonds_new_exact(tr, Pn, cxr[u], cyr[u], czr[u], [&](double *Oq) { reg_o(u, Oq); }, b);
-							add_slot(u, b);
-						}
-					each_far([&](double qx, double qy, double qz, auto load_o) {
-						bonds_new_exact(tr, Pn, qx, qy, qz, load_o, bns);
-					});
-				}
-				// three counts below 1024 in one reduction
-				const int packed = team_sum<T>(bns | (bnm << 10) | (bom << 20));
-				s_new = packed & 1023;
-				bo = sbond[k] + (packed >> 20);
-				bn = s_new + ((packed >> 10) & 1023);
-			}
-			else {
-				bo = 0;
-				bn = 0;
-				bool band = tr.c2 < 0.;
-				auto each_neighbour = [&](auto &&f) {
-#pragma unroll
-					for(int u = 0; u < CPL; u++)
-						if(has_slot(u)) f(cxr[u], cyr[u], czr[u], [&](double *Oq) { reg_o(u, Oq); });
-					each_far(f);
-				};
-				if(!band)
-					each_neighbour([&](double qx, double qy, double qz, auto load_o) {
-						bonds_old_new(tr, Po, Pn, qx, qy, qz, load_o, bo, bn, band);
-					});
-				if(__ballot(band) != 0ull && team_any<T>(band) && band) {
-					bo = 0;
-					bn = 0;
-					each_neighbour([&](double qx, double qy, double qz, auto load_o) {
-						bonds_old_new_exact(tr, Po, Pn, qx, qy, qz, load_o, bo, bn);
-					});
-				}
-				bo = team_sum_small<T>(bo);
-				bn = team_sum_small<T>(bn);
-			}
-			const int db = bn - bo;  // E = -bonds, dE = -db
-			const double dE = (double) (-db);
-			// MC.c:332: accept if dE < 0 or a uniform draw u < exp(-dE/T); dE
-			// is an integer: below ACC_TAB the trial's acceptance bits hold
-			// the comparison with the replica's exp(-dE/T)
-			const int idE = -db;
-			const unsigned am = (unsigned) tv[0];
-			const bool acc = idE < 0 ||
-			                 (idE == 0 ? tv[13] < 1.
-			                           : (idE < ACC_TAB ? ((am >> idE) & 1u) != 0u : tv[13] < exp(-dE / temp)));
-			if(acc) {
-				c_acc++;
-				d_bonds += db;
-				// member k takes the new position, orientation and patches
-				// (O' and P' are contiguous in its record, lane l's at 3 + l)
-				double *wk = own + k * OWN_W;
-				// (the kept form keeps u in the patch slots instead of P')
-				constexpr int NW = KEEP ? 9 : 21;
-				if(lane < NW) wk[3 + lane] = rv;
-				if constexpr(T < NW)
-					if(lane + T < NW) wk[3 + lane + T] = rv2;
-				// (orientations in LDS) and into member k's register slot
-				if constexpr(!REG_ORI)
-					if(lane < 9) ori[lane * T + k] = rv;
-				if(lane == 0) {
-					wk[0] = tr.nx;
-					wk[1] = tr.ny;
-					wk[2] = tr.nz;
-					if constexpr(KEEP) {
-						wk[NCOMP] = cu0;
-						wk[NCOMP + 1] = cu1;
-						wk[NCOMP + 2] = cu2;
-					}
-					if constexpr(KEEP) sbond[k] = s_new;
-				}
-				if constexpr(KEEP) {
-					// member k's bonds with the others are now the new ones
-					const unsigned long long nb_bits =
-					    (__ballot(bnm != 0) >> koff) & (T >= 32 ? 0xffffffffull : ((1ull << T) - 1ull));
-					if(lane < cnt) mbits = lane == k ? (unsigned) nb_bits : ((mbits & ~(1u << k)) | ((unsigned) bnm << k));
-				}
-			}
-			team_sync();
-		}
-		// 6. write the members back, ranked (the ranking permutes the cell's slots)
-		if(c_acc > 0 || cnt > 1) {
-			for(int e = lane; e < cnt * NCOMP; e += T) {
-				int m = e / NCOMP, c = e - m * NCOMP;
-				if constexpr(DD)
-					__hip_atomic_store(part(F, s0 + m) + c, own[m * OWN_W + c], __ATOMIC_RELAXED,
-					                   __HIP_MEMORY_SCOPE_AGENT);
-				else part(F, s0 + m)[c] = own[m * OWN_W + c];
-			}
-			if(lane < cnt) {
-				int rank = 0;
-				for(int m = 0; m < cnt; m++) rank += own_pid[m] < my_pid;
-				PID[s0 + rank] = my_pid;
-			}
-		}
-		if constexpr(DD) {
-			// the members' stores have completed (the wavefront's memory
-			// counter is zero) before the cell is published as done
-			__atomic_signal_fence(__ATOMIC_SEQ_CST);
-			__builtin_amdgcn_s_waitcnt(0);
-			__atomic_signal_fence(__ATOMIC_SEQ_CST);
-			if(lane == 0)
-				__hip_atomic_store(d.done + rp.cell_off + cloc, mark, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-		}
-		if(lane == 0) {
-			const int slot = gi & (NSLOT - 1);
-			atomicAdd(ctr_at(d.ctr, r, C_TRY_ROTO, slot), (unsigned long long) ntrial);
-			if(c_acc) {
-				atomicAdd(ctr_at(d.ctr, r, C_ACC_ROTO, slot), (unsigned long long) c_acc);
-				atomicAdd(ctr_at(d.ctr, r, C_DBONDS, slot), (unsigned long long) (long long) d_bonds);
-			}
+	}
+	if constexpr(DD) {
+		// the members' stores have completed (the wavefront's memory
+		// counter is zero) before the cell is published as done
+		__atomic_signal_fence(__ATOMIC_SEQ_CST);
+		__builtin_amdgcn_s_waitcnt(0);
+		__atomic_signal_fence(__ATOMIC_SEQ_CST);
+		if(lane == 0) __hip_atomic_store(d.done + rp.cell_off + cloc, mark, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+	}
+	if(lane == 0) {
+		const int slot = gi & (NSLOT - 1);
+		atomicAdd(ctr_at(d.ctr, r, C_TRY_ROTO, slot), (unsigned long long) ntrial);
+		if(c_acc) {
+			atomicAdd(ctr_at(d.ctr, r, C_ACC_ROTO, slot), (unsigned long long) c_acc);
+			atomicAdd(ctr_at(d.ctr, r, C_DBONDS, slot), (unsigned long long) (long long) d_bonds);
 		}
 	}
 }
@@ -1432,7 +1217,7 @@ __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int
 // list is in cell order, so XCD x takes the x-th eighth of the entries
 // actually listed (a slab of the box, whose shared neighbour reads its L2
 // then serves); the surplus workgroups of each XCD leave at once.
-template <int T, int CPL, bool KEEP, bool ONE, int CAP = CELL_CAP>
+template <int T, int CPL, bool ONE, int CAP = CELL_CAP>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_pass(PassArgs a) {
 	extern __shared__ double lds[];
 	const int lane = threadIdx.x & (T - 1);
@@ -1444,14 +1229,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 	if(i >= per_xcd) return;
 	const int gi = uni<T>(((blockIdx.x & 7) * per_xcd + i) * tpb + team);
 	if(gi >= total) return;
-	// 16-lane teams with two slots per lane keep the reachable neighbours only
-	pass_cell<T, CPL, KEEP, ONE, false, T == 16 && CPL == 2 && KEEP, CAP>(a.d, a.sweep, a.pass, gi, lane,
-	                                                                       lds + team * team_lds<T, CAP>(), 0u);
+	pass_cell<T, CPL, ONE, false, CAP>(a.d, a.sweep, a.pass, gi, lane, lds + team * team_lds<CAP>(), 0u);
 }
 
 // The cells the small-cell pass deferred (more than SMALL_CAP members), by
 // the general 32-lane form: teams take the listed entries in turn.
-template <bool KEEP, bool ONE>
+template <bool ONE>
 __global__ __launch_bounds__(128) void k_pass_ovf(PassArgs a) {
 	extern __shared__ double lds[];
 	constexpr int T = 32;
@@ -1460,7 +1243,7 @@ __global__ __launch_bounds__(128) void k_pass_ovf(PassArgs a) {
 	const int tpb = blockDim.x / T;
 	const int n = a.d.ovf_n[a.pass];
 	for(int e = blockIdx.x * tpb + team; e < n; e += gridDim.x * tpb)
-		pass_cell<T, 1, KEEP, ONE, false>(a.d, a.sweep, a.pass, a.d.ovf[e], lane, lds + team * team_lds<T>(), 0u);
+		pass_cell<T, 2, ONE, false>(a.d, a.sweep, a.pass, a.d.ovf[e], lane, lds + team * team_lds<>(), 0u);
 }
 
 // The 8 colour passes of a sweep in one launch, driven by dependencies
@@ -1477,7 +1260,7 @@ __global__ __launch_bounds__(128) void k_pass_ovf(PassArgs a) {
 // once.  Results equal the per-pass launches' bit for bit: each cell sees its
 // neighbourhood as the earlier passes left it, and its trials do not depend
 // on timing.
-template <int T, int CPL, bool KEEP, bool ONE>
+template <int T, bool ONE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_pass_dd(PassArgs a) {
 	extern __shared__ double lds[];
 	const DevState &d = a.d;
@@ -1495,7 +1278,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 		base += padded;
 	}
 	if(p == 8 || t - base >= n) return;
-	pass_cell<T, CPL, KEEP, ONE, true>(d, a.sweep, p, t - base, lane, lds + team * team_lds<T>(), a.mark);
+	pass_cell<T, T < 64 ? 2 : 1, ONE, true>(d, a.sweep, p, t - base, lane, lds + team * team_lds<>(), a.mark);
 }
 
 // Grid-wide barrier of a cooperative launch (every workgroup resident).
@@ -1531,7 +1314,7 @@ __device__ __forceinline__ void grid_barrier(unsigned *bar, int *err) {
 
 // The 8 colour passes of a sweep in one cooperative launch, separated by
 // grid barriers.  Team g takes list entries g, g + teams, ... of each pass.
-template <int T, int CPL, bool KEEP>
+template <int T>
 __global__ __launch_bounds__(256) void k_sweep_passes(PassArgs a) {
 	extern __shared__ double lds[];
 	const DevState &d = a.d;
@@ -1540,130 +1323,96 @@ __global__ __launch_bounds__(256) void k_sweep_passes(PassArgs a) {
 	const int tpb = blockDim.x / T;
 	const int nteams = gridDim.x * tpb;
 	const int g0 = uni<T>(blockIdx.x * tpb + team);
-	double *own = lds + team * team_lds<T>();
+	double *own = lds + team * team_lds<>();
 	for(int k = 0; k < 8; k++) {
 		const int total = uni<T>(d.pfx[k * (d.R + 1) + d.R]);
-		for(int gi = g0; gi < total; gi += nteams) pass_cell<T, CPL, KEEP, false, false>(d, a.sweep, k, gi, lane, own, 0u);
+		for(int gi = g0; gi < total; gi += nteams) pass_cell<T, T < 64 ? 2 : 1, false, false>(d, a.sweep, k, gi, lane, own, 0u);
 		if(k < 7) grid_barrier(d.bar, d.err);
 	}
 }
 
-template <int T, int CPL, bool KEEP, bool ONE>
+template <int T, bool ONE>
 static void pass_dd_T(const DevState &d, uint64_t sweep, unsigned mark, int block, hipStream_t s) {
 	const int tpb = block / T;
 	// every pass's largest list, one team per entry (wavefronts past the
 	// sweep's tickets leave at once)
 	const unsigned nb = (unsigned) std::max(1, 8 * ((d.total_act + tpb - 1) / tpb));
-	size_t lds = (size_t) tpb * team_lds<T>() * sizeof(double);
 	PassArgs a{d, sweep, 0, mark};
-	hipLaunchKernelGGL((k_pass_dd<T, CPL, KEEP, ONE>), dim3(nb), dim3(block), lds, s, a);
-}
-
-template <int T, bool KEEP>
-static void pass_dd_TK(const DevState &d, uint64_t sweep, unsigned mark, int block, hipStream_t s) {
-	if(d.R == 1) pass_dd_T<T, 1, KEEP, true>(d, sweep, mark, block, s);
-	else pass_dd_T<T, 1, KEEP, false>(d, sweep, mark, block, s);
+	hipLaunchKernelGGL((k_pass_dd<T, ONE>), dim3(nb), dim3(block), pass_lds_bytes(T, block), s, a);
 }
 
 void launch_passes_dd(const DevState &d, uint64_t sweep, unsigned mark, int T, int block, hipStream_t s) {
-	const bool keep = d.trials_per_cell >= KEEP_MIN_TRIALS;
 	if(T == 32) {
-		if(keep) pass_dd_TK<32, true>(d, sweep, mark, block, s);
-		else pass_dd_TK<32, false>(d, sweep, mark, block, s);
+		if(d.R == 1) pass_dd_T<32, true>(d, sweep, mark, block, s);
+		else pass_dd_T<32, false>(d, sweep, mark, block, s);
 	}
 	else {
-		if(keep) pass_dd_TK<64, true>(d, sweep, mark, block, s);
-		else pass_dd_TK<64, false>(d, sweep, mark, block, s);
+		if(d.R == 1) pass_dd_T<64, true>(d, sweep, mark, block, s);
+		else pass_dd_T<64, false>(d, sweep, mark, block, s);
 	}
 }
 
-template <int T, int CPL, bool KEEP, bool ONE, int CAP = CELL_CAP>
+template <int T, int CPL, bool ONE, int CAP = CELL_CAP>
 static void pass_T(const DevState &d, uint64_t sweep, int pass, int block, hipStream_t s) {
 	const int tpb = block / T;
 	int nb = (d.total_act + tpb - 1) / tpb;
 	nb = (nb + 7) & ~7;  // 8 XCDs x the most workgroups one XCD may need
-	size_t lds = (size_t) tpb * team_lds<T, CAP>() * sizeof(double);
+	size_t lds = (size_t) tpb * team_lds<CAP>() * sizeof(double);
 	PassArgs a{d, sweep, pass, 0u};
-	hipLaunchKernelGGL((k_pass<T, CPL, KEEP, ONE, CAP>), dim3(nb), dim3(block), lds, s, a);
+	hipLaunchKernelGGL((k_pass<T, CPL, ONE, CAP>), dim3(nb), dim3(block), lds, s, a);
 	if constexpr(CAP < CELL_CAP) {
 		// the deferred cells (usually none: the workgroups leave at once)
 		constexpr int OB = 128;
-		hipLaunchKernelGGL((k_pass_ovf<KEEP, ONE>), dim3(256), dim3(OB), (size_t) (OB / 32) * team_lds<32>() * sizeof(double),
-		                   s, a);
+		hipLaunchKernelGGL((k_pass_ovf<ONE>), dim3(256), dim3(OB), pass_lds_bytes(32, OB), s, a);
 	}
 }
 
 int small_cell_cap() { return SMALL_CAP; }
 
-size_t pass_lds_bytes(int T, int block) {
-	return (size_t) (block / T) * (T == 16 ? team_lds<16>() : (T == 32 ? team_lds<32>() : team_lds<64>())) *
-	       sizeof(double);
-}
+size_t pass_lds_bytes(int T, int block) { return (size_t) (block / T) * team_lds<>() * sizeof(double); }
 
-// The form is chosen per context: 32 or 64 lanes per cell, kept static
-// bonds or not, and one replica (its constants then load to scalar registers
-// for every team) or several.
-template <int T, bool KEEP>
+// The form is chosen per context: 16, 32 or 64 lanes per cell, and one
+// replica (its constants then load to scalar registers for every team) or
+// several.
+template <int T>
 static void pass_TK(const DevState &d, uint64_t sweep, int pass, int block, hipStream_t s) {
 	if constexpr(T == 16) {
 		// dilute systems (fewer than 16 candidates in a cell's 27 cells on
 		// average): one register neighbour per lane, the rare rest from memory
 		const double cand = 27. * (double) d.Ntot / (double) std::max(d.C_total, 1);
 		if(cand < 16.) {
-			if(d.R == 1) pass_T<16, 1, KEEP, true, SMALL_CAP>(d, sweep, pass, block, s);
-			else pass_T<16, 1, KEEP, false, SMALL_CAP>(d, sweep, pass, block, s);
+			if(d.R == 1) pass_T<16, 1, true, SMALL_CAP>(d, sweep, pass, block, s);
+			else pass_T<16, 1, false, SMALL_CAP>(d, sweep, pass, block, s);
 			return;
 		}
 	}
-	constexpr int CPL = T < 32 ? 32 / T : 1;  // register neighbours per lane
-	if(d.R == 1) pass_T<T, CPL, KEEP, true>(d, sweep, pass, block, s);
-	else pass_T<T, CPL, KEEP, false>(d, sweep, pass, block, s);
+	constexpr int CPL = T < 64 ? 2 : 1;  // register neighbours per lane
+	if(d.R == 1) pass_T<T, CPL, true>(d, sweep, pass, block, s);
+	else pass_T<T, CPL, false>(d, sweep, pass, block, s);
 }
 
 void launch_pass(const DevState &d, uint64_t sweep, int pass, int T, int block, hipStream_t s) {
-	const bool keep = d.trials_per_cell >= KEEP_MIN_TRIALS;
-	if(T == 16) {
-		if(keep) pass_TK<16, true>(d, sweep, pass, block, s);
-		else pass_TK<16, false>(d, sweep, pass, block, s);
-	}
-	else if(T == 32) {
-		if(keep) pass_TK<32, true>(d, sweep, pass, block, s);
-		else pass_TK<32, false>(d, sweep, pass, block, s);
-	}
-	else {
-		if(keep) pass_TK<64, true>(d, sweep, pass, block, s);
-		else pass_TK<64, false>(d, sweep, pass, block, s);
-	}
+	if(T == 16) pass_TK<16>(d, sweep, pass, block, s);
+	else if(T == 32) pass_TK<32>(d, sweep, pass, block, s);
+	else pass_TK<64>(d, sweep, pass, block, s);
 }
 
-template <int T, int CPL, bool KEEP>
-static int sweep_blocks_T(int block, int cus) {
+static const void *sweep_kernel(int T) {
+	return T == 32 ? (const void *) k_sweep_passes<32> : (const void *) k_sweep_passes<64>;
+}
+
+// co-resident workgroups of the cooperative launch
+int sweep_blocks_max(int T, int block, int cus) {
 	int per_cu = 0;
-	if(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void *) k_sweep_passes<T, CPL, KEEP>, block,
-	                                                pass_lds_bytes(T, block)) != hipSuccess)
+	if(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, sweep_kernel(T), block, pass_lds_bytes(T, block)) != hipSuccess)
 		return 0;
 	return per_cu * cus;
 }
 
-// co-resident workgroups of either form (both must fit: the form is chosen
-// per context at launch)
-int sweep_blocks_max(int T, int block, int cus) {
-	if(T == 32) return std::min(sweep_blocks_T<32, 1, false>(block, cus), sweep_blocks_T<32, 1, true>(block, cus));
-	return std::min(sweep_blocks_T<64, 1, false>(block, cus), sweep_blocks_T<64, 1, true>(block, cus));
-}
-
-template <int T, int CPL, bool KEEP>
-static hipError_t sweep_T(const DevState &d, uint64_t sweep, int block, int blocks, hipStream_t s) {
+hipError_t launch_sweep_passes(const DevState &d, uint64_t sweep, int T, int block, int blocks, hipStream_t s) {
 	PassArgs a{d, sweep, 0, 0u};
 	void *args[] = {&a};
-	return hipLaunchCooperativeKernel((const void *) k_sweep_passes<T, CPL, KEEP>, dim3(blocks), dim3(block), args,
-	                                  (unsigned) pass_lds_bytes(T, block), s);
-}
-
-hipError_t launch_sweep_passes(const DevState &d, uint64_t sweep, int T, int block, int blocks, hipStream_t s) {
-	const bool keep = d.trials_per_cell >= KEEP_MIN_TRIALS;
-	if(T == 32) return keep ? sweep_T<32, 1, true>(d, sweep, block, blocks, s) : sweep_T<32, 1, false>(d, sweep, block, blocks, s);
-	return keep ? sweep_T<64, 1, true>(d, sweep, block, blocks, s) : sweep_T<64, 1, false>(d, sweep, block, blocks, s);
+	return hipLaunchCooperativeKernel(sweep_kernel(T), dim3(blocks), dim3(block), args, (unsigned) pass_lds_bytes(T, block), s);
 }
 
 // ------------------------------------------------------------------------

@@ -174,7 +174,6 @@ extern "C" pp_status pp_energy_snapshot_noalloc(int n, const double *r, const do
 	rp.rc2 = rcut * rcut;  // SQR(1. + delta) (system.c:86)
 	rp.cosmax = kf_cosmax;
 	rp.T = 1.;
-	for(int e = 0; e < ACC_TAB; e++) rp.acc_tab[e] = std::exp(-(double) e);
 	rp.ensemble = PP_NVT;
 	rp.min_n = 3;
 	rp.even = 0;
