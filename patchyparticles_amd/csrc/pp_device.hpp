@@ -90,6 +90,51 @@ __device__ __forceinline__ int wave_incl_scan(int v) {
 	return v;
 }
 
+__device__ __forceinline__ int wrapi(int i, int n) { return i < 0 ? i + n : (i >= n ? i - n : i); }
+
+// The slots of the 26 cells around cell (ix, iy, iz) of an n0 x n1 x n2 grid
+// (st: the replica's cell starts), in the order of the directions m = 9 (dx +
+// 1) + 3 (dy + 1) + dz + 1: row j < 9 holds the cells of directions 3j, 3j + 1
+// and 3j + 2, whose slots are one range, or two where the row wraps around the
+// box or (j = 4) leaves out the cell itself.  The row's candidates are
+// [a1, b1), then [a2, b2).
+__device__ __forceinline__ void row_ranges(const int *st, int ix, int iy, int iz, int n0, int n1, int n2, int j, int &a1,
+                                           int &b1, int &a2, int &b2) {
+	const int cx = wrapi(ix + j / 3 - 1, n0), cy = wrapi(iy + j % 3 - 1, n1);
+	const int *row = st + (size_t) (cx * n1 + cy) * n2;
+	const int zl = wrapi(iz - 1, n2), zh = wrapi(iz + 1, n2);
+	// ends of the first range and starts of the second, as cells of the row
+	int e1 = iz + 2, s2 = zh, e2 = zh;
+	if(j == 4) e1 = zl + 1, e2 = zh + 1;
+	else if(iz == 0) e1 = zl + 1, s2 = 0, e2 = 2;
+	else if(iz == n2 - 1) e1 = n2, e2 = zh + 1;
+	a1 = row[zl];
+	b1 = row[e1];
+	a2 = row[s2];
+	b2 = row[e2];
+}
+
+// Slot of candidate i of those rows, counted through (a record holds the
+// first REC_SLOTS; few cells have more).
+__device__ inline int walk_slot(const int *st, int ix, int iy, int iz, int n0, int n1, int n2, int i) {
+	for(int j = 0; j < 9; j++) {
+		int a1, b1, a2, b2;
+		row_ranges(st, ix, iy, iz, n0, n1, n2, j, a1, b1, a2, b2);
+		if(i < b1 - a1) return a1 + i;
+		i -= b1 - a1;
+		if(i < b2 - a2) return a2 + i;
+		i -= b2 - a2;
+	}
+	return 0;
+}
+
+// Slot of static neighbour i of a record (rec: the record or a copy).
+__device__ __forceinline__ int rec_slot(const DevState &d, const int *rec, int i) {
+	if(i < REC_SLOTS) return rec[REC_HEAD + i];
+	const Rep &rp = d.reps[rec[REC_REP]];
+	return walk_slot(d.start + rp.cell_off, rec[REC_IX], rec[REC_IY], rec[REC_IZ], rp.lg.n[0], rp.lg.n[1], rp.lg.n[2], i);
+}
+
 // A value the compiler knows nothing about: what is computed from it stays
 // where it is written, not in registers across a loop that rarely needs it.
 __device__ __forceinline__ int opaque(int v) {
@@ -134,8 +179,6 @@ __device__ __forceinline__ void team_sync() {
 __device__ __forceinline__ unsigned long long *ctr_at(unsigned long long *ctr, int r, int row, int slot) {
 	return ctr + ((long long) (r * NCTR + row) * NSLOT + slot);
 }
-
-__device__ __forceinline__ int wrapi(int i, int n) { return i < 0 ? i + n : (i >= n ? i - n : i); }
 
 // Uniform axis on the unit sphere by Marsaglia's rejection method (the
 // method of random_vector_on_sphere, utils.c:115-131), fed by Philox blocks

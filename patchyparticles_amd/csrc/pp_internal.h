@@ -20,7 +20,24 @@ constexpr int MAX_TRIALS_PER_CELL = 16;
 constexpr int SCAN_TILE_SMALL = 512;
 constexpr int SCAN_TILE_LARGE = 2048;
 constexpr int SCAN_SMALL_MAX_TILES = 320;  // small tiles up to this many (look-back scan)
-constexpr int REC_W = 64;      // ints of one cell record of a pass
+// one cell record of a pass (ints): a header, then the slots of the cell's
+// first REC_SLOTS static neighbours
+constexpr int REC_W = 64;
+enum RecHead : int {
+	REC_TAG = 0,  // the rebuild that wrote the record (DevState::rec_tag)
+	REC_M,        // static neighbours: particles of the 26 surrounding cells
+	REC_S0,       // first slot and population of the cell
+	REC_CNT,
+	REC_CELL,     // local index of the cell, replica, buffer selector
+	REC_REP,
+	REC_SEL,
+	REC_M0,       // static neighbours in the 13 directions m < 13
+	REC_IX,       // the cell's indices along the axes
+	REC_IY,
+	REC_IZ,
+	REC_HEAD = 12
+};
+constexpr int REC_SLOTS = REC_W - REC_HEAD;
 constexpr int ACC_TAB = 16;    // Metropolis factors exp(-k/T) tabulated per replica, k < ACC_TAB
 
 // per-replica counter rows, each NSLOT wide
@@ -114,7 +131,7 @@ struct PassGeo {
 	double shift[3], side[3];   // of the sweep's cells
 	float inv_side[3];
 	F32Filter filter;           // of the single-precision pair tests
-	int n1, n2;
+	int n[3];
 	int n_thr;                  // entries of thr in use
 	uint32_t thr[ACC_TAB - 1];  // a 32-bit draw w accepts a rise of j bonds iff w <= thr[j - 1]
 };
@@ -225,6 +242,7 @@ struct DevState {
 	int *ccount;       // [R][8] non-empty cells per colour
 	int *pfx;          // [8][R+1] prefix over replicas of the cells pass k works on
 	int *rec;          // [8][total_act][REC_W] records of the cells of each pass, in list order
+	unsigned rec_tag;  // mark of the sweep's records (never 0; differs from every earlier sweep's)
 	unsigned *bar;     // grid barrier of the cooperative sweep kernel: arrivals, generation
 	int *scan_ticket;  // [0]: tiles taken, [1]: tiles done
 	int *tile_sum;     // [ntiles] per-tile sums, then their exclusive prefixes (grids of many tiles)

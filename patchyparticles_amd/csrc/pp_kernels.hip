@@ -103,8 +103,7 @@ __device__ __forceinline__ void set_pass_geo(Rep &rp, const Grid &G, const doubl
 		smax = fmax(smax, p.side[k]);
 	}
 	p.filter = f32_filter(rp.cosmax, rp.rc2, smax);
-	p.n1 = G.n[1];
-	p.n2 = G.n[2];
+	for(int k = 0; k < 3; k++) p.n[k] = G.n[k];
 }
 
 // ONE: a context of one replica, whose table then loads to scalar registers.
@@ -418,123 +417,140 @@ __global__ __launch_bounds__(256) void k_scan(DevState d, int flip, int lists, i
 }
 
 // The layout of the passes' lists, after the scan has counted them:
-// pfx[k][r] = first entry of replica r in the list of pass k (one thread per
-// pass; the kernel boundary makes every workgroup's counts visible).  Also
-// resets the ticket queue of the dependency-driven sweep.
-__device__ __forceinline__ void pass_prefix(const DevState &d, int t) {
-	if(t == 0 && d.ddq) *d.ddq = 0;  // the dependency-driven sweep's tickets
-	if(t < 8) {
-		if(d.ovf_n) d.ovf_n[t] = 0;  // the small-cell pass's deferred cells
-		int acc = 0;
-		d.pfx[t * (d.R + 1)] = 0;
-		for(int r = 0; r < d.R; r++) {
-			const int col = (int) ((d.reps[r].col_perm >> (4 * t)) & 0xFu);
-			acc += d.ccount[r * 8 + col];
-			d.pfx[t * (d.R + 1) + r + 1] = acc;
-		}
+// pfx[k][r] = first entry of replica r in the list of pass k, by wavefront k
+// (the kernel boundary makes every workgroup's counts visible).  Also resets
+// the ticket queue of the dependency-driven sweep and the lists of deferred
+// cells.  A thread per pass adding 256 replicas one by one took 80 us; a
+// wavefront's scan takes 5.
+__device__ __forceinline__ void pass_prefix(const DevState &d, int k, int lane) {
+	if(lane == 0) {
+		if(k == 0 && d.ddq) *d.ddq = 0;
+		if(d.ovf_n) d.ovf_n[k] = 0;
+	}
+	int *pf = d.pfx + k * (d.R + 1);
+	if(lane == 0) pf[0] = 0;
+	int base = 0;
+	for(int r0 = 0; r0 < d.R; r0 += 64) {
+		const int r = r0 + lane;
+		int n = 0;
+		if(r < d.R) n = d.ccount[r * 8 + (int) ((d.reps[r].col_perm >> (4 * k)) & 0xFu)];
+		const int inc = wave_incl_scan(n);
+		if(r < d.R) pf[r + 1] = base + inc;
+		base += __builtin_amdgcn_readlane(inc, 63);
 	}
 }
 
-__global__ void k_pass_prefix(DevState d) { pass_prefix(d, threadIdx.x); }
+__global__ __launch_bounds__(512) void k_pass_prefix(DevState d) { pass_prefix(d, threadIdx.x >> 6, threadIdx.x & 63); }
 
-// Record of entry i of the cell lists (replica r's list of colour col at
-// clist[cell_off + col * act_cap + k]), stored at the entry's position in the
-// list of the pass that works on that colour: the 26 surrounding cells' first
-// slots [0, 26), the exclusive prefix of their populations [32, 59), the
-// cell's first slot, population, local index, replica and buffer selector
-// [59, 64).  A pass finds all its data from this one load.
+// The record of entry gi of pass k's list, by the 16 lanes of a team: lane j <
+// 9 takes row j of the neighbourhood (row_ranges), a prefix sum over the
+// lanes places its slots, lane 9 writes the header.  A pass finds all its
+// data from this one record: its slot list needs no search, and lanes of one
+// team write to one or two cache lines (a thread per record wrote 256 bytes
+// at a time, from 52 loads of its own).
 template <bool ONE>
-__device__ __forceinline__ void build_record(const DevState &d, int i) {
-	int lo = 0, hi = d.R;
-	if constexpr(!ONE)
-		while(hi - lo > 1) {
-			int mid = (lo + hi) >> 1;
-			if(d.reps[mid].cell_off <= i) lo = mid;
-			else hi = mid;
+__device__ __forceinline__ void build_record(const DevState &d, int k, int gi, int lane) {
+	int r = 0;
+	if constexpr(!ONE) {
+		// the replica whose entries of pass k hold gi: the last r with
+		// pfx[r] <= gi, the team's lanes probing 16 places at once
+		const int *pf = d.pfx + k * (d.R + 1);
+		for(int n = d.R; n > 1;) {
+			const int step = (n + 15) / 16, at = r + lane * step;
+			const bool le = lane * step < n && pf[at] <= gi;
+			const int off = threadIdx.x & 63 & ~15;
+			const unsigned m = (unsigned) (ballot(le) >> off) & 0xffffu;  // lane 0 always, then a run
+			const int last = 31 - __clz((int) m);
+			r += last * step;
+			n = min(step, n - last * step);
 		}
-	const Rep &rp = d.reps[lo];
-	const int local = i - rp.cell_off;
-	const int col = local / rp.act_cap, kk = local - col * rp.act_cap;
-	if(col >= 8 || kk >= d.ccount[lo * 8 + col]) return;
-	const int cloc = d.clist[i];
-	int k = 0;
-	while(k < 7 && (int) ((rp.col_perm >> (4 * k)) & 0xFu) != col) k++;
-	const int gi = (ONE ? 0 : d.pfx[k * (d.R + 1) + lo]) + kk;
+	}
+	const Rep &rp = d.reps[r];
+	const int kk = ONE ? gi : gi - d.pfx[k * (d.R + 1) + r];
+	const int col = (int) ((rp.col_perm >> (4 * k)) & 0xFu);
+	const int cloc = d.clist[rp.cell_off + col * rp.act_cap + kk];
 	const int n0 = rp.g.n[0], n1 = rp.g.n[1], n2 = rp.g.n[2];
 	const int ix = cloc / (n1 * n2), iy = (cloc / n2) % n1, iz = cloc % n2;
 	const int *st = d.start + rp.cell_off;
-	int rec[REC_W];
-	int acc = 0;
-#pragma unroll
-	for(int nb = 0; nb < 26; nb++) {
-		const int m = nb < 13 ? nb : nb + 1;
-		const int cx = wrapi(ix + m / 9 - 1, n0), cy = wrapi(iy + (m / 3) % 3 - 1, n1), cz = wrapi(iz + m % 3 - 1, n2);
-		const int cc = (cx * n1 + cy) * n2 + cz;
-		const int a = st[cc], b = st[cc + 1];
-		rec[nb] = a;
-		rec[32 + nb] = acc;
-		acc += b - a;
+	int a1 = 0, b1 = 0, a2 = 0, b2 = 0;
+	if(lane < 9) row_ranges(st, ix, iy, iz, n0, n1, n2, lane, a1, b1, a2, b2);
+	else if(lane == 9) {
+		a1 = st[cloc];
+		b1 = st[cloc + 1];
 	}
-#pragma unroll
-	for(int e = 26; e < 32; e++) rec[e] = 0;
-	const int s0 = st[cloc];
-	rec[58] = acc;
-	rec[59] = s0;
-	rec[60] = st[cloc + 1] - s0;
-	rec[61] = cloc;
-	rec[62] = lo;
-	rec[63] = rp.sel;
-	int4 *out = (int4 *) (d.rec + ((size_t) k * d.total_act + gi) * REC_W);
-#pragma unroll
-	for(int e = 0; e < REC_W / 4; e++) out[e] = make_int4(rec[4 * e], rec[4 * e + 1], rec[4 * e + 2], rec[4 * e + 3]);
+	const int l1 = b1 - a1, len = lane < 9 ? l1 + b2 - a2 : 0;
+	int inc = len;
+	inc += __builtin_amdgcn_update_dpp(0, inc, DPP_ROW_SHR + 1, 0xf, 0xf, true);
+	inc += __builtin_amdgcn_update_dpp(0, inc, DPP_ROW_SHR + 2, 0xf, 0xf, true);
+	inc += __builtin_amdgcn_update_dpp(0, inc, DPP_ROW_SHR + 4, 0xf, 0xf, true);
+	inc += __builtin_amdgcn_update_dpp(0, inc, DPP_ROW_SHR + 8, 0xf, 0xf, true);
+	// candidates before the cell itself, for the header's lane
+	const int m0 = __shfl(inc - len + l1, (int) (threadIdx.x & 63 & ~15) + 4);
+	int *rec = d.rec + ((size_t) k * d.total_act + gi) * REC_W;
+	for(int e = 0, at = REC_HEAD + inc - len; e < len && at < REC_W; e++, at++) rec[at] = e < l1 ? a1 + e : a2 + e - l1;
+	if(lane == 9) {
+		int4 *out = (int4 *) rec;
+		out[0] = make_int4((int) d.rec_tag, inc, a1, l1);
+		out[1] = make_int4(cloc, r, rp.sel, m0);
+		out[2] = make_int4(ix, iy, iz, 0);
+	}
 }
 
+// Workgroups of the scatter that build records (grid-stride over the listed
+// cells): enough to fill the chip.
+constexpr int REC_BLOCKS = 2048;
+constexpr int PART_BLOCK = 256 / (NCOMP / 2);  // particles moved by one workgroup
+
 // Move every particle to its cell's slot range.  After a flipping scan the
-// source is the previous buffer (sel ^ 1); a trial writes into sel ^ 1.
-// With a new grid shift the workers also write the cell records of the
-// sweep's passes.
+// source is the previous buffer (sel ^ 1); a trial writes into sel ^ 1.  Six
+// lanes per particle, 16 bytes each: whole cache lines on both sides.
+// With a new grid shift, workgroups past the particles' write the cell
+// records of the sweep's passes.
 // ONE: one replica, whose lists start at entry 0 of every pass; the first
 // workgroup also writes the pass prefixes (k_pass_prefix's work), which the
 // records then do not need.
 template <bool ONE>
-__global__ void k_scatter(DevState d, int mode, uint64_t sweep) {
-	int j = blockIdx.x * blockDim.x + threadIdx.x;
+__global__ __launch_bounds__(256) void k_scatter(DevState d, int mode, int part_blocks) {
 	if constexpr(ONE)
-		if(mode == REB_SHIFT && blockIdx.x == 0) pass_prefix(d, threadIdx.x);
-	// the particle's loads first, so that they overlap the record's chain of
-	// loads; its stores after the record's
-	bool mv = false, hw = false;
-	int r = 0, dst = 0, pid = 0;
-	double v[NCOMP];
-	double *G = nullptr;
-	int *PG = nullptr;
-	if(j < d.Ntot) {
-		r = ONE ? 0 : d.prep[j];
-		const Rep &rp = d.reps[r];
-		const bool tr = (mode == REB_TRIAL) && trial_rebuilds(rp);
-		if(mode != REB_TRIAL || tr) {
-			mv = true;
-			// the buffer this rebuild switches to holds the live particles first
-			hw = mode != REB_TRIAL && j == rp.p_off;
-			const int sb = tr ? rp.sel : (rp.sel ^ 1);
-			const double *F = pick_buf(d.f, sb);
-			G = pick_buf(d.f, sb ^ 1);
-			PG = pick_buf(d.pid, sb ^ 1);
-			dst = d.start[d.cellid[j]] + d.slot[j];
+		if(mode == REB_SHIFT && blockIdx.x == 0)
+			for(int k = threadIdx.x >> 6; k < 8; k += 4) pass_prefix(d, k, threadIdx.x & 63);
+	if((int) blockIdx.x >= part_blocks) {
+		const int team = (blockIdx.x - part_blocks) * 16 + threadIdx.x / 16, teams = (gridDim.x - part_blocks) * 16;
+		int len[8], total = 0;
 #pragma unroll
-			for(int c = 0; c < NCOMP; c++) {
-				v[c] = part(F, j)[c];
-				if(tr && c < 3) v[c] *= rp.trial_s[c];
-			}
-			pid = pick_buf(d.pid, sb)[j];
+		for(int k = 0; k < 8; k++) {
+			len[k] = ONE ? d.ccount[(d.reps[0].col_perm >> (4 * k)) & 0xFu] : d.pfx[k * (d.R + 1) + d.R];
+			total += len[k];
 		}
+		for(int i = team; i < total; i += teams) {
+			int k = 0, gi = i;
+			while(gi >= len[k]) gi -= len[k++];
+			build_record<ONE>(d, k, gi, threadIdx.x & 15);
+		}
+		return;
 	}
-	if(mode == REB_SHIFT && j < d.C_total) build_record<ONE>(d, j);
-	if(!mv) return;
-#pragma unroll
-	for(int c = 0; c < NCOMP; c++) part(G, dst)[c] = v[c];
-	PG[dst] = pid;
-	if(hw) d.reps[r].np_hw = d.reps[r].np;
+	constexpr int PER = NCOMP / 2;  // lanes per particle
+	const int e = threadIdx.x % PER;
+	const int j = blockIdx.x * PART_BLOCK + threadIdx.x / PER;
+	if((int) threadIdx.x >= PART_BLOCK * PER || j >= d.Ntot) return;
+	const int r = ONE ? 0 : d.prep[j];
+	Rep &rp = d.reps[r];
+	const bool tr = (mode == REB_TRIAL) && trial_rebuilds(rp);
+	if(mode == REB_TRIAL && !tr) return;
+	const int sb = tr ? rp.sel : (rp.sel ^ 1);
+	const int dst = d.start[d.cellid[j]] + d.slot[j];
+	double2 v = ((const double2 *) part((const double *) pick_buf(d.f, sb), j))[e];
+	if(tr) {
+		// (components 0, 1 and 2 are the position)
+		if(e == 0) v.x *= rp.trial_s[0], v.y *= rp.trial_s[1];
+		if(e == 1) v.x *= rp.trial_s[2];
+	}
+	((double2 *) part(pick_buf(d.f, sb ^ 1), dst))[e] = v;
+	if(e == 0) {
+		pick_buf(d.pid, sb ^ 1)[dst] = pick_buf(d.pid, sb)[j];
+		// the buffer this rebuild switches to holds the live particles first
+		if(mode != REB_TRIAL && j == rp.p_off) rp.np_hw = rp.np;
+	}
 }
 
 void launch_rebuild(const DevState &d, int mode, uint64_t sweep, long long trace_pos, hipStream_t s) {
@@ -560,11 +576,12 @@ void launch_rebuild(const DevState &d, int mode, uint64_t sweep, long long trace
 		hipLaunchKernelGGL(k_tile_scan, dim3(1), dim3(1024), 0, s, d);
 		hipLaunchKernelGGL((k_scan<SCAN_TILE_LARGE / 256, false>), dim3(d.ntiles), dim3(256), 0, s, d, flip, lists, 1);
 	}
-	if(mode == REB_SHIFT && d.R != 1) hipLaunchKernelGGL(k_pass_prefix, dim3(1), dim3(64), 0, s, d);
-	unsigned gs = gp;
-	if(mode == REB_SHIFT) gs = std::max(gp, (unsigned) ((d.C_total + B - 1) / B));
-	if(d.R == 1) hipLaunchKernelGGL(k_scatter<true>, dim3(gs), dim3(B), 0, s, d, mode, sweep);
-	else hipLaunchKernelGGL(k_scatter<false>, dim3(gs), dim3(B), 0, s, d, mode, sweep);
+	if(mode == REB_SHIFT && d.R != 1) hipLaunchKernelGGL(k_pass_prefix, dim3(1), dim3(512), 0, s, d);
+	const unsigned pb = (unsigned) std::max(1, (d.Ntot + PART_BLOCK - 1) / PART_BLOCK);
+	unsigned gs = pb;
+	if(mode == REB_SHIFT) gs += (unsigned) std::min<long long>(REC_BLOCKS, (8LL * d.total_act + 15) / 16);
+	if(d.R == 1) hipLaunchKernelGGL(k_scatter<true>, dim3(gs), dim3(B), 0, s, d, mode, (int) pb);
+	else hipLaunchKernelGGL(k_scatter<false>, dim3(gs), dim3(B), 0, s, d, mode, (int) pb);
 }
 
 // ------------------------------------------------------------------------
@@ -586,13 +603,15 @@ struct PassArgs {
 //   OWN the members' exact state, ranked by particle index: x, y, z, O, and
 //       the position relative to the cell's centre
 //   TR  the trials' exact displacement and R
-//   PID particle indices, NB the cell's record (surrounding slot ranges)
+//   PID particle indices
+//   NB  (neighbourhoods beyond the record's list) the rows' slot ranges
 //   GEO constants of the exact arithmetic and the far neighbours, here so
 //       that the trial loop does not hold them in registers
 constexpr int OWN_W = 16;  // x, y, z, O[9], rel[3], one unused
 constexpr int TR_W = 12;   // dx, dy, dz, R[9]
 constexpr int SH_W = 16;   // floats: rel[3], O[9], static bonds, member bond bits, two unused
 constexpr int FT_W = 16;   // floats: dx, dy, dz, the rise it accepts, R[9], rank, two unused
+constexpr int NB_W = 40;   // ints: first slots [0, 18) and exclusive prefix [20, 39) of the rows' ranges
 constexpr int GEO_W = 12;  // box[3], 1 / box[3], the cell's centre[3], rc^2, cosmax, one unused
 template <int CAP>
 struct TeamLds {
@@ -603,7 +622,7 @@ struct TeamLds {
 	static constexpr int TR = OWN + CAP * OWN_W;
 	static constexpr int PID = TR + TRIALS * TR_W;
 	static constexpr int NB = PID + (CAP + 1) / 2;
-	static constexpr int GEO = NB + REC_W / 2;
+	static constexpr int GEO = NB + NB_W / 2;
 	static constexpr int SIZE = GEO + GEO_W;
 	static_assert(FT % 2 == 0 && OWN % 2 == 0 && TR % 2 == 0 && NB % 2 == 0 && SIZE % 2 == 0, "16-byte aligned parts");
 };
@@ -654,24 +673,26 @@ __device__ __forceinline__ double nbld(const double *p) {
 
 // Wait (DD) until every non-empty neighbour cell that an earlier pass of this
 // sweep works on has published `mark` in done[]: lane nb < 26 of the team
-// watches neighbour nb of the cell record (direction m = nb < 13 ? nb : nb +
-// 1, offsets m / 9 - 1, (m / 3) % 3 - 1, m % 3 - 1).  Neighbours of later
-// passes wait for this cell in turn, so none of them writes before this
-// cell's reads.  The wait is bounded: past DD_SPIN_MAX polls the team reports
-// ERR_DEPWAIT and goes on, so the launch always drains.
+// watches the neighbour in direction m = nb < 13 ? nb : nb + 1 (offsets m / 9 -
+// 1, (m / 3) % 3 - 1, m % 3 - 1).  Neighbours of later passes wait for this
+// cell in turn, so none of them writes before this cell's reads.  The wait is
+// bounded: past DD_SPIN_MAX polls the team reports ERR_DEPWAIT and goes on, so
+// the launch always drains.
 template <int T>
-__device__ __forceinline__ void wait_neighbours(const DevState &d, const Rep &rp, const int *nb_tab, int pass, int ix,
-                                                int iy, int iz, int n0, int n1, int n2, unsigned mark, int lane) {
+__device__ __forceinline__ void wait_neighbours(const DevState &d, const Rep &rp, int pass, int ix, int iy, int iz,
+                                                unsigned mark, int lane) {
 	bool need = false;
 	const unsigned *w = nullptr;
 	if(lane < 26) {
+		const int n0 = rp.pg.n[0], n1 = rp.pg.n[1], n2 = rp.pg.n[2];
 		const int m = lane < 13 ? lane : lane + 1;
 		const int cx = wrapi(ix + m / 9 - 1, n0), cy = wrapi(iy + (m / 3) % 3 - 1, n1), cz = wrapi(iz + m % 3 - 1, n2);
 		const int ncol = ((cx & 1) << 2) | ((cy & 1) << 1) | (cz & 1);
 		int np = 0;
 		while(np < 7 && (int) ((rp.col_perm >> (4 * np)) & 0xFu) != ncol) np++;
-		need = np < pass && nb_tab[32 + lane + 1] > nb_tab[32 + lane];
-		w = d.done + rp.cell_off + (cx * n1 + cy) * n2 + cz;
+		const int c = rp.cell_off + (cx * n1 + cy) * n2 + cz;
+		need = np < pass && d.start[c + 1] > d.start[c];
+		w = d.done + c;
 	}
 	int spins = 0;
 	while(team_any<T>(need)) {
@@ -731,16 +752,20 @@ __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int
 	int *own_pid = (int *) (blk + L::PID);
 	int *nb_tab = (int *) (blk + L::NB);
 
-	// 1. the cell's record: surrounding slot ranges, own range, replica
-	const int4 *rec = (const int4 *) (d.rec + ((size_t) pass * d.total_act + gi) * REC_W);
-	for(int e = lane; e < REC_W / 4; e += T) ((int4 *) nb_tab)[e] = rec[e];
-	team_sync();
-	const int M = uni<T>(nb_tab[58]);
-	const int s0 = uni<T>(nb_tab[59]);
-	const int cnt = uni<T>(nb_tab[60]);
-	const int cloc = uni<T>(nb_tab[61]);
-	const int r = ONE ? 0 : uni<T>(nb_tab[62]);
-	const int sel = uni<T>(nb_tab[63]);
+	// 1. the cell's record: its header, and this lane's neighbour; a record of
+	// another sweep lies past the end of the pass's list
+	const int *rec = d.rec + ((size_t) pass * d.total_act + gi) * REC_W;
+	const int4 h0 = ((const int4 *) rec)[0], h1 = ((const int4 *) rec)[1], h2 = ((const int4 *) rec)[2];
+	int cq[CPL];
+	cq[0] = lane < REC_SLOTS ? rec[REC_HEAD + lane] : -1;
+	if(uni<T>(h0.x) != (int) d.rec_tag) return;
+	const int M = uni<T>(h0.y);
+	const int s0 = uni<T>(h0.z);
+	const int cnt = uni<T>(h0.w);
+	const int cloc = uni<T>(h1.x);
+	const int r = ONE ? 0 : uni<T>(h1.y);
+	const int sel = uni<T>(h1.z);
+	const int ix = uni<T>(h2.x), iy = uni<T>(h2.y), iz = uni<T>(h2.z);
 	if constexpr(CAP < CELL_CAP)
 		if(cnt > d.small_cap) {
 			// (entries < total_act: each cell is listed at most once a pass)
@@ -762,52 +787,38 @@ __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int
 	int *PID = pick_buf(d.pid, sel);
 
 	// 2. every load of the cell at once: the members, the static neighbours
-	// and the replica's geometry
+	// and the replica's geometry.  Register slot u (u < CPL) of lane l holds
+	// one neighbour: the last cnt lanes' first slot the cell's members (read
+	// from the shadow records at every trial), the slots before them and the
+	// second ones the static neighbours (l, and T - cnt + l); the rest (dense
+	// neighbourhoods only) are read again at every trial.  A lane thus tests
+	// one neighbour per trial whether the cell holds one member or several.
+	const int nstat = T - cnt;        // first slots of static neighbours
+	const int mi = lane - nstat;      // this lane's member
+	const bool is_mem = mi >= 0;
+	const int nreg = min(M, min(T * CPL - cnt, REC_SLOTS));
 	int my_pid = 0;
 	double mine[NCOMP];
-	if(lane < cnt) {
-		my_pid = PID[s0 + lane];
+	if(is_mem) {
+		my_pid = PID[s0 + mi];
 #pragma unroll
-		for(int c = 0; c < NCOMP; c++) mine[c] = part(F, s0 + lane)[c];
+		for(int c = 0; c < NCOMP; c++) mine[c] = part(F, s0 + mi)[c];
 	}
 	// trials of the cell in this pass: one per member (a sweep is then N
 	// attempts), or a fixed number per non-empty cell
 	const int ntrial = d.trials_per_cell > 0 ? d.trials_per_cell : cnt;
-	// slot of static neighbour i (0 <= i < M)
-	auto nb_slot = [&](int i) {
-		int lo2 = 0, hi2 = 26;
-		while(hi2 - lo2 > 1) {
-			int mid = (lo2 + hi2) >> 1;
-			if(nb_tab[32 + mid] <= i) lo2 = mid;
-			else hi2 = mid;
-		}
-		return nb_tab[lo2] + (i - nb_tab[32 + lo2]);
-	};
-	// Register slot lane + u T (u < CPL) of the team holds one neighbour:
-	// slots below cnt the cell's members (member = lane, read from the
-	// shadow records at every trial), then the first static neighbours; the
-	// rest (dense neighbourhoods only) are read again at every trial.  A lane
-	// thus tests one neighbour per trial whether the cell holds one member or
-	// several.
-	int cq[CPL];  // the static neighbour's slot, -1: a member or none
+	if(is_mem || lane >= nreg) cq[0] = -1;
+	if constexpr(CPL > 1) cq[1] = nstat + lane < nreg ? rec[REC_HEAD + nstat + lane] : -1;
 	double sd[CPL][NCOMP];
 	auto load_static = [&]() {
 #pragma unroll
-		for(int u = 0; u < CPL; u++) {
-			const int i = lane + u * T - cnt;
-			cq[u] = -1;
-			if(i >= 0 && i < M) {
-				const int q = nb_slot(i);
-				cq[u] = q;
+		for(int u = 0; u < CPL; u++)
+			if(cq[u] >= 0)
 #pragma unroll
-				for(int c = 0; c < NCOMP; c++) sd[u][c] = nbld<DD>(part(F, q) + c);
-			}
-		}
+				for(int c = 0; c < NCOMP; c++) sd[u][c] = nbld<DD>(part(F, cq[u]) + c);
 	};
 	if constexpr(!DD) load_static();
 	const PassGeo &pg = rp.pg;
-	const int n1 = uni<T>(pg.n1), n2 = uni<T>(pg.n2);
-	const int ix = cloc / (n1 * n2), iy = (cloc / n2) % n1, iz = cloc % n2;
 	const int col = ((ix & 1) << 2) | ((iy & 1) << 1) | (iz & 1);
 	// the cell's centre
 	const double ce0 = pg.shift[0] + ((double) ix + 0.5) * pg.side[0], ce1 = pg.shift[1] + ((double) iy + 0.5) * pg.side[1],
@@ -849,7 +860,7 @@ __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int
 		if constexpr(sizeof(m) == 8) return (int) __popcll(m);
 		else return (int) __popc(m);
 	};
-	if(lane < cnt) own_pid[lane] = my_pid;
+	if(is_mem) own_pid[mi] = my_pid;
 	if(lane == 0) {
 		const double g[GEO_W] = {pg.box[0], pg.box[1], pg.box[2], pg.inv_box[0], pg.inv_box[1], pg.inv_box[2],
 		                         ce0, ce1, ce2, rp.rc2, rp.cosmax, 0.};
@@ -869,7 +880,7 @@ __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int
 	auto check_o = [&](const float *o) {
 		wild |= !f32_orientation_ok(o);
 	};
-	if(lane < cnt) {
+	if(is_mem) {
 		int rank = 0;
 		for(int m = 0; m < cnt; m++) rank += own_pid[m] < my_pid;
 		double *w = own + rank * OWN_W;
@@ -892,7 +903,7 @@ __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int
 	}
 	if constexpr(DD) {
 		// the neighbours' data once their earlier passes are done
-		wait_neighbours<T>(d, rp, nb_tab, pass, ix, iy, iz, rp.g.n[0], n1, n2, mark, lane);
+		wait_neighbours<T>(d, rp, pass, ix, iy, iz, mark, lane);
 		load_static();
 	}
 	float qx[CPL], qy[CPL], qz[CPL], qo[CPL][9];
@@ -917,9 +928,30 @@ __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int
 	const float is0 = pg.inv_side[0], is1 = pg.inv_side[1], is2 = pg.inv_side[2];
 	// whether any team of the wavefront has neighbours beyond the register
 	// slots (a scalar branch around those loops)
-	const bool wave_far = ballot(M + cnt > T * CPL) != 0ull;
+	const bool wave_far = ballot(M > nreg) != 0ull;
 	// and likewise whether any uses the second slot of its lanes
-	const bool wave_2 = CPL > 1 && ballot(M + cnt > T) != 0ull;
+	const bool wave_2 = CPL > 1 && ballot(nreg > nstat) != 0ull;
+	if(wave_far && M > REC_SLOTS) {
+		// the rows' ranges, for the neighbours past the record's list
+		if(lane < 9) {
+			int a1, b1, a2, b2;
+			row_ranges(d.start + rp.cell_off, ix, iy, iz, pg.n[0], pg.n[1], pg.n[2], lane, a1, b1, a2, b2);
+			nb_tab[2 * lane] = a1;
+			nb_tab[2 * lane + 1] = a2;
+			nb_tab[20 + 2 * lane] = b1 - a1;
+			nb_tab[20 + 2 * lane + 1] = b2 - a2;
+		}
+		team_sync();
+		if(lane == 0) {
+			int acc = 0;
+			for(int e = 0; e < 18; e++) {
+				const int n = nb_tab[20 + e];
+				nb_tab[20 + e] = acc;
+				acc += n;
+			}
+			nb_tab[38] = acc;
+		}
+	}
 	team_sync();
 
 	auto hide = [](int v) { if constexpr(T == 64) return opaque_uniform(v); else return opaque(v); };
@@ -965,13 +997,23 @@ __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int
 		for(int c = 0; c < 9; c++) O[c] = other(3 + c);
 		return kf_any_q(w[0], w[1], w[2], O, cosmax) ? BOND : 0u;
 	};
+	// slot of static neighbour i (0 <= i < M)
+	auto nb_slot = [&](int i) {
+		if(i < REC_SLOTS) return rec[REC_HEAD + i];
+		int lo = 0, hi = 18;
+		while(hi - lo > 1) {
+			const int mid = (lo + hi) >> 1;
+			if(nb_tab[20 + mid] <= i) lo = mid;
+			else hi = mid;
+		}
+		return nb_tab[lo] + (i - nb_tab[20 + lo]);
+	};
 	// within a band of one of the distance thresholds (an empty slot is not)
 	auto near_d2 = [&](float d2) { return f32_near(d2, fl) & (d2 < 0.5f * F32_FAR * F32_FAR); };
 	auto bond_f32 = [&](float e0, float e1, float e2, float dx, float dy, float dz, float d2, const float *Oq) -> unsigned {
 		const int v = f32_bond(e0, e1, e2, dx, dy, dz, d2, Oq, fl);
 		return v == KF_YES ? (unsigned) BOND : (v == KF_NO ? 0u : (unsigned) UNSURE);
 	};
-	const bool is_mem = lane < cnt;
 	const MoveShare ms = move_share(lane);
 	int c_acc = 0, d_bonds = 0;
 	unsigned known = 0;  // members whose bonds are counted in their records
@@ -996,9 +1038,9 @@ __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int
 #pragma unroll
 		for(int c = 0; c < 14; c++) sv[c] = s[c];
 		if(is_mem) {
-			if(lane == k) qx[0] = F32_FAR;
+			if(mi == k) qx[0] = F32_FAR;
 			else {
-				const float *so = shadow + lane * SH_W;
+				const float *so = shadow + mi * SH_W;
 				qx[0] = so[0];
 				qy[0] = so[1];
 				qz[0] = so[2];
@@ -1078,7 +1120,7 @@ __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int
 #pragma unroll
 				for(int u = 0; u < CPL; u++)
 					if((v ? b[u] : bo[u]) == UNSURE) {
-						const unsigned e = exact_pair(k, v ? t : -1, cq[u], u == 0 && is_mem ? lane : -1);
+						const unsigned e = exact_pair(k, v ? t : -1, cq[u], u == 0 && is_mem ? mi : -1);
 						if(v) b[u] = e;
 						else bo[u] = e;
 						late |= v && e == OVERLAP;
@@ -1086,13 +1128,13 @@ __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int
 			late = team_any<T>(late);
 		}
 		// the counts: static neighbours, and the members' bits
-		const unsigned mem_mask = (1u << cnt) - 1u;
+		auto member_bits = [&](auto bits) { return (unsigned) (bits >> nstat); };
 		int s_new = 0, s_old = __float_as_int(sv[12]);
 		unsigned mb = 0, mb_old = __float_as_uint(sv[13]);
 		each_slot([&](int u) {
 			const auto bits = team_bits(ballot(b[u] == BOND));
 			s_new += count_bits(bits);
-			if(u == 0) mb = (unsigned) bits & mem_mask;
+			if(u == 0) mb = member_bits(bits);
 		});
 		s_new -= (int) __popc(mb);
 		if(wave_first) {
@@ -1101,7 +1143,7 @@ __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int
 			each_slot([&](int u) {
 				const auto bits = team_bits(ballot(bo[u] == BOND));
 				so += count_bits(bits);
-				if(u == 0) mo = (unsigned) bits & mem_mask;
+				if(u == 0) mo = member_bits(bits);
 			});
 			mb_old = first ? mo : mb_old;
 			s_old = first ? so - (int) __popc(mo) : s_old;
@@ -1110,7 +1152,7 @@ __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int
 			// the static neighbours beyond the register slots, from HBM
 			int n = 0;  // bonds at the new position, and << 16 at the present one
 			bool ov = false;
-			for(int i = lane + T * CPL - cnt; i < M; i += T) {
+			for(int i = lane + nreg; i < M; i += T) {
 				const int q = opaque(nb_slot(i));
 				float rel[3], Oq[9];
 				wild = false;
@@ -1170,8 +1212,8 @@ __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int
 				    lane == 0 ? __int_as_float(s_new) : (lane == 1 ? __uint_as_float(mb) : (float) rv);
 			}
 			// the other members' bits for member k
-			if(is_mem && lane != k) {
-				unsigned *w = (unsigned *) (shadow + lane * SH_W + 13);
+			if(is_mem && mi != k) {
+				unsigned *w = (unsigned *) (shadow + mi * SH_W + 13);
 				*w = (*w & ~(1u << k)) | ((b[0] >> 1) << k);
 			}
 		}
@@ -1188,7 +1230,7 @@ __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int
 				__hip_atomic_store(part(F, at + m) + c, own[m * OWN_W + c], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 			else part(F, at + m)[c] = own[m * OWN_W + c];
 		}
-		if(lane < cnt) {
+		if(is_mem) {
 			int rank = 0;
 			for(int m = 0; m < cnt; m++) rank += own_pid[m] < my_pid;
 			PID[at + rank] = my_pid;
@@ -1213,22 +1255,22 @@ __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int
 }
 
 // One colour pass per launch, one list entry per team.  The grid is sized
-// for the largest list; workgroups reach the 8 XCDs round-robin, and the
-// list is in cell order, so XCD x takes the x-th eighth of the entries
-// actually listed (a slab of the box, whose shared neighbour reads its L2
-// then serves); the surplus workgroups of each XCD leave at once.
+// for the largest list; teams past the end of the list find a record of
+// another sweep and leave (reading the list's length first cost a dependent
+// load in every workgroup).  Workgroups reach the 8 XCDs round-robin, and the
+// list is in cell order, so each XCD takes runs of XCD_RUN workgroups:
+// neighbouring cells, whose shared neighbours its L2 then serves.
+constexpr int XCD_RUN = 16;
+
 template <int T, int CPL, bool ONE, int CAP = CELL_CAP>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_pass(PassArgs a) {
 	extern __shared__ double lds[];
 	const int lane = threadIdx.x & (T - 1);
 	const int team = threadIdx.x / T;
-	const int tpb = blockDim.x / T;
-	const int total = a.d.pfx[a.pass * (a.d.R + 1) + a.d.R];
-	const int per_xcd = ((total + tpb - 1) / tpb + 7) >> 3;  // workgroups with work on each XCD
 	const int i = blockIdx.x >> 3;
-	if(i >= per_xcd) return;
-	const int gi = uni<T>(((blockIdx.x & 7) * per_xcd + i) * tpb + team);
-	if(gi >= total) return;
+	const int blk = (i / XCD_RUN * 8 + (int) (blockIdx.x & 7)) * XCD_RUN + i % XCD_RUN;
+	const int gi = uni<T>(blk * (int) (blockDim.x / T) + team);
+	if(gi >= a.d.total_act) return;
 	pass_cell<T, CPL, ONE, false, CAP>(a.d, a.sweep, a.pass, gi, lane, lds + team * team_lds<CAP>(), 0u);
 }
 
@@ -1356,7 +1398,7 @@ template <int T, int CPL, bool ONE, int CAP = CELL_CAP>
 static void pass_T(const DevState &d, uint64_t sweep, int pass, int block, hipStream_t s) {
 	const int tpb = block / T;
 	int nb = (d.total_act + tpb - 1) / tpb;
-	nb = (nb + 7) & ~7;  // 8 XCDs x the most workgroups one XCD may need
+	nb = (nb + 8 * XCD_RUN - 1) / (8 * XCD_RUN) * (8 * XCD_RUN);  // whole runs on each XCD
 	size_t lds = (size_t) tpb * team_lds<CAP>() * sizeof(double);
 	PassArgs a{d, sweep, pass, 0u};
 	hipLaunchKernelGGL((k_pass<T, CPL, ONE, CAP>), dim3(nb), dim3(block), lds, s, a);
@@ -1615,6 +1657,22 @@ void launch_energy(const DevState &d, int trial, int per_particle, hipStream_t s
 	else hipLaunchKernelGGL(k_energy<32>, grid(block / 32), dim3(block), 0, s, d, trial, per_particle);
 }
 
+// The pair of work item e of a record: the cell's member j with candidate k
+// of the 13 directions m > 13, or two members; false for the half of the
+// member pairs that is skipped.
+__device__ __forceinline__ bool rec_pair(const DevState &d, const int *rec, int s0, int cnt, int m0, int m2, int e, int &j,
+                                         int &q) {
+	if(e < cnt * m2) {
+		j = s0 + e / m2;
+		q = rec_slot(d, rec, e % m2 + m0);
+		return true;
+	}
+	const int a = (e - cnt * m2) / cnt, b2 = (e - cnt * m2) % cnt;
+	j = s0 + a;
+	q = s0 + b2;
+	return a < b2;
+}
+
 // The energy of box trials on the current lists, from the sweep's cell
 // records instead of per particle: listed cell i (of the 8 passes' lists one
 // after another) pairs its members with each other once and with the
@@ -1645,14 +1703,14 @@ __global__ __launch_bounds__(256) void k_energy_rec(DevState d) {
 		int p = 0, gi = i0;
 		while(gi >= lens[p]) gi -= lens[p++];
 		const int *rec = d.rec + ((size_t) p * d.total_act + gi) * REC_W;
-		const int r = rec[62];
+		const int r = rec[REC_REP];
 		const Rep &rp = d.reps[r];
 		if(!rp.trial_active || !rp.trial_rec) continue;
 		// (the early exit may read a stale flag: it only saves work)
 		if(__hip_atomic_load(&d.vflag[r], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) continue;
-		const int s0 = rec[59], cnt = rec[60];
-		const int m0 = rec[32 + 13], m2 = rec[58] - m0;  // candidates in the 13 directions
-		const double *F = pick_buf(d.f, rec[63]);
+		const int s0 = rec[REC_S0], cnt = rec[REC_CNT];
+		const int m0 = rec[REC_M0], m2 = rec[REC_M] - m0;  // candidates in the 13 directions
+		const double *F = pick_buf(d.f, rec[REC_SEL]);
 		const double t0 = rp.trial_s[0], t1 = rp.trial_s[1], t2 = rp.trial_s[2];
 		const double Lx = rp.tg.box[0], Ly = rp.tg.box[1], Lz = rp.tg.box[2];
 		const double iLx = rp.tg.inv_box[0], iLy = rp.tg.inv_box[1], iLz = rp.tg.inv_box[2];
@@ -1661,19 +1719,7 @@ __global__ __launch_bounds__(256) void k_energy_rec(DevState d) {
 		const int work = cnt * m2 + cnt * cnt;
 		for(int e = lane; e < work; e += TT) {
 			int j, q;
-			if(e < cnt * m2) {
-				j = s0 + e / m2;
-				const int k = e % m2 + m0;  // prefix position among the record's 26 neighbours
-				int nb = 13;
-				while(nb < 25 && rec[32 + nb + 1] <= k) nb++;
-				q = rec[nb] + (k - rec[32 + nb]);
-			}
-			else {
-				const int a = (e - cnt * m2) / cnt, b2 = (e - cnt * m2) % cnt;
-				if(a >= b2) continue;
-				j = s0 + a;
-				q = s0 + b2;
-			}
+			if(!rec_pair(d, rec, s0, cnt, m0, m2, e, j, q)) continue;
 			const double px = part(F, j)[0] * t0, py = part(F, j)[1] * t1, pz = part(F, j)[2] * t2;
 			const double dx = kf_min_image(part(F, q)[0] * t0 - px, Lx, iLx);
 			const double dy = kf_min_image(part(F, q)[1] * t1 - py, Ly, iLy);
@@ -1730,24 +1776,6 @@ void launch_energy_rec(const DevState &d, int cus, hipStream_t s) {
 // pair within the bond range in adjacent cells: the trial's energy is the sum
 // over the listed pairs, pair by pair as k_energy_rec takes it.
 
-// The pair of work item e of a record (k_energy_rec's enumeration): the
-// cell's member j with candidate k of the 13 directions m > 13, or two
-// members; false for the half of the member pairs that is skipped.
-__device__ __forceinline__ bool rec_pair(const int *rec, int s0, int cnt, int m0, int m2, int e, int &j, int &q) {
-	if(e < cnt * m2) {
-		j = s0 + e / m2;
-		const int k = e % m2 + m0;
-		int nb = 13;
-		while(nb < 25 && rec[32 + nb + 1] <= k) nb++;
-		q = rec[nb] + (k - rec[32 + nb]);
-		return true;
-	}
-	const int a = (e - cnt * m2) / cnt, b2 = (e - cnt * m2) % cnt;
-	j = s0 + a;
-	q = s0 + b2;
-	return a < b2;
-}
-
 // Which replicas list their pairs this sweep (box trials on current lists
 // whose records were written by this sweep's rebuild), and an empty list.
 __global__ void k_pairs_reset(DevState d) {
@@ -1789,14 +1817,14 @@ __global__ __launch_bounds__(256) void k_pairs_build(DevState d) {
 			int p = 0, gi = i0;
 			while(gi >= lens[p]) gi -= lens[p++];
 			rec = d.rec + ((size_t) p * d.total_act + gi) * REC_W;
-			const Rep &rp = d.reps[rec[62]];
+			const Rep &rp = d.reps[rec[REC_REP]];
 			on = rp.pl_ok != 0;
 			if(on) {
-				s0 = rec[59];
-				cnt = rec[60];
-				m0 = rec[32 + 13];
-				m2 = rec[58] - m0;
-				F = pick_buf(d.f, rec[63]);
+				s0 = rec[REC_S0];
+				cnt = rec[REC_CNT];
+				m0 = rec[REC_M0];
+				m2 = rec[REC_M] - m0;
+				F = pick_buf(d.f, rec[REC_SEL]);
 				for(int a = 0; a < 3; a++) {
 					L[a] = rp.g.box[a];
 					iL[a] = rp.g.inv_box[a];
@@ -1814,7 +1842,7 @@ __global__ __launch_bounds__(256) void k_pairs_build(DevState d) {
 		int n = 0;
 		for(int e = 0; e < work; e++) {
 			int j, q;
-			if(rec_pair(rec, s0, cnt, m0, m2, e, j, q) && close(j, q)) n++;
+			if(rec_pair(d, rec, s0, cnt, m0, m2, e, j, q) && close(j, q)) n++;
 		}
 		const int incl = wave_incl_scan(n);
 		const int tot = __builtin_amdgcn_readlane(incl, 63);
@@ -1830,7 +1858,7 @@ __global__ __launch_bounds__(256) void k_pairs_build(DevState d) {
 		int pos = base + incl - n;
 		for(int e = 0; e < work; e++) {
 			int j, q;
-			if(rec_pair(rec, s0, cnt, m0, m2, e, j, q) && close(j, q)) d.pl[pos++] = make_int2(j, q);
+			if(rec_pair(d, rec, s0, cnt, m0, m2, e, j, q) && close(j, q)) d.pl[pos++] = make_int2(j, q);
 		}
 	}
 }

@@ -524,25 +524,13 @@ struct CellView {
 __device__ inline CellView cell_view(const DevState &d, int pass, int gi) {
 	CellView v;
 	v.rec = d.rec + ((size_t) pass * d.total_act + gi) * REC_W;
-	v.M = v.rec[58];
-	v.s0 = v.rec[59];
-	v.cnt = v.rec[60];
-	v.cloc = v.rec[61];
-	v.r = v.rec[62];
-	v.sel = v.rec[63];
+	v.M = v.rec[REC_M];
+	v.s0 = v.rec[REC_S0];
+	v.cnt = v.rec[REC_CNT];
+	v.cloc = v.rec[REC_CELL];
+	v.r = v.rec[REC_REP];
+	v.sel = v.rec[REC_SEL];
 	return v;
-}
-
-// slot of static neighbour i < M of the cell (the record's 26 ranges; rec may
-// be the global record or a copy of it in LDS)
-__device__ inline int rec_slot(const int *rec, int i) {
-	int lo = 0, hi = 26;
-	while(hi - lo > 1) {
-		const int mid = (lo + hi) >> 1;
-		if(rec[32 + mid] <= i) lo = mid;
-		else hi = mid;
-	}
-	return rec[lo] + (i - rec[32 + lo]);
 }
 
 // Candidates of one wave's cell, staged in LDS: their slots and positions
@@ -557,13 +545,14 @@ struct CandLds {
 // candidate neighbours of the moving slot j: the cell's static neighbours and
 // the other members of the cell
 struct Cands {
+	const DevState &d;
 	const double *F;
 	CellView v;
 	int j;
 	const CandLds *L = nullptr;  // staged slots / positions (filled by stage())
 	__device__ int count() const { return v.M + v.cnt - 1; }
 	__device__ int slot_of(int i) const {
-		if(i < v.M) return rec_slot(L ? L->rec : v.rec, i);
+		if(i < v.M) return rec_slot(d, L ? L->rec : v.rec, i);
 		const int o = v.s0 + (i - v.M);
 		return o < j ? o : o + 1;
 	}
@@ -698,7 +687,7 @@ __global__ __launch_bounds__(64 * LP_WAVES) void k_learn_pass(DevState d, NetDev
 		}
 		const unsigned long long hm = (__ballot(hit) >> (lane & ~(T - 1))) & ((1ull << T) - 1ull);
 		j = v.s0 + (int) __builtin_ctzll(hm);
-		const Cands c{F, v, j, &CL};
+		const Cands c{d, F, v, j, &CL};
 		c.stage<T>(CL, tl);
 		double p[3];
 		for(int k = 0; k < 3; k++) p[k] = part(F, j)[k];
@@ -711,7 +700,7 @@ __global__ __launch_bounds__(64 * LP_WAVES) void k_learn_pass(DevState d, NetDev
 		}
 	__syncthreads();
 	if(live) {
-		const Cands c{F, v, j, &CL};
+		const Cands c{d, F, v, j, &CL};
 		double p[3], O[9];
 		for(int k = 0; k < 3; k++) p[k] = part(F, j)[k];
 		for(int k = 0; k < 9; k++) O[k] = part(F, j)[3 + k];
@@ -780,13 +769,13 @@ __global__ __launch_bounds__(64 * LP_WAVES) void k_learn_pass(DevState d, NetDev
 		         cell_coord(np[1], rp.g.shift[1], rp.g.inv_box[1], n1) == iy &&
 		         cell_coord(np[2], rp.g.shift[2], rp.g.inv_box[2], n2) == iz;
 		if(inside) {
-			const Cands c{F, v, j, &CL};
+			const Cands c{d, F, v, j, &CL};
 			nv = desc_collect<T>(np, c.count(), [&](int i, double q[3]) { c.pos(i, q); }, L, iL, D, row, tl);
 		}
 	}
 	__syncthreads();
 	if(live && inside) {
-		const Cands c{F, v, j, &CL};
+		const Cands c{d, F, v, j, &CL};
 		const double *pp = S.prop[cell];
 		double np[3], On[9];
 		for(int k = 0; k < 3; k++) np[k] = pp[k];
@@ -843,7 +832,7 @@ __global__ __launch_bounds__(64 * LP_WAVES) void k_learn_pass(DevState d, NetDev
 	double Po[4][3], Pn[4][3];
 	kf_patches(O, Po);
 	kf_patches(On, Pn);
-	const Cands c{Fw, v, j, &CL};
+	const Cands c{d, Fw, v, j, &CL};
 	const int n = c.count();
 	int bo = 0, bn = 0;
 	bool ov = false;
