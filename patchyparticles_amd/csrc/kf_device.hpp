@@ -253,6 +253,7 @@ __device__ __forceinline__ unsigned kf_fast_q1(double dx, double dy, double dz, 
 // within reach takes the exact arithmetic.
 constexpr float F32_BAND_D2 = 4e-6f;  // times s rc
 constexpr float F32_BAND_T = 8e-5f;   // times s rc
+constexpr float F32_ALL = 1e28f;      // a band that holds every pair (but not an empty slot's distance)
 constexpr double F32_MAX_POS = 1e7;
 
 struct F32Filter {
@@ -263,7 +264,7 @@ struct F32Filter {
 __device__ __forceinline__ F32Filter f32_filter(double cosmax, double rc2, double side) {
 	const float cm = (float) cosmax, band = (float) (side * sqrt(rc2));
 	const bool off = !(cosmax >= KF_FILTER_MIN_COS);
-	return {(float) rc2, 3.f * (cm * cm), off ? 1e30f : F32_BAND_D2 * band, off ? 1e30f : F32_BAND_T * band};
+	return {(float) rc2, 3.f * (cm * cm), off ? F32_ALL : F32_BAND_D2 * band, off ? F32_ALL : F32_BAND_T * band};
 }
 
 __device__ __forceinline__ bool f32_orientation_ok(const float *o) {
@@ -299,17 +300,17 @@ __device__ __forceinline__ bool f32_near(float d2, const F32Filter &f) {
 }
 
 // The bond of a pair at separation d, with e the separation in p's body
-// frame: KF_YES, KF_NO or KF_UNSURE.
-__device__ __forceinline__ int f32_bond(float e0, float e1, float e2, float dx, float dy, float dz, float d2,
-                                        const float *Oq, const F32Filter &f) {
+// frame: yes, or unsure, or neither.
+__device__ __forceinline__ void f32_bond(float e0, float e1, float e2, float dx, float dy, float dz, float d2,
+                                         const float *Oq, const F32Filter &f, bool &yes, bool &unsure) {
 	const float thr = f.c3 * d2;
-	const float lo = thr - f.eps_t, hi = thr + f.eps_t;
 	const float gp = patch_top(e0, e1, e2), tp = gp * __builtin_fabsf(gp);
 	float f0, f1, f2;
 	mul_t(Oq, -dx, -dy, -dz, f0, f1, f2);
 	const float gq = patch_top(f0, f1, f2), tq = gq * __builtin_fabsf(gq);
-	const float tm = __builtin_fminf(tp, tq);
-	return tm > hi ? KF_YES : (tm < lo ? KF_NO : KF_UNSURE);
+	const float over = __builtin_fminf(tp, tq) - thr;
+	yes = over > f.eps_t;
+	unsure = !(__builtin_fabsf(over) > f.eps_t);
 }
 
 // Cell coordinate of x on a grid of n cells over [s, s+L) (periodic).

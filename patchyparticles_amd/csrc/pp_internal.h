@@ -131,6 +131,7 @@ struct PassGeo {
 	double shift[3], side[3];   // of the sweep's cells
 	float inv_side[3];
 	F32Filter filter;           // of the single-precision pair tests
+	float margin;               // of the single-precision in-cell test, in cell sides
 	int n[3];
 	int n_thr;                  // entries of thr in use
 	uint32_t thr[ACC_TAB - 1];  // a 32-bit draw w accepts a rise of j bonds iff w <= thr[j - 1]

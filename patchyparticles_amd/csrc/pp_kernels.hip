@@ -103,6 +103,8 @@ __device__ __forceinline__ void set_pass_geo(Rep &rp, const Grid &G, const doubl
 		smax = fmax(smax, p.side[k]);
 	}
 	p.filter = f32_filter(rp.cosmax, rp.rc2, smax);
+	// (a step longer than a cell could come round the box: the exact test)
+	p.margin = rp.disp_max < smax ? 1e-5f : F32_ALL;
 	for(int k = 0; k < 3; k++) p.n[k] = G.n[k];
 }
 
@@ -624,6 +626,7 @@ struct TeamLds {
 	static constexpr int NB = PID + (CAP + 1) / 2;
 	static constexpr int GEO = NB + NB_W / 2;
 	static constexpr int SIZE = GEO + GEO_W;
+	static_assert(TRIALS * FT_W / 2 + FT <= OWN, "a trial's successor is inside the block");
 	static_assert(FT % 2 == 0 && OWN % 2 == 0 && TR % 2 == 0 && NB % 2 == 0 && SIZE % 2 == 0, "16-byte aligned parts");
 };
 // Cells of the small-cell pass (dilute systems, 16-lane teams with one
@@ -639,7 +642,7 @@ constexpr int team_lds() {
 static_assert(16 * team_lds<>() * sizeof(double) <= 160 * 1024, "two pass workgroups per CU");
 static_assert(32 * team_lds<SMALL_CAP>() * sizeof(double) <= 160 * 1024, "eight small-cell workgroups per CU");
 
-constexpr float F32_CELL = 1e-5f;  // in-cell margin of the single-precision test, in cell sides
+constexpr int MOST_EXP = 1 << 16;  // a trial whose draw accepts every tabulated rise
 constexpr float F32_FAR = 1e15f;   // the position of an empty slot
 
 // One lane's share of an accepted move, values v = 0..14 of the moving
@@ -843,7 +846,7 @@ __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int
 		f[0] = (float) tv[1];
 		f[1] = (float) tv[2];
 		f[2] = (float) tv[3];
-		f[3] = __int_as_float(most);
+		f[3] = __int_as_float(most < ACC_TAB - 1 ? most : MOST_EXP);
 #pragma unroll
 		for(int e = 0; e < 9; e++) f[4 + e] = (float) tv[4 + e];
 		f[13] = __int_as_float(k);
@@ -856,6 +859,7 @@ __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int
 		else if constexpr(T == 32) return koff ? (unsigned) (m >> 32) : (unsigned) m;
 		else return (unsigned) (m >> koff) & ((1u << T) - 1u);
 	};
+	auto team_has = [&](unsigned long long m) { return team_bits(m) != 0; };
 	auto count_bits = [](auto m) {
 		if constexpr(sizeof(m) == 8) return (int) __popcll(m);
 		else return (int) __popc(m);
@@ -900,6 +904,7 @@ __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int
 		}
 #pragma unroll
 		for(int c = 0; c < 9; c++) s[3 + c] = of[c];
+		s[12] = __int_as_float(-1);  // bonds not counted yet
 	}
 	if constexpr(DD) {
 		// the neighbours' data once their earlier passes are done
@@ -924,8 +929,8 @@ __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int
 		}
 	}
 	F32Filter fl = pg.filter;
-	if(team_any<T>(wild)) fl.eps_d2 = fl.eps_t = 1e30f;
-	const float is0 = pg.inv_side[0], is1 = pg.inv_side[1], is2 = pg.inv_side[2];
+	if(team_any<T>(wild)) fl.eps_d2 = fl.eps_t = F32_ALL;
+	const float margin = pg.margin, is0 = pg.inv_side[0], is1 = pg.inv_side[1], is2 = pg.inv_side[2];
 	// whether any team of the wavefront has neighbours beyond the register
 	// slots (a scalar branch around those loops)
 	const bool wave_far = ballot(M > nreg) != 0ull;
@@ -1008,35 +1013,22 @@ __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int
 		}
 		return nb_tab[lo] + (i - nb_tab[20 + lo]);
 	};
-	// within a band of one of the distance thresholds (an empty slot is not)
-	auto near_d2 = [&](float d2) { return f32_near(d2, fl) & (d2 < 0.5f * F32_FAR * F32_FAR); };
-	auto bond_f32 = [&](float e0, float e1, float e2, float dx, float dy, float dz, float d2, const float *Oq) -> unsigned {
-		const int v = f32_bond(e0, e1, e2, dx, dy, dz, d2, Oq, fl);
-		return v == KF_YES ? (unsigned) BOND : (v == KF_NO ? 0u : (unsigned) UNSURE);
-	};
 	const MoveShare ms = move_share(lane);
 	int c_acc = 0, d_bonds = 0;
-	unsigned known = 0;  // members whose bonds are counted in their records
-	float ft[14];
-	auto read_trial = [&](int t) {
-		const float *f = ftrial + t * FT_W;
-#pragma unroll
-		for(int e = 0; e < 14; e++) ft[e] = f[e];
-	};
-	read_trial(0);
+	int next_k = __float_as_int(ftrial[13]);
 
 	// 5. the trials
 	for(int t = 0; t < ntrial; t++) {
-		// the trial (read one ahead), the moving member's record, another
-		// member's for a member lane, and the lane's share of the exact move
-		float tv[14];
-#pragma unroll
-		for(int e = 0; e < 14; e++) tv[e] = ft[e];
-		const int k = __float_as_int(tv[13]);
-		const float *s = shadow + k * SH_W;
-		float sv[14];
+		// the moving member's record (its rank was read one trial ahead), the
+		// trial, another member's record for a member lane, and the lane's
+		// share of the exact move
+		const int k = next_k;
+		const float *s = shadow + k * SH_W, *f = ftrial + t * FT_W;
+		float sv[14], tv[13];
 #pragma unroll
 		for(int c = 0; c < 14; c++) sv[c] = s[c];
+#pragma unroll
+		for(int e = 0; e < 13; e++) tv[e] = f[e];
 		if(is_mem) {
 			if(mi == k) qx[0] = F32_FAR;
 			else {
@@ -1050,17 +1042,18 @@ __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int
 		}
 		const double *dt = trials + t * TR_W;
 		const double *me = own + k * OWN_W + ms.o, *tm = dt + ms.r;
-		const double o0 = me[0], o1 = me[ms.dot ? 1 : 0], o2 = me[ms.dot ? 2 : 0];
-		const double r0 = tm[0], r1 = tm[ms.dot ? 3 : 0], r2 = tm[ms.dot ? 6 : 0];
-		read_trial(t + 1 < ntrial ? t + 1 : t);
+		const double o0 = me[0], o1 = me[1], o2 = me[2];
+		const double r0 = tm[0], r1 = tm[3], r2 = tm[6];
+		next_k = __float_as_int(f[FT_W + 13]);  // (past the last trial: not used)
 		const float nx = sv[0] + tv[0], ny = sv[1] + tv[1], nz = sv[2] + tv[2];
 
 		// a trial that leaves the cell, or overlaps a neighbour, is rejected;
 		// what single precision cannot tell stays for the exact arithmetic
 		const float x = __builtin_fmaxf(__builtin_fabsf(nx) * is0, __builtin_fmaxf(__builtin_fabsf(ny) * is1,
 		                                                                         __builtin_fabsf(nz) * is2));
-		const bool close = !(__builtin_fabsf(x - 0.5f) > F32_CELL) | !(x < 1.5f);
-		bool rej = (x > 0.5f) & !close, unsure = close;
+		// (conditions are kept as lane masks in scalar registers)
+		const unsigned long long m_close = ballot(!(__builtin_fabsf(x - 0.5f) > margin));
+		unsigned long long m_rej = ballot(x > 0.5f) & ~m_close, m_unsure = m_close;
 		// slots in use by the wavefront's teams (a scalar branch)
 		auto each_slot = [&](auto &&f) {
 			f(0);
@@ -1068,47 +1061,55 @@ __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int
 				if(wave_2) f(1);
 		};
 		float dx[CPL], dy[CPL], dz[CPL], d2[CPL];
-		bool near[CPL];
+		unsigned long long m_near[CPL] = {}, m_onear[CPL] = {}, m_bond[CPL] = {}, m_obond[CPL] = {};
 		each_slot([&](int u) {
 			dx[u] = qx[u] - nx;
 			dy[u] = qy[u] - ny;
 			dz[u] = qz[u] - nz;
 			d2[u] = norm2(dx[u], dy[u], dz[u]);
-			near[u] = near_d2(d2[u]);
-			rej |= (d2[u] < 1.f) & !near[u];
+			m_near[u] = ballot(f32_near(d2[u], fl));
+			m_rej |= ballot(d2[u] < 1.f) & ~m_near[u];
 		});
-		if(team_any<T>(rej)) continue;
+		if(team_has(m_rej)) continue;
 
 		// bonds at the new position: O'^T d = R^T (O^T d)
-		unsigned b[CPL] = {}, bo[CPL] = {};
 		each_slot([&](int u) {
-			if(d2[u] < fl.rc2) {
+			const unsigned long long m_in = ballot(d2[u] < fl.rc2);
+			if(m_in != 0ull) {
 				float a0, a1, a2, e0, e1, e2;
+				bool yes, unsure;
 				mul_t(sv + 3, dx[u], dy[u], dz[u], a0, a1, a2);
 				mul_t(tv + 4, a0, a1, a2, e0, e1, e2);
-				b[u] = bond_f32(e0, e1, e2, dx[u], dy[u], dz[u], d2[u], qo[u]);
+				f32_bond(e0, e1, e2, dx[u], dy[u], dz[u], d2[u], qo[u], fl, yes, unsure);
+				m_bond[u] = ballot(yes) & m_in & ~m_near[u];
+				m_near[u] |= ballot(unsure) & m_in;
 			}
-			b[u] = near[u] ? (unsigned) UNSURE : b[u];
-			unsure |= b[u] == UNSURE;
+			m_unsure |= m_near[u];
 		});
 		// the bonds at the present position, when not yet counted
-		const bool first = !((known >> k) & 1u);
+		int s_old = __float_as_int(sv[12]);
+		unsigned mb_old = __float_as_uint(sv[13]);
+		const bool first = s_old < 0;
 		const bool wave_first = ballot(first) != 0ull;
 		if(wave_first)
 			each_slot([&](int u) {
 				const float ex = qx[u] - sv[0], ey = qy[u] - sv[1], ez = qz[u] - sv[2];
 				const float e2 = norm2(ex, ey, ez);
-				if(e2 < fl.rc2) {
+				const unsigned long long m_in = ballot(e2 < fl.rc2);
+				m_onear[u] = ballot(f32_near(e2, fl));
+				if(m_in != 0ull) {
 					float a0, a1, a2;
+					bool yes, unsure;
 					mul_t(sv + 3, ex, ey, ez, a0, a1, a2);
-					bo[u] = bond_f32(a0, a1, a2, ex, ey, ez, e2, qo[u]);
+					f32_bond(a0, a1, a2, ex, ey, ez, e2, qo[u], fl, yes, unsure);
+					m_obond[u] = ballot(yes) & m_in & ~m_onear[u];
+					m_onear[u] |= ballot(unsure) & m_in;
 				}
-				bo[u] = near_d2(e2) ? (unsigned) UNSURE : bo[u];
-				unsure |= bo[u] == UNSURE;
+				m_unsure |= m_onear[u];
 			});
 		bool late = false;  // a rejection found by the exact arithmetic
-		if(__builtin_expect(ballot(unsure) != 0ull, 0)) {
-			if(close) {
+		if(__builtin_expect(m_unsure != 0ull, 0)) {
+			if(__builtin_amdgcn_inverse_ballot_w64(m_close)) {
 				const Grid &G = d.reps[hide_rep()].g;
 				const int at[3] = {ix, iy, iz};
 #pragma unroll 1
@@ -1118,35 +1119,36 @@ __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int
 #pragma unroll 1
 			for(int v = 0; v < 2; v++)
 #pragma unroll
-				for(int u = 0; u < CPL; u++)
-					if((v ? b[u] : bo[u]) == UNSURE) {
-						const unsigned e = exact_pair(k, v ? t : -1, cq[u], u == 0 && is_mem ? mi : -1);
-						if(v) b[u] = e;
-						else bo[u] = e;
-						late |= v && e == OVERLAP;
-					}
+				for(int u = 0; u < CPL; u++) {
+					unsigned e = 0;
+					if(__builtin_amdgcn_inverse_ballot_w64(v ? m_near[u] : m_onear[u]))
+						e = exact_pair(k, v ? t : -1, cq[u], u == 0 && is_mem ? mi : -1);
+					const unsigned long long m = ballot(e == BOND);
+					if(v) m_bond[u] |= m;
+					else m_obond[u] |= m;
+					late |= v && e == OVERLAP;
+				}
 			late = team_any<T>(late);
 		}
-		// the counts: static neighbours, and the members' bits
+		// the counts: all bonds, and the members' as bits
 		auto member_bits = [&](auto bits) { return (unsigned) (bits >> nstat); };
-		int s_new = 0, s_old = __float_as_int(sv[12]);
-		unsigned mb = 0, mb_old = __float_as_uint(sv[13]);
+		int n_new = 0;
+		unsigned mb = 0;
 		each_slot([&](int u) {
-			const auto bits = team_bits(ballot(b[u] == BOND));
-			s_new += count_bits(bits);
+			const auto bits = team_bits(m_bond[u]);
+			n_new += count_bits(bits);
 			if(u == 0) mb = member_bits(bits);
 		});
-		s_new -= (int) __popc(mb);
 		if(wave_first) {
-			int so = 0;
+			int n = 0;
 			unsigned mo = 0;
 			each_slot([&](int u) {
-				const auto bits = team_bits(ballot(bo[u] == BOND));
-				so += count_bits(bits);
+				const auto bits = team_bits(m_obond[u]);
+				n += count_bits(bits);
 				if(u == 0) mo = member_bits(bits);
 			});
 			mb_old = first ? mo : mb_old;
-			s_old = first ? so - (int) __popc(mo) : s_old;
+			s_old = first ? n - (int) __popc(mo) : s_old;
 		}
 		if(wave_far) {
 			// the static neighbours beyond the register slots, from HBM
@@ -1174,12 +1176,14 @@ __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int
 					const float gx = fx - (v ? nx : sv[0]), gy = fy - (v ? ny : sv[1]), gz = fz - (v ? nz : sv[2]);
 					const float g2 = v ? gn2 : go2;
 					unsigned bf = g2 < 1.f ? (unsigned) OVERLAP : 0u;
-					if(wild || near_d2(g2)) bf = UNSURE;
+					if(wild || f32_near(g2, fl)) bf = UNSURE;
 					else if(g2 >= 1.f && g2 < fl.rc2) {
 						float a0, a1, a2, e0, e1, e2;
 						mul_t(sv + 3, gx, gy, gz, a0, a1, a2);
 						mul_t(tv + 4, a0, a1, a2, e0, e1, e2);
-						bf = bond_f32(v ? e0 : a0, v ? e1 : a1, v ? e2 : a2, gx, gy, gz, g2, Oq);
+						bool is, maybe;
+						f32_bond(v ? e0 : a0, v ? e1 : a1, v ? e2 : a2, gx, gy, gz, g2, Oq, fl, is, maybe);
+						bf = maybe ? (unsigned) UNSURE : (is ? (unsigned) BOND : 0u);
 					}
 					if(bf == UNSURE) bf = exact_pair(k, v ? t : -1, q, -1);
 					ov |= v && bf == OVERLAP;
@@ -1188,19 +1192,19 @@ __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int
 			}
 			late |= team_any<T>(ov);
 			n = team_sum<T>(n);
-			s_new += n & 0xffff;
+			n_new += n & 0xffff;
 			if(first) s_old += n >> 16;
 		}
-		known |= 1u << k;
-		const int db = s_new + (int) __popc(mb) - s_old - (int) __popc(mb_old);
+		const int db = n_new - (s_old + (int) __popc(mb_old));
 		// MC.c:332: accept if dE <= 0 or a uniform draw u < exp(-dE/T), with
-		// dE = -db an integer: below ACC_TAB the trial holds the comparison
-		bool acc = -db <= __float_as_int(tv[3]);
-		if(ballot(-db >= ACC_TAB) != 0ull && -db >= ACC_TAB) {
+		// dE = -db an integer: the trial holds the largest rise it accepts
+		// (MOST_EXP: at least ACC_TAB - 1, beyond which the factor is formed)
+		bool acc = -db <= __float_as_int(tv[3]) && !late;
+		if(acc && -db >= ACC_TAB) {
 			const u32x4 rb = rng(d.seed, r, sweep, (uint32_t) hide(cloc), TAG_TRIAL_B, (uint32_t) col, (uint32_t) t);
 			acc = u01(rb.w) < exp((double) db / d.reps[hide_rep()].T);
 		}
-		if(acc && !late) {
+		if(acc) {
 			c_acc++;
 			d_bonds += db;
 			// the new state, one value per lane, exact and single precision;
@@ -1209,12 +1213,12 @@ __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int
 			if(lane < 15) {
 				own[k * OWN_W + lane] = rv;
 				shadow[k * SH_W + ms.word] =
-				    lane == 0 ? __int_as_float(s_new) : (lane == 1 ? __uint_as_float(mb) : (float) rv);
+				    lane == 0 ? __int_as_float(n_new - (int) __popc(mb)) : (lane == 1 ? __uint_as_float(mb) : (float) rv);
 			}
 			// the other members' bits for member k
 			if(is_mem && mi != k) {
 				unsigned *w = (unsigned *) (shadow + mi * SH_W + 13);
-				*w = (*w & ~(1u << k)) | ((b[0] >> 1) << k);
+				*w = (*w & ~(1u << k)) | (((mb >> mi) & 1u) << k);
 			}
 		}
 		else if(first && lane < 2)

@@ -53,8 +53,9 @@ __global__ void k_check(const Pair *pairs, int n, double L, double side, double 
 			float a0, a1, a2, e0, e1, e2;
 			mul_t(O, d[0], d[1], d[2], a0, a1, a2);
 			mul_t(R, a0, a1, a2, e0, e1, e2);
-			const int b = f32_bond(e0, e1, e2, d[0], d[1], d[2], d2, Q, fl);
-			got = b == KF_YES ? 1 : (b == KF_NO ? 0 : 2);
+			bool yes, unsure;
+			f32_bond(e0, e1, e2, d[0], d[1], d[2], d2, Q, fl, yes, unsure);
+			got = unsure ? 2 : (yes ? 1 : 0);
 		}
 	}
 	// the reference arithmetic
