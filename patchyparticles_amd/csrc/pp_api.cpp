@@ -308,12 +308,16 @@ pp_status create_impl(int R, const pp_params *prm, const pp_options *opts, const
 	if(R <= 0 || !prm || !n || !box) return fail(PP_ERR_ARG, "bad replica arguments");
 	pp_options o{};
 	if(opts) o = *opts;
+	// left open: 32 lanes per cell (16 on large systems, decided once the
+	// grids are known), one wavefront per workgroup for the per-pass launches
+	// (a pass's few workgroups start sooner: 74 against 77 us per sweep at
+	// N=1000), else the largest workgroup of at most MAX_TEAMS teams
+	const bool per_pass = o.launch != PP_LAUNCH_COOP && o.launch != PP_LAUNCH_DEPS;
+	const bool auto_T = o.threads_per_cell == 0 && per_pass;
 	if(o.threads_per_cell == 0) o.threads_per_cell = 32;
 	if(o.block_size == 0) {
-		// the largest workgroup whose teams' LDS fits
-		o.block_size = 256;
-		while(o.block_size > 64 && pass_lds_bytes(o.threads_per_cell, o.block_size) > MAX_LDS_BYTES)
-			o.block_size /= 2;
+		o.block_size = per_pass ? 64 : 256;
+		while(o.block_size > 64 && o.block_size > MAX_TEAMS * o.threads_per_cell) o.block_size /= 2;
 	}
 	const int Tv = o.threads_per_cell;
 	if(Tv != 16 && Tv != 32 && Tv != 64) return fail(PP_ERR_ARG, "threads_per_cell must be 16, 32 or 64");
@@ -326,9 +330,9 @@ pp_status create_impl(int R, const pp_params *prm, const pp_options *opts, const
 		return fail(PP_ERR_ARG, "the dependency-driven launch form takes 32 or 64 threads per cell");
 	if(o.trials_per_cell < 0 || o.trials_per_cell > MAX_TRIALS_PER_CELL)
 		return fail(PP_ERR_ARG, "trials_per_cell must be in [0, %d]", MAX_TRIALS_PER_CELL);
-	if(pass_lds_bytes(Tv, o.block_size) > MAX_LDS_BYTES)
-		return fail(PP_ERR_ARG, "threads_per_cell %d with block_size %d needs %zu bytes of LDS (max %zu)", Tv,
-		            o.block_size, pass_lds_bytes(Tv, o.block_size), MAX_LDS_BYTES);
+	if(o.block_size > MAX_TEAMS * Tv)
+		return fail(PP_ERR_ARG, "threads_per_cell %d with block_size %d makes %d cells per workgroup (max %d)", Tv,
+		            o.block_size, o.block_size / Tv, MAX_TEAMS);
 
 	// slots per replica: its particles, or for a grand-canonical replica the
 	// most it may hold (GC_N_max)
@@ -460,6 +464,25 @@ pp_status create_impl(int R, const pp_params *prm, const pp_options *opts, const
 	                                                                                   : SCAN_TILE_LARGE;
 	d.ntiles = (d.C_total + d.scan_tile - 1) / d.scan_tile;
 	d.total_act = (int) aoff;
+	if(hipDeviceGetAttribute(&c->cus, hipDeviceAttributeMultiprocessorCount, o.device) != hipSuccess || c->cus <= 0)
+		c->cus = 256;
+	if(auto_T && !c->any_gc && o.block_size <= MAX_TEAMS * 16) {
+		// 16 lanes per cell once a pass's cells are more than 32-lane teams
+		// fit on the chip at two wavefronts per SIMD (16 cells per CU; the
+		// count for independent points, a tenth below that of spheres), unless
+		// the neighbourhoods pass the 32 register slots of such a team.
+		// Steps of 16 trials per cell, 32 against 16 lanes: 196 and 233 us at
+		// N=32768, 309 and 239 at 49152, 339 and 231 at 65536 (rho 0.3); 40
+		// replicas of 2000 at rho 0.6 (31 candidates) 346 and 515.
+		double cells = 0., listed = 0.;
+		for(int k = 0; k < R; k++) {
+			const Grid &g = c->reps[k].g;
+			const double C = (double) g.n[0] * g.n[1] * g.n[2];
+			cells += C;
+			listed += C / 8. * (1. - std::exp(-n[k] / C));
+		}
+		if(listed > 0.9 * 16. * c->cus && 27. * (double) nsum <= 24. * cells) c->T = 16;
+	}
 	{
 		// the kernels carry the base patches as compile-time constants
 		const Base hb = host_base_patches();
@@ -538,8 +561,6 @@ pp_status create_impl(int R, const pp_params *prm, const pp_options *opts, const
 		if(const char *e = getenv("PP_SMALL_CELL_CAP"))
 			if(*e) d.small_cap = std::max(1, std::min(small_cell_cap(), atoi(e)));
 	}
-	if(hipDeviceGetAttribute(&c->cus, hipDeviceAttributeMultiprocessorCount, o.device) != hipSuccess || c->cus <= 0)
-		c->cus = 256;
 	{
 		// every buffer a kernel may touch must exist before the first launch
 		const void *need[] = {d.f[0], d.f[1], d.pid[0], d.pid[1], d.reps, d.prep, d.act_off, d.count, d.start,
@@ -819,7 +840,7 @@ pp_status pp_autotune(pp_ctx *c, int sweeps, int *threads_per_cell, int *block_s
 	const int Ts[3] = {16, 32, 64}, blocks[3] = {64, 128, 256};
 	for(int ti = 0; ti < 3 && st == PP_OK; ti++)
 		for(int bi = 0; bi < 3 && st == PP_OK; bi++) {
-			if(pass_lds_bytes(Ts[ti], blocks[bi]) > MAX_LDS_BYTES || blocks[bi] < Ts[ti]) continue;
+			if(blocks[bi] > MAX_TEAMS * Ts[ti] || blocks[bi] < Ts[ti]) continue;
 			c->T = Ts[ti];
 			c->block = blocks[bi];
 			st = enqueue_sweep(c);  // warm-up of this shape

@@ -309,6 +309,7 @@ hipError_t launch_sweep_passes(const DevState &d, uint64_t sweep, int T, int blo
 int sweep_blocks_max(int T, int block, int cus);  // co-resident workgroups of that launch
 size_t pass_lds_bytes(int T, int block);  // dynamic LDS of one pass workgroup
 constexpr size_t MAX_LDS_BYTES = 65536;
+constexpr int MAX_TEAMS = 6;  // cells one pass workgroup may work on
 void launch_energy(const DevState &d, int trial, int per_particle, hipStream_t s);
 void launch_bond_list(const DevState &d, int max_per, int *count, int *partners, hipStream_t s);
 // volume-move attempt k of sweep `sweep` (NPT replicas only)

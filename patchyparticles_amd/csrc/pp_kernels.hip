@@ -607,14 +607,13 @@ struct PassArgs {
 //   TR  the trials' exact displacement and R
 //   PID particle indices
 //   NB  (neighbourhoods beyond the record's list) the rows' slot ranges
-//   GEO constants of the exact arithmetic and the far neighbours, here so
-//       that the trial loop does not hold them in registers
-constexpr int OWN_W = 16;  // x, y, z, O[9], rel[3], one unused
+//   GEO the cell's centre, for the far neighbours
+constexpr int OWN_W = 15;  // x, y, z, O[9], rel[3]
 constexpr int TR_W = 12;   // dx, dy, dz, R[9]
-constexpr int SH_W = 16;   // floats: rel[3], O[9], static bonds, member bond bits, two unused
-constexpr int FT_W = 16;   // floats: dx, dy, dz, the rise it accepts, R[9], rank, two unused
+constexpr int SH_W = 14;   // floats: rel[3], O[9], static bonds, member bond bits
+constexpr int FT_W = 14;   // floats: dx, dy, dz, the rise it accepts, R[9], rank
 constexpr int NB_W = 40;   // ints: first slots [0, 18) and exclusive prefix [20, 39) of the rows' ranges
-constexpr int GEO_W = 12;  // box[3], 1 / box[3], the cell's centre[3], rc^2, cosmax, one unused
+constexpr int GEO_W = 3;   // the cell's centre
 template <int CAP>
 struct TeamLds {
 	static constexpr int TRIALS = CAP > MAX_TRIALS_PER_CELL ? CAP : MAX_TRIALS_PER_CELL;
@@ -622,25 +621,25 @@ struct TeamLds {
 	static constexpr int FT = SH + CAP * SH_W / 2;
 	static constexpr int OWN = FT + TRIALS * FT_W / 2;
 	static constexpr int TR = OWN + CAP * OWN_W;
-	static constexpr int PID = TR + TRIALS * TR_W;
+	static constexpr int GEO = TR + TRIALS * TR_W;
+	static constexpr int PID = GEO + GEO_W;
 	static constexpr int NB = PID + (CAP + 1) / 2;
-	static constexpr int GEO = NB + NB_W / 2;
-	static constexpr int SIZE = GEO + GEO_W;
-	static_assert(TRIALS * FT_W / 2 + FT <= OWN, "a trial's successor is inside the block");
-	static_assert(FT % 2 == 0 && OWN % 2 == 0 && TR % 2 == 0 && NB % 2 == 0 && SIZE % 2 == 0, "16-byte aligned parts");
+	// (the small-cell pass defers the neighbourhoods that need NB)
+	static constexpr int SIZE = NB + (CAP < CELL_CAP ? 0 : NB_W / 2);
+	static_assert(SH_W % 2 == 0 && FT_W % 2 == 0, "whole words");
 };
-// Cells of the small-cell pass (dilute systems, 16-lane teams with one
-// register slot per lane): half the LDS of a general team, so twice the
-// cells stay resident; fuller cells are deferred to the general pass.
+// The small-cell pass (16-lane teams): cells of up to SMALL_CAP members whose
+// neighbours fit the record's list, in 3.9 KB of LDS per team where a general
+// team takes 8.2, so that the registers and not the LDS limit the wavefronts
+// of a CU; other cells are deferred to the general pass.
 constexpr int SMALL_CAP = 8;
 template <int CAP = CELL_CAP>
 constexpr int team_lds() {
 	return TeamLds<CAP>::SIZE;
 }
-// 16 general teams (four 128-thread workgroups of 32-lane teams, the default
-// shape) share a CU's 160 KiB; 32 small-cell teams do
-static_assert(16 * team_lds<>() * sizeof(double) <= 160 * 1024, "two pass workgroups per CU");
-static_assert(32 * team_lds<SMALL_CAP>() * sizeof(double) <= 160 * 1024, "eight small-cell workgroups per CU");
+static_assert(16 * team_lds<>() * sizeof(double) <= 160 * 1024, "16 general teams per CU");
+static_assert(40 * team_lds<SMALL_CAP>() * sizeof(double) <= 160 * 1024, "40 small-cell teams per CU");
+static_assert(MAX_TEAMS * team_lds<>() * sizeof(double) <= MAX_LDS_BYTES, "a workgroup's teams");
 
 constexpr int MOST_EXP = 1 << 16;  // a trial whose draw accepts every tabulated rise
 constexpr float F32_FAR = 1e15f;   // the position of an empty slot
@@ -659,7 +658,7 @@ __device__ __forceinline__ MoveShare move_share(int v) {
 	m.dot = v >= 3 && v < 12;
 	m.o = m.dot ? 3 + 3 * ((v - 3) / 3) : (v < 15 ? v : 0);
 	m.r = m.dot ? 3 + (v - 3) % 3 : (v < 3 ? v : (v >= 12 && v < 15 ? v - 12 : 0));
-	m.word = v < 3 ? 12 + v : (v < 12 ? v : v - 12);
+	m.word = v < 3 ? (v == 0 ? 12 : 13) : (v < 12 ? v : v - 12);
 	return m;
 }
 
@@ -740,8 +739,9 @@ __device__ __forceinline__ void wait_neighbours(const DevState &d, const Rep &rp
 // writes its members back with agent-scope stores, waits for them to
 // complete, and publishes `mark` for its own cell.
 //
-// CAP < CELL_CAP (the small-cell pass): a cell of more than CAP members is
-// not worked on here but listed for the general pass that follows.
+// CAP < CELL_CAP (the small-cell pass): a cell of more than CAP members, or
+// with more neighbours than its record lists, is not worked on here but
+// listed for the general pass that follows.
 template <int T, int CPL, bool ONE, bool DD, int CAP = CELL_CAP>
 __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int pass, int gi, int lane, double *blk,
                                           unsigned mark) {
@@ -770,7 +770,7 @@ __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int
 	const int sel = uni<T>(h1.z);
 	const int ix = uni<T>(h2.x), iy = uni<T>(h2.y), iz = uni<T>(h2.z);
 	if constexpr(CAP < CELL_CAP)
-		if(cnt > d.small_cap) {
+		if(cnt > d.small_cap || M > REC_SLOTS) {
 			// (entries < total_act: each cell is listed at most once a pass)
 			if(lane == 0) d.ovf[atomicAdd(d.ovf_n + pass, 1)] = gi;
 			return;
@@ -800,27 +800,20 @@ __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int
 	const int mi = lane - nstat;      // this lane's member
 	const bool is_mem = mi >= 0;
 	const int nreg = min(M, min(T * CPL - cnt, REC_SLOTS));
-	int my_pid = 0;
-	double mine[NCOMP];
-	if(is_mem) {
-		my_pid = PID[s0 + mi];
+	if(is_mem || lane >= nreg) cq[0] = -1;
+	if constexpr(CPL > 1) cq[1] = nstat + lane < nreg ? rec[REC_HEAD + nstat + lane] : -1;
+	// the lane's member or first static neighbour, in one set of registers
+	// (second slots follow once that one is converted)
+	const int my_pid = is_mem ? PID[s0 + mi] : 0;
+	double pv[NCOMP];
+	auto load_part = [&](int j) {
 #pragma unroll
-		for(int c = 0; c < NCOMP; c++) mine[c] = part(F, s0 + mi)[c];
-	}
+		for(int c = 0; c < NCOMP; c++) pv[c] = nbld<DD>(part(F, j) + c);
+	};
+	if(is_mem || (!DD && cq[0] >= 0)) load_part(is_mem ? s0 + mi : cq[0]);
 	// trials of the cell in this pass: one per member (a sweep is then N
 	// attempts), or a fixed number per non-empty cell
 	const int ntrial = d.trials_per_cell > 0 ? d.trials_per_cell : cnt;
-	if(is_mem || lane >= nreg) cq[0] = -1;
-	if constexpr(CPL > 1) cq[1] = nstat + lane < nreg ? rec[REC_HEAD + nstat + lane] : -1;
-	double sd[CPL][NCOMP];
-	auto load_static = [&]() {
-#pragma unroll
-		for(int u = 0; u < CPL; u++)
-			if(cq[u] >= 0)
-#pragma unroll
-				for(int c = 0; c < NCOMP; c++) sd[u][c] = nbld<DD>(part(F, cq[u]) + c);
-	};
-	if constexpr(!DD) load_static();
 	const PassGeo &pg = rp.pg;
 	const int col = ((ix & 1) << 2) | ((iy & 1) << 1) | (iz & 1);
 	// the cell's centre
@@ -866,10 +859,9 @@ __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int
 	};
 	if(is_mem) own_pid[mi] = my_pid;
 	if(lane == 0) {
-		const double g[GEO_W] = {pg.box[0], pg.box[1], pg.box[2], pg.inv_box[0], pg.inv_box[1], pg.inv_box[2],
-		                         ce0, ce1, ce2, rp.rc2, rp.cosmax, 0.};
-#pragma unroll
-		for(int e = 0; e < GEO_W; e++) geo[e] = g[e];
+		geo[0] = ce0;
+		geo[1] = ce1;
+		geo[2] = ce2;
 	}
 	team_sync();
 	// 4. members into LDS ranked by particle index; a lane's slots become
@@ -884,59 +876,69 @@ __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int
 	auto check_o = [&](const float *o) {
 		wild |= !f32_orientation_ok(o);
 	};
-	if(is_mem) {
-		int rank = 0;
-		for(int m = 0; m < cnt; m++) rank += own_pid[m] < my_pid;
-		double *w = own + rank * OWN_W;
-		float *s = shadow + rank * SH_W;
+	float qx[CPL], qy[CPL], qz[CPL], qo[CPL][9];
+	// pv in single precision, into slot u
+	auto convert = [&](int u, double *rel) {
+		rel3(pv, rel);
+		qx[u] = (float) rel[0];
+		qy[u] = (float) rel[1];
+		qz[u] = (float) rel[2];
+#pragma unroll
+		for(int c = 0; c < 9; c++) qo[u][c] = (float) pv[3 + c];
+		check_o(qo[u]);
+	};
+	auto empty_slot = [&](int u) {
+		qx[u] = qy[u] = qz[u] = F32_FAR;
+#pragma unroll
+		for(int c = 0; c < 9; c++) qo[u][c] = 0.f;
+	};
+	empty_slot(0);
+	if(is_mem || (!DD && cq[0] >= 0)) {
 		double rel[3];
-		rel3(mine, rel);
-		float of[9];
+		convert(0, rel);
+		if(is_mem) {
+			int rank = 0;
+			for(int m = 0; m < cnt; m++) rank += own_pid[m] < my_pid;
+			double *w = own + rank * OWN_W;
+			float *s = shadow + rank * SH_W;
 #pragma unroll
-		for(int c = 0; c < NCOMP; c++) w[c] = mine[c];
+			for(int c = 0; c < NCOMP; c++) w[c] = pv[c];
 #pragma unroll
-		for(int c = 0; c < 9; c++) of[c] = (float) mine[3 + c];
-		check_o(of);
+			for(int c = 0; c < 3; c++) w[12 + c] = rel[c];
+			s[0] = qx[0];
+			s[1] = qy[0];
+			s[2] = qz[0];
 #pragma unroll
-		for(int c = 0; c < 3; c++) {
-			w[12 + c] = rel[c];
-			s[c] = (float) rel[c];
+			for(int c = 0; c < 9; c++) s[3 + c] = qo[0][c];
+			s[12] = __int_as_float(-1);  // bonds not counted yet
 		}
-#pragma unroll
-		for(int c = 0; c < 9; c++) s[3 + c] = of[c];
-		s[12] = __int_as_float(-1);  // bonds not counted yet
 	}
 	if constexpr(DD) {
 		// the neighbours' data once their earlier passes are done
 		wait_neighbours<T>(d, rp, pass, ix, iy, iz, mark, lane);
-		load_static();
-	}
-	float qx[CPL], qy[CPL], qz[CPL], qo[CPL][9];
-#pragma unroll
-	for(int u = 0; u < CPL; u++) {
-		qx[u] = qy[u] = qz[u] = F32_FAR;
-#pragma unroll
-		for(int c = 0; c < 9; c++) qo[u][c] = 0.f;
-		if(cq[u] >= 0) {
+		if(cq[0] >= 0) {
 			double rel[3];
-			rel3(sd[u], rel);
-			qx[u] = (float) rel[0];
-			qy[u] = (float) rel[1];
-			qz[u] = (float) rel[2];
-#pragma unroll
-			for(int c = 0; c < 9; c++) qo[u][c] = (float) sd[u][3 + c];
-			check_o(qo[u]);
+			load_part(cq[0]);
+			convert(0, rel);
 		}
 	}
+	// whether any team of the wavefront uses the second slot of its lanes, or
+	// has neighbours beyond the register slots (scalar branches)
+	const bool wave_2 = CPL > 1 && ballot(nreg > nstat) != 0ull;
+	const bool wave_far = ballot(M > nreg) != 0ull;
+	if constexpr(CPL > 1)
+		if(wave_2) {
+			empty_slot(1);
+			if(cq[1] >= 0) {
+				double rel[3];
+				load_part(cq[1]);
+				convert(1, rel);
+			}
+		}
 	F32Filter fl = pg.filter;
 	if(team_any<T>(wild)) fl.eps_d2 = fl.eps_t = F32_ALL;
 	const float margin = pg.margin, is0 = pg.inv_side[0], is1 = pg.inv_side[1], is2 = pg.inv_side[2];
-	// whether any team of the wavefront has neighbours beyond the register
-	// slots (a scalar branch around those loops)
-	const bool wave_far = ballot(M > nreg) != 0ull;
-	// and likewise whether any uses the second slot of its lanes
-	const bool wave_2 = CPL > 1 && ballot(nreg > nstat) != 0ull;
-	if(wave_far && M > REC_SLOTS) {
+	if(CAP == CELL_CAP && wave_far && M > REC_SLOTS) {
 		// the rows' ranges, for the neighbours past the record's list
 		if(lane < 9) {
 			int a1, b1, a2, b2;
@@ -969,6 +971,7 @@ __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int
 		q = opaque(q);
 		m = opaque(m);
 		const double *p = own + k * OWN_W, *pm = own + max(m, 0) * OWN_W, *dt = trials + t * TR_W;
+		const Rep &hp = d.reps[hide_rep()];
 		double w[3];
 		// (the member's value is read in either case and kept, so that no
 		// pointer is chosen between LDS and HBM)
@@ -980,24 +983,40 @@ __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int
 		};
 #pragma unroll
 		for(int c = 0; c < 3; c++)
-			w[c] = kf_min_image(other(c) - (t >= 0 ? p[c] + dt[c] : p[c]), geo[c], geo[3 + c]);
-		const double w2 = w[0] * w[0] + w[1] * w[1] + w[2] * w[2], cosmax = geo[10];
+			w[c] = kf_min_image(other(c) - (t >= 0 ? p[c] + dt[c] : p[c]), hp.pg.box[c], hp.pg.inv_box[c]);
+		const double w2 = w[0] * w[0] + w[1] * w[1] + w[2] * w[2], cosmax = hp.cosmax;
 		if(w2 < 1.) return OVERLAP;
-		if(!(w2 < geo[9])) return 0u;
+		if(!(w2 < hp.rc2)) return 0u;
 		kf_unit(w[0], w[1], w[2], w2);
-		double O[9], P[4][3];
-#pragma unroll
-		for(int c = 0; c < 9; c++) O[c] = p[3 + c];
+		// (one row, then one patch at a time: this path sets the kernel's
+		// register count otherwise)
+		double O[9];
 		if(t >= 0) {
-			double R[9], On[9];
+			double R[9];
 #pragma unroll
 			for(int c = 0; c < 9; c++) R[c] = dt[3 + c];
-			mat_mul3(O, R, On);
 #pragma unroll
-			for(int c = 0; c < 9; c++) O[c] = On[c];
+			for(int i = 0; i < 3; i++) {
+				const double a0 = p[3 + 3 * i], a1 = p[4 + 3 * i], a2 = p[5 + 3 * i];
+#pragma unroll
+				for(int j = 0; j < 3; j++) O[3 * i + j] = a0 * R[j] + a1 * R[3 + j] + a2 * R[6 + j];
+				__builtin_amdgcn_sched_barrier(0);
+			}
 		}
-		kf_patches(O, P);
-		if(!kf_any_p(w[0], w[1], w[2], &P[0][0], cosmax)) return 0u;
+		else
+#pragma unroll
+			for(int c = 0; c < 9; c++) O[c] = p[3 + c];
+		bool hit = false;
+#pragma unroll
+		for(int i = 0; i < 4; i++) {
+			double v[3];
+#pragma unroll
+			for(int e = 0; e < 3; e++)
+				v[e] = O[3 * e] * kf_base(i, 0) + O[3 * e + 1] * kf_base(i, 1) + O[3 * e + 2] * kf_base(i, 2);
+			hit |= kf_dot(w[0], w[1], w[2], v[0], v[1], v[2]) > cosmax;
+			__builtin_amdgcn_sched_barrier(0);
+		}
+		if(!hit) return 0u;
 #pragma unroll
 		for(int c = 0; c < 9; c++) O[c] = other(3 + c);
 		return kf_any_q(w[0], w[1], w[2], O, cosmax) ? BOND : 0u;
@@ -1156,12 +1175,13 @@ __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int
 			bool ov = false;
 			for(int i = lane + nreg; i < M; i += T) {
 				const int q = opaque(nb_slot(i));
+				const Rep &hp = d.reps[hide_rep()];
 				float rel[3], Oq[9];
 				wild = false;
 #pragma unroll
 				for(int c = 0; c < 3; c++) {
 					const double p = nbld<DD>(part(F, q) + c);
-					rel[c] = (float) kf_min_image(p - geo[6 + c], geo[c], geo[3 + c]);
+					rel[c] = (float) kf_min_image(p - geo[c], hp.pg.box[c], hp.pg.inv_box[c]);
 					wild |= !(__builtin_fabs(p) < F32_MAX_POS);
 				}
 				const float fx = rel[0], fy = rel[1], fz = rel[2];
@@ -1208,12 +1228,12 @@ __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int
 			c_acc++;
 			d_bonds += db;
 			// the new state, one value per lane, exact and single precision;
-			// lanes 0 and 1 write the new static count and member bits
+			// lanes 0 to 2 write the new static count and member bits
 			const double rv = ms.dot ? o0 * r0 + o1 * r1 + o2 * r2 : o0 + r0;
 			if(lane < 15) {
 				own[k * OWN_W + lane] = rv;
 				shadow[k * SH_W + ms.word] =
-				    lane == 0 ? __int_as_float(n_new - (int) __popc(mb)) : (lane == 1 ? __uint_as_float(mb) : (float) rv);
+				    lane == 0 ? __int_as_float(n_new - (int) __popc(mb)) : (lane <= 2 ? __uint_as_float(mb) : (float) rv);
 			}
 			// the other members' bits for member k
 			if(is_mem && mi != k) {
@@ -1423,12 +1443,11 @@ size_t pass_lds_bytes(int T, int block) { return (size_t) (block / T) * team_lds
 template <int T>
 static void pass_TK(const DevState &d, uint64_t sweep, int pass, int block, hipStream_t s) {
 	if constexpr(T == 16) {
-		// dilute systems (fewer than 16 candidates in a cell's 27 cells on
-		// average): one register neighbour per lane, the rare rest from memory
-		const double cand = 27. * (double) d.Ntot / (double) std::max(d.C_total, 1);
-		if(cand < 16.) {
-			if(d.R == 1) pass_T<16, 1, true, SMALL_CAP>(d, sweep, pass, block, s);
-			else pass_T<16, 1, false, SMALL_CAP>(d, sweep, pass, block, s);
+		// at most one particle per cell on average: cells that the small-cell
+		// pass defers are rare
+		if(d.Ntot <= d.C_total) {
+			if(d.R == 1) pass_T<16, 2, true, SMALL_CAP>(d, sweep, pass, block, s);
+			else pass_T<16, 2, false, SMALL_CAP>(d, sweep, pass, block, s);
 			return;
 		}
 	}
