@@ -1577,7 +1577,7 @@ pp_status pp_net_train(pp_ctx *c, pp_net *net, int steps, int batch, double lr, 
 	HIPCHECK(hipStreamSynchronize(net->stream));
 	std::vector<float> hl(batch);
 	auto mean_loss = [&](double *out) -> pp_status {
-		HIPCHECK(hipMemcpyAsync(hl.data(), net->loss, sizeof(float) * batch, hipMemcpyDeviceToHost, c->stream));
+		HIPCHECK(hipMemcpyAsync(hl.data(), net->q.loss, sizeof(float) * batch, hipMemcpyDeviceToHost, c->stream));
 		HIPCHECK(hipStreamSynchronize(c->stream));
 		double sum = 0.;
 		for(float v : hl) sum += v;
@@ -1588,16 +1588,17 @@ pp_status pp_net_train(pp_ctx *c, pp_net *net, int steps, int batch, double lr, 
 	for(int s = 0; s < steps; s++) {
 		if(s > 0)
 			for(int k = 0; k < sweeps_between; k++) TRY(enqueue_sweep(c));
-		// the cell ranges of the current state (an NPT trial may have left
-		// those of its trial grid)
-		rebuild_now(c);
+		// the cell ranges of the current state: those of the last sweep hold
+		// (its passes move no particle out of its cell), unless a box trial
+		// has left those of its trial grid
+		if(s == 0 || c->any_npt || c->any_lx) rebuild_now(c);
 		launch_train_samples(c->d, tseed, (uint64_t) net->step, batch, pos_noise, theta_max, net->x, net->target,
 		                     c->stream);
-		launch_net_loss_grad(net->d, net->x, net->target, batch, net->h, net->y, net->dy, net->dh, net->loss, c->stream);
+		launch_net_train(net->d, net->x, net->target, batch, net->q, c->stream);
 		if(s == 0 && loss_first) TRY(mean_loss(loss_first));
 		if(s == steps - 1 && loss_last) TRY(mean_loss(loss_last));
 		net->step++;
-		launch_net_adam(net->d, net->step, (float) lr, c->stream);
+		launch_net_adam(net->d, batch, net->q, net->step, (float) lr, c->stream);
 	}
 	HIPCHECK(hipStreamSynchronize(c->stream));
 	TRY(collect_timing(c));

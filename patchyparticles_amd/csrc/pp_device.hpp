@@ -135,6 +135,45 @@ __device__ __forceinline__ int rec_slot(const DevState &d, const int *rec, int i
 	return walk_slot(d.start + rp.cell_off, rec[REC_IX], rec[REC_IY], rec[REC_IZ], rp.lg.n[0], rp.lg.n[1], rp.lg.n[2], i);
 }
 
+// The record of cell cloc = (ix, iy, iz) of a grid of n0 x n1 x n2 cells (st:
+// its cells' first slots), by 16 lanes of a DPP row: lane j < 9 takes row j of
+// the neighbourhood (row_ranges), a prefix sum over the lanes places its
+// slots, lane 9 writes the header.  A pass finds all its data from this one
+// record: its slot list needs no search, and lanes of one team write to one or
+// two cache lines (a thread per record wrote 256 bytes at a time, from 52
+// loads of its own).
+__device__ __forceinline__ void write_record(int *rec, int tag, const int *st, int cloc, int ix, int iy, int iz, int n0,
+                                             int n1, int n2, int r, int sel, int lane) {
+	int a1 = 0, b1 = 0, a2 = 0, b2 = 0;
+	if(lane < 9) row_ranges(st, ix, iy, iz, n0, n1, n2, lane, a1, b1, a2, b2);
+	else if(lane == 9) {
+		a1 = st[cloc];
+		b1 = st[cloc + 1];
+	}
+	const int l1 = b1 - a1, len = lane < 9 ? l1 + b2 - a2 : 0;
+	int inc = len;
+	inc += __builtin_amdgcn_update_dpp(0, inc, DPP_ROW_SHR + 1, 0xf, 0xf, true);
+	inc += __builtin_amdgcn_update_dpp(0, inc, DPP_ROW_SHR + 2, 0xf, 0xf, true);
+	inc += __builtin_amdgcn_update_dpp(0, inc, DPP_ROW_SHR + 4, 0xf, 0xf, true);
+	inc += __builtin_amdgcn_update_dpp(0, inc, DPP_ROW_SHR + 8, 0xf, 0xf, true);
+	// candidates before the cell itself, for the header's lane
+	const int m0 = __shfl(inc - len + l1, (int) (threadIdx.x & 63 & ~15) + 4);
+	for(int e = 0, at = REC_HEAD + inc - len; e < len && at < REC_W; e++, at++) rec[at] = e < l1 ? a1 + e : a2 + e - l1;
+	if(lane == 9) {
+		rec[REC_TAG] = tag;
+		rec[REC_M] = inc;
+		rec[REC_S0] = a1;
+		rec[REC_CNT] = l1;
+		rec[REC_CELL] = cloc;
+		rec[REC_REP] = r;
+		rec[REC_SEL] = sel;
+		rec[REC_M0] = m0;
+		rec[REC_IX] = ix;
+		rec[REC_IY] = iy;
+		rec[REC_IZ] = iz;
+	}
+}
+
 // A value the compiler knows nothing about: what is computed from it stays
 // where it is written, not in registers across a loop that rarely needs it.
 __device__ __forceinline__ int opaque(int v) {

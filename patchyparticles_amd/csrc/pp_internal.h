@@ -83,6 +83,13 @@ struct NetDev {
 	__bf16 *frag, *fragT;
 };
 
+// Scratch of one gradient evaluation of m_pad rows (a multiple of 32).
+struct NetScratch {
+	__bf16 *at, *zt;  // the layers' inputs and output gradients, transposed (k_net_grad)
+	float *part;      // [net_grad_slices(m_pad)][NN_W + NN_B] partial gradients
+	float *loss;      // [m_pad]
+};
+
 constexpr int NN_PROP_W = 16;  // doubles of one drawn proposal
 
 // Per-context state of the learned passes (scratch sized for the largest list).
@@ -291,15 +298,16 @@ void launch_pass(const DevState &d, uint64_t sweep, int pass, int T, int block, 
 void launch_passes_dd(const DevState &d, uint64_t sweep, unsigned mark, int T, int block, hipStream_t s);
 // learned proposal (pp_learn.hip)
 void launch_learned_pass(const DevState &d, const NetDev &net, uint64_t sweep, int pass, hipStream_t s);
-void launch_net_forward(const NetDev &net, const __bf16 *x, int m, const int *m_dev, float *y, __bf16 *h,
-                        hipStream_t s);
+void launch_net_forward(const NetDev &net, const float *x, int m, float *y, hipStream_t s);
 void launch_net_pack(const NetDev &net, hipStream_t s);
-// m rows (padded to a multiple of 32, rows >= m of x zero): forward with the
-// hidden layers kept, per-row -log q (loss[m_pad]), backward, gradients of
-// the mean loss into net.gw / net.gb
-void launch_net_loss_grad(const NetDev &net, const __bf16 *x, const float *target, int m, __bf16 *h, float *y,
-                          __bf16 *dy, __bf16 *dh, float *loss, hipStream_t s);
-void launch_net_adam(const NetDev &net, int step, float lr, hipStream_t s);
+// loss of each of m rows and the gradients of their mean into net.gw / net.gb
+void launch_net_loss_grad(const NetDev &net, const float *x, const float *target, int m, const NetScratch &q,
+                          hipStream_t s);
+// a training step on m samples (x: BF16 rows): losses and the gradients'
+// partial sums, then the step itself
+void launch_net_train(const NetDev &net, const __bf16 *x, const float *target, int m, const NetScratch &q, hipStream_t s);
+void launch_net_adam(const NetDev &net, int m, const NetScratch &q, int step, float lr, hipStream_t s);
+int net_grad_slices(int m_pad);  // slices of the rows the gradients are summed in
 void launch_descriptor(int n, const double *r, const double *O, const Grid &g, int m, const int *idx, __bf16 *x,
                        hipStream_t s);
 void launch_train_samples(const DevState &d, uint64_t seed, uint64_t step, int m, double pos_noise, double theta_max,

@@ -444,12 +444,7 @@ __device__ __forceinline__ void pass_prefix(const DevState &d, int k, int lane) 
 
 __global__ __launch_bounds__(512) void k_pass_prefix(DevState d) { pass_prefix(d, threadIdx.x >> 6, threadIdx.x & 63); }
 
-// The record of entry gi of pass k's list, by the 16 lanes of a team: lane j <
-// 9 takes row j of the neighbourhood (row_ranges), a prefix sum over the
-// lanes places its slots, lane 9 writes the header.  A pass finds all its
-// data from this one record: its slot list needs no search, and lanes of one
-// team write to one or two cache lines (a thread per record wrote 256 bytes
-// at a time, from 52 loads of its own).
+// The record of entry gi of pass k's list, by the 16 lanes of a team.
 template <bool ONE>
 __device__ __forceinline__ void build_record(const DevState &d, int k, int gi, int lane) {
 	int r = 0;
@@ -473,29 +468,8 @@ __device__ __forceinline__ void build_record(const DevState &d, int k, int gi, i
 	const int cloc = d.clist[rp.cell_off + col * rp.act_cap + kk];
 	const int n0 = rp.g.n[0], n1 = rp.g.n[1], n2 = rp.g.n[2];
 	const int ix = cloc / (n1 * n2), iy = (cloc / n2) % n1, iz = cloc % n2;
-	const int *st = d.start + rp.cell_off;
-	int a1 = 0, b1 = 0, a2 = 0, b2 = 0;
-	if(lane < 9) row_ranges(st, ix, iy, iz, n0, n1, n2, lane, a1, b1, a2, b2);
-	else if(lane == 9) {
-		a1 = st[cloc];
-		b1 = st[cloc + 1];
-	}
-	const int l1 = b1 - a1, len = lane < 9 ? l1 + b2 - a2 : 0;
-	int inc = len;
-	inc += __builtin_amdgcn_update_dpp(0, inc, DPP_ROW_SHR + 1, 0xf, 0xf, true);
-	inc += __builtin_amdgcn_update_dpp(0, inc, DPP_ROW_SHR + 2, 0xf, 0xf, true);
-	inc += __builtin_amdgcn_update_dpp(0, inc, DPP_ROW_SHR + 4, 0xf, 0xf, true);
-	inc += __builtin_amdgcn_update_dpp(0, inc, DPP_ROW_SHR + 8, 0xf, 0xf, true);
-	// candidates before the cell itself, for the header's lane
-	const int m0 = __shfl(inc - len + l1, (int) (threadIdx.x & 63 & ~15) + 4);
-	int *rec = d.rec + ((size_t) k * d.total_act + gi) * REC_W;
-	for(int e = 0, at = REC_HEAD + inc - len; e < len && at < REC_W; e++, at++) rec[at] = e < l1 ? a1 + e : a2 + e - l1;
-	if(lane == 9) {
-		int4 *out = (int4 *) rec;
-		out[0] = make_int4((int) d.rec_tag, inc, a1, l1);
-		out[1] = make_int4(cloc, r, rp.sel, m0);
-		out[2] = make_int4(ix, iy, iz, 0);
-	}
+	write_record(d.rec + ((size_t) k * d.total_act + gi) * REC_W, (int) d.rec_tag, d.start + rp.cell_off, cloc, ix, iy, iz,
+	             n0, n1, n2, r, rp.sel, lane);
 }
 
 // Workgroups of the scatter that build records (grid-stride over the listed

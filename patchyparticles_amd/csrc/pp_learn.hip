@@ -255,21 +255,39 @@ __host__ __device__ inline size_t fragT_at(int l, int kb, int nt, int lane) {
 
 constexpr int ACT_LD = NN_H + 8;  // LDS row stride of the activations (bf16)
 
-// One wave per 16 rows: every layer of the MLP, activations in LDS.  m rows
-// (or *m_dev if given); y: [rows][NN_OUT_PAD]; h (optional): the three
-// hidden layers, [3][hs][NN_H], for the backward pass.
-__global__ __launch_bounds__(64) void k_net_fwd(NetDev net, const __bf16 *x, int m, const int *m_dev, float *y,
-                                                __bf16 *h, int hs) {
+// One row of network inputs as the host gives it, or as the samplers write it
+// (NN_IN_PAD BF16 values): 8 consecutive inputs from column c (a multiple of 8).
+__device__ __forceinline__ bf16x8 load_inputs(const __bf16 *x, size_t row, int c) {
+	return *(const bf16x8 *) (x + row * NN_IN_PAD + c);
+}
+__device__ __forceinline__ bf16x8 load_inputs(const float *x, size_t row, int c) {
+	// (rows of 84 floats: 16-byte aligned, and column 80 has four left)
+	static_assert(NN_IN % 4 == 0 && NN_IN_PAD - NN_IN == 12, "whole vectors of four");
+	const f32x4 *p = (const f32x4 *) (x + row * NN_IN + c);
+	f32x4 lo = {}, hi = {};
+	if(c < NN_IN) lo = p[0];
+	if(c + 4 < NN_IN) hi = p[1];
+	bf16x8 v;
+#pragma unroll
+	for(int e = 0; e < 4; e++) {
+		v[e] = (__bf16) lo[e];
+		v[4 + e] = (__bf16) hi[e];
+	}
+	return v;
+}
+
+// One wave per 16 rows: every layer of the MLP, activations in LDS.
+// y: [rows][NN_OUT_PAD].
+__global__ __launch_bounds__(64) void k_net_fwd(NetDev net, const float *x, int rows, float *y) {
 	__shared__ __attribute__((aligned(16))) __bf16 act[2][16 * ACT_LD];
 	const int lane = threadIdx.x;
-	const int rows = m_dev ? *m_dev : m;
 	const int row0 = blockIdx.x * 16;
 	if(row0 >= rows) return;
 	const int r = lane & 15, g = lane >> 4;
 	bf16x8 a0[NN_IN_PAD / 32];
 	for(int kb = 0; kb < NN_IN_PAD / 32; kb++) {
 		bf16x8 v = {};
-		if(row0 + r < rows) v = *(const bf16x8 *) (x + (size_t) (row0 + r) * NN_IN_PAD + kb * 32 + g * 8);
+		if(row0 + r < rows) v = load_inputs(x, (size_t) (row0 + r), kb * 32 + g * 8);
 		a0[kb] = v;
 	}
 	int cur = 0;
@@ -286,13 +304,8 @@ __global__ __launch_bounds__(64) void k_net_fwd(NetDev net, const __bf16 *x, int
 			const float bias = net.b[nn_boff(l) + col];
 			for(int j = 0; j < 4; j++) {
 				const int row = g * 4 + j;
-				float v = acc[j] + bias;
-				if(l < NN_LAYERS - 1) {
-					v = fmaxf(v, 0.f);
-					const __bf16 bv = (__bf16) v;
-					act[cur ^ 1][row * ACT_LD + col] = bv;
-					if(h && row0 + row < rows) h[((size_t) l * hs + row0 + row) * NN_H + col] = bv;
-				}
+				const float v = acc[j] + bias;
+				if(l < NN_LAYERS - 1) act[cur ^ 1][row * ACT_LD + col] = (__bf16) fmaxf(v, 0.f);
 				else if(row0 + row < rows)
 					y[(size_t) (row0 + row) * NN_OUT_PAD + col] = v;
 			}
@@ -302,165 +315,310 @@ __global__ __launch_bounds__(64) void k_net_fwd(NetDev net, const __bf16 *x, int
 	}
 }
 
-// -log q of each training row (and its gradient, scaled by 1/m, as BF16 for
-// the backward kernels); rows in [m, m_pad) get zero gradients.
-__global__ void k_net_loss(const float *y, const float *target, int m, int m_pad, __bf16 *dy, float *loss) {
-	const int i = blockIdx.x * blockDim.x + threadIdx.x;
-	if(i >= m_pad) return;
-	float g[NN_OUT_PAD];
-	float l = 0.f;
-	if(i < m) {
-		const float *t = target + (size_t) i * 6;
-		l = prop_loss_grad(y + (size_t) i * NN_OUT_PAD, t, t + 3, g);
-		for(int e = 0; e < NN_OUT_PAD; e++) g[e] *= 1.f / (float) m;
-	}
-	else
-		for(int e = 0; e < NN_OUT_PAD; e++) g[e] = 0.f;
-	for(int e = 0; e < NN_OUT_PAD; e++) dy[(size_t) i * NN_OUT_PAD + e] = (__bf16) g[e];
-	loss[i] = l;
+// ------------------------------------------------------------------------
+// gradients of the mean loss
+//
+// k_net_grad takes rows through the whole network and back and leaves each
+// layer's inputs and output gradients for k_net_wgrad, transposed: blocks of
+// 32 rows, in a block the 32 values of one column together.  An operand
+// fragment of dW = A^T dZ (8 rows of one column per lane) is then one 16-byte
+// load and a wavefront's fragment 1 KB in one piece; from row-major arrays it
+// took eight 2-byte loads, and the gradients of a batch of 4096 49 us.
+
+// value (row, col) of layer l's inputs / output gradients, m_pad rows in all
+__host__ __device__ constexpr int nn_koff(int l) { return l == 0 ? 0 : nn_koff(l - 1) + nn_k(l - 1); }
+__device__ __forceinline__ __bf16 *at_ptr(__bf16 *at, int m_pad, int l, int row, int col) {
+	return at + (size_t) nn_koff(l) * m_pad + ((size_t) (row >> 5) * nn_k(l) + col) * 32 + (row & 31);
+}
+__device__ __forceinline__ __bf16 *zt_ptr(__bf16 *zt, int m_pad, int l, int row, int col) {
+	return zt + (size_t) nn_boff(l) * m_pad + ((size_t) (row >> 5) * nn_n(l) + col) * 32 + (row & 31);
 }
 
-// One wave per 16 rows: dH3 = (dY W4^T) * [H3 > 0], dH2 = (dH3 W3^T) * [H2 > 0],
-// dH1 = (dH2 W2^T) * [H1 > 0]; dh: [3][hs][NN_H].
-__global__ __launch_bounds__(64) void k_net_bwd(NetDev net, const __bf16 *dy, const __bf16 *h, int m_pad, int hs,
-                                                __bf16 *dh) {
-	__shared__ __attribute__((aligned(16))) __bf16 act[2][16 * ACT_LD];
-	const int lane = threadIdx.x;
-	const int row0 = blockIdx.x * 16;
-	if(row0 >= m_pad) return;
-	const int r = lane & 15, g = lane >> 4;
-	const bf16x8 gy = *(const bf16x8 *) (dy + (size_t) (row0 + r) * NN_OUT_PAD + g * 8);
-	int cur = 0;
-	for(int l = NN_LAYERS - 1; l >= 1; l--) {
-		// input gradient of layer l: K' = nn_n(l), N' = nn_k(l) = NN_H
-		const int nkb = nn_n(l) / 32, nnt = nn_k(l) / 16;
-		for(int nt = 0; nt < nnt; nt++) {
-			f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-			for(int kb = 0; kb < nkb; kb++) {
-				const bf16x8 a = l == NN_LAYERS - 1 ? gy : *(const bf16x8 *) (&act[cur][r * ACT_LD + kb * 32 + g * 8]);
-				const bf16x8 b = *(const bf16x8 *) (net.fragT + fragT_at(l, kb, nt, lane));
-				acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc, 0, 0, 0);
-			}
-			const int col = nt * 16 + r;
-			for(int j = 0; j < 4; j++) {
-				const int row = g * 4 + j;
-				const size_t at = ((size_t) (l - 1) * hs + row0 + row) * NN_H + col;
-				const float mask = (float) h[at] > 0.f ? 1.f : 0.f;
-				const __bf16 v = (__bf16) (acc[j] * mask);
-				act[cur ^ 1][row * ACT_LD + col] = v;
-				dh[at] = v;
-			}
+typedef __attribute__((__vector_size__(4 * sizeof(__bf16)))) __bf16 bf16x4;
+
+constexpr int NG_ROWS = 16;             // rows of a tile
+constexpr int NG_WAVES = NN_H / 16;     // one 16-column tile of a hidden layer per wavefront
+constexpr int NG_BLOCKS = 256;          // a workgroup per CU, which takes every NG_BLOCKS-th tile
+
+// -log q of each row, and the gradient of its mean over m rows with respect
+// to every layer's output before the activation (BF16, as the MFMA operands
+// of the weight gradients); rows in [m, m_pad) have none.  X: float (rows of
+// the caller) or __bf16 (samples on the device, padded to m_pad rows).
+//
+// Bound by the chain of seven layers, not by the matrix cores (a batch of 4096
+// is 1.2 GFLOP): each of the 8 wavefronts computes 16 columns of every layer
+// with its weights (24 operand fragments, forward and transposed) held in
+// registers from the start, so a layer costs its LDS exchange and at most
+// four dependent MFMAs.  One kernel instead of three: the activations stay in
+// LDS and registers, and ReLU's mask is the wavefront's own columns.
+// Forward, loss and backward of 4096 rows: 58 -> 10.9 us.
+template <class X>
+__global__ __launch_bounds__(64 * NG_WAVES) void k_net_grad(NetDev net, const X *x, const float *target, int m, int m_pad,
+                                                            __bf16 *at, __bf16 *zt, float *loss) {
+	__shared__ __attribute__((aligned(16))) __bf16 xs[NG_ROWS * ACT_LD], act[2][NG_ROWS * ACT_LD];
+	__shared__ __attribute__((aligned(16))) __bf16 dys[NG_ROWS * (NN_OUT_PAD + 8)];
+	__shared__ float ys[NG_ROWS * NN_OUT_PAD];
+	constexpr int DY_LD = NN_OUT_PAD + 8;
+	const int t = threadIdx.x, lane = t & 63, w = t >> 6, r = lane & 15, g = lane >> 4;
+	const int col = w * 16 + r;  // the lane's column of a hidden layer
+	// the weights of this wavefront's columns
+	bf16x8 f0[3], f1[4], f2[4], f3[4], b3, b2[4], b1[4];
+	float bias[4];
+#pragma unroll
+	for(int kb = 0; kb < 3; kb++) f0[kb] = *(const bf16x8 *) (net.frag + frag_at(0, kb, w, lane));
+#pragma unroll
+	for(int kb = 0; kb < 4; kb++) {
+		f1[kb] = *(const bf16x8 *) (net.frag + frag_at(1, kb, w, lane));
+		f2[kb] = *(const bf16x8 *) (net.frag + frag_at(2, kb, w, lane));
+		f3[kb] = *(const bf16x8 *) (net.frag + frag_at(3, kb, w & 1, lane));
+		b2[kb] = *(const bf16x8 *) (net.fragT + fragT_at(2, kb, w, lane));
+		b1[kb] = *(const bf16x8 *) (net.fragT + fragT_at(1, kb, w, lane));
+	}
+	b3 = *(const bf16x8 *) (net.fragT + fragT_at(3, 0, w, lane));
+#pragma unroll
+	for(int l = 0; l < 4; l++) bias[l] = net.b[nn_boff(l) + (l < 3 ? col : (w & 1) * 16 + r)];
+
+	for(int row0 = blockIdx.x * NG_ROWS; row0 < m_pad; row0 += gridDim.x * NG_ROWS) {
+		// the rows, and their transpose
+		constexpr int XV = NN_IN_PAD / 8;
+		if(t < NG_ROWS * XV) {
+			const int row = t / XV, c = (t % XV) * 8;
+			bf16x8 v = {};
+			if(row0 + row < m) v = load_inputs(x, (size_t) (row0 + row), c);
+			*(bf16x8 *) (xs + row * ACT_LD + c) = v;
 		}
 		__syncthreads();
-		cur ^= 1;
+		if(t < 2 * NN_IN_PAD) {
+			const int c = t % NN_IN_PAD, h = t / NN_IN_PAD * 8;
+			bf16x8 v;
+#pragma unroll
+			for(int e = 0; e < 8; e++) v[e] = xs[(h + e) * ACT_LD + c];
+			*(bf16x8 *) at_ptr(at, m_pad, 0, row0 + h, c) = v;
+		}
+		// forward; the lane's values of hidden layer l + 1 in hv[l]
+		bf16x4 hv[3];
+		auto forward = [&](const __bf16 *A, const bf16x8 *f, int nkb, float b, f32x4 &out) {
+			f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+			for(int kb = 0; kb < nkb; kb++) {
+				const bf16x8 a = *(const bf16x8 *) (A + r * ACT_LD + kb * 32 + g * 8);
+				acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, f[kb], acc, 0, 0, 0);
+			}
+#pragma unroll
+			for(int j = 0; j < 4; j++) out[j] = acc[j] + b;
+		};
+		auto hidden = [&](const f32x4 &v, int l, __bf16 *to) {
+#pragma unroll
+			for(int j = 0; j < 4; j++) {
+				hv[l][j] = (__bf16) fmaxf(v[j], 0.f);
+				to[(g * 4 + j) * ACT_LD + col] = hv[l][j];
+			}
+			*(bf16x4 *) at_ptr(at, m_pad, l + 1, row0 + g * 4, col) = hv[l];
+			__syncthreads();
+		};
+		f32x4 v;
+		forward(xs, f0, 3, bias[0], v);
+		hidden(v, 0, act[0]);
+		forward(act[0], f1, 4, bias[1], v);
+		hidden(v, 1, act[1]);
+		forward(act[1], f2, 4, bias[2], v);
+		hidden(v, 2, act[0]);
+		if(w < NN_OUT_PAD / 16) {
+			forward(act[0], f3, 4, bias[3], v);
+#pragma unroll
+			for(int j = 0; j < 4; j++) ys[(g * 4 + j) * NN_OUT_PAD + col] = v[j];
+		}
+		__syncthreads();
+		// the loss and its gradient with respect to the outputs, a row per lane
+		if(t < NG_ROWS) {
+			const int i = row0 + t;
+			float gr[NN_OUT_PAD], l = 0.f;
+			if(i < m) {
+				const float *tg = target + (size_t) i * 6;
+				l = prop_loss_grad(ys + t * NN_OUT_PAD, tg, tg + 3, gr);
+#pragma unroll
+				for(int e = 0; e < NN_OUT_PAD; e++) gr[e] *= 1.f / (float) m;
+			}
+			else
+#pragma unroll
+				for(int e = 0; e < NN_OUT_PAD; e++) gr[e] = 0.f;
+#pragma unroll
+			for(int e = 0; e < NN_OUT_PAD; e++) dys[t * DY_LD + e] = (__bf16) gr[e];
+			loss[i] = l;
+		}
+		__syncthreads();
+		if(t < 2 * NN_OUT_PAD) {
+			const int c = t % NN_OUT_PAD, h = t / NN_OUT_PAD * 8;
+			bf16x8 o;
+#pragma unroll
+			for(int e = 0; e < 8; e++) o[e] = dys[(h + e) * DY_LD + c];
+			*(bf16x8 *) zt_ptr(zt, m_pad, 3, row0 + h, c) = o;
+		}
+		// backward: dH3 = (dY W4^T) * [H3 > 0], then dH2, dH1
+		auto masked = [&](const f32x4 &acc, int l, __bf16 *to) {
+			bf16x4 z;
+#pragma unroll
+			for(int j = 0; j < 4; j++) {
+				z[j] = (__bf16) (acc[j] * ((float) hv[l][j] > 0.f ? 1.f : 0.f));
+				if(to) to[(g * 4 + j) * ACT_LD + col] = z[j];
+			}
+			*(bf16x4 *) zt_ptr(zt, m_pad, l, row0 + g * 4, col) = z;
+			__syncthreads();
+		};
+		{
+			const bf16x8 a = *(const bf16x8 *) (dys + r * DY_LD + g * 8);
+			const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+			v = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b3, zero, 0, 0, 0);
+		}
+		masked(v, 2, act[1]);
+		forward(act[1], b2, 4, 0.f, v);
+		masked(v, 1, act[0]);
+		forward(act[0], b1, 4, 0.f, v);
+		masked(v, 0, nullptr);
 	}
 }
 
-// Weight gradients dW_l = A_l^T dZ_l summed over the m_pad rows (A: x, H1,
-// H2, H3; dZ: dH1, dH2, dH3, dY); one wave per 16 x 16 tile of one layer.
-__global__ __launch_bounds__(64) void k_net_wgrad(NetDev net, const __bf16 *x, const __bf16 *h, const __bf16 *dy,
-                                                  const __bf16 *dh, int m_pad, int hs) {
-	int t = blockIdx.x, l = 0;
-	while(l < NN_LAYERS && t >= (nn_k(l) / 16) * (nn_n(l) / 16)) {
-		t -= (nn_k(l) / 16) * (nn_n(l) / 16);
+// Weight and bias gradients: dW_l = A_l^T dZ_l and the column sums of dZ_l.
+// A wavefront takes a 32 x 32 tile of one layer over one slice of the rows
+// (two fragments of either operand for four MFMAs) and leaves partial sums:
+// part[slice][NN_W + NN_B].  The 48 tiles alone would leave the chip idle, so
+// the rows are cut into slices of at least NW_ROWS (a chain of 8 blocks), at
+// most NW_SLICES of them, whose sums the next kernel adds in a fixed order.
+// The bias sums are one MFMA with a matrix of ones, stored by the tiles of
+// the first rows.  Batch of 4096: 49 + 11 us (a tile over all rows; the biases in
+// a kernel of their own) -> 6.4 us.
+constexpr int NW_ROWS = 256, NW_SLICES = 32;
+constexpr int nw_tiles(int l) { return l < 0 ? 0 : nw_tiles(l - 1) + (nn_k(l) / 32) * (nn_n(l) / 32); }
+constexpr int NW_TILES = nw_tiles(NN_LAYERS - 1);
+constexpr int NW_WAVES = 4;
+static_assert(NW_TILES % NW_WAVES == 0, "whole workgroups");
+constexpr int NN_G = NN_W + NN_B;
+
+int net_grad_slices(int m_pad) { return std::max(1, std::min(m_pad / NW_ROWS, NW_SLICES)); }
+
+__global__ __launch_bounds__(64 * NW_WAVES) void k_net_wgrad(const __bf16 *at, const __bf16 *zt, int m_pad, float *part) {
+	int t = blockIdx.x * NW_WAVES + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = 0;
+	while(t >= (nn_k(l) / 32) * (nn_n(l) / 32)) {
+		t -= (nn_k(l) / 32) * (nn_n(l) / 32);
 		l++;
 	}
-	if(l >= NN_LAYERS) return;
-	const int nnt = nn_n(l) / 16;
-	const int kt = t / nnt, nt = t % nnt;
-	const int lane = threadIdx.x, r = lane & 15, g = lane >> 4;
-	const __bf16 *A = l == 0 ? x : h + (size_t) (l - 1) * hs * NN_H;
-	const int lda = l == 0 ? NN_IN_PAD : NN_H;
-	const __bf16 *Z = l == NN_LAYERS - 1 ? dy : dh + (size_t) l * hs * NN_H;
-	const int ldz = l == NN_LAYERS - 1 ? NN_OUT_PAD : NN_H;
-	f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-	for(int c = 0; c < m_pad; c += 32) {
-		bf16x8 a, b;
-		for(int i = 0; i < 8; i++) {
-			const size_t row = (size_t) (c + g * 8 + i);
-			a[i] = A[row * lda + kt * 16 + r];
-			b[i] = Z[row * ldz + nt * 16 + r];
-		}
-		acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc, 0, 0, 0);
+	const int K = nn_k(l), N = nn_n(l);
+	const int k0 = t / (N / 32) * 32, n0 = t % (N / 32) * 32;
+	const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+	const __bf16 *A = at + (size_t) nn_koff(l) * m_pad + (k0 + r) * 32 + g * 8;
+	const __bf16 *Z = zt + (size_t) nn_boff(l) * m_pad + (n0 + r) * 32 + g * 8;
+	const int blocks = m_pad / 32, S = gridDim.y, s = blockIdx.y;
+	const int lo = (int) ((long long) blocks * s / S), hi = (int) ((long long) blocks * (s + 1) / S);
+	f32x4 acc[2][2] = {}, sum[2] = {};
+	bf16x8 ones;
+#pragma unroll
+	for(int e = 0; e < 8; e++) ones[e] = (__bf16) 1.f;
+	for(int b = lo; b < hi; b++) {
+		const __bf16 *pa = A + (size_t) b * K * 32, *pz = Z + (size_t) b * N * 32;
+		const bf16x8 a0 = *(const bf16x8 *) pa, a1 = *(const bf16x8 *) (pa + 512);
+		const bf16x8 z0 = *(const bf16x8 *) pz, z1 = *(const bf16x8 *) (pz + 512);
+		acc[0][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, z0, acc[0][0], 0, 0, 0);
+		acc[0][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, z1, acc[0][1], 0, 0, 0);
+		acc[1][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, z0, acc[1][0], 0, 0, 0);
+		acc[1][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, z1, acc[1][1], 0, 0, 0);
+		sum[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, z0, sum[0], 0, 0, 0);
+		sum[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, z1, sum[1], 0, 0, 0);
 	}
-	for(int j = 0; j < 4; j++) net.gw[nn_woff(l) + (size_t) (kt * 16 + g * 4 + j) * nn_n(l) + nt * 16 + r] = acc[j];
+	float *gw = part + (size_t) s * NN_G + nn_woff(l), *gb = part + (size_t) s * NN_G + NN_W + nn_boff(l);
+#pragma unroll
+	for(int i = 0; i < 2; i++)
+#pragma unroll
+		for(int c = 0; c < 2; c++)
+#pragma unroll
+			for(int j = 0; j < 4; j++) gw[(size_t) (k0 + i * 16 + g * 4 + j) * N + n0 + c * 16 + r] = acc[i][c][j];
+	// (every row of the product with ones holds the column sums)
+	if(k0 == 0 && g == 0) {
+		gb[n0 + r] = sum[0][0];
+		gb[n0 + 16 + r] = sum[1][0];
+	}
 }
 
-// Bias gradients: one workgroup per bias, a tree sum over the rows.
-__global__ __launch_bounds__(256) void k_net_bgrad(NetDev net, const __bf16 *dy, const __bf16 *dh, int m_pad, int hs) {
-	__shared__ float part[256];
-	const int i = blockIdx.x;
-	int l = 0;
-	while(l + 1 < NN_LAYERS && i >= nn_boff(l + 1)) l++;
-	const int n = i - nn_boff(l);
-	const __bf16 *Z = l == NN_LAYERS - 1 ? dy : dh + (size_t) l * hs * NN_H;
-	const int ldz = l == NN_LAYERS - 1 ? NN_OUT_PAD : NN_H;
-	float s = 0.f;
-	for(int row = threadIdx.x; row < m_pad; row += 256) s += (float) Z[(size_t) row * ldz + n];
-	part[threadIdx.x] = s;
-	__syncthreads();
-	for(int o = 128; o > 0; o >>= 1) {
-		if((int) threadIdx.x < o) part[threadIdx.x] += part[threadIdx.x + o];
-		__syncthreads();
-	}
-	if(threadIdx.x == 0) net.gb[i] = part[0];
+// gradient e of the slices' partial sums (e < NN_W: a weight, else a bias)
+__device__ __forceinline__ float slice_sum(const float *part, int slices, int e) {
+	float g = 0.f;
+	for(int s = 0; s < slices; s++) g += part[(size_t) s * NN_G + e];
+	return g;
 }
 
-// BF16 operand fragments of W (forward) and W^T (backward) from the FP32 weights.
-__global__ void k_net_pack(NetDev net) {
+__global__ void k_net_reduce(const float *part, int slices, float *gw, float *gb) {
 	const int e = blockIdx.x * blockDim.x + threadIdx.x;
-	if(e >= NN_W) return;
+	if(e >= NN_G) return;
+	const float g = slice_sum(part, slices, e);
+	if(e < NN_W) gw[e] = g;
+	else gb[e - NN_W] = g;
+}
+
+// BF16 operand fragments of W (forward) and W^T (backward): those of weight e.
+__device__ __forceinline__ void pack_weight(const NetDev &net, int e, float w) {
 	int l = 0;
 	while(l + 1 < NN_LAYERS && e >= nn_woff(l + 1)) l++;
 	const int loc = e - nn_woff(l), N = nn_n(l);
 	const int k = loc / N, n = loc % N;
-	const __bf16 v = (__bf16) net.w[e];
+	const __bf16 v = (__bf16) w;
 	net.frag[frag_at(l, k / 32, n / 16, ((k % 32) / 8) * 16 + n % 16) + k % 8] = v;
 	net.fragT[fragT_at(l, n / 32, k / 16, ((n % 32) / 8) * 16 + k % 16) + n % 8] = v;
 }
 
-// Adam (Kingma & Ba) on every weight and bias; step t >= 1.
-__global__ void k_net_adam(NetDev net, int t, float lr) {
+__global__ void k_net_pack(NetDev net) {
 	const int e = blockIdx.x * blockDim.x + threadIdx.x;
-	if(e >= NN_W + NN_B) return;
+	if(e < NN_W) pack_weight(net, e, net.w[e]);
+}
+
+// Adam (Kingma & Ba) on every weight and bias, from the gradients' partial
+// sums; step t >= 1.  Leaves the operand fragments of the new weights.
+__global__ void k_net_adam(NetDev net, const float *part, int slices, int t, float lr) {
+	const int e = blockIdx.x * blockDim.x + threadIdx.x;
+	if(e >= NN_G) return;
 	const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
 	const bool isw = e < NN_W;
 	const int i = isw ? e : e - NN_W;
 	float *w = isw ? net.w : net.b, *m = isw ? net.mw : net.mb, *v = isw ? net.vw : net.vb;
-	const float g = isw ? net.gw[i] : net.gb[i];
+	const float g = slice_sum(part, slices, e);
 	m[i] = b1 * m[i] + (1.f - b1) * g;
 	v[i] = b2 * v[i] + (1.f - b2) * g * g;
 	const float mh = m[i] / (1.f - powf(b1, (float) t)), vh = v[i] / (1.f - powf(b2, (float) t));
-	w[i] -= lr * mh / (sqrtf(vh) + eps);
+	const float nw = w[i] - lr * mh / (sqrtf(vh) + eps);
+	w[i] = nw;
+	if(isw) pack_weight(net, e, nw);
 }
 
-void launch_net_forward(const NetDev &net, const __bf16 *x, int m, const int *m_dev, float *y, __bf16 *h,
-                        hipStream_t s) {
+void launch_net_forward(const NetDev &net, const float *x, int m, float *y, hipStream_t s) {
 	const int blocks = (m + 15) / 16;
-	if(blocks > 0) hipLaunchKernelGGL(k_net_fwd, dim3(blocks), dim3(64), 0, s, net, x, m, m_dev, y, h, m);
+	if(blocks > 0) hipLaunchKernelGGL(k_net_fwd, dim3(blocks), dim3(64), 0, s, net, x, m, y);
 }
 
 void launch_net_pack(const NetDev &net, hipStream_t s) {
 	hipLaunchKernelGGL(k_net_pack, dim3((NN_W + 255) / 256), dim3(256), 0, s, net);
 }
 
-// m_pad (a multiple of 32) rows of x (rows >= m zero): forward with stored
-// activations, loss, backward, gradients into net.gw / net.gb; loss[m_pad].
-void launch_net_loss_grad(const NetDev &net, const __bf16 *x, const float *target, int m, __bf16 *h, float *y,
-                          __bf16 *dy, __bf16 *dh, float *loss, hipStream_t s) {
+template <class X>
+static void net_grad(const NetDev &net, const X *x, const float *target, int m, const NetScratch &q, hipStream_t s) {
 	const int m_pad = (m + 31) & ~31;
-	hipLaunchKernelGGL(k_net_fwd, dim3(m_pad / 16), dim3(64), 0, s, net, x, m_pad, (const int *) nullptr, y, h, m_pad);
-	hipLaunchKernelGGL(k_net_loss, dim3((m_pad + 255) / 256), dim3(256), 0, s, y, target, m, m_pad, dy, loss);
-	hipLaunchKernelGGL(k_net_bwd, dim3(m_pad / 16), dim3(64), 0, s, net, dy, h, m_pad, m_pad, dh);
-	int tiles = 0;
-	for(int l = 0; l < NN_LAYERS; l++) tiles += (nn_k(l) / 16) * (nn_n(l) / 16);
-	hipLaunchKernelGGL(k_net_wgrad, dim3(tiles), dim3(64), 0, s, net, x, h, dy, dh, m_pad, m_pad);
-	hipLaunchKernelGGL(k_net_bgrad, dim3(NN_B), dim3(256), 0, s, net, dy, dh, m_pad, m_pad);
+	hipLaunchKernelGGL(k_net_grad<X>, dim3(std::min(m_pad / NG_ROWS, NG_BLOCKS)), dim3(64 * NG_WAVES), 0, s, net, x, target,
+	                   m, m_pad, q.at, q.zt, q.loss);
+	hipLaunchKernelGGL(k_net_wgrad, dim3(NW_TILES / NW_WAVES, net_grad_slices(m_pad)), dim3(64 * NW_WAVES), 0, s,
+	                   (const __bf16 *) q.at, (const __bf16 *) q.zt, m_pad, q.part);
 }
 
-void launch_net_adam(const NetDev &net, int step, float lr, hipStream_t s) {
-	hipLaunchKernelGGL(k_net_adam, dim3((NN_W + NN_B + 255) / 256), dim3(256), 0, s, net, step, lr);
-	launch_net_pack(net, s);
+void launch_net_loss_grad(const NetDev &net, const float *x, const float *target, int m, const NetScratch &q,
+                          hipStream_t s) {
+	net_grad(net, x, target, m, q, s);
+	hipLaunchKernelGGL(k_net_reduce, dim3((NN_G + 255) / 256), dim3(256), 0, s, (const float *) q.part,
+	                   net_grad_slices((m + 31) & ~31), net.gw, net.gb);
+}
+
+void launch_net_train(const NetDev &net, const __bf16 *x, const float *target, int m, const NetScratch &q, hipStream_t s) {
+	net_grad(net, x, target, m, q, s);
+}
+
+void launch_net_adam(const NetDev &net, int m, const NetScratch &q, int step, float lr, hipStream_t s) {
+	hipLaunchKernelGGL(k_net_adam, dim3((NN_G + 255) / 256), dim3(256), 0, s, net, (const float *) q.part,
+	                   net_grad_slices((m + 31) & ~31), step, lr);
 }
 
 // ------------------------------------------------------------------------
@@ -900,7 +1058,9 @@ void launch_descriptor(int n, const double *r, const double *O, const Grid &g, i
 // rotated at random (the "current" state of a move), its descriptor there,
 // and as target the move back: displacement in the perturbed body frame and
 // the rotation axis (-a; the angle is uniform in both directions).  One wave
-// per sample.
+// per sample, which finds its neighbours as a pass does, from a record (here in
+// LDS) and positions staged once: a search through 27 ranges for every read of
+// a candidate took 33 us for 4096 samples, this 18.
 
 constexpr int TS_WAVES = 4;
 
@@ -908,33 +1068,19 @@ __global__ __launch_bounds__(64 * TS_WAVES) void k_train_samples(DevState d, uin
                                                                  int m_pad, double pos_noise, double theta_max,
                                                                  __bf16 *x, float *target) {
 	__shared__ DescLds Ds[TS_WAVES];
+	__shared__ __attribute__((aligned(16))) CandLds Cs[TS_WAVES];
 	const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 	const int b = blockIdx.x * TS_WAVES + wave;
 	__bf16 *row = x + (size_t) b * NN_IN_PAD;
 	const bool live = b < m;
 	int nv = 0;
 	double pt[3], Ot[9];
-	// the slot's cell neighbourhood (27 cells, the particle itself left out)
-	int st[27], cn[27], self = -1, j = 0, tot = 0;
+	CellView v{};
+	int j = 0;
 	const double *F = nullptr;
 	double L[3], iL[3];
-	auto slot_of = [&](int i) {
-		if(self >= 0 && i >= self) i++;
-		int nb = 0;
-		while(nb < 26 && i >= cn[nb]) {
-			i -= cn[nb];
-			nb++;
-		}
-		return st[nb] + i;
-	};
-	auto pos = [&](int i, double q[3]) {
-		const int s2 = slot_of(i);
-		for(int k = 0; k < 3; k++) q[k] = part(F, s2)[k];
-	};
-	auto ori = [&](int i, double Oq[9]) {
-		const int s2 = slot_of(i);
-		for(int k = 0; k < 9; k++) Oq[k] = part(F, s2)[3 + k];
-	};
+	CandLds &CL = Cs[wave];
+	auto cands = [&]() { return Cands{d, F, v, j, &CL}; };
 	if(b < m_pad && !live) {
 		if(lane < NN_IN_PAD / 2) {
 			row[2 * lane] = (__bf16) 0.f;
@@ -959,20 +1105,22 @@ __global__ __launch_bounds__(64 * TS_WAVES) void k_train_samples(DevState d, uin
 		for(int k = 0; k < 3; k++) p[k] = part(F, j)[k];
 		for(int k = 0; k < 9; k++) O[k] = part(F, j)[3 + k];
 		// its cell on the current grid (particles never leave their cells
-		// between rebuilds) and the 27 cells around it
+		// between rebuilds) and the cells around it, as a pass's record
 		const int n0 = rp.g.n[0], n1 = rp.g.n[1], n2 = rp.g.n[2];
 		const int ix = cell_coord(p[0], rp.g.shift[0], rp.g.inv_box[0], n0);
 		const int iy = cell_coord(p[1], rp.g.shift[1], rp.g.inv_box[1], n1);
 		const int iz = cell_coord(p[2], rp.g.shift[2], rp.g.inv_box[2], n2);
-		for(int nb = 0; nb < 27; nb++) {
-			const int cx = wrapi(ix + nb / 9 - 1, n0), cy = wrapi(iy + (nb / 3) % 3 - 1, n1),
-			          cz = wrapi(iz + nb % 3 - 1, n2);
-			const int cc = rp.cell_off + (cx * n1 + cy) * n2 + cz;
-			st[nb] = d.start[cc];
-			cn[nb] = d.start[cc + 1] - st[nb];
-			if(self < 0 && j >= st[nb] && j < st[nb] + cn[nb]) self = tot + (j - st[nb]);
-			tot += cn[nb];
-		}
+		v.rec = CL.rec;
+		v.cloc = (ix * n1 + iy) * n2 + iz;
+		v.r = d.prep[j];
+		v.sel = rp.sel;
+		if(lane < 16)
+			write_record(CL.rec, 0, d.start + rp.cell_off, v.cloc, ix, iy, iz, n0, n1, n2, v.r, v.sel, lane);
+		team_sync();
+		v.M = CL.rec[REC_M];
+		v.s0 = CL.rec[REC_S0];
+		v.cnt = CL.rec[REC_CNT];
+		cands().stage<64>(CL, lane);
 		// the perturbed state: Gaussian displacement, rotation by an angle
 		// uniform in [0, theta_max) about a uniform axis
 		double z[6];
@@ -994,10 +1142,16 @@ __global__ __launch_bounds__(64 * TS_WAVES) void k_train_samples(DevState d, uin
 				t[k] = (float) (Ot[3 * k] * (p[0] - pt[0]) + Ot[3 * k + 1] * (p[1] - pt[1]) + Ot[3 * k + 2] * (p[2] - pt[2]));
 			for(int k = 0; k < 3; k++) t[3 + k] = (float) -ax[k];
 		}
-		nv = desc_collect<64>(pt, self >= 0 ? tot - 1 : tot, pos, L, iL, Ds[wave], row, lane);
+		const Cands c = cands();
+		nv = desc_collect<64>(pt, c.count(), [&](int i, double q[3]) { c.pos(i, q); }, L, iL, Ds[wave], row, lane);
 	}
 	__syncthreads();
-	if(live) desc_fill<64>(pt, Ot, nv, pos, ori, L, iL, Ds[wave], row, lane);
+	if(live) {
+		const Cands c = cands();
+		desc_fill<64>(
+			pt, Ot, nv, [&](int i, double q[3]) { c.pos(i, q); }, [&](int i, double Oq[9]) { c.ori(i, Oq); }, L, iL, Ds[wave],
+			row, lane);
+	}
 }
 
 void launch_train_samples(const DevState &d, uint64_t seed, uint64_t step, int m, double pos_noise, double theta_max,

@@ -47,15 +47,6 @@ pp_status nalloc(pp_net *n, Tp **p, size_t count) {
 	return PP_OK;
 }
 
-// round to nearest even
-uint16_t to_bf16(float f) {
-	uint32_t u;
-	std::memcpy(&u, &f, 4);
-	if((u & 0x7fffffffu) > 0x7f800000u) return (uint16_t) ((u >> 16) | 0x40);  // NaN stays NaN
-	u += 0x7fffu + ((u >> 16) & 1u);
-	return (uint16_t) (u >> 16);
-}
-
 float from_bf16(uint16_t b) {
 	uint32_t u = (uint32_t) b << 16;
 	float f;
@@ -99,7 +90,7 @@ int ppd::net_reserve(pp_net *n, int m) {
 	if(need <= n->cap) return PP_OK;
 	// the smaller scratch of earlier calls goes (the stream is idle: every
 	// call that used it synchronised)
-	void *old[] = {n->x, n->h, n->dy, n->dh, n->y, n->target, n->loss};
+	void *old[] = {n->x, n->xh, n->y, n->target, n->q.at, n->q.zt, n->q.part, n->q.loss};
 	for(void *p : old) {
 		if(!p) continue;
 		for(size_t k = 0; k < n->allocs.size(); k++)
@@ -109,14 +100,16 @@ int ppd::net_reserve(pp_net *n, int m) {
 				break;
 			}
 	}
-	n->x = n->h = n->dy = n->dh = nullptr;
-	n->y = n->target = n->loss = nullptr;
+	n->x = nullptr;
+	n->xh = n->y = n->target = nullptr;
+	n->q = NetScratch{};
 	n->cap = 0;
 	const size_t r = (size_t) need;
 	pp_status st;
-	if((st = nalloc(n, &n->x, r * NN_IN_PAD)) || (st = nalloc(n, &n->h, 3 * r * NN_H)) ||
-	   (st = nalloc(n, &n->dy, r * NN_OUT_PAD)) || (st = nalloc(n, &n->dh, 3 * r * NN_H)) ||
-	   (st = nalloc(n, &n->y, r * NN_OUT_PAD)) || (st = nalloc(n, &n->target, r * 6)) || (st = nalloc(n, &n->loss, r)))
+	if((st = nalloc(n, &n->x, r * NN_IN_PAD)) || (st = nalloc(n, &n->xh, r * NN_IN)) ||
+	   (st = nalloc(n, &n->y, r * NN_OUT_PAD)) || (st = nalloc(n, &n->target, r * 6)) ||
+	   (st = nalloc(n, &n->q.at, r * (NN_IN_PAD + 3 * NN_H))) || (st = nalloc(n, &n->q.zt, r * NN_B)) ||
+	   (st = nalloc(n, &n->q.part, (size_t) net_grad_slices(need) * (NN_W + NN_B))) || (st = nalloc(n, &n->q.loss, r)))
 		return st;
 	n->cap = need;
 	return PP_OK;
@@ -189,22 +182,14 @@ pp_status pp_net_get(pp_net *n, float *w, float *b) {
 	return PP_OK;
 }
 
-static pp_status upload_inputs(pp_net *n, int m, const float *x) {
-	const int m_pad = (m + 31) & ~31;
-	std::vector<uint16_t> hx((size_t) m_pad * NN_IN_PAD, 0);
-	for(int i = 0; i < m; i++)
-		for(int e = 0; e < NN_IN; e++) hx[(size_t) i * NN_IN_PAD + e] = to_bf16(x[(size_t) i * NN_IN + e]);
-	NCHECK(hipMemcpy(n->x, hx.data(), hx.size() * 2, hipMemcpyHostToDevice));
-	return PP_OK;
-}
-
 pp_status pp_net_forward(pp_net *n, int m, const float *x, float *y) {
 	if(!n || m < 0 || (m > 0 && (!x || !y))) return nfail(PP_ERR_ARG, "bad arguments");
 	if(m == 0) return PP_OK;
 	NCHECK(hipSetDevice(n->device));
 	pp_status st;
-	if((st = (pp_status) net_reserve(n, m)) || (st = upload_inputs(n, m, x))) return st;
-	launch_net_forward(n->d, n->x, m, nullptr, n->y, nullptr, n->stream);
+	if((st = (pp_status) net_reserve(n, m)) != PP_OK) return st;
+	NCHECK(hipMemcpy(n->xh, x, sizeof(float) * NN_IN * (size_t) m, hipMemcpyHostToDevice));
+	launch_net_forward(n->d, n->xh, m, n->y, n->stream);
 	NCHECK(hipStreamSynchronize(n->stream));
 	NCHECK(hipGetLastError());
 	std::vector<float> hy((size_t) m * NN_OUT_PAD);
@@ -218,14 +203,15 @@ pp_status pp_net_loss_grad(pp_net *n, int m, const float *x, const float *target
 	if(!n || m <= 0 || !x || !target) return nfail(PP_ERR_ARG, "bad arguments");
 	NCHECK(hipSetDevice(n->device));
 	pp_status st;
-	if((st = (pp_status) net_reserve(n, m)) || (st = upload_inputs(n, m, x))) return st;
+	if((st = (pp_status) net_reserve(n, m)) != PP_OK) return st;
+	NCHECK(hipMemcpy(n->xh, x, sizeof(float) * NN_IN * (size_t) m, hipMemcpyHostToDevice));
 	NCHECK(hipMemcpy(n->target, target, sizeof(float) * 6 * (size_t) m, hipMemcpyHostToDevice));
-	launch_net_loss_grad(n->d, n->x, n->target, m, n->h, n->y, n->dy, n->dh, n->loss, n->stream);
+	launch_net_loss_grad(n->d, n->xh, n->target, m, n->q, n->stream);
 	NCHECK(hipStreamSynchronize(n->stream));
 	NCHECK(hipGetLastError());
 	if(loss) {
 		std::vector<float> hl(m);
-		NCHECK(hipMemcpy(hl.data(), n->loss, sizeof(float) * m, hipMemcpyDeviceToHost));
+		NCHECK(hipMemcpy(hl.data(), n->q.loss, sizeof(float) * m, hipMemcpyDeviceToHost));
 		double s = 0.;
 		for(float v : hl) s += v;
 		*loss = s / m;

@@ -12,8 +12,9 @@ struct pp_net {
 	int step = 0;  // Adam steps taken
 	// device scratch of host-driven calls and of training batches
 	int cap = 0;  // rows (multiple of 32)
-	__bf16 *x = nullptr, *h = nullptr, *dy = nullptr, *dh = nullptr;
-	float *y = nullptr, *target = nullptr, *loss = nullptr;
+	__bf16 *x = nullptr;                                // training samples
+	float *xh = nullptr, *y = nullptr, *target = nullptr;  // a caller's rows, their outputs, the targets
+	ppd::NetScratch q{};
 	std::vector<void *> allocs;
 	~pp_net();
 };

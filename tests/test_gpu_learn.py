@@ -111,6 +111,32 @@ def test_loss_and_gradients_match_oracle(pp):
             assert not gw[no.W_OFF[3]:].reshape(no.H, no.OUT_PAD)[:, no.OUT:].any()
 
 
+@pytest.mark.parametrize("m", [1, 16, 31, 33, 511, 513, 4129, 9000])
+def test_gradients_at_tile_and_slice_edges(pp, m):
+    """One row, part of a tile, one and two row slices, more tiles than
+    workgroups, the most slices: every row counts once.  BF16 activations in
+    both, so the bounds are those of the test above."""
+    rng = np.random.default_rng(m)
+    with pp.ProposalNet(seed=4) as net:
+        w, b = net.get()
+        w = w.copy()
+        w[no.W_OFF[3]:] *= 10
+        net.set(w, b)
+        x = _rand_inputs(rng, m)
+        t = np.hstack([rng.normal(scale=0.05, size=(m, 3)), rng.normal(size=(m, 3))])
+        t[:, 3:] /= np.linalg.norm(t[:, 3:], axis=1, keepdims=True)
+        loss, gw, gb = net.loss_grad(x, t)
+        lo, ow, ob = no.loss_and_grads(w, b, x, t.astype(np.float32).astype(np.float64))
+        assert abs(loss - lo) < 1e-3 * (1 + abs(lo)), (m, loss, lo)
+        for g, o in ((gw, ow), (gb, ob)):
+            g = g.astype(np.float64)
+            cos = g @ o / (np.linalg.norm(g) * np.linalg.norm(o))
+            assert cos > 0.999, (m, cos)
+            assert abs(np.linalg.norm(g) / np.linalg.norm(o) - 1) < 0.02
+        again = net.loss_grad(x, t)
+        assert again[0] == loss and np.array_equal(again[1], gw) and np.array_equal(again[2], gb)
+
+
 def _skewed_net(pp, seed, drift=0.08, spread=(0.4, 0.05, 0.1), kappa=20.0, hidden_scale=1.0):
     """A network whose proposal is far from symmetric: a drift along the body
     x axis, anisotropic spread, an axis concentrated around body z, and (with
