@@ -1588,10 +1588,9 @@ pp_status pp_net_train(pp_ctx *c, pp_net *net, int steps, int batch, double lr, 
 	for(int s = 0; s < steps; s++) {
 		if(s > 0)
 			for(int k = 0; k < sweeps_between; k++) TRY(enqueue_sweep(c));
-		// the cell ranges of the current state: those of the last sweep hold
-		// (its passes move no particle out of its cell), unless a box trial
-		// has left those of its trial grid
-		if(s == 0 || c->any_npt || c->any_lx) rebuild_now(c);
+		// the cell ranges of the current state (an NPT trial may have left
+		// those of its trial grid)
+		rebuild_now(c);
 		launch_train_samples(c->d, tseed, (uint64_t) net->step, batch, pos_noise, theta_max, net->x, net->target,
 		                     c->stream);
 		launch_net_train(net->d, net->x, net->target, batch, net->q, c->stream);
