@@ -117,6 +117,7 @@ __device__ __forceinline__ void row_ranges(const int *st, int ix, int iy, int iz
 // Slot of candidate i of those rows, counted through (a record holds the
 // first REC_SLOTS; few cells have more).
 __device__ inline int walk_slot(const int *st, int ix, int iy, int iz, int n0, int n1, int n2, int i) {
+#pragma unroll 1  // (rare: nine copies at every use only displace the code that runs)
 	for(int j = 0; j < 9; j++) {
 		int a1, b1, a2, b2;
 		row_ranges(st, ix, iy, iz, n0, n1, n2, j, a1, b1, a2, b2);

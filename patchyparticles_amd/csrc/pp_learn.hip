@@ -65,20 +65,53 @@ __device__ inline float log_vmf(float lk, float c) {
 	return lk - LOG_2PI - k - logf(-expm1f(-2.f * k)) + k * c;
 }
 
-__device__ inline float prop_logq(const Prop &p, const float d[3], const float a[3]) {
+// The same by the lanes of a cell's team: lane tl decodes mixture component
+// tl % NN_MIX and the four meet within their quad, in the order of the
+// components, so that every lane has the values of the serial form.
+static_assert(NN_MIX == 4, "a quad of lanes");
+struct PropLane {
+	float mu[3], ls[3];
+	float dir[3], k, lk, lw;  // of the lane's component (k = exp(lk))
+};
+
+template <int c>
+__device__ __forceinline__ float quad_get(float v) {
+	return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), c * 0x55, 0xf, 0xf, true));
+}
+
+// (every lane of the quad active)
+__device__ __forceinline__ float quad_log_sum_exp(float l) {
+	const float mx = fmaxf(fmaxf(fmaxf(fmaxf(-3.0e38f, quad_get<0>(l)), quad_get<1>(l)), quad_get<2>(l)), quad_get<3>(l));
+	const float e = expf(l - mx);
+	return mx + logf(quad_get<0>(e) + quad_get<1>(e) + quad_get<2>(e) + quad_get<3>(e));
+}
+
+__device__ __forceinline__ void prop_decode_lane(const float *y, int tl, PropLane &p) {
+#pragma unroll
+	for(int k = 0; k < 3; k++) {
+		p.mu[k] = y[k];
+		p.ls[k] = fminf(fmaxf(y[3 + k], NN_LS_MIN), NN_LS_MAX);
+	}
+	const float *u = y + 6 + 5 * (tl & (NN_MIX - 1));
+	const float n = sqrtf(u[0] * u[0] + u[1] * u[1] + u[2] * u[2] + 1e-12f);
+#pragma unroll
+	for(int j = 0; j < 3; j++) p.dir[j] = u[j] / n;
+	p.lk = fminf(fmaxf(u[3], NN_LK_MIN), NN_LK_MAX);
+	p.k = expf(p.lk);
+	p.lw = u[4] - quad_log_sum_exp(u[4]);
+}
+
+__device__ __forceinline__ float prop_logq_lane(const PropLane &p, const float d[3], const float a[3]) {
 	float lg = 0.f;
+#pragma unroll
 	for(int k = 0; k < 3; k++) {
 		const float z = (d[k] - p.mu[k]) * expf(-p.ls[k]);
 		lg += -0.5f * z * z - p.ls[k] - 0.5f * LOG_2PI;
 	}
-	float l[NN_MIX], mx = -3.0e38f;
-	for(int c = 0; c < NN_MIX; c++) {
-		l[c] = p.lw[c] + log_vmf(p.lk[c], p.dir[c][0] * a[0] + p.dir[c][1] * a[1] + p.dir[c][2] * a[2]);
-		mx = fmaxf(mx, l[c]);
-	}
-	float se = 0.f;
-	for(int c = 0; c < NN_MIX; c++) se += expf(l[c] - mx);
-	return lg + mx + logf(se);
+	const float l = p.lw + log_vmf(p.lk, p.dir[0] * a[0] + p.dir[1] * a[1] + p.dir[2] * a[2]);
+	const float mx = fmaxf(fmaxf(fmaxf(fmaxf(-3.0e38f, quad_get<0>(l)), quad_get<1>(l)), quad_get<2>(l)), quad_get<3>(l));
+	const float e = expf(l - mx);
+	return lg + mx + logf(quad_get<0>(e) + quad_get<1>(e) + quad_get<2>(e) + quad_get<3>(e));
 }
 
 // -log q and its gradient with respect to the raw outputs y (g[NN_OUT_PAD])
@@ -121,38 +154,27 @@ __device__ inline float prop_loss_grad(const float *y, const float d[3], const f
 // ------------------------------------------------------------------------
 // descriptor
 
-// Quaternion (x, y, z, w), w >= 0, of the rotation matrix M (rows).
+// Quaternion (x, y, z, w), w >= 0, of the rotation matrix M (rows), from its
+// largest component.  The four cases choose operands: one square root and
+// three divisions, where lanes of different cases ran them four times.
 __device__ inline void quat_of(const double M[9], float q[4]) {
-	double x, y, z, w;
 	const double tr = M[0] + M[4] + M[8];
-	if(tr > 0.) {
-		const double S = sqrt(tr + 1.) * 2.;
-		w = 0.25 * S;
-		x = (M[7] - M[5]) / S;
-		y = (M[2] - M[6]) / S;
-		z = (M[3] - M[1]) / S;
-	}
-	else if(M[0] > M[4] && M[0] > M[8]) {
-		const double S = sqrt(1. + M[0] - M[4] - M[8]) * 2.;
-		w = (M[7] - M[5]) / S;
-		x = 0.25 * S;
-		y = (M[1] + M[3]) / S;
-		z = (M[2] + M[6]) / S;
-	}
-	else if(M[4] > M[8]) {
-		const double S = sqrt(1. + M[4] - M[0] - M[8]) * 2.;
-		w = (M[2] - M[6]) / S;
-		x = (M[1] + M[3]) / S;
-		y = 0.25 * S;
-		z = (M[5] + M[7]) / S;
-	}
-	else {
-		const double S = sqrt(1. + M[8] - M[0] - M[4]) * 2.;
-		w = (M[3] - M[1]) / S;
-		x = (M[2] + M[6]) / S;
-		y = (M[5] + M[7]) / S;
-		z = 0.25 * S;
-	}
+	const bool cw = tr > 0.;
+	const bool cx = !cw && M[0] > M[4] && M[0] > M[8];
+	const bool cy = !cw && !cx && M[4] > M[8];
+	const double d0 = cx ? M[0] : (cy ? M[4] : M[8]);  // its diagonal element, then the others
+	const double d1 = cx ? M[4] : M[0];
+	const double d2 = cx || cy ? M[8] : M[4];
+	const double S = sqrt(cw ? tr + 1. : 1. + d0 - d1 - d2) * 2.;
+	const double big = 0.25 * S;
+	const double a0 = M[7] - M[5], a1 = M[2] - M[6], a2 = M[3] - M[1];
+	const double s01 = M[1] + M[3], s02 = M[2] + M[6], s12 = M[5] + M[7];
+	const double e0 = (cw || cx ? a0 : (cy ? s01 : s02)) / S;
+	const double e1 = (cw || cy ? a1 : (cx ? s01 : s12)) / S;
+	const double e2 = (cw ? a2 : (cx ? s02 : (cy ? s12 : a2))) / S;
+	const bool cz = !cw && !cx && !cy;
+	const double x = cx ? big : e0, y = cy ? big : e1, z = cz ? big : e2;
+	const double w = cw ? big : (cx ? e0 : (cy ? e1 : e2));
 	const double sg = w < 0. ? -1. : 1.;
 	q[0] = (float) (sg * x);
 	q[1] = (float) (sg * y);
@@ -177,14 +199,16 @@ struct DescLds {
 	int i[DESC_CAND];    // its candidate index
 };
 
-// T: lanes per particle (64: a wavefront, 32: half of one); tl = lane % T.
+template <int T>
+__device__ __forceinline__ void zero_row(__bf16 *row, int tl) {
+	for(int e = tl; e < NN_IN_PAD / 8; e += T) *(bf16x8 *) (row + 8 * e) = bf16x8{};
+}
+
+// T: lanes per particle (64: a wavefront, 16: a quarter of one); tl = lane % T.
 template <int T, class Pos>
 __device__ int desc_collect(const double p[3], int n, Pos pos, const double L[3], const double iL[3], DescLds &S,
                             __bf16 *row, int tl) {
-	for(int e = tl; e < NN_IN_PAD / 2; e += T) {
-		row[2 * e] = (__bf16) 0.f;
-		row[2 * e + 1] = (__bf16) 0.f;
-	}
+	zero_row<T>(row, tl);
 	const double rc2 = NN_RCUT * NN_RCUT;
 	const int off = (threadIdx.x & 63) & ~(T - 1);
 	const unsigned long long tm = T == 64 ? ~0ull : ((1ull << T) - 1ull);
@@ -693,7 +717,7 @@ __device__ inline CellView cell_view(const DevState &d, int pass, int gi) {
 
 // Candidates of one wave's cell, staged in LDS: their slots and positions
 // (the first CAND_MAX; the rest are read from the record and global memory).
-constexpr int CAND_MAX = 128;
+constexpr int CAND_MAX = 64;
 struct CandLds {
 	double x[CAND_MAX], y[CAND_MAX], z[CAND_MAX];
 	int slot[CAND_MAX];
@@ -745,7 +769,7 @@ struct Cands {
 
 constexpr int PROP_W = NN_PROP_W;  // p'[3], O'[9], log q forward, axis[3]
 constexpr int LP_ROWS = 16;        // rows of the MFMA tile = cells of one workgroup
-constexpr int LP_TEAM = 32;        // lanes per cell: two cells per wavefront
+constexpr int LP_TEAM = 16;        // lanes per cell: four cells per wavefront
 constexpr int LP_WAVES = LP_ROWS * LP_TEAM / 64;
 
 // LDS of one learned-pass workgroup
@@ -755,47 +779,91 @@ struct LpLds {
 	float y[LP_ROWS * NN_OUT_PAD];    // network outputs
 	DescLds desc[LP_ROWS];
 	double prop[LP_ROWS][PROP_W];     // the drawn proposal of each cell
+	double cur[LP_ROWS][NCOMP];       // the moving particle
 	CandLds cand[LP_ROWS];
 };
 
-// The network on the workgroup's 16 rows, S.x -> S.y; wave w computes the
-// 16-column tiles w, w + LP_WAVES, ... of each layer; a barrier after each.
-__device__ void lp_forward(const NetDev &net, LpLds &S, int wave, int lane) {
-	const int r = lane & 15, g = lane >> 4;
-	int cur = 0;
-	for(int l = 0; l < NN_LAYERS; l++) {
-		const int nkb = nn_k(l) / 32, nnt = nn_n(l) / 16;
-		const __bf16 *A = l == 0 ? S.x : S.act[cur];
-		for(int nt = wave; nt < nnt; nt += LP_WAVES) {
-			f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-			for(int kb = 0; kb < nkb; kb++) {
-				const bf16x8 a = *(const bf16x8 *) (A + r * ACT_LD + kb * 32 + g * 8);
-				const bf16x8 b = *(const bf16x8 *) (net.frag + frag_at(l, kb, nt, lane));
-				acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc, 0, 0, 0);
-			}
-			const int col = nt * 16 + r;
-			const float bias = net.b[nn_boff(l) + col];
-			for(int j = 0; j < 4; j++) {
-				const int row = g * 4 + j;
-				const float v = acc[j] + bias;
-				if(l < NN_LAYERS - 1) S.act[cur ^ 1][row * ACT_LD + col] = (__bf16) fmaxf(v, 0.f);
-				else S.y[row * NN_OUT_PAD + col] = v;
-			}
-		}
-		__syncthreads();
-		cur ^= 1;
+// The operand fragments and biases of a wavefront's columns of one layer:
+// 16-column tiles w and w + LP_WAVES, as far as the layer has them.
+constexpr int LP_TILES = NN_H / 16 / LP_WAVES;
+struct LayerOps {
+	bf16x8 f[LP_TILES][NN_H / 32];
+	float bias[LP_TILES];
+};
+template <int l>
+__device__ __forceinline__ void load_ops(const NetDev &net, int wave, int lane, LayerOps &o) {
+#pragma unroll
+	for(int u = 0; u < LP_TILES; u++) {
+		const int nt = wave + u * LP_WAVES;
+		if(nt >= nn_n(l) / 16) return;
+#pragma unroll
+		for(int kb = 0; kb < nn_k(l) / 32; kb++) o.f[u][kb] = *(const bf16x8 *) (net.frag + frag_at(l, kb, nt, lane));
+		o.bias[u] = net.b[nn_boff(l) + nt * 16 + (lane & 15)];
 	}
 }
 
+// Layer l on the workgroup's 16 rows, A -> S.act / S.y, and a barrier; the
+// next layer's weights are under way before that barrier, so that a layer
+// waits for LDS and MFMAs only.
+template <int l>
+__device__ __forceinline__ void lp_layer(const NetDev &net, LpLds &S, int wave, int lane, LayerOps &o) {
+	const int r = lane & 15, g = lane >> 4;
+	const __bf16 *A = l == 0 ? S.x : S.act[l & 1];
+	LayerOps next;
+	if constexpr(l + 1 < NN_LAYERS) load_ops<l + 1>(net, wave, lane, next);
+	bf16x8 a[nn_k(l) / 32];
+#pragma unroll
+	for(int kb = 0; kb < nn_k(l) / 32; kb++) a[kb] = *(const bf16x8 *) (A + r * ACT_LD + kb * 32 + g * 8);
+#pragma unroll
+	for(int u = 0; u < LP_TILES; u++) {
+		const int nt = wave + u * LP_WAVES, col = nt * 16 + r;
+		if(nt >= nn_n(l) / 16) break;
+		f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+		for(int kb = 0; kb < nn_k(l) / 32; kb++)
+			acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[kb], o.f[u][kb], acc, 0, 0, 0);
+#pragma unroll
+		for(int j = 0; j < 4; j++) {
+			const int row = g * 4 + j;
+			const float v = acc[j] + o.bias[u];
+			if constexpr(l < NN_LAYERS - 1) S.act[(l & 1) ^ 1][row * ACT_LD + col] = (__bf16) fmaxf(v, 0.f);
+			else S.y[row * NN_OUT_PAD + col] = v;
+		}
+	}
+	__syncthreads();
+	if constexpr(l + 1 < NN_LAYERS) o = next;
+}
+
+// The network on the workgroup's 16 rows, S.x -> S.y, after a barrier.
+__device__ __forceinline__ void lp_forward(const NetDev &net, LpLds &S, int wave, int lane) {
+	static_assert(LP_TILES * LP_WAVES * 16 == NN_H && NN_LAYERS == 4, "whole column tiles per wavefront");
+	LayerOps o;
+	load_ops<0>(net, wave, lane, o);
+	__syncthreads();
+	lp_layer<0>(net, S, wave, lane, o);
+	lp_layer<1>(net, S, wave, lane, o);
+	lp_layer<2>(net, S, wave, lane, o);
+	lp_layer<3>(net, S, wave, lane, o);
+}
+
 // The whole learned pass in one kernel: a workgroup takes 16 cells of the
-// pass's list (the rows of one MFMA tile), 32 lanes per cell:
+// pass's list (the rows of one MFMA tile), 16 lanes per cell:
 //   A  pick the moving member (uniform by rank of particle index, as the plain
 //      pass), descriptor of the current state;      network forward (MFMA)
 //   B  draw the proposal from the outputs; a move that leaves the cell is
 //      rejected; descriptor of the proposed state;  network forward (MFMA)
 //   C  reverse density, Kern-Frenkel energy change over the cell's
 //      candidates (the reference's pair test), Metropolis-Hastings.
-__global__ __launch_bounds__(64 * LP_WAVES) void k_learn_pass(DevState d, NetDev net, uint64_t sweep, int pass) {
+// Bound by instruction issue: a wavefront runs some 8000 instructions, most
+// of them FP64 or the densities' transcendentals, whatever the share of its
+// lanes that have a candidate.  With 32 lanes per cell (about 10 candidates
+// within reach) and 95 KB of LDS, N=65536 at rho 0.3 was 409 workgroups on
+// 256 CUs in two rounds, 55 us.  16 lanes and 67 KB halve the instructions
+// and let every workgroup run at once; the mixture's components are one per
+// lane; code that rarely runs (slots past a record's list) is no longer
+// unrolled into every use, since the kernel exceeds the instruction cache.
+// 26 us.  (32 lanes in 128 registers, two workgroups per CU: 60 us, spills.)
+__global__ __launch_bounds__(64 * LP_WAVES, 2) void k_learn_pass(DevState d, NetDev net, uint64_t sweep, int pass) {
 	__shared__ __attribute__((aligned(16))) LpLds S;
 	constexpr int T = LP_TEAM;
 	const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -811,17 +879,18 @@ __global__ __launch_bounds__(64 * LP_WAVES) void k_learn_pass(DevState d, NetDev
 	__bf16 *row = S.x + cell * ACT_LD;
 	DescLds &D = S.desc[cell];
 	CandLds &CL = S.cand[cell];
+	double *cur = S.cur[cell];
 	double L[3], iL[3];
 	if(live) {
 		v = cell_view(d, pass, gi);
-		// a cell of more members than a team holds (one per lane) is not
-		// moved and is reported; its threads stay for the barriers below
-		if(v.cnt > CELL_CAP || v.cnt > T) {
+		// a cell of more members than the passes work on is not moved and is
+		// reported; its threads stay for the barriers below
+		if(v.cnt > CELL_CAP) {
 			if(tl == 0) atomicOr(d.err, (int) ERR_CELL_CAP);
 			live = false;
 		}
 		else
-			for(int e = tl; e < REC_W; e += T) CL.rec[e] = v.rec[e];
+			for(int e = tl; e < REC_W / 4; e += T) ((int4 *) CL.rec)[e] = ((const int4 *) v.rec)[e];
 	}
 	__syncthreads();
 
@@ -836,45 +905,46 @@ __global__ __launch_bounds__(64 * LP_WAVES) void k_learn_pass(DevState d, NetDev
 		const int *PID = pick_buf(d.pid, v.sel);
 		const u32x4 ra = rng(d.seed, v.r, sweep, (uint32_t) v.cloc, TAG_LEARN_A, (uint32_t) pass, 0);
 		const int target = (int) __umulhi(ra.x, (uint32_t) v.cnt);
-		bool hit = false;
-		if(tl < v.cnt) {
-			const int me = PID[v.s0 + tl];
-			int rk = 0;
-			for(int b = 0; b < v.cnt; b++) rk += PID[v.s0 + b] < me;
-			hit = rk == target;
+		// (few cells hold more members than the team has lanes)
+		for(int m0 = 0; m0 < v.cnt; m0 += T) {
+			bool hit = false;
+			if(m0 + tl < v.cnt) {
+				const int me = PID[v.s0 + m0 + tl];
+				int rk = 0;
+				for(int b = 0; b < v.cnt; b++) rk += PID[v.s0 + b] < me;
+				hit = rk == target;
+			}
+			const unsigned long long hm = (__ballot(hit) >> (lane & ~(T - 1))) & ((1ull << T) - 1ull);
+			if(hm) j = v.s0 + m0 + (int) __builtin_ctzll(hm);
 		}
-		const unsigned long long hm = (__ballot(hit) >> (lane & ~(T - 1))) & ((1ull << T) - 1ull);
-		j = v.s0 + (int) __builtin_ctzll(hm);
+		if(tl < NCOMP) cur[tl] = part(F, j)[tl];
 		const Cands c{d, F, v, j, &CL};
 		c.stage<T>(CL, tl);
+		team_sync();
 		double p[3];
-		for(int k = 0; k < 3; k++) p[k] = part(F, j)[k];
+		for(int k = 0; k < 3; k++) p[k] = cur[k];
 		nv = desc_collect<T>(p, c.count(), [&](int i, double q[3]) { c.pos(i, q); }, L, iL, D, row, tl);
 	}
 	else
-		for(int e = tl; e < NN_IN_PAD / 2; e += T) {
-			row[2 * e] = (__bf16) 0.f;
-			row[2 * e + 1] = (__bf16) 0.f;
-		}
+		zero_row<T>(row, tl);
 	__syncthreads();
 	if(live) {
 		const Cands c{d, F, v, j, &CL};
 		double p[3], O[9];
-		for(int k = 0; k < 3; k++) p[k] = part(F, j)[k];
-		for(int k = 0; k < 9; k++) O[k] = part(F, j)[3 + k];
+		for(int k = 0; k < 3; k++) p[k] = cur[k];
+		for(int k = 0; k < 9; k++) O[k] = cur[3 + k];
 		desc_fill<T>(
 			p, O, nv, [&](int i, double q[3]) { c.pos(i, q); }, [&](int i, double Oq[9]) { c.ori(i, Oq); }, L, iL, D, row,
 			tl);
 	}
-	__syncthreads();
 	lp_forward(net, S, wave, lane);
 
 	// ---- B
 	bool inside = false;
 	if(live) {
 		const Rep &rp = d.reps[v.r];
-		Prop pr;
-		prop_decode(S.y + cell * NN_OUT_PAD, pr);
+		PropLane pr;
+		prop_decode_lane(S.y + cell * NN_OUT_PAD, tl, pr);
 		const u32x4 ra = rng(d.seed, v.r, sweep, (uint32_t) v.cloc, TAG_LEARN_A, (uint32_t) pass, 1);
 		const u32x4 rb = rng(d.seed, v.r, sweep, (uint32_t) v.cloc, TAG_LEARN_B, (uint32_t) pass, 0);
 		float z[4];
@@ -883,29 +953,18 @@ __global__ __launch_bounds__(64 * LP_WAVES) void k_learn_pass(DevState d, NetDev
 		float dbody[3];
 		for(int k = 0; k < 3; k++) dbody[k] = pr.mu[k] + expf(pr.ls[k]) * z[k];
 		// mixture component by its weight, then the axis
-		const float uc = u01f(rb.x);
-		int comp = NN_MIX - 1;
-		float acc = 0.f;
-		for(int c = 0; c < NN_MIX; c++) {
-			acc += expf(pr.lw[c]);
-			if(uc < acc) {
-				comp = c;
-				break;
-			}
-		}
-		float dir[3], kap = expf(pr.lk[0]);
-		for(int k = 0; k < 3; k++) dir[k] = pr.dir[0][k];
-		for(int c = 1; c < NN_MIX; c++)
-			if(c == comp) {
-				for(int k = 0; k < 3; k++) dir[k] = pr.dir[c][k];
-				kap = expf(pr.lk[c]);
-			}
+		const float uc = u01f(rb.x), wc = expf(pr.lw);
+		const float c0 = quad_get<0>(wc), c1 = c0 + quad_get<1>(wc), c2 = c1 + quad_get<2>(wc);
+		const int comp = uc < c0 ? 0 : (uc < c1 ? 1 : (uc < c2 ? 2 : 3)), from = (lane & ~(NN_MIX - 1)) + comp;
+		float dir[3];
+		for(int k = 0; k < 3; k++) dir[k] = __shfl(pr.dir[k], from);
+		const float kap = __shfl(pr.k, from);
 		float axf[3];
 		vmf_sample(dir, kap, u01f(rb.y), u01f(rb.z), axf);
 		const double ang = u01(rb.w) * d.learn.theta_max;
 		double p[3], O[9];
-		for(int k = 0; k < 3; k++) p[k] = part(F, j)[k];
-		for(int k = 0; k < 9; k++) O[k] = part(F, j)[3 + k];
+		for(int k = 0; k < 3; k++) p[k] = cur[k];
+		for(int k = 0; k < 9; k++) O[k] = cur[3 + k];
 		// body -> lab: O^T d; O' = O R(a, angle) (utils.c:186-209)
 		double np[3];
 		for(int k = 0; k < 3; k++) np[k] = p[k] + (O[k] * dbody[0] + O[3 + k] * dbody[1] + O[6 + k] * dbody[2]);
@@ -915,10 +974,11 @@ __global__ __launch_bounds__(64 * LP_WAVES) void k_learn_pass(DevState d, NetDev
 		rotation_matrix(axd, st, ct, R);
 		mat_mul3(O, R, On);
 		double *out = S.prop[cell];
+		const float logq = prop_logq_lane(pr, dbody, axf);
 		if(tl == 0) {
 			for(int k = 0; k < 3; k++) out[k] = np[k];
 			for(int k = 0; k < 9; k++) out[3 + k] = On[k];
-			out[12] = prop_logq(pr, dbody, axf);
+			out[12] = logq;
 			for(int k = 0; k < 3; k++) out[13 + k] = axd[k];
 		}
 		const int n0 = rp.g.n[0], n1 = rp.g.n[1], n2 = rp.g.n[2];
@@ -942,7 +1002,6 @@ __global__ __launch_bounds__(64 * LP_WAVES) void k_learn_pass(DevState d, NetDev
 			np, On, nv, [&](int i, double q[3]) { c.pos(i, q); }, [&](int i, double Oq[9]) { c.ori(i, Oq); }, L, iL, D, row,
 			tl);
 	}
-	__syncthreads();
 	lp_forward(net, S, wave, lane);
 
 	// ---- C (no barrier below: teams leave independently)
@@ -957,8 +1016,8 @@ __global__ __launch_bounds__(64 * LP_WAVES) void k_learn_pass(DevState d, NetDev
 	double *Fw = pick_buf(d.f, v.sel);
 	const double *pp = S.prop[cell];
 	double p[3], O[9], np[3], On[9];
-	for(int k = 0; k < 3; k++) p[k] = part(Fw, j)[k];
-	for(int k = 0; k < 9; k++) O[k] = part(Fw, j)[3 + k];
+	for(int k = 0; k < 3; k++) p[k] = cur[k];
+	for(int k = 0; k < 9; k++) O[k] = cur[3 + k];
 	for(int k = 0; k < 3; k++) np[k] = pp[k];
 	for(int k = 0; k < 9; k++) On[k] = pp[3 + k];
 	// reverse: displacement p - p' in the body frame of O', axis -a
@@ -966,9 +1025,9 @@ __global__ __launch_bounds__(64 * LP_WAVES) void k_learn_pass(DevState d, NetDev
 	for(int k = 0; k < 3; k++)
 		rbody[k] = (float) (On[3 * k] * (p[0] - np[0]) + On[3 * k + 1] * (p[1] - np[1]) + On[3 * k + 2] * (p[2] - np[2]));
 	const float rax[3] = {(float) -pp[13], (float) -pp[14], (float) -pp[15]};
-	Prop pr;
-	prop_decode(S.y + cell * NN_OUT_PAD, pr);
-	const double log_ratio = (double) prop_logq(pr, rbody, rax) - pp[12];
+	PropLane pr;
+	prop_decode_lane(S.y + cell * NN_OUT_PAD, tl, pr);
+	const double log_ratio = (double) prop_logq_lane(pr, rbody, rax) - pp[12];
 	// energy change over the static neighbours and the other members, one
 	// candidate per lane of the team
 	Trial t;
@@ -1082,10 +1141,7 @@ __global__ __launch_bounds__(64 * TS_WAVES) void k_train_samples(DevState d, uin
 	CandLds &CL = Cs[wave];
 	auto cands = [&]() { return Cands{d, F, v, j, &CL}; };
 	if(b < m_pad && !live) {
-		if(lane < NN_IN_PAD / 2) {
-			row[2 * lane] = (__bf16) 0.f;
-			row[2 * lane + 1] = (__bf16) 0.f;
-		}
+		zero_row<64>(row, lane);
 		if(lane < 6) target[(size_t) b * 6 + lane] = 0.f;
 	}
 	if(live) {
