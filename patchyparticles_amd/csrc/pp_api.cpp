@@ -112,6 +112,12 @@ struct pp_ctx {
 	int snap_n = 0;
 	bool snap_gc = false;
 	double snap_box[3] = {0., 0., 0.};
+	// downloads: a replica in index order on the device, two pinned chunks
+	// through which it reaches the caller's memory
+	double *dl_dev = nullptr;  // UNPACK_HEAD + NCOMP x dl_cap
+	char *dl_host = nullptr;   // 2 x DL_CHUNK
+	hipEvent_t dl_ev[2] = {nullptr, nullptr};
+	int dl_cap = 0;
 	int cus = 256;           // compute units of the device
 
 	~pp_ctx() {
@@ -124,6 +130,9 @@ struct pp_ctx {
 		if(h_vslow) (void) hipHostFree(h_vslow);
 		if(snap_host) (void) hipHostFree(snap_host);
 		if(snap_host_pid) (void) hipHostFree(snap_host_pid);
+		if(dl_host) (void) hipHostFree(dl_host);
+		for(hipEvent_t e : dl_ev)
+			if(e) (void) hipEventDestroy(e);
 		if(snap_ready) (void) hipEventDestroy(snap_ready);
 		if(snap_done) (void) hipEventDestroy(snap_done);
 		if(copy_stream) (void) hipStreamDestroy(copy_stream);
@@ -953,15 +962,71 @@ pp_status pp_check_energy(pp_ctx *c, double *energy_per_rep) {
 	return result;
 }
 
+// Download of a replica of fixed size.  The device puts the particles in index
+// order; the copy goes through two pinned chunks, one filled by the copy engine
+// while the host empties the other.  A copy straight into the caller's pageable
+// memory ran at 2.4 GB/s up to 1 MB and 18 GB/s beyond (0.8 MB: 322 us, 12.6 MB:
+// 681 us); this one at 18 and 27 GB/s (44 and 461 us).
+constexpr size_t DL_CHUNK = 1 << 20;
+
+static pp_status download_fixed(pp_ctx *c, int rep, double *r, double *O, double box[3]) {
+	const int n = c->reps[rep].np;
+	if(!c->dl_cap) {
+		// (each piece is kept as it is made; dl_cap is set once all exist)
+		int cap = 1;
+		for(int k = 0; k < c->R; k++) cap = std::max(cap, c->reps[k].np);
+		if(!c->dl_dev) TRY(dev_alloc(c, &c->dl_dev, UNPACK_HEAD + (size_t) NCOMP * cap));
+		for(hipEvent_t &e : c->dl_ev)
+			if(!e) HIPCHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+		if(!c->dl_host && hipHostMalloc((void **) &c->dl_host, 2 * DL_CHUNK, hipHostMallocDefault) != hipSuccess) {
+			c->dl_host = nullptr;
+			return fail(PP_ERR_NOMEM, "pinned download buffer");
+		}
+		c->dl_cap = cap;
+	}
+	launch_unpack(c->d, rep, r || O ? n : 0, c->dl_dev, c->stream);
+	const size_t head = sizeof(double) * UNPACK_HEAD, rb = sizeof(double) * 3 * (size_t) n, ob = 3 * rb;
+	const size_t total = r || O ? head + rb + ob : head, chunks = (total + DL_CHUNK - 1) / DL_CHUNK;
+	const char *dev = (const char *) c->dl_dev;
+	auto fetch = [&](size_t k) -> pp_status {
+		const size_t at = k * DL_CHUNK;
+		HIPCHECK(hipMemcpyAsync(c->dl_host + (k & 1) * DL_CHUNK, dev + at, std::min(DL_CHUNK, total - at),
+		                        hipMemcpyDeviceToHost, c->stream));
+		HIPCHECK(hipEventRecord(c->dl_ev[k & 1], c->stream));
+		return PP_OK;
+	};
+	double bad = 0.;
+	TRY(fetch(0));
+	if(chunks > 1) TRY(fetch(1));
+	for(size_t k = 0; k < chunks; k++) {
+		HIPCHECK(hipEventSynchronize(c->dl_ev[k & 1]));
+		const char *src = c->dl_host + (k & 1) * DL_CHUNK;
+		const size_t lo = k * DL_CHUNK, hi = std::min(total, lo + DL_CHUNK);
+		// the part of this chunk in [from, from + bytes) of the whole
+		auto give = [&](size_t from, size_t bytes, void *to) {
+			const size_t a = std::max(lo, from), b = std::min(hi, from + bytes);
+			if(to && a < b) std::memcpy((char *) to + (a - from), src + (a - lo), b - a);
+		};
+		if(k == 0) {
+			std::memcpy(&bad, src + sizeof(double) * UNPACK_BAD, sizeof bad);
+			if(box) std::memcpy(box, src + sizeof(double) * UNPACK_BOX, 3 * sizeof(double));
+		}
+		give(head, rb, r);
+		give(head + rb, ob, O);
+		if(k + 2 < chunks) TRY(fetch(k + 2));
+	}
+	if(bad != 0.) return fail(PP_ERR_HIP, "corrupt particle index %d", (int) (bad - 1.));
+	return PP_OK;
+}
+
 pp_status pp_download(pp_ctx *c, int rep, double *r, double *O, double box[3]) {
 	if(!c) return fail(PP_ERR_ARG, "ctx is NULL");
 	if(rep < 0 || rep >= c->R) return fail(PP_ERR_ARG, "replica %d out of range", rep);
 	HIPCHECK(hipSetDevice(c->device));
-	if(c->any_gc) {
-		// grand-canonical replicas: their live particles first (a rebuild)
-		rebuild_now(c);
-		HIPCHECK(hipStreamSynchronize(c->stream));
-	}
+	if(!c->reps[rep].gc) return download_fixed(c, rep, r, O, box);
+	// a grand-canonical replica: its live particles first (a rebuild)
+	rebuild_now(c);
+	HIPCHECK(hipStreamSynchronize(c->stream));
 	TRY(pull_reps(c));
 	const Rep &rp = c->reps[rep];
 	const int n = rp.np, off = rp.p_off;
@@ -972,7 +1037,7 @@ pp_status pp_download(pp_ctx *c, int rep, double *r, double *O, double box[3]) {
 		                   hipMemcpyDeviceToHost));
 	TRY(slot_indices(c, rep, hp, sorted));
 	for(int j = 0; j < n; j++) {
-		const int i = rp.gc ? rank_of(sorted, hp[j]) : hp[j];
+		const int i = rank_of(sorted, hp[j]);
 		if(r)
 			for(int a = 0; a < 3; a++) r[3 * i + a] = h[(size_t) NCOMP * j + a];
 		if(O)

@@ -357,5 +357,8 @@ void launch_energy_pairs(const DevState &d, int cus, hipStream_t s);
 // grand-canonical insertions and removals of the sweep (GC replicas only)
 void launch_gc_phase(const DevState &d, uint64_t sweep, hipStream_t s);
 void launch_gram_schmidt(const DevState &d, hipStream_t s);
+// replica rep (np particles, not grand-canonical) in index order: out[UNPACK_HEAD + NCOMP np]
+enum Unpack : int { UNPACK_BOX = 0, UNPACK_BAD = 3, UNPACK_HEAD = 8 };
+void launch_unpack(const DevState &d, int rep, int np, double *out, hipStream_t s);
 
 }  // namespace ppd

@@ -66,3 +66,24 @@ def test_snapshot_misuse_is_refused(pp, oracle):
         s.snapshot_finish()
         with pytest.raises(pp.PPError):
             s.snapshot_start(7)
+
+
+@pytest.mark.parametrize("n", [40, 10921, 10922, 10923, 21844, 21846, 40000])
+def test_download_equals_the_snapshot(pp, n):
+    """A download puts particles in index order on the device and copies them in
+    chunks of 1 MiB; a snapshot orders them on the host.  Sizes at the chunks'
+    edges (8 doubles, then 12 per particle); either array alone."""
+    r, O, box = pp.generate(n, 0.1, 3)
+    with pp.System.batch([r, r], [O, O], [box, box], [dict(T=0.2)] * 2, seed=5) as s:
+        s.do_ensemble(3)
+        for k in (1, 0):
+            s.snapshot_start(k)
+            want = s.snapshot_finish()
+            got = s.state(k)
+            for a, b in zip(got, want):
+                assert np.array_equal(a, b)
+            r1, O1, b1 = np.zeros((n, 3)), np.zeros((n, 3, 3)), np.zeros(3)
+            assert pp.lib().pp_download(s._h, k, r1.ctypes.data, None, None) == 0
+            assert pp.lib().pp_download(s._h, k, None, O1.ctypes.data, None) == 0
+            assert pp.lib().pp_download(s._h, k, None, None, b1.ctypes.data) == 0
+            assert np.array_equal(r1, want[0]) and np.array_equal(O1, want[1]) and np.array_equal(b1, want[2])
