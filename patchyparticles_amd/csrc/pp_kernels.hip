@@ -773,12 +773,23 @@ __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int
 	int *own_pid = (int *) (blk + L::PID);
 	int *nb_tab = (int *) (blk + L::NB);
 
-	// 1. the cell's record: its header, and this lane's neighbour; a record of
-	// another sweep lies past the end of the pass's list
+	// 1. the cell's record: its header, and this lane's neighbours; a record of
+	// another sweep lies past the end of the pass's list.  Everything is read
+	// at once and pinned here: the compiler would move all but the tag behind
+	// the check, one more round trip to memory, and a pass waits for memory
+	// during 60 % of its time when its cells make one trial per member.
 	const int *rec = d.rec + ((size_t) pass * d.total_act + gi) * REC_W;
-	const int4 h0 = ((const int4 *) rec)[0], h1 = ((const int4 *) rec)[1], h2 = ((const int4 *) rec)[2];
-	int cq[CPL];
-	cq[0] = lane < REC_SLOTS ? rec[REC_HEAD + lane] : -1;
+	int4 h0 = ((const int4 *) rec)[0], h1 = ((const int4 *) rec)[1], h2 = ((const int4 *) rec)[2];
+	int e0 = rec[REC_HEAD + min(lane, REC_SLOTS - 1)], e1 = 0;
+	if constexpr(CPL > 1) e1 = rec[REC_HEAD + min(T + lane, REC_SLOTS - 1)];
+	// (not volatile: the scalar loads below stay scalar)
+	asm("" : "+v"(h0.x) : "v"(h0.y), "v"(h0.z), "v"(h0.w), "v"(h1.x), "v"(h1.y), "v"(h1.z), "v"(h2.x), "v"(h2.y), "v"(h2.z), "v"(e0), "v"(e1));
+	if constexpr(ONE) {
+		// (the lines of the replica's constants, into the scalar cache)
+		const Rep &rq = d.reps[0];
+		asm("" : "+v"(h0.x) : "s"(rq.T), "s"(rq.pg.box[0]), "s"(rq.pg.shift[2]), "s"(rq.pg.inv_side[0]), "s"(rq.pg.thr[0]),
+		             "s"(rq.pg.thr[ACC_TAB - 2]));
+	}
 	if(uni<T>(h0.x) != (int) d.rec_tag) return;
 	const int M = uni<T>(h0.y);
 	const int s0 = uni<T>(h0.z);
@@ -818,17 +829,20 @@ __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int
 	const int mi = lane - nstat;      // this lane's member
 	const bool is_mem = mi >= 0;
 	const int nreg = min(M, min(T * CPL - cnt, REC_SLOTS));
-	if(is_mem || lane >= nreg) cq[0] = -1;
-	if constexpr(CPL > 1) cq[1] = nstat + lane < nreg ? rec[REC_HEAD + nstat + lane] : -1;
+	int cq[CPL];
+	cq[0] = is_mem || lane >= nreg ? -1 : e0;
+	if constexpr(CPL > 1) cq[1] = -1;
 	// the lane's member or first static neighbour, in one set of registers
-	// (second slots follow once that one is converted)
-	const int my_pid = is_mem ? PID[s0 + mi] : 0;
+	// (second slots follow once that one is converted).  Lanes without one
+	// read the first member: a load under a condition would be waited for at
+	// its end, before the trials are drawn.
 	double pv[NCOMP];
 	auto load_part = [&](int j) {
 #pragma unroll
 		for(int c = 0; c < NCOMP; c++) pv[c] = nbld<DD>(part(F, j) + c);
 	};
-	if(is_mem || (!DD && cq[0] >= 0)) load_part(is_mem ? s0 + mi : cq[0]);
+	load_part(is_mem ? s0 + mi : (!DD && cq[0] >= 0 ? cq[0] : s0));
+	const int my_pid = PID[s0 + max(mi, 0)];
 	// trials of the cell in this pass: one per member (a sweep is then N
 	// attempts), or a fixed number per non-empty cell
 	const int ntrial = d.trials_per_cell > 0 ? d.trials_per_cell : cnt;
@@ -946,6 +960,10 @@ __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int
 	const bool wave_far = ballot(M > nreg) != 0ull;
 	if constexpr(CPL > 1)
 		if(wave_2) {
+			// (entry nstat + lane of the record's list)
+			const int from = koff + ((nstat + lane) & (T - 1));
+			const int x0 = __shfl(e0, from), x1 = __shfl(e1, from);
+			cq[1] = nstat + lane < nreg ? (nstat + lane < T ? x0 : x1) : -1;
 			empty_slot(1);
 			if(cq[1] >= 0) {
 				double rel[3];
