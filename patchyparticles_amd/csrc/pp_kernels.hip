@@ -171,7 +171,21 @@ __global__ void k_count(DevState d, int mode, uint64_t sweep, long long trace_po
 		c = rp.cell_off + (ix * G.n[1] + iy) * G.n[2] + iz;
 	}
 	d.cellid[j] = c;
-	d.slot[j] = atomicAdd(&d.count[c], 1);
+	// the slots a grand-canonical replica does not use all go to one cell: a
+	// wavefront's together (one by one, 900 of them took 8 us of a 12 us kernel)
+	const bool parked = c == rp.cell_off + rp.cell_cap;
+	for(unsigned long long left = ballot(parked); left != 0ull;) {
+		const int cl = __builtin_amdgcn_readlane(c, (int) __builtin_ctzll(left));
+		const unsigned long long mates = ballot(parked && c == cl);
+		if(parked && c == cl) {
+			const int before = __popcll(mates & ((1ull << (threadIdx.x & 63)) - 1ull));
+			int base = 0;
+			if(before == 0) base = atomicAdd(&d.count[c], __popcll(mates));
+			d.slot[j] = __builtin_amdgcn_readlane(base, (int) __builtin_ctzll(mates)) + before;
+		}
+		left &= ~mates;
+	}
+	if(!parked) d.slot[j] = atomicAdd(&d.count[c], 1);
 }
 
 // (replica, colour) keys of the non-empty-cell lists counted per scan workgroup
