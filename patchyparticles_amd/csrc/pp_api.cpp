@@ -768,17 +768,15 @@ pp_status enqueue_sweep(pp_ctx *c) {
 		if(c->vol_run_ahead && c->d.pl) {
 			// every attempt enqueued on the close-pair list, which serves
 			// every fast trial in the common case; the host then learns once
-			// where, if anywhere, an attempt needed more (k_vol_gate), and
+			// where, if anywhere, an attempt needed more (attempt_stopped), and
 			// goes on from that attempt's standing proposal as below
 			for(int k = 0; k < nvol; k++) {
 				hipEvent_t v{};
 				tic(c, TK_VOLUME, &v);
 				launch_vol_propose(c->d, sw, k, c->stream);
-				launch_vol_gate(c->d, k, c->stream);
-				launch_energy_rows_zero(c->d, c->stream);
-				launch_energy_pairs(c->d, c->cus, c->stream);
-				launch_vol_decide(c->d, sw, k, c->stream);
-				launch_vol_apply(c->d, c->stream);
+				launch_energy_pairs(c->d, c->cus, 1, c->stream);
+				launch_vol_decide(c->d, sw, k, 1, c->stream);
+				launch_vol_apply(c->d, k, 1, c->stream);
 				toc(c, TK_VOLUME, v);
 			}
 			const unsigned seq = (++c->vol_seq) & 0x7FFFFFu;
@@ -802,11 +800,10 @@ pp_status enqueue_sweep(pp_ctx *c) {
 			TRY(wait_published(c, 0, 4, seq, &need));
 			if(need & NEED_REBUILD) launch_rebuild(c->d, REB_TRIAL, sw, -1, c->stream);
 			if(need & NEED_PARTICLES) launch_energy(c->d, 1, 0, c->stream);
-			else launch_energy_rows_zero(c->d, c->stream);
 			if(need & NEED_RECORDS) launch_energy_rec(c->d, c->cus, c->stream);
-			if(need & NEED_PAIRS) launch_energy_pairs(c->d, c->cus, c->stream);
-			launch_vol_decide(c->d, sw, k, c->stream);
-			launch_vol_apply(c->d, c->stream);
+			if(need & NEED_PAIRS) launch_energy_pairs(c->d, c->cus, 0, c->stream);
+			launch_vol_decide(c->d, sw, k, 0, c->stream);
+			launch_vol_apply(c->d, k, 0, c->stream);
 			toc(c, TK_VOLUME, v);
 		}
 	}

@@ -320,14 +320,15 @@ constexpr size_t MAX_LDS_BYTES = 65536;
 constexpr int MAX_TEAMS = 6;  // cells one pass workgroup may work on
 void launch_energy(const DevState &d, int trial, int per_particle, hipStream_t s);
 void launch_bond_list(const DevState &d, int max_per, int *count, int *partners, hipStream_t s);
-// volume-move attempt k of sweep `sweep` (NPT replicas only)
+// volume-move attempt k of sweep `sweep` (NPT replicas only); clears the energy rows
 void launch_vol_propose(const DevState &d, uint64_t sweep, int k, hipStream_t s);
 // write (seq << 4) | the TrialNeed bits of the attempt just proposed into the
 // host's pinned word (host_word: its device address); seq < 2^27
 void launch_vol_publish(const DevState &d, int *host_word, unsigned seq, hipStream_t s);
-void launch_vol_decide(const DevState &d, uint64_t sweep, int k, hipStream_t s);
-// rescale the positions of replicas whose fast trial was accepted
-void launch_vol_apply(const DevState &d, hipStream_t s);
+// (ahead: the attempt stops unless the close-pair list serves every trial)
+void launch_vol_decide(const DevState &d, uint64_t sweep, int k, int ahead, hipStream_t s);
+// rescale the positions of replicas whose fast trial was accepted; the end of attempt k
+void launch_vol_apply(const DevState &d, int k, int ahead, hipStream_t s);
 // the energy of the box trials whose replicas take it from the cell records
 // (trial_rec), one listed cell per team; `cus` sizes the grid
 void launch_energy_rec(const DevState &d, int cus, hipStream_t s);
@@ -338,10 +339,8 @@ void launch_colour_conflicts(const DevState &d, int rep, int slots, const int *n
                              hipStream_t s);
 // zero the energy rows (C_EBONDS, C_OVL) of every replica
 void launch_energy_rows_zero(const DevState &d, hipStream_t s);
-// run-ahead box attempts: stop the sequence at attempt k when it needs more
-// than the close-pair list; report the stop (attempt + 1, 0 for none) with
-// `seq` into the host's pinned word and clear it
-void launch_vol_gate(const DevState &d, int k, hipStream_t s);
+// the end of run-ahead box attempts: report where they stopped (attempt + 1, 0
+// for nowhere) with `seq` into the host's pinned word and clear it
 void launch_vol_report(const DevState &d, int *host_word, unsigned seq, hipStream_t s);
 // the trial-energy paths a box attempt needs, as the host reads them from
 // vslow after k_vol_propose: a trial rebuild, the per-particle trial energy,
@@ -350,10 +349,10 @@ enum TrialNeed : int { NEED_REBUILD = 1, NEED_PARTICLES = 2, NEED_RECORDS = 4, N
 // the close-pair list keeps the pairs of adjacent cells closer than
 // PAIR_LIST_FACTOR bond ranges at its build
 constexpr double PAIR_LIST_FACTOR = 1.1;
-// build the sweep's close-pair list (and reset the replicas' pair state)
+// build the sweep's close-pair list (and set the replicas' pair state)
 void launch_pairs_build(const DevState &d, int cus, hipStream_t s);
 // the energy of the box trials that take it from the close-pair list
-void launch_energy_pairs(const DevState &d, int cus, hipStream_t s);
+void launch_energy_pairs(const DevState &d, int cus, int ahead, hipStream_t s);
 // grand-canonical insertions and removals of the sweep (GC replicas only)
 void launch_gc_phase(const DevState &d, uint64_t sweep, hipStream_t s);
 void launch_gram_schmidt(const DevState &d, hipStream_t s);

@@ -47,10 +47,8 @@ void launch_fill_u64(unsigned long long *p, unsigned long long v, long long n, h
 	hipLaunchKernelGGL(k_fill_u64, dim3((unsigned) ((n + 255) / 256)), dim3(256), 0, s, p, v, n);
 }
 
-// Zero the energy-kernel rows (C_EBONDS, C_OVL) of every replica (nothing
-// once a run-ahead sequence of box attempts has stopped: *stop >= 0).
-__global__ void k_zero_energy_rows(unsigned long long *ctr, int R, const int *stop) {
-	if(stop && *stop >= 0) return;
+// Zero the energy-kernel rows (C_EBONDS, C_OVL) of every replica.
+__global__ void k_zero_energy_rows(unsigned long long *ctr, int R) {
 	int i = blockIdx.x * blockDim.x + threadIdx.x;
 	if(i >= R * 2 * NSLOT) return;
 	int r = i / (2 * NSLOT), k = i % (2 * NSLOT);
@@ -117,6 +115,11 @@ __global__ void k_count(DevState d, int mode, uint64_t sweep, long long trace_po
 	for(int t = j; t < d.R * 8; t += gridDim.x * blockDim.x) d.ccount[t] = 0;
 	if(j == 0) {
 		d.scan_ticket[0] = 0;
+		if(mode == REB_SHIFT && d.pl_n) {
+			// the sweep's list of close pairs, built after its passes
+			d.pl_n[0] = 0;
+			d.pl_n[1] = 0;
+		}
 	}
 	if(mode == REB_TRIAL)
 		// replicas without a trial rebuild keep their lists as they are:
@@ -787,23 +790,30 @@ __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int
 	int *own_pid = (int *) (blk + L::PID);
 	int *nb_tab = (int *) (blk + L::NB);
 
-	// 1. the cell's record: its header, and this lane's neighbours; a record of
-	// another sweep lies past the end of the pass's list.  Everything is read
-	// at once and pinned here: the compiler would move all but the tag behind
-	// the check, one more round trip to memory, and a pass waits for memory
-	// during 60 % of its time when its cells make one trial per member.
+	// 1. the cell's record: its header, and this lane's neighbour; a record of
+	// another sweep lies past the end of the pass's list.
+	// One replica (ONE): few wavefronts, which wait for memory during 60 % of a
+	// pass when cells make one trial per member.  Everything is then read at
+	// once and pinned here: the compiler would move all but the tag behind the
+	// check, one more round trip (N=32768: 11.6 -> 11.3 us; N=65536 at rho 0.3
+	// with 16 lanes 12.8 -> 12.0).  A batch's many wavefronts hide that round
+	// trip, and pay for the second slots' line and the idle lanes' loads (16 x
+	// 131072 at rho 0.05: 830 -> 869 us).
 	const int *rec = d.rec + ((size_t) pass * d.total_act + gi) * REC_W;
 	int4 h0 = ((const int4 *) rec)[0], h1 = ((const int4 *) rec)[1], h2 = ((const int4 *) rec)[2];
-	int e0 = rec[REC_HEAD + min(lane, REC_SLOTS - 1)], e1 = 0;
-	if constexpr(CPL > 1) e1 = rec[REC_HEAD + min(T + lane, REC_SLOTS - 1)];
-	// (not volatile: the scalar loads below stay scalar)
-	asm("" : "+v"(h0.x) : "v"(h0.y), "v"(h0.z), "v"(h0.w), "v"(h1.x), "v"(h1.y), "v"(h1.z), "v"(h2.x), "v"(h2.y), "v"(h2.z), "v"(e0), "v"(e1));
+	int e0, e1 = 0;
 	if constexpr(ONE) {
-		// (the lines of the replica's constants, into the scalar cache)
+		e0 = rec[REC_HEAD + min(lane, REC_SLOTS - 1)];
+		if constexpr(CPL > 1) e1 = rec[REC_HEAD + min(T + lane, REC_SLOTS - 1)];
+		// (not volatile: the scalar loads below stay scalar; the second
+		// statement brings the lines of the replica's constants into the
+		// scalar cache)
 		const Rep &rq = d.reps[0];
+		asm("" : "+v"(h0.x) : "v"(h0.y), "v"(h0.z), "v"(h0.w), "v"(h1.x), "v"(h1.y), "v"(h1.z), "v"(h2.x), "v"(h2.y), "v"(h2.z), "v"(e0), "v"(e1));
 		asm("" : "+v"(h0.x) : "s"(rq.T), "s"(rq.pg.box[0]), "s"(rq.pg.shift[2]), "s"(rq.pg.inv_side[0]), "s"(rq.pg.thr[0]),
 		             "s"(rq.pg.thr[ACC_TAB - 2]));
 	}
+	else e0 = lane < REC_SLOTS ? rec[REC_HEAD + lane] : -1;
 	if(uni<T>(h0.x) != (int) d.rec_tag) return;
 	const int M = uni<T>(h0.y);
 	const int s0 = uni<T>(h0.z);
@@ -845,18 +855,20 @@ __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int
 	const int nreg = min(M, min(T * CPL - cnt, REC_SLOTS));
 	int cq[CPL];
 	cq[0] = is_mem || lane >= nreg ? -1 : e0;
-	if constexpr(CPL > 1) cq[1] = -1;
+	// (ONE finds the second slots' entries among the lanes, when it needs them)
+	if constexpr(CPL > 1) cq[1] = !ONE && nstat + lane < nreg ? rec[REC_HEAD + nstat + lane] : -1;
 	// the lane's member or first static neighbour, in one set of registers
-	// (second slots follow once that one is converted).  Lanes without one
-	// read the first member: a load under a condition would be waited for at
-	// its end, before the trials are drawn.
+	// (second slots follow once that one is converted).  ONE: lanes without one
+	// read the first member, since a load under a condition would be waited for
+	// at its end, before the trials are drawn.
 	double pv[NCOMP];
 	auto load_part = [&](int j) {
 #pragma unroll
 		for(int c = 0; c < NCOMP; c++) pv[c] = nbld<DD>(part(F, j) + c);
 	};
-	load_part(is_mem ? s0 + mi : (!DD && cq[0] >= 0 ? cq[0] : s0));
-	const int my_pid = PID[s0 + max(mi, 0)];
+	int my_pid = 0;
+	if(ONE || is_mem) my_pid = PID[s0 + max(mi, 0)];
+	if(ONE || is_mem || (!DD && cq[0] >= 0)) load_part(is_mem ? s0 + mi : (!DD && cq[0] >= 0 ? cq[0] : s0));
 	// trials of the cell in this pass: one per member (a sweep is then N
 	// attempts), or a fixed number per non-empty cell
 	const int ntrial = d.trials_per_cell > 0 ? d.trials_per_cell : cnt;
@@ -974,10 +986,12 @@ __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int
 	const bool wave_far = ballot(M > nreg) != 0ull;
 	if constexpr(CPL > 1)
 		if(wave_2) {
-			// (entry nstat + lane of the record's list)
-			const int from = koff + ((nstat + lane) & (T - 1));
-			const int x0 = __shfl(e0, from), x1 = __shfl(e1, from);
-			cq[1] = nstat + lane < nreg ? (nstat + lane < T ? x0 : x1) : -1;
+			if constexpr(ONE) {
+				// (entry nstat + lane of the record's list)
+				const int from = koff + ((nstat + lane) & (T - 1));
+				const int x0 = __shfl(e0, from), x1 = __shfl(e1, from);
+				cq[1] = nstat + lane < nreg ? (nstat + lane < T ? x0 : x1) : -1;
+			}
 			empty_slot(1);
 			if(cq[1] >= 0) {
 				double rel[3];
@@ -1712,8 +1726,7 @@ void launch_bond_list(const DevState &d, int max_per, int *count, int *partners,
 }
 
 void launch_energy_rows_zero(const DevState &d, hipStream_t s) {
-	hipLaunchKernelGGL(k_zero_energy_rows, dim3((d.R * 2 * NSLOT + 255) / 256), dim3(256), 0, s, d.ctr, d.R,
-	                   (const int *) (d.vslow ? d.vslow + 1 : nullptr));
+	hipLaunchKernelGGL(k_zero_energy_rows, dim3((d.R * 2 * NSLOT + 255) / 256), dim3(256), 0, s, d.ctr, d.R);
 }
 
 // Lanes per particle: 32 where the 27 cells hold many candidates, 8 in dilute
@@ -1851,16 +1864,94 @@ void launch_energy_rec(const DevState &d, int cus, hipStream_t s) {
 
 // Which replicas list their pairs this sweep (box trials on current lists
 // whose records were written by this sweep's rebuild), and an empty list.
-__global__ void k_pairs_reset(DevState d) {
-	const int r = blockIdx.x * blockDim.x + threadIdx.x;
-	if(r == 0) {
-		d.pl_n[0] = 0;
-		d.pl_n[1] = 0;
+__device__ __forceinline__ bool lists_pairs(const Rep &rp) {
+	return (rp.ensemble == 5 || rp.lx_move) && rp.rec_ok && rp.lists_ok;
+}
+
+// The replicas' pair state at the start of the sweep's box trials, by the
+// building kernel's first workgroup (the rebuild has emptied the list).
+__device__ __forceinline__ void pairs_reset(const DevState &d) {
+	if(blockIdx.x != 0) return;
+	for(int r = threadIdx.x; r < d.R; r += blockDim.x) {
+		Rep &rp = d.reps[r];
+		rp.pl_ok = lists_pairs(rp) ? 1 : 0;
+		rp.pl_scale[0] = rp.pl_scale[1] = rp.pl_scale[2] = 1.;
 	}
-	if(r >= d.R) return;
-	Rep &rp = d.reps[r];
-	rp.pl_ok = ((rp.ensemble == 5 || rp.lx_move) && rp.rec_ok && rp.lists_ok) ? 1 : 0;
-	rp.pl_scale[0] = rp.pl_scale[1] = rp.pl_scale[2] = 1.;
+}
+
+// Few cells: 16 lanes per listed cell share its pairs, and remember those they
+// found close (a bit per step) while the workgroup reserves its places with
+// one atomic.  A lane per cell walks a cell's pairs one after the other, two
+// dependent loads each, twice: 28 us for N=1331 at rho 0.3, this 5.7.
+__global__ __launch_bounds__(256) void k_pairs_build_team(DevState d) {
+	constexpr int T = 16;
+	__shared__ int wsum[4], base;
+	pairs_reset(d);
+	const int tl = threadIdx.x & (T - 1), lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+	int lens[8];
+	int total = 0;
+#pragma unroll
+	for(int p = 0; p < 8; p++) {
+		lens[p] = d.pfx[p * (d.R + 1) + d.R];
+		total += lens[p];
+	}
+	for(int g0 = blockIdx.x * (256 / T); g0 < total; g0 += gridDim.x * (256 / T)) {
+		const int i0 = g0 + threadIdx.x / T;
+		const int *rec = d.rec;
+		int s0 = 0, cnt = 0, m0 = 0, m2 = 0, work = 0;
+		const double *F = d.f[0];
+		double L[3] = {1., 1., 1.}, iL[3] = {1., 1., 1.}, rl2 = 0.;
+		if(i0 < total) {
+			int p = 0, gi = i0;
+			while(gi >= lens[p]) gi -= lens[p++];
+			rec = d.rec + ((size_t) p * d.total_act + gi) * REC_W;
+			const Rep &rp = d.reps[rec[REC_REP]];
+			s0 = rec[REC_S0];
+			cnt = rec[REC_CNT];
+			m0 = rec[REC_M0];
+			m2 = rec[REC_M] - m0;
+			F = pick_buf(d.f, rec[REC_SEL]);
+			for(int a = 0; a < 3; a++) {
+				L[a] = rp.g.box[a];
+				iL[a] = rp.g.inv_box[a];
+			}
+			rl2 = rp.rc2 * (PAIR_LIST_FACTOR * PAIR_LIST_FACTOR);
+			if(lists_pairs(rp)) work = cnt * m2 + cnt * cnt;
+		}
+		// pair e, if it is one and close (bits: the first 32 steps' results)
+		auto close = [&](int e, int &j, int &q) {
+			if(!rec_pair(d, rec, s0, cnt, m0, m2, e, j, q)) return false;
+			const double dx = kf_min_image(part(F, q)[0] - part(F, j)[0], L[0], iL[0]);
+			const double dy = kf_min_image(part(F, q)[1] - part(F, j)[1], L[1], iL[1]);
+			const double dz = kf_min_image(part(F, q)[2] - part(F, j)[2], L[2], iL[2]);
+			return dx * dx + dy * dy + dz * dz < rl2;
+		};
+		int n = 0, j, q;
+		unsigned bits = 0;
+		for(int e = tl, k = 0; e < work; e += T, k++)
+			if(close(e, j, q)) {
+				n++;
+				if(k < 32) bits |= 1u << k;
+			}
+		const int incl = wave_incl_scan(n);
+		if(lane == 63) wsum[wave] = incl;
+		__syncthreads();
+		const int tot = wsum[0] + wsum[1] + wsum[2] + wsum[3];
+		if(threadIdx.x == 0) base = tot > 0 ? atomicAdd(d.pl_n, tot) : 0;
+		__syncthreads();
+		int pos = base + incl - n;
+		for(int w = 0; w < wave; w++) pos += wsum[w];
+		if(base + tot > d.pl_cap) {
+			if(threadIdx.x == 0) d.pl_n[1] = 1;
+		}
+		else
+			for(int e = tl, k = 0; e < work; e += T, k++) {
+				if(k < 32 ? !((bits >> k) & 1u) : !close(e, j, q)) continue;
+				rec_pair(d, rec, s0, cnt, m0, m2, e, j, q);
+				d.pl[pos++] = make_int2(j, q);
+			}
+		__syncthreads();  // (wsum and base are written again)
+	}
 }
 
 // One lane per listed cell, the wavefront's lanes in step: each counts its
@@ -1869,6 +1960,7 @@ __global__ void k_pairs_reset(DevState d) {
 // list that would pass pl_cap is marked as overflowed; the trials then take
 // their energy from the records.
 __global__ __launch_bounds__(256) void k_pairs_build(DevState d) {
+	pairs_reset(d);
 	const int lane = threadIdx.x & 63;
 	const int wave = (xcd_remap(blockIdx.x, gridDim.x) * blockDim.x + (int) threadIdx.x) >> 6;
 	const int waves = gridDim.x * (blockDim.x >> 6);
@@ -1891,7 +1983,7 @@ __global__ __launch_bounds__(256) void k_pairs_build(DevState d) {
 			while(gi >= lens[p]) gi -= lens[p++];
 			rec = d.rec + ((size_t) p * d.total_act + gi) * REC_W;
 			const Rep &rp = d.reps[rec[REC_REP]];
-			on = rp.pl_ok != 0;
+			on = lists_pairs(rp);
 			if(on) {
 				s0 = rec[REC_S0];
 				cnt = rec[REC_CNT];
@@ -1937,16 +2029,37 @@ __global__ __launch_bounds__(256) void k_pairs_build(DevState d) {
 }
 
 void launch_pairs_build(const DevState &d, int cus, hipStream_t s) {
-	hipLaunchKernelGGL(k_pairs_reset, dim3((unsigned) ((d.R + 255) / 256)), dim3(256), 0, s, d);
+	// 16 lanes per cell while a lane per cell (at most one cell per particle)
+	// would leave the chip idle, and where cells have many pairs; big dilute
+	// systems, about one pair per cell, take a lane.  16 lanes / one lane, us:
+	// N=60000 at rho 0.3 46 / 361, 120000 at 0.05 75 / 86, 400000 at 0.3 295 /
+	// 691, at 0.1 291 / 224, 10^6 at 0.15 725 / 593, 2.1 10^6 at 0.05 1316 / 437.
+	if(d.Ntot < cus * 512 || 27. * d.Ntot >= 6. * d.C_total) {
+		const int blocks = std::max(1, std::min((d.Ntot + 15) / 16, cus * 8));
+		hipLaunchKernelGGL(k_pairs_build_team, dim3((unsigned) blocks), dim3(256), 0, s, d);
+		return;
+	}
 	const int blocks = std::max(8, cus * 8) & ~7;
 	hipLaunchKernelGGL(k_pairs_build, dim3((unsigned) blocks), dim3(256), 0, s, d);
+}
+
+// Run-ahead box attempts (ahead: enqueued without the host reading each
+// attempt's paths): an attempt proceeds on the close-pair list alone, which
+// serves every fast trial in the common case; if some replica's trial needs
+// more, the sequence stops there: the kernels of this and the later attempts
+// leave at once, the proposal stays in place and its paths stay in vslow[0]
+// for the host to take over from.  The attempt's own kernels read that from
+// vslow[0]; its last one (k_vol_apply) marks the stop in vslow[1] before a
+// later proposal could add to it.
+__device__ __forceinline__ bool attempt_stopped(const DevState &d, int ahead) {
+	return d.vslow[1] >= 0 || (ahead && (d.vslow[0] & ~(int) NEED_PAIRS));
 }
 
 // The trial energies from the close-pair list: one lane per pair, the
 // separation and the bond decision as k_energy_rec forms them; a bonded pair
 // adds 2 to the bond rows, an overlapping pair 1 to the overlap row.
-__global__ __launch_bounds__(256) void k_energy_pairs(DevState d) {
-	if(d.vslow[1] >= 0) return;  // a run-ahead sequence of attempts stopped
+__global__ __launch_bounds__(256) void k_energy_pairs(DevState d, int ahead) {
+	if(attempt_stopped(d, ahead)) return;
 	const int n = min(d.pl_n[0], d.pl_cap);
 	const int stride = gridDim.x * blockDim.x;
 	for(int k = xcd_remap(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x; k < n; k += stride) {
@@ -1985,9 +2098,9 @@ __global__ __launch_bounds__(256) void k_energy_pairs(DevState d) {
 	}
 }
 
-void launch_energy_pairs(const DevState &d, int cus, hipStream_t s) {
+void launch_energy_pairs(const DevState &d, int cus, int ahead, hipStream_t s) {
 	const int blocks = std::max(8, cus * 8) & ~7;
-	hipLaunchKernelGGL(k_energy_pairs, dim3((unsigned) blocks), dim3(256), 0, s, d);
+	hipLaunchKernelGGL(k_energy_pairs, dim3((unsigned) blocks), dim3(256), 0, s, d, ahead);
 }
 
 // ------------------------------------------------------------------------
@@ -2078,9 +2191,14 @@ __device__ __forceinline__ void choose_trial_path(const DevState &d, Rep &rp, co
 	                       : (int) (NEED_REBUILD | NEED_PARTICLES));
 }
 
-__global__ void k_vol_propose(DevState d, uint64_t sweep, int k) {
-	int r = blockIdx.x * blockDim.x + threadIdx.x;
-	if(r >= d.R || d.vslow[1] >= 0) return;
+// One wavefront per replica; its lanes also clear the replica's energy rows for
+// the trial energies.
+__global__ __launch_bounds__(64) void k_vol_propose(DevState d, uint64_t sweep, int k) {
+	const int r = blockIdx.x;
+	if(d.vslow[1] >= 0) return;
+	*ctr_at(d.ctr, r, C_EBONDS, threadIdx.x) = 0ull;
+	*ctr_at(d.ctr, r, C_OVL, threadIdx.x) = 0ull;
+	if(threadIdx.x != 0) return;
 	Rep &rp = d.reps[r];
 	rp.trial_active = 0;
 	rp.trial_fast = 0;
@@ -2162,20 +2280,6 @@ void launch_vol_publish(const DevState &d, int *host_word, unsigned seq, hipStre
 	hipLaunchKernelGGL(k_vol_publish, dim3(1), dim3(64), 0, s, d, host_word, seq);
 }
 
-// Run-ahead box attempts (enqueued without the host reading each attempt's
-// paths): attempt k proceeds on the close-pair list alone, which serves
-// every fast trial in the common case; if some replica's trial needs more,
-// the sequence stops here (vslow[1] = k), and the kernels of this and the
-// later attempts leave at once: the attempt's proposal stays in place and
-// its paths stay in vslow[0] for the host to take over from.
-__global__ void k_vol_gate(DevState d, int k) {
-	if(threadIdx.x == 0 && d.vslow[1] < 0 && (d.vslow[0] & ~(int) NEED_PAIRS)) d.vslow[1] = k;
-}
-
-void launch_vol_gate(const DevState &d, int k, hipStream_t s) {
-	hipLaunchKernelGGL(k_vol_gate, dim3(1), dim3(64), 0, s, d, k);
-}
-
 // The end of a run-ahead sequence: where it stopped (attempt + 1, 0 if it
 // ran through) with the host's sequence number into the pinned word; the
 // stop is cleared for the attempts that follow.
@@ -2193,20 +2297,23 @@ void launch_vol_report(const DevState &d, int *host_word, unsigned seq, hipStrea
 }
 
 void launch_vol_propose(const DevState &d, uint64_t sweep, int k, hipStream_t s) {
-	hipLaunchKernelGGL(k_vol_propose, dim3((d.R + 63) / 64), dim3(64), 0, s, d, sweep, k);
+	static_assert(NSLOT == 64, "a lane per slot");
+	hipLaunchKernelGGL(k_vol_propose, dim3(d.R), dim3(64), 0, s, d, sweep, k);
 }
 
-__global__ void k_vol_decide(DevState d, uint64_t sweep, int k) {
-	int r = blockIdx.x * blockDim.x + threadIdx.x;
-	if(r >= d.R || d.vslow[1] >= 0) return;
+// One wavefront per replica, a lane per counter slot.
+__global__ __launch_bounds__(64) void k_vol_decide(DevState d, uint64_t sweep, int k, int ahead) {
+	const int r = blockIdx.x;
 	Rep &rp = d.reps[r];
-	if(!rp.trial_active) return;
-	unsigned long long eb = 0, ov = 0, db = 0;
-	for(int s = 0; s < NSLOT; s++) {
-		eb += *ctr_at(d.ctr, r, C_EBONDS, s);
-		ov += *ctr_at(d.ctr, r, C_OVL, s);
-		db += *ctr_at(d.ctr, r, C_DBONDS, s);
+	unsigned long long eb = *ctr_at(d.ctr, r, C_EBONDS, threadIdx.x), ov = *ctr_at(d.ctr, r, C_OVL, threadIdx.x),
+	                   db = *ctr_at(d.ctr, r, C_DBONDS, threadIdx.x);
+	if(attempt_stopped(d, ahead) || !rp.trial_active) return;
+	for(int o = 32; o > 0; o >>= 1) {
+		eb += __shfl_xor(eb, o);
+		ov += __shfl_xor(ov, o);
+		db += __shfl_xor(db, o);
 	}
+	if(threadIdx.x != 0) return;
 	const long long B1 = (long long) eb / 2;
 	const long long B0 = rp.bonds_base + (long long) db;
 	const double dE = (double) (B0 - B1);  // E' - E with E = -bonds
@@ -2247,16 +2354,20 @@ __global__ void k_vol_decide(DevState d, uint64_t sweep, int k) {
 	rp.trial_active = 0;
 }
 
-void launch_vol_decide(const DevState &d, uint64_t sweep, int k, hipStream_t s) {
-	hipLaunchKernelGGL(k_vol_decide, dim3((d.R + 63) / 64), dim3(64), 0, s, d, sweep, k);
+void launch_vol_decide(const DevState &d, uint64_t sweep, int k, int ahead, hipStream_t s) {
+	hipLaunchKernelGGL(k_vol_decide, dim3(d.R), dim3(64), 0, s, d, sweep, k, ahead);
 }
 
 // The accepted fast trials: every position component times its trial scale,
 // as the trial rebuild writes it (x * 1 is x).  Clears the trial paths for
-// the next attempt.
-__global__ void k_vol_apply(DevState d) {
+// the next attempt, or marks where a run-ahead sequence stopped; either way
+// the other workgroups find the same answer before and after.
+__global__ void k_vol_apply(DevState d, int k, int ahead) {
 	const int j = blockIdx.x * blockDim.x + threadIdx.x;
-	if(d.vslow[1] >= 0) return;  // a run-ahead sequence of attempts stopped
+	if(attempt_stopped(d, ahead)) {
+		if(j == 0 && d.vslow[1] < 0) d.vslow[1] = k;
+		return;
+	}
 	if(j == 0) *d.vslow = 0;
 	if(j >= d.Ntot) return;
 	const Rep &rp = d.reps[d.prep[j]];
@@ -2265,8 +2376,8 @@ __global__ void k_vol_apply(DevState d) {
 	for(int c = 0; c < 3; c++) part(F, j)[c] *= rp.trial_s[c];
 }
 
-void launch_vol_apply(const DevState &d, hipStream_t s) {
-	hipLaunchKernelGGL(k_vol_apply, dim3((unsigned) std::max(1, (d.Ntot + 255) / 256)), dim3(256), 0, s, d);
+void launch_vol_apply(const DevState &d, int k, int ahead, hipStream_t s) {
+	hipLaunchKernelGGL(k_vol_apply, dim3((unsigned) std::max(1, (d.Ntot + 255) / 256)), dim3(256), 0, s, d, k, ahead);
 }
 
 // ------------------------------------------------------------------------

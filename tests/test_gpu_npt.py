@@ -95,3 +95,13 @@ def test_box_trials_on_current_lists_keep_the_trajectory(pp, oracle, monkeypatch
         b, ov, tot, anyo = fast[2][k]
         ob, oov, otot = oracle.energy(rr, OO, bb)
         assert np.array_equal(b, ob) and not anyo and tot == otot == c["bonds"][k], k
+
+
+@pytest.mark.parametrize("n, rho", [(60000, 0.3), (140000, 0.05)])
+def test_pair_list_of_large_systems(pp, monkeypatch, n, rho):
+    """The two forms of the list's build: 16 lanes per cell, here more cells
+    than one round of its workgroups takes, and a lane per cell of a big dilute
+    system; either gives the records' trajectory."""
+    r, O, box = pp.generate(n, rho, 7)
+    make = lambda: pp.System(r, O, box, T=0.2, P=0.2, rescale_factor_max=1e-3, seed=3, trials_per_cell=2, **NPT)
+    _same_runs(_run(pp, monkeypatch, "records", make, 4), _run(pp, monkeypatch, "pairs", make, 4))
