@@ -79,7 +79,6 @@ constexpr float NN_LK_MAX = 8.0f;
 struct NetDev {
 	float *w, *b;
 	float *mw, *vw, *mb, *vb;
-	float *gw, *gb;
 	__bf16 *frag, *fragT;
 };
 
@@ -300,8 +299,8 @@ void launch_passes_dd(const DevState &d, uint64_t sweep, unsigned mark, int T, i
 void launch_learned_pass(const DevState &d, const NetDev &net, uint64_t sweep, int pass, hipStream_t s);
 void launch_net_forward(const NetDev &net, const float *x, int m, float *y, hipStream_t s);
 void launch_net_pack(const NetDev &net, hipStream_t s);
-// loss of each of m rows and the gradients of their mean into net.gw / net.gb
-void launch_net_loss_grad(const NetDev &net, const float *x, const float *target, int m, const NetScratch &q,
+// loss of each of m rows (q.loss) and the gradients of their mean: out[NN_W + NN_B]
+void launch_net_loss_grad(const NetDev &net, const float *x, const float *target, int m, const NetScratch &q, float *out,
                           hipStream_t s);
 // a training step on m samples (x: BF16 rows): losses and the gradients'
 // partial sums, then the step itself

@@ -569,12 +569,9 @@ __device__ __forceinline__ float slice_sum(const float *part, int slices, int e)
 	return g;
 }
 
-__global__ void k_net_reduce(const float *part, int slices, float *gw, float *gb) {
+__global__ void k_net_reduce(const float *part, int slices, float *out) {
 	const int e = blockIdx.x * blockDim.x + threadIdx.x;
-	if(e >= NN_G) return;
-	const float g = slice_sum(part, slices, e);
-	if(e < NN_W) gw[e] = g;
-	else gb[e - NN_W] = g;
+	if(e < NN_G) out[e] = slice_sum(part, slices, e);
 }
 
 // BF16 operand fragments of W (forward) and W^T (backward): those of weight e.
@@ -629,11 +626,11 @@ static void net_grad(const NetDev &net, const X *x, const float *target, int m, 
 	                   (const __bf16 *) q.at, (const __bf16 *) q.zt, m_pad, q.part);
 }
 
-void launch_net_loss_grad(const NetDev &net, const float *x, const float *target, int m, const NetScratch &q,
+void launch_net_loss_grad(const NetDev &net, const float *x, const float *target, int m, const NetScratch &q, float *out,
                           hipStream_t s) {
 	net_grad(net, x, target, m, q, s);
 	hipLaunchKernelGGL(k_net_reduce, dim3((NN_G + 255) / 256), dim3(256), 0, s, (const float *) q.part,
-	                   net_grad_slices((m + 31) & ~31), net.gw, net.gb);
+	                   net_grad_slices((m + 31) & ~31), out);
 }
 
 void launch_net_train(const NetDev &net, const __bf16 *x, const float *target, int m, const NetScratch &q, hipStream_t s) {

@@ -15,6 +15,9 @@ struct pp_net {
 	__bf16 *x = nullptr;                                // training samples
 	float *xh = nullptr, *y = nullptr, *target = nullptr;  // a caller's rows, their outputs, the targets
 	ppd::NetScratch q{};
+	// pinned: the gradients (NN_W + NN_B) and the rows' losses of a loss_grad
+	// call, which its kernels write straight into host memory
+	float *h_out = nullptr, *d_h_out = nullptr;  // host and device address
 	std::vector<void *> allocs;
 	~pp_net();
 };
