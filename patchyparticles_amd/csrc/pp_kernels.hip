@@ -106,6 +106,56 @@ __device__ __forceinline__ void set_pass_geo(Rep &rp, const Grid &G, const doubl
 	for(int k = 0; k < 3; k++) p.n[k] = G.n[k];
 }
 
+// The start of a sweep (REB_SHIFT) in a replica's table: the grid shift, the
+// colour order and the passes' constants.
+__device__ __forceinline__ void begin_sweep(const DevState &d, Rep &rp, int r, uint64_t sweep, const double sh[3]) {
+	for(int k = 0; k < 3; k++) rp.g.shift[k] = sh[k];
+	// random colour order of this sweep's 8 passes
+	u32x4 v = rng(d.seed, r, sweep, 0, TAG_COLOUR, 0, 0);
+	const uint32_t w4[4] = {v.x, v.y, v.z, v.w};
+	rp.col_perm = colour_perm_from(w4);
+	set_pass_geo(rp, rp.g, sh);
+}
+
+// The lists a rebuild of the current state (not a trial) makes are by
+// membership in the grid of shift sh.
+__device__ __forceinline__ void begin_lists(Rep &rp, int mode, const double sh[3]) {
+	rp.lg = rp.g;
+	for(int k = 0; k < 3; k++) rp.lg.shift[k] = sh[k];
+	rp.lists_ok = 1;
+	rp.rec_ok = mode == REB_SHIFT;  // only that rebuild writes the cell records
+}
+
+// Empty what is collected anew in a sweep.
+__device__ __forceinline__ void reset_sweep_lists(const DevState &d, int mode) {
+	d.scan_ticket[0] = 0;
+	if(mode == REB_SHIFT && d.pl_n) {
+		// the sweep's list of close pairs, built after its passes
+		d.pl_n[0] = 0;
+		d.pl_n[1] = 0;
+	}
+}
+
+// The place of a slot in cell c, counted in `count`.  The slots a
+// grand-canonical replica does not use all go to one cell (parked): a
+// wavefront's together (one by one, 900 of them took 8 us of a 12 us kernel).
+__device__ __forceinline__ int take_place(int *count, int c, bool parked) {
+	int at = 0;
+	for(unsigned long long left = ballot(parked); left != 0ull;) {
+		const int cl = __builtin_amdgcn_readlane(c, (int) __builtin_ctzll(left));
+		const unsigned long long mates = ballot(parked && c == cl);
+		if(parked && c == cl) {
+			const int before = __popcll(mates & ((1ull << (threadIdx.x & 63)) - 1ull));
+			int base = 0;
+			if(before == 0) base = atomicAdd(&count[c], __popcll(mates));
+			at = __builtin_amdgcn_readlane(base, (int) __builtin_ctzll(mates)) + before;
+		}
+		left &= ~mates;
+	}
+	if(!parked) at = atomicAdd(&count[c], 1);
+	return at;
+}
+
 // ONE: a context of one replica, whose table then loads to scalar registers.
 template <bool ONE>
 __global__ void k_count(DevState d, int mode, uint64_t sweep, long long trace_pos) {
@@ -113,14 +163,7 @@ __global__ void k_count(DevState d, int mode, uint64_t sweep, long long trace_po
 	// reset the scan's look-back state for the scan that follows
 	for(int t = j; t < d.ntiles; t += gridDim.x * blockDim.x) d.scan_status[t] = 0ull;
 	for(int t = j; t < d.R * 8; t += gridDim.x * blockDim.x) d.ccount[t] = 0;
-	if(j == 0) {
-		d.scan_ticket[0] = 0;
-		if(mode == REB_SHIFT && d.pl_n) {
-			// the sweep's list of close pairs, built after its passes
-			d.pl_n[0] = 0;
-			d.pl_n[1] = 0;
-		}
-	}
+	if(j == 0) reset_sweep_lists(d, mode);
 	if(mode == REB_TRIAL)
 		// replicas without a trial rebuild keep their lists as they are:
 		// their cells' counts are the current populations, so the scan
@@ -143,23 +186,10 @@ __global__ void k_count(DevState d, int mode, uint64_t sweep, long long trace_po
 				for(int k = 0; k < NSLOT; k++) db += *ctr_at(d.ctr, r, C_DBONDS, k);
 				d.trace[(long long) r * d.trace_cap + trace_pos] = rp.bonds_base + (long long) db;
 			}
-			rp.g.shift[0] = sh[0];
-			rp.g.shift[1] = sh[1];
-			rp.g.shift[2] = sh[2];
-			// random colour order of this sweep's 8 passes
-			u32x4 v = rng(d.seed, r, sweep, 0, TAG_COLOUR, 0, 0);
-			const uint32_t w4[4] = {v.x, v.y, v.z, v.w};
-			rp.col_perm = colour_perm_from(w4);
-			set_pass_geo(rp, G, sh);
+			begin_sweep(d, rp, r, sweep, sh);
 		}
 	}
-	if(!tr && j == rp.p_off) {
-		// the lists the scan and scatter build are by membership in this grid
-		rp.lg = rp.g;
-		for(int k = 0; k < 3; k++) rp.lg.shift[k] = sh[k];
-		rp.lists_ok = 1;
-		rp.rec_ok = mode == REB_SHIFT;  // only that rebuild writes the cell records
-	}
+	if(!tr && j == rp.p_off) begin_lists(rp, mode, sh);
 	// a free or removed slot of a grand-canonical replica goes to the
 	// replica's parking cell
 	int c = rp.cell_off + rp.cell_cap;
@@ -174,25 +204,8 @@ __global__ void k_count(DevState d, int mode, uint64_t sweep, long long trace_po
 		c = rp.cell_off + (ix * G.n[1] + iy) * G.n[2] + iz;
 	}
 	d.cellid[j] = c;
-	// the slots a grand-canonical replica does not use all go to one cell: a
-	// wavefront's together (one by one, 900 of them took 8 us of a 12 us kernel)
-	const bool parked = c == rp.cell_off + rp.cell_cap;
-	for(unsigned long long left = ballot(parked); left != 0ull;) {
-		const int cl = __builtin_amdgcn_readlane(c, (int) __builtin_ctzll(left));
-		const unsigned long long mates = ballot(parked && c == cl);
-		if(parked && c == cl) {
-			const int before = __popcll(mates & ((1ull << (threadIdx.x & 63)) - 1ull));
-			int base = 0;
-			if(before == 0) base = atomicAdd(&d.count[c], __popcll(mates));
-			d.slot[j] = __builtin_amdgcn_readlane(base, (int) __builtin_ctzll(mates)) + before;
-		}
-		left &= ~mates;
-	}
-	if(!parked) d.slot[j] = atomicAdd(&d.count[c], 1);
+	d.slot[j] = take_place(d.count, c, c == rp.cell_off + rp.cell_cap);
 }
-
-// (replica, colour) keys of the non-empty-cell lists counted per scan workgroup
-constexpr int SCAN_KEYS = 512;
 
 // A lane's PER consecutive cells of a tile: whole vectors where all PER
 // are in the grid (base is a multiple of PER, the arrays 16-byte aligned).
@@ -233,6 +246,103 @@ __device__ __forceinline__ void store_cells(int *p, int base, int n, const int v
 		for(int e = 0; e < PER; e++)
 			if(base + e < n) p[base + e] = v[e];
 }
+
+// Count and scan of one small replica in one workgroup, the cells' counts in
+// LDS (d.count stays clear).  k_count and k_scan are mostly round trips to
+// memory (the ticket, the counts, the look-back, the lists' atomics); here
+// each round of 1024 particles costs about 2 us, so it ends at three.  Both
+// kernels against this one: N=300 (512 cells) 9.1 -> 4.9 us, N=1000 (5832
+// cells) 9.9 -> 7.3, N=2700 9.3 -> 8.8, N=4000 9.7 -> 11.6.
+constexpr int CS_CELLS = 8192;     // cells, the parking cell included
+constexpr int CS_PARTICLES = 3072;
+constexpr int CS_THREADS = 1024, CS_PER = CS_CELLS / CS_THREADS;
+
+__global__ __launch_bounds__(CS_THREADS) void k_count_scan(DevState d, int mode, uint64_t sweep, long long trace_pos) {
+	__shared__ __attribute__((aligned(16))) int cnt[CS_CELLS];
+	__shared__ int wsum[CS_THREADS / 64];
+	const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+	Rep &rp = d.reps[0];
+#pragma unroll
+	for(int e = 0; e < CS_PER; e += 4) *(int4 *) (cnt + t * CS_PER + e) = make_int4(0, 0, 0, 0);
+	const int n0 = rp.g.n[0], n1 = rp.g.n[1], n2 = rp.g.n[2], sel = rp.sel, parking = rp.cell_cap;
+	double sh[3] = {rp.g.shift[0], rp.g.shift[1], rp.g.shift[2]};
+	if(mode == REB_SHIFT) sweep_shift(d, 0, rp.g, sweep, sh);
+	const double i0 = rp.g.inv_box[0], i1 = rp.g.inv_box[1], i2 = rp.g.inv_box[2];
+	__syncthreads();
+	for(int j = t; j < d.Ntot; j += CS_THREADS) {
+		int c = parking;
+		if(j < rp.np_hw && pick_buf(d.pid, sel)[j] >= 0) {
+			const double *p = part((const double *) pick_buf(d.f, sel), j);
+			c = (cell_coord(p[0], sh[0], i0, n0) * n1 + cell_coord(p[1], sh[1], i1, n1)) * n2 + cell_coord(p[2], sh[2], i2, n2);
+		}
+		d.cellid[j] = c;
+		d.slot[j] = take_place(cnt, c, c == parking);
+	}
+	__syncthreads();
+	// first slots
+	int v[CS_PER], tot = 0;
+#pragma unroll
+	for(int e = 0; e < CS_PER; e++) {
+		v[e] = cnt[t * CS_PER + e];
+		tot += v[e];
+	}
+	const int inc = wave_incl_scan(tot);
+	if(lane == 63) wsum[w] = inc;
+	__syncthreads();
+	int run = inc - tot;
+	for(int k = 0; k < w; k++) run += wsum[k];
+	int first[CS_PER];
+#pragma unroll
+	for(int e = 0; e < CS_PER; e++) {
+		first[e] = run;
+		run += v[e];
+	}
+	if(t * CS_PER < d.C_total) store_cells<CS_PER>(d.start, t * CS_PER, d.C_total, first);
+	// the table's entries for this rebuild (every thread has read the old
+	// ones), by wavefronts that make no list
+	if(t == CS_THREADS - 64) {
+		reset_sweep_lists(d, mode);
+		if(mode == REB_SHIFT) begin_sweep(d, rp, 0, sweep, sh);
+		begin_lists(rp, mode, sh);
+		rp.sel = sel ^ 1;
+		d.start[d.C_total] = d.Ntot;
+	}
+	if(w == 8 && mode == REB_SHIFT && d.trace && trace_pos >= 0 && trace_pos < d.trace_cap) {
+		// energy trace: bonded pairs as they stand after the previous sweep
+		static_assert(NSLOT == 64, "a lane per slot");
+		unsigned long long db = *ctr_at(d.ctr, 0, C_DBONDS, lane);
+		for(int o = 32; o > 0; o >>= 1) db += __shfl_xor(db, o);
+		if(lane == 0) d.trace[trace_pos] = rp.bonds_base + (long long) db;
+	}
+	if(mode != REB_SHIFT || w >= 8) return;
+	// the passes' lists: wavefront w takes the cells of colour w in order
+	const int h1 = n1 / 2, h2 = n2 / 2, cells = n0 / 2 * h1 * h2;
+	const int sa = 64 / (h1 * h2), sb = 64 % (h1 * h2) / h2, sc = 64 % h2;  // 64 cells on, per axis
+	int a = lane / (h1 * h2), b = lane / h2 % h1, c = lane % h2, n = 0;
+	int *list = d.clist + w * rp.act_cap;
+	for(int k = lane; __any(k < cells); k += 64) {
+		const int cloc = ((2 * a + (w >> 2)) * n1 + 2 * b + ((w >> 1) & 1)) * n2 + 2 * c + (w & 1);
+		const bool on = k < cells && cnt[cloc] > 0;
+		const unsigned long long m = ballot(on);
+		if(on) list[n + __popcll(m & ((1ull << lane) - 1ull))] = cloc;
+		n += __popcll(m);
+		c += sc;
+		b += sb;
+		a += sa;
+		if(c >= h2) {
+			c -= h2;
+			b++;
+		}
+		if(b >= h1) {
+			b -= h1;
+			a++;
+		}
+	}
+	if(lane == 0) d.ccount[w] = n;
+}
+
+// (replica, colour) keys of the non-empty-cell lists counted per scan workgroup
+constexpr int SCAN_KEYS = 512;
 
 // Exclusive scan of the cell counts in one pass (decoupled look-back):
 // workgroups take tiles in dispatch order from a ticket, publish their tile
@@ -546,11 +656,24 @@ __global__ __launch_bounds__(256) void k_scatter(DevState d, int mode, int part_
 	}
 }
 
+static void launch_scatter(const DevState &d, int mode, hipStream_t s) {
+	const unsigned pb = (unsigned) std::max(1, (d.Ntot + PART_BLOCK - 1) / PART_BLOCK);
+	unsigned gs = pb;
+	if(mode == REB_SHIFT) gs += (unsigned) std::min<long long>(REC_BLOCKS, (8LL * d.total_act + 15) / 16);
+	if(d.R == 1) hipLaunchKernelGGL(k_scatter<true>, dim3(gs), dim3(256), 0, s, d, mode, (int) pb);
+	else hipLaunchKernelGGL(k_scatter<false>, dim3(gs), dim3(256), 0, s, d, mode, (int) pb);
+}
+
 void launch_rebuild(const DevState &d, int mode, uint64_t sweep, long long trace_pos, hipStream_t s) {
 	const int B = 256;
 	unsigned gp = (unsigned) ((d.Ntot + B - 1) / B);
 	if(gp == 0) gp = 1;
 	const int flip = mode != REB_TRIAL;
+	if(flip && d.R == 1 && d.Ntot <= CS_PARTICLES && d.C_total <= CS_CELLS) {
+		hipLaunchKernelGGL(k_count_scan, dim3(1), dim3(CS_THREADS), 0, s, d, mode, sweep, trace_pos);
+		launch_scatter(d, mode, s);
+		return;
+	}
 	if(d.R == 1) hipLaunchKernelGGL(k_count<true>, dim3(gp), dim3(B), 0, s, d, mode, sweep, trace_pos);
 	else hipLaunchKernelGGL(k_count<false>, dim3(gp), dim3(B), 0, s, d, mode, sweep, trace_pos);
 	const int lists = mode == REB_SHIFT ? 1 : 0;
@@ -570,11 +693,7 @@ void launch_rebuild(const DevState &d, int mode, uint64_t sweep, long long trace
 		hipLaunchKernelGGL((k_scan<SCAN_TILE_LARGE / 256, false>), dim3(d.ntiles), dim3(256), 0, s, d, flip, lists, 1);
 	}
 	if(mode == REB_SHIFT && d.R != 1) hipLaunchKernelGGL(k_pass_prefix, dim3(1), dim3(512), 0, s, d);
-	const unsigned pb = (unsigned) std::max(1, (d.Ntot + PART_BLOCK - 1) / PART_BLOCK);
-	unsigned gs = pb;
-	if(mode == REB_SHIFT) gs += (unsigned) std::min<long long>(REC_BLOCKS, (8LL * d.total_act + 15) / 16);
-	if(d.R == 1) hipLaunchKernelGGL(k_scatter<true>, dim3(gs), dim3(B), 0, s, d, mode, (int) pb);
-	else hipLaunchKernelGGL(k_scatter<false>, dim3(gs), dim3(B), 0, s, d, mode, (int) pb);
+	launch_scatter(d, mode, s);
 }
 
 // ------------------------------------------------------------------------

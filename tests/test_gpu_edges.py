@@ -153,3 +153,42 @@ def test_over_full_cell_is_reported_by_every_pass(pp, learned_fraction):
         with pytest.raises(pp.PPError) as e:
             s.do_ensemble(1)
         assert e.value.status == 5  # PP_ERR_CELL_CAP
+
+
+def _lattice(box, spacing, seed):
+    """Particles on a lattice of the box, at most one diameter short of it."""
+    rng = np.random.default_rng(seed)
+    m = [int(b // spacing) for b in box]
+    r = np.stack(np.meshgrid(*[(np.arange(k) + 0.5) * (b / k) for k, b in zip(m, box)], indexing="ij"), -1).reshape(-1, 3)
+    q, _ = np.linalg.qr(rng.normal(size=(len(r), 3, 3)))
+    q[np.linalg.det(q) < 0, :, 0] *= -1
+    return r + rng.uniform(-0.04, 0.04, r.shape), q, np.array(box)
+
+
+@pytest.mark.parametrize("case", ["one", "n1024", "n1025", "n3072", "n3073", "cells_8000", "cells_10648", "flat", "long_z",
+                                  "long_x"])
+def test_small_rebuild_gives_the_general_one_s_trajectory(case):
+    """One workgroup counts, scans and lists a single small replica (up to 3072
+    particles in 8191 cells); the same system as replica 0 of a batch takes the
+    general kernels.  Same trajectory, counters and energy trace to the bit."""
+    import patchyparticles_amd as pp
+
+    if case == "one":
+        r, O, box = np.array([[1.0, 2.0, 3.0]]), np.eye(3)[None], np.full(3, 6.0)
+    elif case[0] == "n":
+        r, O, box = pp.generate(int(case[1:]), 0.4, 11)
+    elif case == "cells_8000":
+        r, O, box = pp.generate(500, 500 / 23.0 ** 3, 12)
+    elif case == "cells_10648":
+        r, O, box = pp.generate(500, 500 / 25.0 ** 3, 13)
+    else:
+        r, O, box = _lattice({"flat": (20.0, 20.0, 5.2), "long_z": (5.2, 9.1, 78.0), "long_x": (78.0, 5.2, 9.1)}[case], 1.28, 14)
+    got = []
+    for copies in (1, 2):
+        with pp.System.batch([r] * copies, [O] * copies, [box] * copies, [dict(T=0.15)] * copies, seed=9) as s:
+            s.set_trace(12)
+            s.do_ensemble(12)
+            c = s.counters(0)
+            got.append((s.trace(0), s.state(0), c["tries"], c["accepted"], c["bonds"]))
+    (ta, (ra, Oa, _), *ca), (tb, (rb, Ob, _), *cb) = got
+    assert np.array_equal(ta, tb) and np.array_equal(ra, rb) and np.array_equal(Oa, Ob) and ca == cb
