@@ -659,18 +659,10 @@ __device__ inline void gauss2(uint32_t u1, uint32_t u2, double &z0, double &z1) 
 // density is evaluated at (body-frame displacement and axis as floats), so
 // the precision of the transforms only shapes the proposal, not the
 // acceptance rule.
-__device__ inline void gauss2f(uint32_t u1, uint32_t u2, float &z0, float &z1) {
-	const float a = ((float) (u1 >> 8) + 0.5f) * 5.9604644775390625e-8f;  // (0, 1)
-	const float b = (float) (u2 >> 8) * 5.9604644775390625e-8f;
-	const float rr = sqrtf(-2.f * logf(a));
-	float sn, cs;
-	sincosf(6.2831853f * b, &sn, &cs);
-	z0 = rr * cs;
-	z1 = rr * sn;
-}
 
-// vMF sample on S^2 around unit mu (Wood 1994: the cosine by inverse CDF)
-__device__ inline void vmf_sample(const float mu[3], float kappa, float u1, float u2, float out[3]) {
+// Wood 1994's cosine to the mean of a vMF sample (inverse CDF), and the sample
+// from it and the azimuth's sine and cosine.
+__device__ inline void vmf_sample(const float mu[3], float kappa, float u1, float sn, float cs, float out[3]) {
 	float w;
 	if(kappa < 1e-4f) w = 2.f * u1 - 1.f;
 	else w = 1.f + logf(expf(-2.f * kappa) + u1 * (-expm1f(-2.f * kappa))) / kappa;
@@ -682,8 +674,6 @@ __device__ inline void vmf_sample(const float mu[3], float kappa, float u1, floa
 	const float n1 = sqrtf(e1[0] * e1[0] + e1[1] * e1[1] + e1[2] * e1[2]);
 	for(int k = 0; k < 3; k++) e1[k] /= n1;
 	const float e2[3] = {mu[1] * e1[2] - mu[2] * e1[1], mu[2] * e1[0] - mu[0] * e1[2], mu[0] * e1[1] - mu[1] * e1[0]};
-	float sn, cs;
-	sincosf(6.2831853f * u2, &sn, &cs);
 	const float sw = sqrtf(fmaxf(0.f, 1.f - w * w));
 	for(int k = 0; k < 3; k++) out[k] = w * mu[k] + sw * (cs * e1[k] + sn * e2[k]);
 	const float no = sqrtf(out[0] * out[0] + out[1] * out[1] + out[2] * out[2]);
@@ -799,15 +789,11 @@ __device__ __forceinline__ void load_ops(const NetDev &net, int wave, int lane, 
 	}
 }
 
-// Layer l on the workgroup's 16 rows, A -> S.act / S.y, and a barrier; the
-// next layer's weights are under way before that barrier, so that a layer
-// waits for LDS and MFMAs only.
+// Layer l on the workgroup's 16 rows, A -> S.act / S.y, and a barrier.
 template <int l>
-__device__ __forceinline__ void lp_layer(const NetDev &net, LpLds &S, int wave, int lane, LayerOps &o) {
+__device__ __forceinline__ void lp_layer(LpLds &S, int wave, int lane, const LayerOps &o) {
 	const int r = lane & 15, g = lane >> 4;
 	const __bf16 *A = l == 0 ? S.x : S.act[l & 1];
-	LayerOps next;
-	if constexpr(l + 1 < NN_LAYERS) load_ops<l + 1>(net, wave, lane, next);
 	bf16x8 a[nn_k(l) / 32];
 #pragma unroll
 	for(int kb = 0; kb < nn_k(l) / 32; kb++) a[kb] = *(const bf16x8 *) (A + r * ACT_LD + kb * 32 + g * 8);
@@ -828,19 +814,23 @@ __device__ __forceinline__ void lp_layer(const NetDev &net, LpLds &S, int wave, 
 		}
 	}
 	__syncthreads();
-	if constexpr(l + 1 < NN_LAYERS) o = next;
 }
 
-// The network on the workgroup's 16 rows, S.x -> S.y, after a barrier.
+// The network on the workgroup's 16 rows, S.x -> S.y, after a barrier.  The
+// weights come from L2 two layers ahead, so that a layer waits for LDS and
+// MFMAs only.
 __device__ __forceinline__ void lp_forward(const NetDev &net, LpLds &S, int wave, int lane) {
 	static_assert(LP_TILES * LP_WAVES * 16 == NN_H && NN_LAYERS == 4, "whole column tiles per wavefront");
-	LayerOps o;
-	load_ops<0>(net, wave, lane, o);
+	LayerOps o0, o1, o2, o3;
+	load_ops<0>(net, wave, lane, o0);
+	load_ops<1>(net, wave, lane, o1);
 	__syncthreads();
-	lp_layer<0>(net, S, wave, lane, o);
-	lp_layer<1>(net, S, wave, lane, o);
-	lp_layer<2>(net, S, wave, lane, o);
-	lp_layer<3>(net, S, wave, lane, o);
+	load_ops<2>(net, wave, lane, o2);
+	lp_layer<0>(S, wave, lane, o0);
+	load_ops<3>(net, wave, lane, o3);
+	lp_layer<1>(S, wave, lane, o1);
+	lp_layer<2>(S, wave, lane, o2);
+	lp_layer<3>(S, wave, lane, o3);
 }
 
 // The whole learned pass in one kernel: a workgroup takes 16 cells of the
@@ -859,17 +849,22 @@ __device__ __forceinline__ void lp_forward(const NetDev &net, LpLds &S, int wave
 // and let every workgroup run at once; the mixture's components are one per
 // lane; code that rarely runs (slots past a record's list) is no longer
 // unrolled into every use, since the kernel exceeds the instruction cache.
-// 26 us.  (32 lanes in 128 registers, two workgroups per CU: 60 us, spills.)
+// The Gaussian pairs and the axis' azimuth are likewise one draw per lane, and
+// the weights come two layers ahead.  24.8 us.  (32 lanes in 128 registers, two
+// workgroups per CU: 60 us, spills.)
 __global__ __launch_bounds__(64 * LP_WAVES, 2) void k_learn_pass(DevState d, NetDev net, uint64_t sweep, int pass) {
 	__shared__ __attribute__((aligned(16))) LpLds S;
 	constexpr int T = LP_TEAM;
 	const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 	const int tl = lane & (T - 1), cell = threadIdx.x / T;
-	const int count = d.pfx[pass * (d.R + 1) + d.R];
 	const int g0 = blockIdx.x * LP_ROWS;
-	if(g0 >= count) return;  // the whole workgroup: before any barrier
 	const int gi = g0 + cell;
-	bool live = gi < count;
+	// a record of another sweep lies past the end of the pass's list (no read
+	// of its length first); the whole workgroup leaves before any barrier
+	const int *recs = d.rec + (size_t) pass * d.total_act * REC_W;
+	const bool any = recs[(size_t) g0 * REC_W + REC_TAG] == (int) d.rec_tag;
+	bool live = gi < d.total_act && recs[(size_t) min(gi, d.total_act - 1) * REC_W + REC_TAG] == (int) d.rec_tag;
+	if(!any) return;
 	CellView v{};
 	const double *F = nullptr;
 	int j = 0, nv = 0;
@@ -902,15 +897,13 @@ __global__ __launch_bounds__(64 * LP_WAVES, 2) void k_learn_pass(DevState d, Net
 		const int *PID = pick_buf(d.pid, v.sel);
 		const u32x4 ra = rng(d.seed, v.r, sweep, (uint32_t) v.cloc, TAG_LEARN_A, (uint32_t) pass, 0);
 		const int target = (int) __umulhi(ra.x, (uint32_t) v.cnt);
-		// (few cells hold more members than the team has lanes)
+		const int me = tl < v.cnt ? PID[v.s0 + tl] : 0;
 		for(int m0 = 0; m0 < v.cnt; m0 += T) {
-			bool hit = false;
-			if(m0 + tl < v.cnt) {
-				const int me = PID[v.s0 + m0 + tl];
-				int rk = 0;
-				for(int b = 0; b < v.cnt; b++) rk += PID[v.s0 + b] < me;
-				hit = rk == target;
-			}
+			// (few cells hold more members than the team has lanes)
+			const int id = m0 == 0 ? me : (m0 + tl < v.cnt ? PID[v.s0 + m0 + tl] : 0);
+			int rk = 0;
+			for(int b = 0; b < v.cnt; b++) rk += (b < T ? __shfl(me, (lane & ~(T - 1)) + b) : PID[v.s0 + b]) < id;
+			const bool hit = m0 + tl < v.cnt && rk == target;
 			const unsigned long long hm = (__ballot(hit) >> (lane & ~(T - 1))) & ((1ull << T) - 1ull);
 			if(hm) j = v.s0 + m0 + (int) __builtin_ctzll(hm);
 		}
@@ -944,9 +937,14 @@ __global__ __launch_bounds__(64 * LP_WAVES, 2) void k_learn_pass(DevState d, Net
 		prop_decode_lane(S.y + cell * NN_OUT_PAD, tl, pr);
 		const u32x4 ra = rng(d.seed, v.r, sweep, (uint32_t) v.cloc, TAG_LEARN_A, (uint32_t) pass, 1);
 		const u32x4 rb = rng(d.seed, v.r, sweep, (uint32_t) v.cloc, TAG_LEARN_B, (uint32_t) pass, 0);
-		float z[4];
-		gauss2f(ra.x, ra.y, z[0], z[1]);
-		gauss2f(ra.z, ra.w, z[2], z[3]);
+		// the Gaussian pairs (Box-Muller) by lanes 0 and 1 of each quad, the
+		// azimuth of the axis by lane 2: one logarithm and one sine and cosine
+		const int ql = tl & 3;
+		const uint32_t ub = ql == 0 ? ra.y : (ql == 1 ? ra.w : rb.z);
+		float sn, cs;
+		sincosf(6.2831853f * u01f(ub), &sn, &cs);
+		const float rr = sqrtf(-2.f * logf(((float) ((ql == 0 ? ra.x : ra.z) >> 8) + 0.5f) * 5.9604644775390625e-8f));
+		const float z[3] = {quad_get<0>(rr * cs), quad_get<0>(rr * sn), quad_get<1>(rr * cs)};
 		float dbody[3];
 		for(int k = 0; k < 3; k++) dbody[k] = pr.mu[k] + expf(pr.ls[k]) * z[k];
 		// mixture component by its weight, then the axis
@@ -957,7 +955,7 @@ __global__ __launch_bounds__(64 * LP_WAVES, 2) void k_learn_pass(DevState d, Net
 		for(int k = 0; k < 3; k++) dir[k] = __shfl(pr.dir[k], from);
 		const float kap = __shfl(pr.k, from);
 		float axf[3];
-		vmf_sample(dir, kap, u01f(rb.y), u01f(rb.z), axf);
+		vmf_sample(dir, kap, u01f(rb.y), quad_get<2>(sn), quad_get<2>(cs), axf);
 		const double ang = u01(rb.w) * d.learn.theta_max;
 		double p[3], O[9];
 		for(int k = 0; k < 3; k++) p[k] = cur[k];
