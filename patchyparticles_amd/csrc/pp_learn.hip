@@ -1111,20 +1111,22 @@ void launch_descriptor(int n, const double *r, const double *O, const Grid &g, i
 // training samples: a random particle of the current state, displaced and
 // rotated at random (the "current" state of a move), its descriptor there,
 // and as target the move back: displacement in the perturbed body frame and
-// the rotation axis (-a; the angle is uniform in both directions).  One wave
-// per sample, which finds its neighbours as a pass does, from a record (here in
+// the rotation axis (-a; the angle is uniform in both directions).  16 lanes
+// per sample, which find its neighbours as a pass does, from a record (here in
 // LDS) and positions staged once: a search through 27 ranges for every read of
-// a candidate took 33 us for 4096 samples, this 18.
+// a candidate, by a wavefront per sample, took 33 us for 4096 samples; with the
+// record 18; four samples per wavefront 10.6.
 
-constexpr int TS_WAVES = 4;
+constexpr int TS_LANES = 16;               // lanes per sample
+constexpr int TS_BLOCK = 256 / TS_LANES;   // samples of a workgroup
 
-__global__ __launch_bounds__(64 * TS_WAVES) void k_train_samples(DevState d, uint64_t seed, uint64_t step, int m,
-                                                                 int m_pad, double pos_noise, double theta_max,
-                                                                 __bf16 *x, float *target) {
-	__shared__ DescLds Ds[TS_WAVES];
-	__shared__ __attribute__((aligned(16))) CandLds Cs[TS_WAVES];
-	const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-	const int b = blockIdx.x * TS_WAVES + wave;
+__global__ __launch_bounds__(256) void k_train_samples(DevState d, uint64_t seed, uint64_t step, int m, int m_pad,
+                                                       double pos_noise, double theta_max, __bf16 *x, float *target) {
+	constexpr int T = TS_LANES;
+	__shared__ DescLds Ds[TS_BLOCK];
+	__shared__ __attribute__((aligned(16))) CandLds Cs[TS_BLOCK];
+	const int lane = threadIdx.x & (T - 1), team = threadIdx.x / T;
+	const int b = blockIdx.x * TS_BLOCK + team;
 	__bf16 *row = x + (size_t) b * NN_IN_PAD;
 	const bool live = b < m;
 	int nv = 0;
@@ -1133,10 +1135,10 @@ __global__ __launch_bounds__(64 * TS_WAVES) void k_train_samples(DevState d, uin
 	int j = 0;
 	const double *F = nullptr;
 	double L[3], iL[3];
-	CandLds &CL = Cs[wave];
+	CandLds &CL = Cs[team];
 	auto cands = [&]() { return Cands{d, F, v, j, &CL}; };
 	if(b < m_pad && !live) {
-		zero_row<64>(row, lane);
+		zero_row<T>(row, lane);
 		if(lane < 6) target[(size_t) b * 6 + lane] = 0.f;
 	}
 	if(live) {
@@ -1165,13 +1167,12 @@ __global__ __launch_bounds__(64 * TS_WAVES) void k_train_samples(DevState d, uin
 		v.cloc = (ix * n1 + iy) * n2 + iz;
 		v.r = d.prep[j];
 		v.sel = rp.sel;
-		if(lane < 16)
-			write_record(CL.rec, 0, d.start + rp.cell_off, v.cloc, ix, iy, iz, n0, n1, n2, v.r, v.sel, lane);
+		write_record(CL.rec, 0, d.start + rp.cell_off, v.cloc, ix, iy, iz, n0, n1, n2, v.r, v.sel, lane);
 		team_sync();
 		v.M = CL.rec[REC_M];
 		v.s0 = CL.rec[REC_S0];
 		v.cnt = CL.rec[REC_CNT];
-		cands().stage<64>(CL, lane);
+		cands().stage<T>(CL, lane);
 		// the perturbed state: Gaussian displacement, rotation by an angle
 		// uniform in [0, theta_max) about a uniform axis
 		double z[6];
@@ -1194,13 +1195,13 @@ __global__ __launch_bounds__(64 * TS_WAVES) void k_train_samples(DevState d, uin
 			for(int k = 0; k < 3; k++) t[3 + k] = (float) -ax[k];
 		}
 		const Cands c = cands();
-		nv = desc_collect<64>(pt, c.count(), [&](int i, double q[3]) { c.pos(i, q); }, L, iL, Ds[wave], row, lane);
+		nv = desc_collect<T>(pt, c.count(), [&](int i, double q[3]) { c.pos(i, q); }, L, iL, Ds[team], row, lane);
 	}
 	__syncthreads();
 	if(live) {
 		const Cands c = cands();
-		desc_fill<64>(
-			pt, Ot, nv, [&](int i, double q[3]) { c.pos(i, q); }, [&](int i, double Oq[9]) { c.ori(i, Oq); }, L, iL, Ds[wave],
+		desc_fill<T>(
+			pt, Ot, nv, [&](int i, double q[3]) { c.pos(i, q); }, [&](int i, double Oq[9]) { c.ori(i, Oq); }, L, iL, Ds[team],
 			row, lane);
 	}
 }
@@ -1208,8 +1209,8 @@ __global__ __launch_bounds__(64 * TS_WAVES) void k_train_samples(DevState d, uin
 void launch_train_samples(const DevState &d, uint64_t seed, uint64_t step, int m, double pos_noise, double theta_max,
                           __bf16 *x, float *target, hipStream_t s) {
 	const int m_pad = (m + 31) & ~31;
-	hipLaunchKernelGGL(k_train_samples, dim3((m_pad + TS_WAVES - 1) / TS_WAVES), dim3(64 * TS_WAVES), 0, s, d, seed,
-	                   step, m, m_pad, pos_noise, theta_max, x, target);
+	hipLaunchKernelGGL(k_train_samples, dim3((m_pad + TS_BLOCK - 1) / TS_BLOCK), dim3(256), 0, s, d, seed, step, m, m_pad,
+	                   pos_noise, theta_max, x, target);
 }
 
 }  // namespace ppd
