@@ -1606,21 +1606,8 @@ pp_status pp_net_attach(pp_ctx *c, pp_net *net, double learned_fraction, double 
 	if(!(learned_fraction >= 0. && learned_fraction <= 1.)) return fail(PP_ERR_ARG, "learned_fraction must lie in [0, 1]");
 	if(!(theta_max > 0. && theta_max <= M_PI)) return fail(PP_ERR_ARG, "theta_max must lie in (0, pi]");
 	HIPCHECK(hipSetDevice(c->device));
-	LearnDev &L = c->d.learn;
-	if(!L.xf) {
-		const size_t m = (size_t) std::max(c->d.total_act, 1);
-		TRY(dev_alloc(c, &L.xf, m * NN_IN_PAD));
-		TRY(dev_alloc(c, &L.xr, m * NN_IN_PAD));
-		TRY(dev_alloc(c, &L.yf, m * NN_OUT_PAD));
-		TRY(dev_alloc(c, &L.yr, m * NN_OUT_PAD));
-		TRY(dev_alloc(c, &L.prop, m * NN_PROP_W));
-		TRY(dev_alloc(c, &L.slot, m));
-		HIPCHECK(hipMemsetAsync(L.xf, 0, m * NN_IN_PAD * sizeof(__bf16), c->stream));
-		HIPCHECK(hipMemsetAsync(L.xr, 0, m * NN_IN_PAD * sizeof(__bf16), c->stream));
-		HIPCHECK(hipStreamSynchronize(c->stream));
-	}
-	L.on = 1;
-	L.theta_max = theta_max;
+	c->d.learn.on = 1;
+	c->d.learn.theta_max = theta_max;
 	c->net = net;
 	c->learned_fraction = learned_fraction;
 	return PP_OK;

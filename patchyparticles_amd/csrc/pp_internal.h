@@ -89,16 +89,10 @@ struct NetScratch {
 	float *loss;      // [m_pad]
 };
 
-constexpr int NN_PROP_W = 16;  // doubles of one drawn proposal
-
-// Per-context state of the learned passes (scratch sized for the largest list).
+// Per-context state of the learned passes.
 struct LearnDev {
 	int on;
 	double theta_max;    // rotation angle of a learned move, uniform in [0, theta_max)
-	__bf16 *xf, *xr;     // [total_act][NN_IN_PAD] descriptors at the current / proposed state
-	float *yf, *yr;      // [total_act][NN_OUT_PAD] network outputs
-	double *prop;        // [total_act][NN_PROP_W] p'[3], O'[9], log q forward, a[3] of the proposal
-	int *slot;           // [total_act] moving slot (-1: no move)
 };
 
 // device error bits

@@ -754,7 +754,7 @@ struct Cands {
 	}
 };
 
-constexpr int PROP_W = NN_PROP_W;  // p'[3], O'[9], log q forward, axis[3]
+constexpr int PROP_W = 16;         // one drawn proposal: p'[3], O'[9], log q forward, axis[3]
 constexpr int LP_ROWS = 16;        // rows of the MFMA tile = cells of one workgroup
 constexpr int LP_TEAM = 16;        // lanes per cell: four cells per wavefront
 constexpr int LP_WAVES = LP_ROWS * LP_TEAM / 64;
