@@ -234,9 +234,9 @@ __device__ __forceinline__ u32x4 axis_block(uint64_t seed, int r, uint64_t sweep
 }
 
 // v: block 0 of the draw (callers form it among their other draws, so that
-// the Philox rounds of all of them overlap).
-__device__ __forceinline__ void sphere_axis_from(u32x4 v, uint64_t seed, int r, uint64_t sweep, uint32_t cell,
-                                                 uint32_t col, uint32_t t, double a[3]) {
+// the Philox rounds of all of them overlap); have_next: block 1 is `next`.
+__device__ __forceinline__ void sphere_axis_from(u32x4 v, bool have_next, u32x4 next, uint64_t seed, int r, uint64_t sweep,
+                                                 uint32_t cell, uint32_t col, uint32_t t, double a[3]) {
 	for(uint32_t blk = 0;;) {
 		// the block's first accepted pair
 		const double p1 = 1. - 2. * u01(v.x), p2 = 1. - 2. * u01(v.y), s1 = 1. - 2. * u01(v.z), s2 = 1. - 2. * u01(v.w);
@@ -251,7 +251,8 @@ __device__ __forceinline__ void sphere_axis_from(u32x4 v, uint64_t seed, int r, 
 			return;
 		}
 		if(++blk == AXIS_BLOCKS) break;
-		v = axis_block(seed, r, sweep, cell, col, t, blk);
+		if(have_next && blk == 1) v = next;
+		else v = axis_block(seed, r, sweep, cell, col, t, blk);
 	}
 	v = rng(seed, r, sweep, cell, TAG_AXIS_FALLBACK, col, t);
 	a[0] = 0.;
@@ -261,7 +262,16 @@ __device__ __forceinline__ void sphere_axis_from(u32x4 v, uint64_t seed, int r, 
 
 __device__ __forceinline__ void sphere_axis(uint64_t seed, int r, uint64_t sweep, uint32_t cell, uint32_t col,
                                             uint32_t t, double a[3]) {
-	sphere_axis_from(axis_block(seed, r, sweep, cell, col, t, 0), seed, r, sweep, cell, col, t, a);
+	sphere_axis_from(axis_block(seed, r, sweep, cell, col, t, 0), false, u32x4{}, seed, r, sweep, cell, col, t, a);
+}
+
+template <int c>
+__device__ __forceinline__ uint32_t quad_word(uint32_t v) {
+	return (uint32_t) __builtin_amdgcn_update_dpp(0, (int) v, c * 0x55, 0xf, 0xf, true);
+}
+template <int c>
+__device__ __forceinline__ u32x4 quad_block(u32x4 v) {
+	return u32x4{quad_word<c>(v.x), quad_word<c>(v.y), quad_word<c>(v.z), quad_word<c>(v.w)};
 }
 
 // Trial t of cell cloc (colour col) in sweep `sweep`: member rank among
@@ -269,14 +279,30 @@ __device__ __forceinline__ void sphere_axis(uint64_t seed, int r, uint64_t sweep
 // by an angle uniform in [0, theta_max) about an axis uniform on the sphere
 // (MC.c:321-325, utils.c:186-202).  Returns the 32 bits of the acceptance
 // draw u = w 2^-32 (MC.c:332).
+// by_quads (uniform): the four lanes of a quad make the same trial together,
+// each drawing one of its blocks (the axis' second among them).  A lane alone
+// draws three, one after the other where few wavefronts share the SIMD.
 __device__ __forceinline__ uint32_t make_trial(const DevState &d, const Rep &rp, int r, uint64_t sweep, int cloc, int col,
-                                               int t, int cnt, double out[TRIAL_W]) {
-	const u32x4 ra = rng(d.seed, r, sweep, (uint32_t) cloc, TAG_TRIAL_A, (uint32_t) col, (uint32_t) t);
-	const u32x4 rb = rng(d.seed, r, sweep, (uint32_t) cloc, TAG_TRIAL_B, (uint32_t) col, (uint32_t) t);
-	const u32x4 rc = axis_block(d.seed, r, sweep, (uint32_t) cloc, (uint32_t) col, (uint32_t) t, 0);
+                                               int t, int cnt, bool by_quads, double out[TRIAL_W]) {
+	u32x4 ra, rb, rc, rd{};
+	if(by_quads) {
+		const uint32_t q = threadIdx.x & 3u;
+		const u32x4 v = rng(d.seed, r, sweep, (uint32_t) cloc | (q == 3u ? 1u << 24 : 0u),
+		                    q == 0u ? (uint32_t) TAG_TRIAL_A : (q == 1u ? (uint32_t) TAG_TRIAL_B : (uint32_t) TAG_AXIS),
+		                    (uint32_t) col, (uint32_t) t);
+		ra = quad_block<0>(v);
+		rb = quad_block<1>(v);
+		rc = quad_block<2>(v);
+		rd = quad_block<3>(v);
+	}
+	else {
+		ra = rng(d.seed, r, sweep, (uint32_t) cloc, TAG_TRIAL_A, (uint32_t) col, (uint32_t) t);
+		rb = rng(d.seed, r, sweep, (uint32_t) cloc, TAG_TRIAL_B, (uint32_t) col, (uint32_t) t);
+		rc = axis_block(d.seed, r, sweep, (uint32_t) cloc, (uint32_t) col, (uint32_t) t, 0);
+	}
 	double axis[3], st, ct, R[9];
 	sincos(u01(rb.x) * rp.theta_max, &st, &ct);
-	sphere_axis_from(rc, d.seed, r, sweep, (uint32_t) cloc, (uint32_t) col, (uint32_t) t, axis);
+	sphere_axis_from(rc, by_quads, rd, d.seed, r, sweep, (uint32_t) cloc, (uint32_t) col, (uint32_t) t, axis);
 	out[0] = (double) __umulhi(ra.x, (uint32_t) cnt);
 	out[1] = (u01(ra.y) - 0.5) * rp.disp_max;
 	out[2] = (u01(ra.z) - 0.5) * rp.disp_max;
