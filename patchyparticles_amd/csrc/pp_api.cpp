@@ -677,7 +677,7 @@ void colour_check_now(pp_ctx *c) {
 }
 
 // Wait for the device to publish `seq` in pinned word `w` (k_vol_publish:
-// an attempt's trial paths in the low 4 bits; k_vol_report: where a
+// an attempt's trial paths in the low 4 bits; k_vol_apply: where a
 // run-ahead sequence stopped in the low 8): a spin on host memory, with the
 // stream polled now and then so that a failed launch is reported instead of
 // waited for.
@@ -770,17 +770,16 @@ pp_status enqueue_sweep(pp_ctx *c) {
 			// every fast trial in the common case; the host then learns once
 			// where, if anywhere, an attempt needed more (attempt_stopped), and
 			// goes on from that attempt's standing proposal as below
+			const unsigned seq = (++c->vol_seq) & 0x7FFFFFu;
 			for(int k = 0; k < nvol; k++) {
 				hipEvent_t v{};
 				tic(c, TK_VOLUME, &v);
 				launch_vol_propose(c->d, sw, k, c->stream);
 				launch_energy_pairs(c->d, c->cus, 1, c->stream);
 				launch_vol_decide(c->d, sw, k, 1, c->stream);
-				launch_vol_apply(c->d, k, 1, c->stream);
+				launch_vol_apply(c->d, k, 1, k == nvol - 1 ? c->d_vslow_host + 1 : nullptr, seq, c->stream);
 				toc(c, TK_VOLUME, v);
 			}
-			const unsigned seq = (++c->vol_seq) & 0x7FFFFFu;
-			launch_vol_report(c->d, c->d_vslow_host + 1, seq, c->stream);
 			int stop = 0;
 			TRY(wait_published(c, 1, 8, seq, &stop));
 			k0 = stop > 0 ? stop - 1 : nvol;
@@ -803,7 +802,7 @@ pp_status enqueue_sweep(pp_ctx *c) {
 			if(need & NEED_RECORDS) launch_energy_rec(c->d, c->cus, c->stream);
 			if(need & NEED_PAIRS) launch_energy_pairs(c->d, c->cus, 0, c->stream);
 			launch_vol_decide(c->d, sw, k, 0, c->stream);
-			launch_vol_apply(c->d, k, 0, c->stream);
+			launch_vol_apply(c->d, k, 0, nullptr, 0u, c->stream);
 			toc(c, TK_VOLUME, v);
 		}
 	}

@@ -320,8 +320,10 @@ void launch_vol_propose(const DevState &d, uint64_t sweep, int k, hipStream_t s)
 void launch_vol_publish(const DevState &d, int *host_word, unsigned seq, hipStream_t s);
 // (ahead: the attempt stops unless the close-pair list serves every trial)
 void launch_vol_decide(const DevState &d, uint64_t sweep, int k, int ahead, hipStream_t s);
-// rescale the positions of replicas whose fast trial was accepted; the end of attempt k
-void launch_vol_apply(const DevState &d, int k, int ahead, hipStream_t s);
+// rescale the positions of replicas whose fast trial was accepted; the end of
+// attempt k.  host_word (the last run-ahead attempt): report where they stopped
+// (attempt + 1, 0 for nowhere) with `seq` into the host's pinned word
+void launch_vol_apply(const DevState &d, int k, int ahead, int *host_word, unsigned seq, hipStream_t s);
 // the energy of the box trials whose replicas take it from the cell records
 // (trial_rec), one listed cell per team; `cus` sizes the grid
 void launch_energy_rec(const DevState &d, int cus, hipStream_t s);
@@ -332,9 +334,6 @@ void launch_colour_conflicts(const DevState &d, int rep, int slots, const int *n
                              hipStream_t s);
 // zero the energy rows (C_EBONDS, C_OVL) of every replica
 void launch_energy_rows_zero(const DevState &d, hipStream_t s);
-// the end of run-ahead box attempts: report where they stopped (attempt + 1, 0
-// for nowhere) with `seq` into the host's pinned word and clear it
-void launch_vol_report(const DevState &d, int *host_word, unsigned seq, hipStream_t s);
 // the trial-energy paths a box attempt needs, as the host reads them from
 // vslow after k_vol_propose: a trial rebuild, the per-particle trial energy,
 // the per-record trial energy

@@ -2404,22 +2404,6 @@ void launch_vol_publish(const DevState &d, int *host_word, unsigned seq, hipStre
 	hipLaunchKernelGGL(k_vol_publish, dim3(1), dim3(64), 0, s, d, host_word, seq);
 }
 
-// The end of a run-ahead sequence: where it stopped (attempt + 1, 0 if it
-// ran through) with the host's sequence number into the pinned word; the
-// stop is cleared for the attempts that follow.
-__global__ void k_vol_report(DevState d, int *host_word, unsigned seq) {
-	if(threadIdx.x == 0) {
-		const int stop = d.vslow[1];
-		d.vslow[1] = -1;
-		__hip_atomic_store(host_word, (int) ((seq << 8) | (unsigned) (stop + 1)), __ATOMIC_RELAXED,
-		                   __HIP_MEMORY_SCOPE_SYSTEM);
-	}
-}
-
-void launch_vol_report(const DevState &d, int *host_word, unsigned seq, hipStream_t s) {
-	hipLaunchKernelGGL(k_vol_report, dim3(1), dim3(64), 0, s, d, host_word, seq);
-}
-
 void launch_vol_propose(const DevState &d, uint64_t sweep, int k, hipStream_t s) {
 	static_assert(NSLOT == 64, "a lane per slot");
 	hipLaunchKernelGGL(k_vol_propose, dim3(d.R), dim3(64), 0, s, d, sweep, k);
@@ -2486,22 +2470,34 @@ void launch_vol_decide(const DevState &d, uint64_t sweep, int k, int ahead, hipS
 // as the trial rebuild writes it (x * 1 is x).  Clears the trial paths for
 // the next attempt, or marks where a run-ahead sequence stopped; either way
 // the other workgroups find the same answer before and after.
-__global__ void k_vol_apply(DevState d, int k, int ahead) {
+// host_word (the last attempt of a run-ahead sequence): where it stopped
+// (attempt + 1, 0 if it ran through) with the host's sequence number goes into
+// that pinned word, and the stop is cleared for the attempts that follow (the
+// paths in vslow[0] still hold this kernel's other workgroups back).
+__global__ void k_vol_apply(DevState d, int k, int ahead, int *host_word, unsigned seq) {
 	const int j = blockIdx.x * blockDim.x + threadIdx.x;
-	if(attempt_stopped(d, ahead)) {
-		if(j == 0 && d.vslow[1] < 0) d.vslow[1] = k;
-		return;
+	const bool stopped = attempt_stopped(d, ahead);
+	if(j == 0) {
+		int stop = 0;
+		if(stopped) {
+			const int at = d.vslow[1] < 0 ? k : d.vslow[1];
+			stop = at + 1;
+			d.vslow[1] = host_word ? -1 : at;
+		}
+		else *d.vslow = 0;
+		if(host_word)
+			__hip_atomic_store(host_word, (int) ((seq << 8) | (unsigned) stop), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 	}
-	if(j == 0) *d.vslow = 0;
-	if(j >= d.Ntot) return;
+	if(stopped || j >= d.Ntot) return;
 	const Rep &rp = d.reps[d.prep[j]];
 	if(!rp.vol_apply) return;
 	double *F = pick_buf(d.f, rp.sel);
 	for(int c = 0; c < 3; c++) part(F, j)[c] *= rp.trial_s[c];
 }
 
-void launch_vol_apply(const DevState &d, int k, int ahead, hipStream_t s) {
-	hipLaunchKernelGGL(k_vol_apply, dim3((unsigned) std::max(1, (d.Ntot + 255) / 256)), dim3(256), 0, s, d, k, ahead);
+void launch_vol_apply(const DevState &d, int k, int ahead, int *host_word, unsigned seq, hipStream_t s) {
+	hipLaunchKernelGGL(k_vol_apply, dim3((unsigned) std::max(1, (d.Ntot + 255) / 256)), dim3(256), 0, s, d, k, ahead, host_word,
+	                   seq);
 }
 
 // ------------------------------------------------------------------------
