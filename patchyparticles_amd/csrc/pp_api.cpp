@@ -580,29 +580,28 @@ pp_status create_impl(int R, const pp_params *prm, const pp_options *opts, const
 			if(!q) return bail(fail(PP_ERR_NOMEM, "a device buffer was not allocated"));
 	}
 
-	// host staging: particles in index order, slot j = particle j; the
-	// free slots of grand-canonical replicas hold no particle (index -1)
+	// particles in index order, slot j = particle j; the free slots of
+	// grand-canonical replicas hold no particle (index -1).  The caller's
+	// arrays go up as they are, into the spare buffer (as large as all slots),
+	// and a kernel places them: interleaving them on the host and uploading
+	// three index tables took 0.4 ms of a snapshot's 0.94 at N=32768
 	{
-		std::vector<double> h((size_t) NCOMP * d.stride, 0.);
-		std::vector<int> hp(d.stride, -1), hr(d.stride, 0);
+		std::vector<int> src_off(R);
 		long long src = 0;  // the caller's arrays hold the replicas' particles back to back
 		for(int k = 0; k < R; k++) {
-			for(int i = 0; i < cap[k]; i++) hr[c->p_off[k] + i] = k;
-			for(int i = 0; i < n[k]; i++, src++) {
-				long long j = c->p_off[k] + i;
-				for(int a = 0; a < 3; a++) h[(size_t) NCOMP * j + a] = r[3 * src + a];
-				for(int a = 0; a < 9; a++) h[(size_t) NCOMP * j + 3 + a] = O[9 * src + a];
-				hp[j] = i;
-			}
+			src_off[k] = (int) src;
+			src += n[k];
 		}
-		if(hipMemcpy(d.f[0], h.data(), h.size() * sizeof(double), hipMemcpyHostToDevice) != hipSuccess ||
-		   hipMemcpy(d.pid[0], hp.data(), hp.size() * sizeof(int), hipMemcpyHostToDevice) != hipSuccess ||
-		   hipMemcpy(d.pid[1], hp.data(), hp.size() * sizeof(int), hipMemcpyHostToDevice) != hipSuccess ||
-		   hipMemcpy((void *) d.prep, hr.data(), hr.size() * sizeof(int), hipMemcpyHostToDevice) != hipSuccess ||
+		double *rs = d.f[1], *Os = d.f[1] + 3 * src;
+		// (pfx: scratch of at least R + 1 words until the first rebuild)
+		if((src > 0 && (hipMemcpy(rs, r, 3 * src * sizeof(double), hipMemcpyHostToDevice) != hipSuccess ||
+		                hipMemcpy(Os, O, 9 * src * sizeof(double), hipMemcpyHostToDevice) != hipSuccess)) ||
+		   hipMemcpy(d.pfx, src_off.data(), R * sizeof(int), hipMemcpyHostToDevice) != hipSuccess ||
 		   hipMemcpy((void *) d.act_off, c->act_off.data(), (R + 1) * sizeof(int), hipMemcpyHostToDevice) !=
 		       hipSuccess ||
 		   hipMemcpy(d.reps, c->reps.data(), R * sizeof(Rep), hipMemcpyHostToDevice) != hipSuccess)
 			return bail(fail(PP_ERR_HIP, "initial upload failed"));
+		launch_place(d, (int *) d.prep, d.pfx, rs, Os, c->stream);
 	}
 	launch_fill_i32(d.count, 0, d.C_total + 1, c->stream);
 	launch_fill_i32(d.err, 0, 1, c->stream);

@@ -348,6 +348,9 @@ void launch_energy_pairs(const DevState &d, int cus, int ahead, hipStream_t s);
 // grand-canonical insertions and removals of the sweep (GC replicas only)
 void launch_gc_phase(const DevState &d, uint64_t sweep, hipStream_t s);
 void launch_gram_schmidt(const DevState &d, hipStream_t s);
+// at creation: particles of the callers' arrays r[3 n], O[9 n] (device copies,
+// replica k's from src_off[k]) into the slots, the index tables and prep
+void launch_place(const DevState &d, int *prep, const int *src_off, const double *r, const double *O, hipStream_t s);
 // replica rep (np particles, not grand-canonical) in index order: out[UNPACK_HEAD + NCOMP np]
 enum Unpack : int { UNPACK_BOX = 0, UNPACK_BAD = 3, UNPACK_HEAD = 8 };
 void launch_unpack(const DevState &d, int rep, int np, double *out, hipStream_t s);

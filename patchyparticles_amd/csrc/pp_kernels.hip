@@ -697,6 +697,41 @@ void launch_rebuild(const DevState &d, int mode, uint64_t sweep, long long trace
 }
 
 // ------------------------------------------------------------------------
+// the callers' arrays into slots, at creation
+
+// Slot j of every replica: particle i of its replica (j = p_off + i) in both
+// index tables and the first buffer, or a free slot (index -1).  r and O hold
+// the replicas' particles back to back (replica k's from src_off[k]); 12 lanes
+// per slot.
+__global__ __launch_bounds__(256) void k_place(DevState d, int *prep, const int *src_off, const double *r, const double *O) {
+	const long long t = (long long) blockIdx.x * 256 + threadIdx.x;
+	const int j = (int) (t / NCOMP), e = (int) (t % NCOMP);
+	if(j >= d.Ntot) return;
+	int lo = 0, hi = d.R;
+	while(hi - lo > 1) {
+		const int mid = (lo + hi) >> 1;
+		if(d.reps[mid].p_off <= j) lo = mid;
+		else hi = mid;
+	}
+	const Rep &rp = d.reps[lo];
+	const int i = j - rp.p_off;
+	const bool there = i < rp.np;
+	const size_t src = (size_t) src_off[lo] + (there ? i : 0);
+	double v = 0.;
+	if(there) v = e < 3 ? r[3 * src + e] : O[9 * src + e - 3];
+	part(d.f[0], j)[e] = v;
+	if(e == 0) {
+		d.pid[0][j] = d.pid[1][j] = there ? i : -1;
+		prep[j] = lo;
+	}
+}
+
+void launch_place(const DevState &d, int *prep, const int *src_off, const double *r, const double *O, hipStream_t s) {
+	const long long t = (long long) d.Ntot * NCOMP;
+	if(t > 0) hipLaunchKernelGGL(k_place, dim3((unsigned) ((t + 255) / 256)), dim3(256), 0, s, d, prep, src_off, r, O);
+}
+
+// ------------------------------------------------------------------------
 // particles in index order, for a download
 
 // The slot (from the replica's first) of each particle index, in d.slot
