@@ -755,8 +755,8 @@ __global__ __launch_bounds__(256) void k_index_slots(DevState d, int rep, double
 // with the copies now.
 __global__ __launch_bounds__(256) void k_unpack(DevState d, int rep, double *out) {
 	const Rep &rp = d.reps[rep];
-	const unsigned t = blockIdx.x * 256u + threadIdx.x;
-	const unsigned i = t / NCOMP, e = t % NCOMP, n = (unsigned) rp.np;
+	const unsigned long long t = blockIdx.x * 256ull + threadIdx.x;
+	const unsigned i = (unsigned) (t / NCOMP), e = (unsigned) (t % NCOMP), n = (unsigned) rp.np;
 	if(i >= n) return;
 	const unsigned j = (unsigned) d.slot[rp.p_off + i];
 	if(j >= n || pick_buf(d.pid, rp.sel)[rp.p_off + j] != (int) i) {
