@@ -7,6 +7,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -57,6 +58,15 @@ Base host_base_patches() {
 }
 
 }  // namespace
+
+// Devices of this process, asked of the runtime until it has found some (the
+// question takes 90 us each time); 0 if there are none.
+int pp_device_count() {
+	static std::atomic<int> found{0};
+	int n = found.load(std::memory_order_relaxed);
+	if(n <= 0 && hipGetDeviceCount(&n) == hipSuccess && n > 0) found.store(n, std::memory_order_relaxed);
+	return n > 0 ? n : 0;
+}
 
 // the error message of the calling thread, set by the other translation units
 pp_status pp_set_error(pp_status s, const char *msg) {
@@ -364,8 +374,8 @@ pp_status create_impl(int R, const pp_params *prm, const pp_options *opts, const
 	if(Ntot > (1LL << 30)) return fail(PP_ERR_ARG, "too many particles");
 	if(nsum > 0 && (!r || !O)) return fail(PP_ERR_ARG, "positions/orientations are NULL");
 
-	int ndev = 0;
-	if(hipGetDeviceCount(&ndev) != hipSuccess || ndev <= 0) return fail(PP_ERR_HIP, "no HIP device available");
+	const int ndev = pp_device_count();
+	if(ndev <= 0) return fail(PP_ERR_HIP, "no HIP device available");
 	if(o.device < 0 || o.device >= ndev) return fail(PP_ERR_ARG, "device %d out of range", o.device);
 
 	pp_ctx *c = new pp_ctx();
@@ -542,12 +552,15 @@ pp_status create_impl(int R, const pp_params *prm, const pp_options *opts, const
 		d.pl_cap = (int) std::min<long long>(8LL * d.stride, 0x7fffff00LL);
 		if((st = dev_alloc(c, &d.pl, (size_t) d.pl_cap)) || (st = dev_alloc(c, &d.pl_n, 2))) return bail(st);
 	}
-	if(hipHostMalloc((void **) &c->h_vslow, 2 * sizeof(int), hipHostMallocDefault) != hipSuccess) c->h_vslow = nullptr;
-	if(!c->h_vslow || hipHostGetDevicePointer((void **) &c->d_vslow_host, c->h_vslow, 0) != hipSuccess ||
-	   !c->d_vslow_host)
-		return bail(fail(PP_ERR_NOMEM, "pinned host flag allocation failed"));
-	c->h_vslow[0] = 0;
-	c->h_vslow[1] = 0;
+	if(!energy_only) {
+		// (only sweeps wait on these words)
+		if(hipHostMalloc((void **) &c->h_vslow, 2 * sizeof(int), hipHostMallocDefault) != hipSuccess) c->h_vslow = nullptr;
+		if(!c->h_vslow || hipHostGetDevicePointer((void **) &c->d_vslow_host, c->h_vslow, 0) != hipSuccess ||
+		   !c->d_vslow_host)
+			return bail(fail(PP_ERR_NOMEM, "pinned host flag allocation failed"));
+		c->h_vslow[0] = 0;
+		c->h_vslow[1] = 0;
+	}
 	// diagnostic switches for the box trials' energy, which must give the
 	// same trajectories: PP_NPT_FULL_TRIAL=1 regroups the particles into the
 	// spare buffer for every trial; PP_NPT_PARTICLE_TRIAL=1 evaluates fast

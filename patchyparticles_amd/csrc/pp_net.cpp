@@ -20,6 +20,7 @@ static_assert(PP_NET_INPUTS == NN_IN && PP_NET_OUTPUTS == NN_OUT && PP_NET_WEIGH
               "the C ABI's network sizes");
 
 pp_status pp_set_error(pp_status s, const char *msg);  // pp_api.cpp
+int pp_device_count();
 
 namespace {
 
@@ -129,8 +130,8 @@ extern "C" {
 pp_status pp_net_create(int device, uint64_t seed, pp_net **out) {
 	if(!out) return nfail(PP_ERR_ARG, "out is NULL");
 	*out = nullptr;
-	int ndev = 0;
-	if(hipGetDeviceCount(&ndev) != hipSuccess || ndev <= 0) return nfail(PP_ERR_HIP, "no HIP device available");
+	const int ndev = pp_device_count();
+	if(ndev <= 0) return nfail(PP_ERR_HIP, "no HIP device available");
 	if(device < 0 || device >= ndev) return nfail(PP_ERR_ARG, "device %d out of range", device);
 	pp_net *n = new pp_net();
 	n->device = device;
