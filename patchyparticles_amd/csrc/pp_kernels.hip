@@ -1159,8 +1159,11 @@ __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int
 			}
 		}
 	F32Filter fl = pg.filter;
-	if(team_any<T>(wild)) fl.eps_d2 = fl.eps_t = F32_ALL;
-	const float margin = pg.margin, is0 = pg.inv_side[0], is1 = pg.inv_side[1], is2 = pg.inv_side[2];
+	float margin = pg.margin;
+	// (the in-cell test too: from about 10^10 on, the roundings of cell_coord
+	// itself pass its margin)
+	if(team_any<T>(wild)) fl.eps_d2 = fl.eps_t = margin = F32_ALL;
+	const float is0 = pg.inv_side[0], is1 = pg.inv_side[1], is2 = pg.inv_side[2];
 	if(CAP == CELL_CAP && wave_far && M > REC_SLOTS) {
 		// the rows' ranges, for the neighbours past the record's list
 		if(lane < 9) {

@@ -1,0 +1,61 @@
+"""Colour passes on states outside the single-precision filter's bounds
+(kf_device.hpp, F32Filter): their decisions are the exact arithmetic's."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def pp():
+    import patchyparticles_amd as pp
+    pp.lib()
+    return pp
+
+
+TAG_TRIAL_A, TAG_SHIFT, TAG_COLOUR = 0, 8, 9
+
+
+def _cell_coord(x, shift, inv_box, n):
+    t = (x - shift) * inv_box
+    t = t - np.floor(t)
+    i = int(t * float(n)) if t == t else 0
+    return min(i, n - 1)
+
+
+def _free_particle(oracle, p, box, n, sweeps, trials, seed, disp_max):
+    """The walk of a single particle: a trial is accepted if it stays in the
+    cell of the sweep's grid (cell_coord, FP64).  Returns its end and the
+    number of accepted trials."""
+    u01 = lambda w: float(w) * 2.0 ** -32
+    key = [seed, 0]
+    p, inv, accepted = [float(v) for v in p], 1.0 / box, 0
+    for sweep in range(sweeps):
+        w = oracle.philox([0, TAG_SHIFT, sweep, 0], key)
+        shift = [u01(w[k]) * (box / n) for k in range(3)]
+        at = [_cell_coord(p[k], shift[k], inv, n) for k in range(3)]
+        colour = (at[0] & 1) << 2 | (at[1] & 1) << 1 | at[2] & 1
+        ctr = np.array([[(at[0] * n + at[1]) * n + at[2], TAG_TRIAL_A | colour << 8 | t << 16, sweep, 0] for t in range(trials)])
+        for w in oracle.philox_n(ctr, np.array([key] * trials)):
+            q = [p[k] + (u01(w[1 + k]) - 0.5) * disp_max for k in range(3)]
+            if all(_cell_coord(q[k], shift[k], inv, n) == at[k] for k in range(3)):
+                p, accepted = q, accepted + 1
+    return np.array(p), accepted
+
+
+@pytest.mark.parametrize("disp_max", [0.3, 1.1])
+@pytest.mark.parametrize("at", [3.0, -5e6, 3e7, 1e11, -1e13, 1e14])
+def test_in_cell_test_at_large_coordinates(pp, oracle, at, disp_max):
+    """One particle at coordinates whose own spacing is up to 1/64: it leaves or
+    stays in its cell as FP64 says, trial by trial, in every team width."""
+    box, n, sweeps, trials, seed = 8.0, 6, 150, 16, 5
+    p = np.array([at, 1.5 + at, 2.25 - at])
+    want, accepted = _free_particle(oracle, p, box, n, sweeps, trials, seed, disp_max)
+    assert 0.2 * sweeps * trials < accepted < sweeps * trials
+    for kw in (dict(threads_per_cell=16, block_size=64), dict(threads_per_cell=32), dict(threads_per_cell=64), dict(launch=3)):
+        with pp.System(p[None], np.eye(3)[None], np.full(3, box), T=0.1, seed=seed, disp_max=disp_max, trials_per_cell=trials,
+                       **kw) as s:
+            assert s.grid()[0] == [n] * 3
+            s.do_ensemble(sweeps)
+            r, _, _ = s.state()
+            assert s.counters()["accepted"][0] == accepted and np.array_equal(r[0], want), kw
