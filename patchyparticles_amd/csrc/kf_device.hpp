@@ -256,6 +256,14 @@ constexpr float F32_BAND_T = 8e-5f;   // times s rc
 constexpr float F32_ALL = 1e28f;      // a band that holds every pair (but not an empty slot's distance)
 constexpr double F32_MAX_POS = 1e7;
 
+// A position or displacement of the filter: finite also where the value is
+// not, or too large (there the exact arithmetic decides), so that no distance
+// is a NaN and none between particles as large as an empty slot's.
+constexpr float F32_POS_LIM = 1e12f;
+__device__ __forceinline__ float f32_pos(double v) {
+	return __builtin_amdgcn_fmed3f((float) v, -F32_POS_LIM, F32_POS_LIM);  // (a NaN: the lower limit)
+}
+
 struct F32Filter {
 	float rc2, c3;        // bond range squared, 3 cosmax^2
 	float eps_d2, eps_t;  // bands

@@ -831,7 +831,10 @@ static_assert(40 * team_lds<SMALL_CAP>() * sizeof(double) <= 160 * 1024, "40 sma
 static_assert(MAX_TEAMS * team_lds<>() * sizeof(double) <= MAX_LDS_BYTES, "a workgroup's teams");
 
 constexpr int MOST_EXP = 1 << 16;  // a trial whose draw accepts every tabulated rise
-constexpr float F32_FAR = 1e15f;   // the position of an empty slot
+constexpr float F32_FAR = 1e15f;   // the position of an empty slot, in no band of any trial's
+static_assert(3.f * (3.f * F32_POS_LIM) * (3.f * F32_POS_LIM) < F32_ALL &&
+                  F32_ALL < (F32_FAR - 2.f * F32_POS_LIM) * (F32_FAR - 2.f * F32_POS_LIM),
+              "the infinite band holds every particle and no empty slot");
 
 // One lane's share of an accepted move, values v = 0..14 of the moving
 // member's record: v < 3 the position, v < 12 O' = O R in the reference's
@@ -1053,9 +1056,9 @@ __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int
 		float *f = ftrial + mt * FT_W;
 #pragma unroll
 		for(int e = 0; e < TR_W; e++) w[e] = tv[1 + e];
-		f[0] = (float) tv[1];
-		f[1] = (float) tv[2];
-		f[2] = (float) tv[3];
+		f[0] = f32_pos(tv[1]);
+		f[1] = f32_pos(tv[2]);
+		f[2] = f32_pos(tv[3]);
 		f[3] = __int_as_float(most < ACC_TAB - 1 ? most : MOST_EXP);
 #pragma unroll
 		for(int e = 0; e < 9; e++) f[4 + e] = (float) tv[4 + e];
@@ -1088,7 +1091,8 @@ __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int
 		q[0] = kf_min_image(p[0] - ce0, pg.box[0], pg.inv_box[0]);
 		q[1] = kf_min_image(p[1] - ce1, pg.box[1], pg.inv_box[1]);
 		q[2] = kf_min_image(p[2] - ce2, pg.box[2], pg.inv_box[2]);
-		wild |= !(__builtin_fmax(__builtin_fabs(p[0]), __builtin_fmax(__builtin_fabs(p[1]), __builtin_fabs(p[2]))) < F32_MAX_POS);
+		// (a sum, which a NaN passes through)
+		wild |= !(__builtin_fabs(p[0]) + __builtin_fabs(p[1]) + __builtin_fabs(p[2]) < F32_MAX_POS);
 	};
 	auto check_o = [&](const float *o) {
 		wild |= !f32_orientation_ok(o);
@@ -1097,9 +1101,9 @@ __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int
 	// pv in single precision, into slot u
 	auto convert = [&](int u, double *rel) {
 		rel3(pv, rel);
-		qx[u] = (float) rel[0];
-		qy[u] = (float) rel[1];
-		qz[u] = (float) rel[2];
+		qx[u] = f32_pos(rel[0]);
+		qy[u] = f32_pos(rel[1]);
+		qz[u] = f32_pos(rel[2]);
 #pragma unroll
 		for(int c = 0; c < 9; c++) qo[u][c] = (float) pv[3 + c];
 		check_o(qo[u]);
@@ -1459,7 +1463,7 @@ __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int
 			if(lane < 15) {
 				own[k * OWN_W + lane] = rv;
 				shadow[k * SH_W + ms.word] =
-				    lane == 0 ? __int_as_float(n_new - (int) __popc(mb)) : (lane <= 2 ? __uint_as_float(mb) : (float) rv);
+				    lane == 0 ? __int_as_float(n_new - (int) __popc(mb)) : (lane <= 2 ? __uint_as_float(mb) : f32_pos(rv));
 			}
 			// the other members' bits for member k
 			if(is_mem && mi != k) {

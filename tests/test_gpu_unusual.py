@@ -1,5 +1,6 @@
 """Colour passes on states outside the single-precision filter's bounds
-(kf_device.hpp, F32Filter): their decisions are the exact arithmetic's."""
+(kf_device.hpp, F32Filter): their decisions are the exact arithmetic's,
+and every read stays inside the particles' arrays."""
 import numpy as np
 import pytest
 
@@ -59,3 +60,39 @@ def test_in_cell_test_at_large_coordinates(pp, oracle, at, disp_max):
             s.do_ensemble(sweeps)
             r, _, _ = s.state()
             assert s.counters()["accepted"][0] == accepted and np.array_equal(r[0], want), kw
+
+
+COOP, DEPS = 2, 3
+
+
+@pytest.mark.parametrize("rho,occupancy", [(0.05, 0.0), (0.3, 0.0), (0.3, 6.0)])
+@pytest.mark.parametrize("trials", [0, 16])
+def test_coordinates_that_are_not_finite(pp, oracle, rho, occupancy, trials):
+    """A particle with a NaN or infinite coordinate has no neighbour: its moves
+    find no overlap and no bond, and the other particles move as without it in
+    reach.  Cells of few and of many neighbours (the occupancies), so that
+    teams have empty slots, full ones and neighbours beyond them; every form
+    of the passes gives the same trajectory."""
+    r, O, box = pp.generate(1500, rho, 21)
+    bad = [3, 40, 41, 333, 1499]
+    r[bad, [0, 1, 2, 0, 1]] = [np.nan, np.inf, -np.inf, np.nan, np.nan]
+    r[333] = np.nan
+    fine = np.setdiff1d(np.arange(len(r)), bad)
+    got = []
+    for kw in (dict(threads_per_cell=32), dict(threads_per_cell=16, block_size=64), dict(threads_per_cell=64),
+               dict(launch=COOP), dict(launch=DEPS), dict(copies=2), dict(copies=2, threads_per_cell=16, block_size=64)):
+        copies = kw.pop("copies", 1)
+        with pp.System.batch([r] * copies, [O] * copies, [box] * copies, [dict(T=0.12)] * copies, seed=9,
+                             cell_occupancy=occupancy, trials_per_cell=trials, **kw) as s:
+            s.do_ensemble(20)
+            bonds, ov, total, any_ov = s.energy(0)
+            rr, OO, _ = s.state(0)
+            c = s.counters(0)
+            assert not any_ov and c["bonds"] == total and not bonds[bad].any(), kw
+            ob, oov, ototal = oracle.energy(rr[fine], OO[fine], box)
+            assert np.array_equal(bonds[fine], ob) and not oov.any() and ototal == total, kw
+            got.append((rr, OO, c["tries"], c["accepted"]))
+    assert not np.isfinite(got[0][0][bad]).all(axis=1).any() and np.isfinite(got[0][0][fine]).all()
+    for x in got[1:]:
+        for a, b in zip(got[0], x):
+            assert np.array_equal(a, b, equal_nan=True)
