@@ -91,7 +91,7 @@ __device__ __forceinline__ bool trial_rebuilds(const Rep &rp) { return rp.trial_
 
 __device__ __forceinline__ void set_pass_geo(Rep &rp, const Grid &G, const double sh[3]) {
 	PassGeo &p = rp.pg;
-	double smax = 0.;
+	double smax = 0., gap = G.box[0];
 	for(int k = 0; k < 3; k++) {
 		p.box[k] = G.box[k];
 		p.inv_box[k] = G.inv_box[k];
@@ -99,10 +99,16 @@ __device__ __forceinline__ void set_pass_geo(Rep &rp, const Grid &G, const doubl
 		p.side[k] = G.box[k] / (double) G.n[k];
 		p.inv_side[k] = (float) ((double) G.n[k] / G.box[k]);
 		smax = fmax(smax, p.side[k]);
+		gap = fmin(gap, G.box[k] - p.side[k]);
 	}
 	p.filter = f32_filter(rp.cosmax, rp.rc2, smax);
-	// (a step longer than a cell could come round the box: the exact test)
-	p.margin = rp.disp_max < smax ? 1e-5f : F32_ALL;
+	p.margin = 1e-5f;
+	// A step of the box less a cell comes round the box into its own cell,
+	// where the filter has the particle a box length away from its neighbours
+	// (shorter ones that leave the cell are rejected by the in-cell test,
+	// whatever their length); an infinite angle makes no rotation.  Everything
+	// is exact then.
+	if(!(0.5 * rp.disp_max < 0.999 * gap) || !(rp.theta_max < 1e300)) p.filter.eps_d2 = p.filter.eps_t = p.margin = F32_ALL;
 	for(int k = 0; k < 3; k++) p.n[k] = G.n[k];
 }
 

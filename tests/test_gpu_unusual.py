@@ -96,3 +96,33 @@ def test_coordinates_that_are_not_finite(pp, oracle, rho, occupancy, trials):
     for x in got[1:]:
         for a, b in zip(got[0], x):
             assert np.array_equal(a, b, equal_nan=True)
+
+
+@pytest.mark.parametrize("disp_max", [0.9, 1.2, 2.5, 6.9, 7.1, 9.3, 40.0])
+def test_steps_longer_than_a_cell_and_round_the_box(pp, oracle, disp_max):
+    """Steps (up to disp_max / 2 per axis) that leave the cell, and from
+    disp_max 6.96 on some that come round the 4-cell box into it: one particle
+    walks as FP64 says, and many never overlap and keep their bonds' count, in
+    every form of the passes."""
+    r, O, box = pp.generate(20, 0.2, 4)
+    sweeps, trials, seed = 400, 16, 11
+    want, accepted = _free_particle(oracle, r[0], float(box[0]), 4, sweeps, trials, seed, disp_max)
+    got = []
+    for kw in (dict(threads_per_cell=16, block_size=64), dict(threads_per_cell=32), dict(threads_per_cell=64), dict(launch=COOP),
+               dict(launch=DEPS)):
+        kw.update(T=0.12, seed=seed, disp_max=disp_max, trials_per_cell=trials)
+        with pp.System(r[:1], O[:1], box, **kw) as s:
+            assert s.grid()[0] == [4] * 3
+            s.do_ensemble(sweeps)
+            assert s.counters()["accepted"][0] == accepted and np.array_equal(s.state()[0][0], want), kw
+        with pp.System(r, O, box, **kw) as s:
+            for _ in range(8):
+                s.do_ensemble(sweeps // 8)
+                rr, OO, _ = s.state()
+                b, ov, total, any_ov = s.energy()
+                ob, oov, ototal = oracle.energy(rr, OO, box, brute=True)
+                assert not any_ov and not oov.any() and np.array_equal(b, ob), kw
+                assert s.counters()["bonds"] == total == ototal, kw
+            got.append((rr, OO, s.counters()["accepted"]))
+    for x in got[1:]:
+        assert all(np.array_equal(a, b) for a, b in zip(got[0], x))
