@@ -126,3 +126,29 @@ def test_steps_longer_than_a_cell_and_round_the_box(pp, oracle, disp_max):
             got.append((rr, OO, s.counters()["accepted"]))
     for x in got[1:]:
         assert all(np.array_equal(a, b) for a, b in zip(got[0], x))
+
+
+@pytest.mark.parametrize("scale", [1.0, 1.015, 1.3])
+@pytest.mark.parametrize("offset", [0, 10 ** 6, 10 ** 9])
+def test_orientations_and_coordinates_past_the_bounds(pp, oracle, scale, offset):
+    """Particles some boxes away from the first (coordinates to 10^10) and
+    matrices whose entries pass 1.01: bonds are the exact arithmetic's, and the
+    team widths agree."""
+    r, O, _ = pp.generate(600, 0.4, 8)
+    box = np.full(3, 11.5)
+    r = r * (11.5 / (600 / 0.4) ** (1 / 3))
+    rng = np.random.default_rng(3)
+    r = r + box * rng.integers(-offset, offset + 1, r.shape)
+    O = O * scale
+    got = []
+    for kw in (dict(threads_per_cell=16, block_size=64), dict(threads_per_cell=32), dict(threads_per_cell=64), dict(launch=DEPS)):
+        with pp.System(r, O, box, T=0.12, seed=2, trials_per_cell=8, **kw) as s:
+            s.do_ensemble(40)
+            rr, OO, _ = s.state()
+            b, ov, total, any_ov = s.energy()
+            ob, oov, ototal = oracle.energy(rr, OO, box)
+            assert not any_ov and not oov.any() and np.array_equal(b, ob), kw
+            assert s.counters()["bonds"] == total == ototal > 0, kw
+            got.append((rr, OO, s.counters()["accepted"]))
+    for x in got[1:]:
+        assert all(np.array_equal(a, b) for a, b in zip(got[0], x))
