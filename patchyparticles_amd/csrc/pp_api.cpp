@@ -625,7 +625,7 @@ pp_status create_impl(int R, const pp_params *prm, const pp_options *opts, const
 	launch_fill_i32((int *) d.done, 0, d.C_total + 1, c->stream);
 	launch_fill_i32(d.ddq, 0, 1, c->stream);
 	launch_fill_i32(d.ovf_n, 0, 8, c->stream);
-	launch_fill_i32(d.rec, 0, 8LL * std::max(d.total_act, 1) * REC_W, c->stream);  // (tag 0: no sweep's)
+	launch_clear_tags(d, c->stream);
 	launch_fill_u64(d.ccheck, 0ull, 2, c->stream);
 	if(d.pl_n) launch_fill_i32(d.pl_n, 0, 2, c->stream);
 	launch_fill_u64(d.ctr, 0ull, (long long) R * NCTR * NSLOT, c->stream);
@@ -725,7 +725,7 @@ pp_status enqueue_sweep(pp_ctx *c) {
 	if(c->trace_len >= 0 && c->trace_len < c->d.trace_cap) tp = c->trace_len++;
 	if(++c->d.rec_tag == 0u) {
 		// (the tags wrap: the old records go)
-		launch_fill_i32(c->d.rec, 0, 8LL * std::max(c->d.total_act, 1) * REC_W, c->stream);
+		launch_clear_tags(c->d, c->stream);
 		c->d.rec_tag = 1u;
 	}
 	launch_rebuild(c->d, REB_SHIFT, sw, tp, c->stream);

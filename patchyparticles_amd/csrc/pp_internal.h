@@ -282,6 +282,8 @@ struct DevState {
 int small_cell_cap();  // members a small-cell pass team stages in LDS
 void launch_fill_i32(int *p, int v, long long n, hipStream_t s);
 void launch_fill_u64(unsigned long long *p, unsigned long long v, long long n, hipStream_t s);
+// mark every cell record as no sweep's
+void launch_clear_tags(const DevState &d, hipStream_t s);
 // regroup slots by cell (mode REB_*); REB_SHIFT draws the grid shift of
 // `sweep` and records the energy trace entry trace_pos (if >= 0)
 void launch_rebuild(const DevState &d, int mode, uint64_t sweep, long long trace_pos, hipStream_t s);

@@ -27,24 +27,37 @@ namespace ppd {
 // ------------------------------------------------------------------------
 // fills
 
-__global__ void k_fill_i32(int *p, int v, long long n) {
-	long long i = (long long) blockIdx.x * blockDim.x + threadIdx.x;
-	if(i < n) p[i] = v;
+// Workgroups of 256 threads for n values, which they take in turn: a launch
+// has fewer than 2^32 threads (10^8 particles have 10^10 record words).
+constexpr long long FILL_BLOCKS = 1 << 20;
+static dim3 fill_grid(long long n) { return dim3((unsigned) std::min((n + 255) / 256, FILL_BLOCKS)); }
+__device__ __forceinline__ long long fill_first() { return (long long) blockIdx.x * 256 + threadIdx.x; }
+__device__ __forceinline__ long long fill_step() { return (long long) gridDim.x * 256; }
+
+__global__ __launch_bounds__(256) void k_fill_i32(int *p, int v, long long n) {
+	for(long long i = fill_first(); i < n; i += fill_step()) p[i] = v;
 }
 
-__global__ void k_fill_u64(unsigned long long *p, unsigned long long v, long long n) {
-	long long i = (long long) blockIdx.x * blockDim.x + threadIdx.x;
-	if(i < n) p[i] = v;
+__global__ __launch_bounds__(256) void k_fill_u64(unsigned long long *p, unsigned long long v, long long n) {
+	for(long long i = fill_first(); i < n; i += fill_step()) p[i] = v;
 }
 
 void launch_fill_i32(int *p, int v, long long n, hipStream_t s) {
-	if(n <= 0) return;
-	hipLaunchKernelGGL(k_fill_i32, dim3((unsigned) ((n + 255) / 256)), dim3(256), 0, s, p, v, n);
+	if(n > 0) hipLaunchKernelGGL(k_fill_i32, fill_grid(n), dim3(256), 0, s, p, v, n);
 }
 
 void launch_fill_u64(unsigned long long *p, unsigned long long v, long long n, hipStream_t s) {
-	if(n <= 0) return;
-	hipLaunchKernelGGL(k_fill_u64, dim3((unsigned) ((n + 255) / 256)), dim3(256), 0, s, p, v, n);
+	if(n > 0) hipLaunchKernelGGL(k_fill_u64, fill_grid(n), dim3(256), 0, s, p, v, n);
+}
+
+// Mark every cell record as no sweep's (tag 0).
+__global__ __launch_bounds__(256) void k_clear_tags(int *rec, long long n) {
+	for(long long i = fill_first(); i < n; i += fill_step()) rec[i * REC_W + REC_TAG] = 0;
+}
+
+void launch_clear_tags(const DevState &d, hipStream_t s) {
+	const long long n = 8LL * std::max(d.total_act, 1);
+	hipLaunchKernelGGL(k_clear_tags, fill_grid(n), dim3(256), 0, s, d.rec, n);
 }
 
 // Zero the energy-kernel rows (C_EBONDS, C_OVL) of every replica.
@@ -710,31 +723,32 @@ void launch_rebuild(const DevState &d, int mode, uint64_t sweep, long long trace
 // the replicas' particles back to back (replica k's from src_off[k]); 12 lanes
 // per slot.
 __global__ __launch_bounds__(256) void k_place(DevState d, int *prep, const int *src_off, const double *r, const double *O) {
-	const long long t = (long long) blockIdx.x * 256 + threadIdx.x;
-	const int j = (int) (t / NCOMP), e = (int) (t % NCOMP);
-	if(j >= d.Ntot) return;
-	int lo = 0, hi = d.R;
-	while(hi - lo > 1) {
-		const int mid = (lo + hi) >> 1;
-		if(d.reps[mid].p_off <= j) lo = mid;
-		else hi = mid;
-	}
-	const Rep &rp = d.reps[lo];
-	const int i = j - rp.p_off;
-	const bool there = i < rp.np;
-	const size_t src = (size_t) src_off[lo] + (there ? i : 0);
-	double v = 0.;
-	if(there) v = e < 3 ? r[3 * src + e] : O[9 * src + e - 3];
-	part(d.f[0], j)[e] = v;
-	if(e == 0) {
-		d.pid[0][j] = d.pid[1][j] = there ? i : -1;
-		prep[j] = lo;
+	const long long n = (long long) d.Ntot * NCOMP;
+	for(long long t = fill_first(); t < n; t += fill_step()) {
+		const int j = (int) (t / NCOMP), e = (int) (t % NCOMP);
+		int lo = 0, hi = d.R;
+		while(hi - lo > 1) {
+			const int mid = (lo + hi) >> 1;
+			if(d.reps[mid].p_off <= j) lo = mid;
+			else hi = mid;
+		}
+		const Rep &rp = d.reps[lo];
+		const int i = j - rp.p_off;
+		const bool there = i < rp.np;
+		const size_t src = (size_t) src_off[lo] + (there ? i : 0);
+		double v = 0.;
+		if(there) v = e < 3 ? r[3 * src + e] : O[9 * src + e - 3];
+		part(d.f[0], j)[e] = v;
+		if(e == 0) {
+			d.pid[0][j] = d.pid[1][j] = there ? i : -1;
+			prep[j] = lo;
+		}
 	}
 }
 
 void launch_place(const DevState &d, int *prep, const int *src_off, const double *r, const double *O, hipStream_t s) {
 	const long long t = (long long) d.Ntot * NCOMP;
-	if(t > 0) hipLaunchKernelGGL(k_place, dim3((unsigned) ((t + 255) / 256)), dim3(256), 0, s, d, prep, src_off, r, O);
+	if(t > 0) hipLaunchKernelGGL(k_place, fill_grid(t), dim3(256), 0, s, d, prep, src_off, r, O);
 }
 
 // ------------------------------------------------------------------------
@@ -761,24 +775,25 @@ __global__ __launch_bounds__(256) void k_index_slots(DevState d, int rep, double
 // with the copies now.
 __global__ __launch_bounds__(256) void k_unpack(DevState d, int rep, double *out) {
 	const Rep &rp = d.reps[rep];
-	const unsigned long long t = blockIdx.x * 256ull + threadIdx.x;
-	const unsigned i = (unsigned) (t / NCOMP), e = (unsigned) (t % NCOMP), n = (unsigned) rp.np;
-	if(i >= n) return;
-	const unsigned j = (unsigned) d.slot[rp.p_off + i];
-	if(j >= n || pick_buf(d.pid, rp.sel)[rp.p_off + j] != (int) i) {
-		out[UNPACK_BAD] = 1. + (double) i;
-		return;
-	}
+	const unsigned n = (unsigned) rp.np;
 	double *r = out + UNPACK_HEAD, *O = r + 3 * (size_t) n;
-	const double v = part((const double *) pick_buf(d.f, rp.sel), rp.p_off + (int) j)[e];
-	if(e < 3) r[3 * (size_t) i + e] = v;
-	else O[9 * (size_t) i + e - 3] = v;
+	for(long long t = fill_first(); t < (long long) n * NCOMP; t += fill_step()) {
+		const unsigned i = (unsigned) (t / NCOMP), e = (unsigned) (t % NCOMP);
+		const unsigned j = (unsigned) d.slot[rp.p_off + i];
+		if(j >= n || pick_buf(d.pid, rp.sel)[rp.p_off + j] != (int) i) {
+			out[UNPACK_BAD] = 1. + (double) i;
+			continue;
+		}
+		const double v = part((const double *) pick_buf(d.f, rp.sel), rp.p_off + (int) j)[e];
+		if(e < 3) r[3 * (size_t) i + e] = v;
+		else O[9 * (size_t) i + e - 3] = v;
+	}
 }
 
 void launch_unpack(const DevState &d, int rep, int np, double *out, hipStream_t s) {
 	const long long t = (long long) np * NCOMP;
 	hipLaunchKernelGGL(k_index_slots, dim3((unsigned) std::max(1, (np + 255) / 256)), dim3(256), 0, s, d, rep, out);
-	if(np > 0) hipLaunchKernelGGL(k_unpack, dim3((unsigned) ((t + 255) / 256)), dim3(256), 0, s, d, rep, out);
+	if(np > 0) hipLaunchKernelGGL(k_unpack, fill_grid(t), dim3(256), 0, s, d, rep, out);
 }
 
 // ------------------------------------------------------------------------

@@ -1,0 +1,75 @@
+"""The library's host side without a GPU: what it allocates and launches, on a
+HIP runtime whose kernels do nothing (tests/host_checks/fake_hip.c)."""
+import os
+import subprocess
+import sys
+
+import numpy as np
+import pytest
+
+from conftest import ROOT
+
+HEAD = """
+import ctypes, os, numpy as np
+fake = ctypes.CDLL(os.environ["FAKE_HIP"])
+fake.fake_hip_log.restype = ctypes.c_char_p
+fake.fake_hip_limit.argtypes = [ctypes.c_size_t]
+import patchyparticles_amd as pp
+def log():
+    return [w.split() for w in fake.fake_hip_log().decode().splitlines()]
+def launches():
+    # (kernel, threads along x)
+    return [(w[1], int(w[2]) * int(w[5])) for w in log() if w[0] == "launch"]
+"""
+
+
+@pytest.fixture(scope="module")
+def run(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("fake") / "fake_hip.so")
+    src = os.path.join(ROOT, "tests", "host_checks", "fake_hip.c")
+    subprocess.run(["gcc", "-O1", "-Wall", "-shared", "-fPIC", src, "-o", so], check=True)
+    env = dict(os.environ, FAKE_HIP=so, PYTHONPATH=ROOT, LD_PRELOAD=" ".join(filter(None, [os.environ.get("LD_PRELOAD"), so])))
+
+    def go(script):
+        res = subprocess.run([sys.executable, "-c", HEAD + script], env=env, cwd=ROOT, capture_output=True, text=True, timeout=120)
+        assert res.returncode == 0, res.stdout + res.stderr
+        return res.stdout
+    return go
+
+
+@pytest.mark.parametrize("replicas,ensemble", [(26, "NPT"), (40, "NVT")])
+def test_systems_of_many_cells_start(run, replicas, ensemble):
+    """Replicas of 138^3 cells (122^3 in NVT), more than 2^26 in all: a launch
+    of a thread per word of the cells' records would pass 2^32 threads, which
+    HIP refuses."""
+    run(f"""
+one = [np.full((1, 3), 1.0)] * {replicas}, [np.eye(3)[None]] * {replicas}, [np.full(3, 137.9)] * {replicas}
+prm = [dict(T=0.11, P=0.02, ensemble=pp.{ensemble}, rescale_factor_max=0.01)] * {replicas}
+with pp.System.batch(*one, prm, trials_per_cell=16) as s:
+    if "{ensemble}" == "NVT":
+        s.do_ensemble(2)
+got = launches()
+assert len(got) > 10 and max(n for _, n in got) < 1 << 32
+cells = [int(w[1]) for w in log() if w[0] == "malloc"]
+assert max(cells) >= 8 * (1 << 23) * 256  # the records
+""")
+
+
+@pytest.mark.gpu
+def test_systems_of_many_cells_move():
+    """The same 40 replicas with a few particles each: replica k moves as in a
+    batch of the first two."""
+    import patchyparticles_amd as pp
+    rng = np.random.default_rng(1)
+    r = np.arange(6)[:, None] * 1.15 + rng.uniform(0, 0.05, (6, 3))
+    O = np.linalg.qr(rng.normal(size=(6, 3, 3)))[0]
+    got = []
+    for copies in (2, 40):
+        with pp.System.batch([r] * copies, [O] * copies, [np.full(3, 137.9)] * copies, [dict(T=0.11)] * copies, seed=3,
+                             trials_per_cell=16) as s:
+            assert s.grid()[0] == [122] * 3
+            s.do_ensemble(3)
+            got.append([s.state(k) + (s.counters(k),) for k in (0, 1)])
+            assert s.counters_all()["tries"][-1, 0] > 0
+    for a, b in zip(*got):
+        assert all(np.array_equal(x, y) for x, y in zip(a[:3], b[:3])) and a[3] == b[3]
