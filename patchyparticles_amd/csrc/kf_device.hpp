@@ -261,7 +261,7 @@ constexpr double F32_MAX_POS = 1e7;
 // is a NaN and none between particles as large as an empty slot's.
 constexpr float F32_POS_LIM = 1e12f;
 __device__ __forceinline__ float f32_pos(double v) {
-	return __builtin_amdgcn_fmed3f((float) v, -F32_POS_LIM, F32_POS_LIM);  // (a NaN: the lower limit)
+	return __builtin_fminf(__builtin_fmaxf((float) v, -F32_POS_LIM), F32_POS_LIM);  // (a NaN: the lower limit)
 }
 
 struct F32Filter {

@@ -1215,7 +1215,9 @@ __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int
 	auto hide = [](int v) { if constexpr(T == 64) return opaque_uniform(v); else return opaque(v); };
 	auto hide_rep = [&]() { if constexpr(ONE) return opaque_uniform(0); else return hide(r); };
 	// The exact arithmetic of one pair: member k moved by trial t (t < 0: as
-	// it stands) and static slot q, or member m >= 0.  OVERLAP, BOND or 0.
+	// it stands) and static slot q, or member m >= 0.  OVERLAP (of a moved
+	// member: where pairs overlap as they stand, which only a refused upload
+	// leaves behind, their bond counts as any other), BOND or 0.
 	enum : unsigned { OVERLAP = 1, BOND = 2, UNSURE = 4 };
 	auto exact_pair = [&](int k, int t, int q, int m) -> unsigned {
 		k = opaque(k);
@@ -1236,7 +1238,7 @@ __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int
 		for(int c = 0; c < 3; c++)
 			w[c] = kf_min_image(other(c) - (t >= 0 ? p[c] + dt[c] : p[c]), hp.pg.box[c], hp.pg.inv_box[c]);
 		const double w2 = w[0] * w[0] + w[1] * w[1] + w[2] * w[2], cosmax = hp.cosmax;
-		if(w2 < 1.) return OVERLAP;
+		if(w2 < (t >= 0 ? 1. : 0.)) return OVERLAP;
 		if(!(w2 < hp.rc2)) return 0u;
 		kf_unit(w[0], w[1], w[2], w2);
 		// (one row, then one patch at a time: this path sets the kernel's
@@ -1446,9 +1448,9 @@ __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int
 				for(int v = first ? 0 : 1; v < 2; v++) {
 					const float gx = fx - (v ? nx : sv[0]), gy = fy - (v ? ny : sv[1]), gz = fz - (v ? nz : sv[2]);
 					const float g2 = v ? gn2 : go2;
-					unsigned bf = g2 < 1.f ? (unsigned) OVERLAP : 0u;
+					unsigned bf = v && g2 < 1.f ? (unsigned) OVERLAP : 0u;
 					if(wild || f32_near(g2, fl)) bf = UNSURE;
-					else if(g2 >= 1.f && g2 < fl.rc2) {
+					else if(bf == 0u && g2 < fl.rc2) {
 						float a0, a1, a2, e0, e1, e2;
 						mul_t(sv + 3, gx, gy, gz, a0, a1, a2);
 						mul_t(tv + 4, a0, a1, a2, e0, e1, e2);
@@ -1481,10 +1483,11 @@ __device__ __forceinline__ void pass_cell(const DevState &d, uint64_t sweep, int
 			// the new state, one value per lane, exact and single precision;
 			// lanes 0 to 2 write the new static count and member bits
 			const double rv = ms.dot ? o0 * r0 + o1 * r1 + o2 * r2 : o0 + r0;
+			const float rf = f32_pos(rv);
 			if(lane < 15) {
 				own[k * OWN_W + lane] = rv;
 				shadow[k * SH_W + ms.word] =
-				    lane == 0 ? __int_as_float(n_new - (int) __popc(mb)) : (lane <= 2 ? __uint_as_float(mb) : f32_pos(rv));
+				    lane == 0 ? __int_as_float(n_new - (int) __popc(mb)) : (lane <= 2 ? __uint_as_float(mb) : rf);
 			}
 			// the other members' bits for member k
 			if(is_mem && mi != k) {

@@ -152,3 +152,25 @@ def test_orientations_and_coordinates_past_the_bounds(pp, oracle, scale, offset)
             got.append((rr, OO, s.counters()["accepted"]))
     for x in got[1:]:
         assert all(np.array_equal(a, b) for a, b in zip(got[0], x))
+
+
+@pytest.mark.parametrize("trials", [0, 8])
+@pytest.mark.parametrize("occupancy", [0.0, 6.0])
+def test_overlaps_left_by_a_refused_upload(pp, occupancy, trials):
+    """A refused upload leaves its particles: the passes then move them apart,
+    and a bond that an overlapping pair has at the present position counts
+    wherever the pair is found, in a lane's slots or beyond them (occupancy 6:
+    more neighbours than any team's slots)."""
+    r, O, box = pp.generate(1500, 0.5, 6)
+    O[:] = O[0]
+    got = []
+    for kw in (dict(threads_per_cell=16, block_size=64), dict(threads_per_cell=32), dict(threads_per_cell=64), dict(launch=DEPS)):
+        with pp.System(r, O, box, T=0.12, seed=2, cell_occupancy=occupancy, trials_per_cell=trials, kf_cosmax=0.5, **kw) as s:
+            with pytest.raises(pp.PPError) as e:
+                s.upload(0, r * 0.97, O, box * 0.97)
+            assert e.value.status == 3  # PP_ERR_OVERLAP
+            s.do_ensemble(30)
+            got.append(s.state() + (s.counters()["accepted"],))
+    assert got[0][3][0] > 10000
+    for x in got[1:]:
+        assert all(np.array_equal(a, b) for a, b in zip(got[0], x))
