@@ -625,7 +625,7 @@ pp_status create_impl(int R, const pp_params *prm, const pp_options *opts, const
 	launch_fill_i32((int *) d.done, 0, d.C_total + 1, c->stream);
 	launch_fill_i32(d.ddq, 0, 1, c->stream);
 	launch_fill_i32(d.ovf_n, 0, 8, c->stream);
-	launch_clear_tags(d, c->stream);
+	if(!energy_only) launch_clear_tags(d, c->stream);  // (only sweeps read the records)
 	launch_fill_u64(d.ccheck, 0ull, 2, c->stream);
 	if(d.pl_n) launch_fill_i32(d.pl_n, 0, 2, c->stream);
 	launch_fill_u64(d.ctr, 0ull, (long long) R * NCTR * NSLOT, c->stream);

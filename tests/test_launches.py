@@ -55,6 +55,18 @@ assert max(cells) >= 8 * (1 << 23) * 256  # the records
 """)
 
 
+def test_snapshot_clears_no_records(run):
+    """A snapshot's context never sweeps: of what creation clears, none is as
+    large as the records (64 words a cell; here 32 x 32 x 32 cells)."""
+    run("""
+rng = np.random.default_rng(1)
+r = rng.uniform(0, 36.0, (2000, 3))
+pp.energy_snapshot(r, np.broadcast_to(np.eye(3), (2000, 3, 3)), np.full(3, 36.0))
+cleared = [n for k, n in launches() if "fill" in k or "clear" in k]
+assert cleared and sum(cleared) < 2 * 32 ** 3 + 8192, cleared  # (two tables of a word a cell)
+""")
+
+
 @pytest.mark.gpu
 def test_systems_of_many_cells_move():
     """The same 40 replicas with a few particles each: replica k moves as in a
