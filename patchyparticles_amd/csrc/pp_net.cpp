@@ -79,6 +79,23 @@ pp_status push(pp_net *n, const std::vector<float> &w, const std::vector<float> 
 	return PP_OK;
 }
 
+// The pinned results of a loss_grad call, for as many rows as the scratch: made
+// by the first such call (forward and training never read them).
+pp_status reserve_out(pp_net *n) {
+	if(n->h_cap >= n->cap) return PP_OK;
+	if(n->h_out) (void) hipHostFree(n->h_out);
+	n->h_out = n->d_h_out = nullptr;
+	n->h_cap = 0;
+	if(hipHostMalloc((void **) &n->h_out, sizeof(float) * (NN_W + NN_B + (size_t) n->cap), hipHostMallocMapped) != hipSuccess) {
+		n->h_out = nullptr;
+		return nfail(PP_ERR_NOMEM, "pinned gradient buffer");
+	}
+	if(hipHostGetDevicePointer((void **) &n->d_h_out, n->h_out, 0) != hipSuccess)
+		return nfail(PP_ERR_HIP, "device address of the gradient buffer");
+	n->h_cap = n->cap;
+	return PP_OK;
+}
+
 }  // namespace
 
 pp_net::~pp_net() {
@@ -105,8 +122,6 @@ int ppd::net_reserve(pp_net *n, int m) {
 	n->x = nullptr;
 	n->xh = n->y = n->target = nullptr;
 	n->q = NetScratch{};
-	if(n->h_out) (void) hipHostFree(n->h_out);
-	n->h_out = n->d_h_out = nullptr;
 	n->cap = 0;
 	const size_t r = (size_t) need;
 	pp_status st;
@@ -115,12 +130,6 @@ int ppd::net_reserve(pp_net *n, int m) {
 	   (st = nalloc(n, &n->q.at, r * (NN_IN_PAD + 3 * NN_H))) || (st = nalloc(n, &n->q.zt, r * NN_B)) ||
 	   (st = nalloc(n, &n->q.part, (size_t) net_grad_slices(need) * (NN_W + NN_B))) || (st = nalloc(n, &n->q.loss, r)))
 		return st;
-	if(hipHostMalloc((void **) &n->h_out, sizeof(float) * (NN_W + NN_B + r), hipHostMallocMapped) != hipSuccess) {
-		n->h_out = nullptr;
-		return nfail(PP_ERR_NOMEM, "pinned gradient buffer");
-	}
-	if(hipHostGetDevicePointer((void **) &n->d_h_out, n->h_out, 0) != hipSuccess)
-		return nfail(PP_ERR_HIP, "device address of the gradient buffer");
 	n->cap = need;
 	return PP_OK;
 }
@@ -212,7 +221,7 @@ pp_status pp_net_loss_grad(pp_net *n, int m, const float *x, const float *target
 	if(!n || m <= 0 || !x || !target) return nfail(PP_ERR_ARG, "bad arguments");
 	NCHECK(hipSetDevice(n->device));
 	pp_status st;
-	if((st = (pp_status) net_reserve(n, m)) != PP_OK) return st;
+	if((st = (pp_status) net_reserve(n, m)) || (st = reserve_out(n))) return st;
 	NCHECK(hipMemcpy(n->xh, x, sizeof(float) * NN_IN * (size_t) m, hipMemcpyHostToDevice));
 	NCHECK(hipMemcpy(n->target, target, sizeof(float) * 6 * (size_t) m, hipMemcpyHostToDevice));
 	// the kernels write their results to the pinned buffer: three copies to

@@ -18,6 +18,7 @@ struct pp_net {
 	// pinned: the gradients (NN_W + NN_B) and the rows' losses of a loss_grad
 	// call, which its kernels write straight into host memory
 	float *h_out = nullptr, *d_h_out = nullptr;  // host and device address
+	int h_cap = 0;                               // rows
 	std::vector<void *> allocs;
 	~pp_net();
 };

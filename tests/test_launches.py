@@ -67,6 +67,29 @@ assert cleared and sum(cleared) < 2 * 32 ** 3 + 8192, cleared  # (two tables of 
 """)
 
 
+def test_only_loss_grad_pins_its_results(run):
+    """Pinning host memory is dear: a network that is evaluated or trained pins
+    none, the first loss_grad call its gradients and losses, later ones of no
+    more rows nothing."""
+    run("""
+r, O, box = pp.generate(500, 0.1, 1)
+x, t = np.zeros((100, 84), np.float32), np.zeros((100, 6), np.float32)
+with pp.System(r, O, box, T=0.1) as s, pp.ProposalNet(seed=1) as net:
+    pins = lambda: [int(w[1]) for w in log() if w[0] == "hostmalloc"]
+    fake.fake_hip_clear()
+    net.forward(x)
+    s.train(net, steps=2, batch=1000)
+    assert pins() == []
+    net.loss_grad(x, t)
+    assert pins() == [4 * (49152 + 416 + 1024)]
+    net.forward(np.zeros((1024, 84), np.float32))
+    net.loss_grad(np.zeros((1024, 84), np.float32), np.zeros((1024, 6), np.float32))
+    assert len(pins()) == 1
+    net.loss_grad(np.zeros((1025, 84), np.float32), np.zeros((1025, 6), np.float32))
+    assert pins()[1:] == [4 * (49152 + 416 + 1056)]
+""")
+
+
 @pytest.mark.gpu
 def test_systems_of_many_cells_move():
     """The same 40 replicas with a few particles each: replica k moves as in a
