@@ -984,21 +984,26 @@ pp_status pp_check_energy(pp_ctx *c, double *energy_per_rep) {
 // 681 us); this one at 18 and 27 GB/s (44 and 461 us).
 constexpr size_t DL_CHUNK = 1 << 20;
 
+// The buffers of download_fixed, made by the first download; false if there is
+// no memory for them.
+static bool download_buffers(pp_ctx *c) {
+	if(c->dl_cap) return true;
+	// (each piece is kept as it is made; dl_cap is set once all exist)
+	int cap = 1;
+	for(int k = 0; k < c->R; k++) cap = std::max(cap, c->reps[k].np);
+	bool ok = c->dl_dev || dev_alloc(c, &c->dl_dev, UNPACK_HEAD + (size_t) NCOMP * cap) == PP_OK;
+	for(hipEvent_t &e : c->dl_ev) ok = ok && (e || hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess);
+	if(ok && !c->dl_host && hipHostMalloc((void **) &c->dl_host, 2 * DL_CHUNK, hipHostMallocDefault) != hipSuccess) {
+		c->dl_host = nullptr;
+		ok = false;
+	}
+	if(ok) c->dl_cap = cap;
+	else (void) hipGetLastError();  // (a later call would report it as its own)
+	return ok;
+}
+
 static pp_status download_fixed(pp_ctx *c, int rep, double *r, double *O, double box[3]) {
 	const int n = c->reps[rep].np;
-	if(!c->dl_cap) {
-		// (each piece is kept as it is made; dl_cap is set once all exist)
-		int cap = 1;
-		for(int k = 0; k < c->R; k++) cap = std::max(cap, c->reps[k].np);
-		if(!c->dl_dev) TRY(dev_alloc(c, &c->dl_dev, UNPACK_HEAD + (size_t) NCOMP * cap));
-		for(hipEvent_t &e : c->dl_ev)
-			if(!e) HIPCHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-		if(!c->dl_host && hipHostMalloc((void **) &c->dl_host, 2 * DL_CHUNK, hipHostMallocDefault) != hipSuccess) {
-			c->dl_host = nullptr;
-			return fail(PP_ERR_NOMEM, "pinned download buffer");
-		}
-		c->dl_cap = cap;
-	}
 	launch_unpack(c->d, rep, r || O ? n : 0, c->dl_dev, c->stream);
 	const size_t head = sizeof(double) * UNPACK_HEAD, rb = sizeof(double) * 3 * (size_t) n, ob = 3 * rb;
 	const size_t total = r || O ? head + rb + ob : head, chunks = (total + DL_CHUNK - 1) / DL_CHUNK;
@@ -1038,9 +1043,10 @@ pp_status pp_download(pp_ctx *c, int rep, double *r, double *O, double box[3]) {
 	if(!c) return fail(PP_ERR_ARG, "ctx is NULL");
 	if(rep < 0 || rep >= c->R) return fail(PP_ERR_ARG, "replica %d out of range", rep);
 	HIPCHECK(hipSetDevice(c->device));
-	if(!c->reps[rep].gc) return download_fixed(c, rep, r, O, box);
-	// a grand-canonical replica: its live particles first (a rebuild)
-	rebuild_now(c);
+	if(!c->reps[rep].gc && download_buffers(c)) return download_fixed(c, rep, r, O, box);
+	// ordered on the host: where the device has no memory left for a copy, and
+	// a grand-canonical replica, its live particles first (a rebuild)
+	if(c->reps[rep].gc) rebuild_now(c);
 	HIPCHECK(hipStreamSynchronize(c->stream));
 	TRY(pull_reps(c));
 	const Rep &rp = c->reps[rep];
@@ -1052,7 +1058,7 @@ pp_status pp_download(pp_ctx *c, int rep, double *r, double *O, double box[3]) {
 		                   hipMemcpyDeviceToHost));
 	TRY(slot_indices(c, rep, hp, sorted));
 	for(int j = 0; j < n; j++) {
-		const int i = rank_of(sorted, hp[j]);
+		const size_t i = (size_t) rank_of(sorted, hp[j]);
 		if(r)
 			for(int a = 0; a < 3; a++) r[3 * i + a] = h[(size_t) NCOMP * j + a];
 		if(O)

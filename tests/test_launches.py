@@ -90,6 +90,24 @@ with pp.System(r, O, box, T=0.1) as s, pp.ProposalNet(seed=1) as net:
 """)
 
 
+def test_download_without_device_memory(run):
+    """A context that leaves no device memory is downloaded all the same, and
+    the allocation that failed is no later call's error.  (One particle: its
+    index is 0, as the memory that no kernel has written.)"""
+    run("""
+with pp.System(np.ones((1, 3)), np.eye(3)[None], np.full(3, 9.0), T=0.1) as s:
+    fake.fake_hip_limit(0)
+    for _ in range(2):
+        r, O, box = s.state()
+        assert box.tolist() == [9.0] * 3
+        s.do_ensemble(1)
+    fake.fake_hip_limit(1 << 30)
+    fake.fake_hip_clear()
+    s.state()
+    assert "k_unpack" in fake.fake_hip_log().decode()
+""")
+
+
 @pytest.mark.gpu
 def test_systems_of_many_cells_move():
     """The same 40 replicas with a few particles each: replica k moves as in a
