@@ -317,7 +317,7 @@ __device__ __forceinline__ uint32_t make_trial(const DevState &d, const Rep &rp,
 struct Trial {
 	double px, py, pz, nx, ny, nz;
 	double Lx, Ly, Lz, iLx, iLy, iLz, rc2, cosmax;
-	double c2;  // cosmax^2 for the filtered angular tests, -1: exact tests only
+	double c2;  // cosmax^2 for the filter's check (a trial's own tests are exact)
 };
 
 // Minimum-image separation of q from the trial's new position, and its
@@ -369,39 +369,69 @@ __device__ __forceinline__ void bonds_old_new_exact(const Trial &t, const double
 	}
 }
 
-// Bonds of neighbour q with the new position only: the filtered decision
-// (a pair inside the filter band sets `band`) and the reference's arithmetic
-// (MC.c:242-262), for the separation (wx, wy, wz) = sep_new(q) and its square
-// w2.
+// The bond decision of a pair closer than the bond range (MC_would_interact's
+// angular part, MC.c:248-262), seen from p with separation (dx, dy, dz) towards
+// q, its square d2 and p's patches P.  Seen from q the decision is the same
+// (every step is the exact negation of p's).  q's orientation is read only
+// when p's patches pass.
+//
+// The filter's answer, for c2 = cosmax^2: KF_YES, KF_NO, or KF_UNSURE inside
+// its band.
+template <class LoadO>
+__device__ __forceinline__ unsigned pair_filter(double dx, double dy, double dz, double d2, const double *P, double c2,
+                                                LoadO load_q) {
+	const KfBand bd = kf_band(c2, d2);
+	const unsigned fp = kf_fast_p(dx, dy, dz, P, bd);
+	unsigned yes = 0u, unsure = fp >> 1;
+	if(fp & 1u) {
+		double Oq[9];
+		load_q(Oq);
+		const unsigned fq = kf_fast_q1(dx, dy, dz, kf_band_q(bd), Oq);
+		unsure |= fq >> 1;
+		yes = fq & 1u;
+	}
+	return unsure ? (unsigned) KF_UNSURE : yes;
+}
+
+// The reference's arithmetic.
+template <class LoadO>
+__device__ __forceinline__ bool pair_exact(double dx, double dy, double dz, double d2, const double *P, double cosmax,
+                                           LoadO load_q) {
+	kf_unit(dx, dy, dz, d2);
+	if(!kf_any_p(dx, dy, dz, P, cosmax)) return false;
+	double Oq[9];
+	load_q(Oq);
+	return kf_any_q(dx, dy, dz, Oq, cosmax);
+}
+
+// The filter, and the reference's arithmetic where it is unsure or not in use
+// (c2 < 0).
+template <class LoadO>
+__device__ __forceinline__ bool pair_bonded(double dx, double dy, double dz, double d2, const double *P, double c2,
+                                            double cosmax, LoadO load_q) {
+	const unsigned f = c2 < 0. ? (unsigned) KF_UNSURE : pair_filter(dx, dy, dz, d2, P, c2, load_q);
+	if(f == KF_UNSURE) return pair_exact(dx, dy, dz, d2, P, cosmax, load_q);
+	return f == KF_YES;
+}
+
+// Bonds of neighbour q with a trial's new position by either half of
+// pair_bonded, as the check of the filter at its thresholds asks for them:
+// the filter's (a pair inside its band sets `band`) for the separation (wx, wy,
+// wz) = sep_new(q) and its square w2, and the reference's.
 template <class LoadO>
 __device__ __forceinline__ void bonds_new_sep(const Trial &t, const double *Pn, double wx, double wy, double wz,
                                               double w2, LoadO load_o, int &bn, bool &band) {
-	const KfBand bd = kf_band(t.c2, w2);
-	const unsigned fn = w2 < t.rc2 ? kf_fast_p(wx, wy, wz, Pn, bd) : 0u;
-	unsigned unsure = (fn >> 1) & 1u;
-	if(fn & 1u) {
-		double Oq[9];
-		load_o(Oq);
-		const unsigned qn = kf_fast_q1(wx, wy, wz, kf_band_q(bd), Oq);
-		unsure |= (qn >> 1) & 1u;
-		bn += (int) (qn & 1u);
-	}
-	band |= unsure != 0u;
+	const unsigned f = w2 < t.rc2 ? pair_filter(wx, wy, wz, w2, Pn, t.c2, load_o) : (unsigned) KF_NO;
+	bn += f == KF_YES;
+	band |= f == KF_UNSURE;
 }
 
 template <class LoadO>
 __device__ __forceinline__ void bonds_new_exact(const Trial &t, const double *Pn, double qx, double qy, double qz,
                                                 LoadO load_o, int &bn) {
-	double wx = kf_min_image(qx - t.nx, t.Lx, t.iLx);
-	double wy = kf_min_image(qy - t.ny, t.Ly, t.iLy);
-	double wz = kf_min_image(qz - t.nz, t.Lz, t.iLz);
-	double w2 = wx * wx + wy * wy + wz * wz;
-	if(!(w2 < t.rc2)) return;
-	kf_unit(wx, wy, wz, w2);
-	if(!kf_any_p(wx, wy, wz, Pn, t.cosmax)) return;
-	double Oq[9];
-	load_o(Oq);
-	bn += kf_any_q(wx, wy, wz, Oq, t.cosmax);
+	double wx, wy, wz;
+	const double w2 = sep_new(t, qx, qy, qz, wx, wy, wz);
+	if(w2 < t.rc2) bn += pair_exact(wx, wy, wz, w2, Pn, t.cosmax, load_o);
 }
 
 }  // namespace ppd

@@ -1754,41 +1754,6 @@ struct NbLayout {
 // whatever the bonds are: the replica's later teams stop at once.
 // Workgroups reach the XCDs round-robin: each XCD takes a contiguous range of
 // slots (neighbouring cells share its L2).
-// The bond decision of a pair of particles closer than the bond range but
-// not overlapping (MC_would_interact's angular part, MC.c:248-262), seen from
-// p with separation (dx, dy, dz) towards q and p's patches P: the filtered
-// test, and the reference's arithmetic only inside the filter's band or
-// without the filter.  Seen from q the decision is the same (every step is
-// the exact negation of p's).
-template <class LoadO>
-__device__ __forceinline__ bool pair_bonded(double dx, double dy, double dz, double d2, const double *P, double c2,
-                                            double cosmax, LoadO load_q) {
-	bool unsure = c2 < 0.;
-	bool bonded = false;
-	if(!unsure) {
-		const KfBand bd = kf_band(c2, d2);
-		const unsigned fp = kf_fast_p(dx, dy, dz, P, bd);
-		unsure = (fp >> 1) != 0u;
-		if(fp & 1u) {
-			double Oq[9];
-			load_q(Oq);
-			const unsigned fq = kf_fast_q1(dx, dy, dz, kf_band_q(bd), Oq);
-			unsure |= (fq >> 1) != 0u;
-			if(!unsure) bonded = (fq & 1u) != 0u;
-		}
-	}
-	if(unsure) {
-		kf_unit(dx, dy, dz, d2);
-		bonded = false;
-		if(kf_any_p(dx, dy, dz, P, cosmax)) {
-			double Oq[9];
-			load_q(Oq);
-			bonded = kf_any_q(dx, dy, dz, Oq, cosmax);
-		}
-	}
-	return bonded;
-}
-
 template <int T>
 __global__ __launch_bounds__(256) void k_energy(DevState d, int trial, int per_particle) {
 	using NB = NbLayout<T>;

@@ -1040,7 +1040,6 @@ __global__ __launch_bounds__(64 * LP_WAVES, 2) void k_learn_pass(DevState d, Net
 	t.iLz = iL[2];
 	t.rc2 = rp.rc2;
 	t.cosmax = rp.cosmax;
-	t.c2 = -1.;
 	double Po[4][3], Pn[4][3];
 	kf_patches(O, Po);
 	kf_patches(On, Pn);
