@@ -532,7 +532,7 @@ def main():
             "workload": f"plain NVT checkerboard rototranslation, N={N}, rho={RHO}, T={T}, KF_delta={DELTA}, "
                         f"KF_cosmax={COSMAX}, Disp_max={DISP}, Theta_max={THETA}, FP64",
             "grid": nside, "cell_side": round(side[0], 5),
-            "threads_per_cell": args.tpc or 32, "trials_per_cell": args.trials_per_cell,
+            "threads_per_cell": args.tpc or "chosen by size", "trials_per_cell": args.trials_per_cell,
             "step": "rebuild on a randomly shifted grid + 8 colour passes",
             "equilibration_steps": args.equil,
             "attempts": attempts, "attempts_per_step": round(attempts / args.steps, 1),

@@ -106,7 +106,9 @@ typedef struct pp_options {
 	int threads_per_cell;    /* lanes that work on one sweep cell: 16, 32 or 64 (0: 32, or 16 on systems
 	                            of many cells); 16 needs
 	                            at most 16 particles per sweep cell and the per-pass launch form */
-	int block_size;          /* threads per workgroup: 64/128/256 (0: 64) */
+	int block_size;          /* threads per workgroup, a multiple of 64 up to 256, at most 6 cells per
+	                            workgroup (0: 64 with a launch per pass; in the other launch forms
+	                            the largest of 256 and 128 that fits) */
 	double cell_occupancy;   /* target particles per sweep cell; 0: smallest cells (side >= 1+delta) */
 	int device;              /* HIP device ordinal */
 	int launch;              /* PP_LAUNCH_*: how the 8 colour passes of a sweep are launched */

@@ -248,9 +248,11 @@ __device__ __forceinline__ unsigned kf_fast_q1(double dx, double dy, double dz, 
 //   e = O'^T d by two 3 x 3 products, g = +-e0 +-e1 +-e2 <= 5.2e-6 s, and
 //     g|g| - 3 cosmax^2 d^2 <= 2.2e-5 s rc (entries of O at most 1.01)
 // The bands hold these errors three times over.  Where an orientation entry
-// is larger or a coordinate beyond F32_MAX_POS (whose FP64 spacing would
-// matter), and below KF_FILTER_MIN_COS, the bands are infinite: every pair
-// within reach takes the exact arithmetic.
+// is larger or a particle's coordinates add up to F32_MAX_POS (their FP64
+// spacing would matter) or are not finite, and where a step may come round the
+// box into its own cell (set_pass_geo), the bands and the margin of the in-cell
+// test are infinite: the team's pairs and its in-cell tests take the exact
+// arithmetic.  Below KF_FILTER_MIN_COS the pairs do.
 constexpr float F32_BAND_D2 = 4e-6f;  // times s rc
 constexpr float F32_BAND_T = 8e-5f;   // times s rc
 constexpr float F32_ALL = 1e28f;      // a band that holds every pair (but not an empty slot's distance)

@@ -108,8 +108,8 @@ pp_status na_scratch(int dev, unsigned char **out) {
 }
 
 // Particles from the caller's layout (r[3j + k], O[9j + k], copied as they
-// are into the second particle buffer) into the kernels' SoA layout in the
-// first buffer, slot j = particle j of replica 0.
+// are into the second particle buffer) into the first buffer, the 12 components
+// of a slot together, slot j = particle j of replica 0.
 __global__ void k_na_stage(const double *aos, int n, double *f0, int *pid0, int *prep) {
 	const int j = blockIdx.x * blockDim.x + threadIdx.x;
 	if(j >= n) return;
@@ -225,7 +225,7 @@ extern "C" pp_status pp_energy_snapshot_noalloc(int n, const double *r, const do
 	d.out_bonds = (int32_t *) at(P_BONDS);
 	d.out_ovl = (uint8_t *) at(P_OVL);
 
-	// the caller's arrays into the second buffer as they are, then the SoA
+	// the caller's arrays into the second buffer as they are, then the slots'
 	// layout into the first; the table of the one replica; zeroed counts and
 	// error word (the array holds the previous call's values)
 	hipStream_t s = nullptr;
