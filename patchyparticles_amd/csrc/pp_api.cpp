@@ -27,14 +27,21 @@ namespace {
 
 thread_local std::string g_err;
 
+// An allocation that failed is this call's error: the runtime keeps it until
+// asked, and a later call would report it as its own (check_err).
+pp_status set_error(pp_status s, const char *msg) {
+	g_err = msg;
+	if(s == PP_ERR_NOMEM) (void) hipGetLastError();
+	return s;
+}
+
 pp_status fail(pp_status s, const char *fmt, ...) {
 	char buf[512];
 	va_list ap;
 	va_start(ap, fmt);
 	vsnprintf(buf, sizeof buf, fmt, ap);
 	va_end(ap);
-	g_err = buf;
-	return s;
+	return set_error(s, buf);
 }
 
 #define HIPCHECK(call)                                                                                    \
@@ -69,10 +76,7 @@ int pp_device_count() {
 }
 
 // the error message of the calling thread, set by the other translation units
-pp_status pp_set_error(pp_status s, const char *msg) {
-	g_err = msg;
-	return s;
-}
+pp_status pp_set_error(pp_status s, const char *msg) { return set_error(s, msg); }
 
 struct pp_ctx {
 	int device = 0;

@@ -108,6 +108,25 @@ with pp.System(np.ones((1, 3)), np.eye(3)[None], np.full(3, 9.0), T=0.1) as s:
 """)
 
 
+def test_a_failed_allocation_is_no_later_call_s_error(run):
+    run("""
+r, O, box = pp.generate(2000, 0.1, 1)
+x = np.zeros((4000, 84), np.float32)
+with pp.ProposalNet(seed=1) as net:
+    for refused in (lambda: pp.System(r, O, box, T=0.1), lambda: net.forward(np.zeros((40000, 84), np.float32))):
+        fake.fake_hip_limit(1 << 16)
+        try:
+            refused()
+            assert False
+        except pp.PPError as e:
+            assert e.status == 7, e  # PP_ERR_NOMEM
+        fake.fake_hip_limit(1 << 30)
+        with pp.System(r, O, box, T=0.1) as s:
+            s.do_ensemble(1)
+        assert net.forward(x).shape == (4000, 26)
+""")
+
+
 @pytest.mark.gpu
 def test_systems_of_many_cells_move():
     """The same 40 replicas with a few particles each: replica k moves as in a
